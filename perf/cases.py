@@ -294,3 +294,92 @@ def tolerance(case):
     """16-bit results: a rounding of the weight, where a product takes them rounded, and one of the result. 32-bit ones: the
     order of sums. Experts, orders and packed codes are whole numbers that do not depend on either."""
     return dict(rel={"bf16": 1e-2, "f16": 2e-3, "f32": 1e-5}[case["dtype"]])
+
+
+class Exact:
+    """The same inputs in plain torch, in 64 bits."""
+
+    def __init__(self, case, make):
+        self.bits, self.group = case["bits"], case["group"]
+        self.at = {t.data_ptr(): t for t in make.keep}
+
+    def value(self, address, *shape):
+        return self.at[address].double().reshape(shape or (-1,))
+
+    def rows(self, matrix, k, lo, hi):
+        """Rows lo..hi of a matrix in the packed format, k columns."""
+        w, s, b = (self.at[p] for p in matrix)
+        words = w.reshape(-1, k * self.bits // 32)[lo:hi].reshape(-1, self.bits).long() & 0xFFFFFFFF
+        codes = torch.empty(words.shape[0], 32, dtype=torch.float64, device=w.device)
+        for i in range(32):  # 32 codes of any width are a whole number of words
+            at, shift = divmod(i * self.bits, 32)
+            c = words[:, at] >> shift
+            if shift + self.bits > 32:
+                c = c | words[:, at + 1] << (32 - shift)
+            codes[:, i] = (c & ((1 << self.bits) - 1)).double()
+        s, b = (t.reshape(-1, k // self.group)[lo:hi].double().reshape(-1, 1) for t in (s, b))
+        return (codes.reshape(-1, self.group) * s + b).reshape(hi - lo, k)
+
+    def product(self, matrix, x, n, first=0):
+        """x [m, k] times the transpose of the matrix's n rows from `first` on."""
+        step = max(1, (1 << 24) // x.shape[1])
+        return torch.cat([x @ self.rows(matrix, x.shape[1], first + lo, first + min(n, lo + step)).T for lo in range(0, n, step)], 1)
+
+    def rms_norm(self, x, weight):
+        return x * torch.rsqrt((x * x).mean(-1, keepdim=True) + float(torch.tensor(1e-5, dtype=torch.float32))) * weight
+
+
+def exact(case, seed):
+    """What `run` returns for these inputs in 64 bits; None where it returns whole numbers."""
+    c, s = case, prepare(case, seed)
+    e = Exact(c, s["make"])
+    kind = c["kind"]
+    if kind == "delta":
+        x = e.value(s["x"], 1, -1)
+        z = e.value(s["z"], c["hv"], -1)
+        inner = e.rms_norm(e.value(s["y"], c["hv"], -1), e.value(s["norm"])) * z * torch.sigmoid(z)
+        return [e.product(m, x, n)[0] for m, n in zip(zip(s["ws"], s["ss"], s["bs"]), s["n"])] + [e.product(s["o"], inner.reshape(1, -1), c["hidden"])[0]]
+    if kind in ("decode", "prefill"):
+        q, kv, hidden, inter, got = c["q"], c["kv"], c["hidden"], c["inter"], []
+        for at in s["layers"]:
+            x, h, attn, act = (e.value(at[name], c["rows"], -1) for name in ("x", "h", "attn", "act"))
+            got += [e.product(at["o"], attn, hidden), e.product(at["down"], act, hidden)]
+            if _fused(c):
+                got += [e.product(at["qkv"], e.rms_norm(x, e.value(at["norm1"])), q + 2 * kv), e.product(at["gate_up"], e.rms_norm(h, e.value(at["norm2"])), 2 * inter)]
+            else:
+                got += [e.product(m, x, n) for m, n in zip(zip(*at["qkv"]), (q, kv, kv))] + [e.product(m, h, inter) for m in zip(*at["gate_up"])]
+        return got
+    if kind == "moe":
+        tokens, hidden, inter, experts, top = (c[k] for k in ("tokens", "hidden", "inter", "experts", "top"))
+        logits = e.value(s["logits"], tokens, experts)
+        ids = torch.sort(logits, dim=1, descending=True, stable=True)[1][:, :top]  # of equal ones the first
+        weights = torch.softmax(logits.gather(1, ids), 1)
+        order = torch.sort(ids.reshape(-1), stable=True)[1] if not _one_token(c) else torch.arange(top, device=ids.device)
+        chosen = ids.reshape(-1)[order].tolist()
+        rows_in, act = e.value(s["x"], tokens, hidden)[order // top], e.value(s["act"], tokens * top, inter)
+        got = dict(ids=None, weights=weights, rows_in=rows_in)
+
+        def through(matrix, x, n):
+            out = torch.empty(x.shape[0], n, dtype=x.dtype, device=x.device)
+            for expert in sorted(set(chosen)):
+                at = torch.tensor([p for p, i in enumerate(chosen) if i == expert], device=x.device)
+                out[at] = e.product(matrix, x[at], n, first=expert * n)
+            return out
+
+        got.update(gate_out=through(s["gate"], rows_in, inter), up_out=through(s["up"], rows_in, inter))
+        down = through(s["down"], act if not _one_token(c) else got["gate_out"] * torch.sigmoid(got["gate_out"]) * got["up_out"], hidden)
+        got["out"] = (down[torch.argsort(order)].reshape(tokens, top, hidden) * weights[:, :, None]).sum(1)
+        if not _one_token(c):
+            got.update(order=None, inverse=None, offsets=None, down_out=down)
+        return got
+    if kind == "vocab":
+        ids = e.at[s["ids"]].tolist()
+        x = e.rms_norm(e.value(s["x"], 1, -1), e.value(s["norm"]))
+        return [torch.cat([e.rows(s["table"], c["hidden"], i, i + 1) for i in ids]), e.product(s["table"], x, c["vocab"])[0]]
+    v = e.value(s["w"], -1, c["group"])
+    low, high, most = v.amin(1, keepdim=True), v.amax(1, keepdim=True), (1 << c["bits"]) - 1
+    scale = (high - low) / most
+    scale = torch.where(scale < 1e-7, torch.ones_like(scale), scale)
+    codes = torch.floor(((v - low) / scale + 0.5).clamp(0, most))
+    held = [t.to(DTYPES[c["dtype"]][1]).double() for t in (scale, low)]  # the packed format holds them in the element type
+    return [None, scale.reshape(-1), low.reshape(-1), (codes * held[0] + held[1]).reshape(-1)]
