@@ -205,7 +205,7 @@ MTQ_API int mtq_qmv_batched(int dtype, int bits, uint32_t group_size, int n_mats
  * (crates/metaltile-std/src/ffai/batched_4_qmm.rs:61-85), whose row count is the grid's second dimension (under those
  * names here too when mtq_dispatch is given a grid other than the all-ones placeholder, and `x` may then hold more rows;
  * without one: the rows `x` holds) and whose constraints (K % 512 == 0, N % 8 == 0, group 64, 4-bit) are not required.
- * One mtq_qmm per matrix, in order, with mtq_qmm's routing and arithmetic: outputs are bit-equal to single calls.
+ * mtq_qmm's routing and arithmetic for each matrix: outputs are bit-equal to single calls.
  * Dispatched under the reference names the matrices run on the qmv family at every M, which keeps those kernels'
  * exact-dequant arithmetic (as the `mt_qmm*` names do). w / scales / biases / outs / N are HOST arrays of device pointers / row counts. */
 MTQ_API int mtq_qmm_batched(int dtype, int bits, uint32_t group_size, int n_mats, const void *const *w,
@@ -436,6 +436,9 @@ MTQ_API int mtq_flush_cache(void);
  *   "gather.wide"          expert-routed rows on the 16-row matrix-core GEMV (4-bit g64 f16 / bf16, K <= 4608): 0 = where
  *                          it is the fastest kernel (large experts, at least 4 rows per expert, below the tile
  *                          kernel's crossover or under an exact-dequant name), 1 = never, 2 = wherever the shape allows
+ *   "qmv.runs"             K-run matrix-core GEMV for batches of up to 16 rows (4- and 8-bit codes, f16 / bf16, K % 128 == 0,
+ *                          K <= 8192, 5120 for 8-bit codes; the matrices of mtq_qmm_batched in one launch): 0 = where it is
+ *                          the fastest kernel, 1 = never, 2 = wherever the shape allows
  *   "qmv.wide"             16-row matrix-core GEMV for batches of 5..16 rows (4-bit codes, f16 / bf16, K % 512 == 0):
  *                          0 = where it is the fastest kernel, 1 = never, 2 = wherever the shape allows
  *   "qmv.wide_kp"          that kernel: waves that share a row block, 0 = choose, or 1 / 2 / 4 / 8 / 16

@@ -287,6 +287,37 @@ static int try_wide(int dtype, int bits, uint32_t G, const void* w, const void* 
     return launch_qmv_wide(q, lc, need ? (char*)g.scratch_buf + g.scratch_held : nullptr);
 }
 
+// The matrices of a batch that the K-run kernel is for, in one launch: taken[j] says which those are. The rule looks at one
+// matrix at a time, so that a matrix gives the same bits alone and in a batch.
+static int run_runs(int dtype, int bits, uint32_t G, int n, const void* const* w, const void* const* s, const void* const* b,
+                    const void* x, void* const* outs, uint32_t M, const uint32_t* N, uint32_t K, bool* taken, const LaunchCtx& lc) {
+    const Options& o = options();
+    for (int j = 0; j < n; j++) taken[j] = false;
+    // a route of another kernel that the caller has asked for stands
+    if (o.qmv_runs == 1 || (o.qmv_runs == 0 && (o.qmv_wide == 2 || o.qmv_mfma == 2 || o.qmv_kernel || o.qmm_kernel || o.qmm_kgroups || o.qmm_ksplit ||
+                                                o.qmm_tile_rows || o.qmm_dma || o.qmm_splits)))
+        return ERR_OK;
+    QmvParams p;
+    p.dtype = dtype; p.bits = bits; p.group_size = G; p.x = x; p.M = M; p.K = K;
+    QmvBatch all;
+    all.n = 0;
+    int left = n;
+    for (int j = 0; j < n; j++) {
+        QmvBatch one;
+        one.n = 1;
+        one.w[0] = w[j]; one.scales[0] = s[j]; one.biases[0] = b[j]; one.out[0] = outs[j]; one.N[0] = N[j];
+        if ((o.qmv_runs != 2 && !qmv_runs_preferred(bits, M, N[j], K)) || !qmv_runs_takes(p, one)) continue;
+        taken[j] = true;
+        left--;
+        const int i = all.n++;
+        all.w[i] = w[j]; all.scales[i] = s[j]; all.biases[i] = b[j]; all.out[i] = outs[j]; all.N[i] = N[j];
+    }
+    if (all.n == 0) return ERR_OK;
+    LaunchCtx l2 = lc;
+    if (left) l2.stop = nullptr;   // (first in the call)
+    return launch_qmv_runs(p, all, l2);
+}
+
 static int op_qmv(int dtype, int bits, uint32_t G, const void* w, const void* s, const void* b,
                   const void* x, void* out, uint32_t M, uint32_t N, uint32_t K, const LaunchCtx& lc) {
     int rc = check_common(dtype, bits, G, N, K);
@@ -328,6 +359,9 @@ static int op_qmm(int dtype, int bits, uint32_t G, const void* w, const void* s,
     // 4096 x 14336 26 / 22 us, 1024 x 4096 14 / 10, 8192 x 28672 107 / 62, 28672 x 8192 56 / 39; but
     // 14336 x 4096 12 / 14, 128256 x 4096 70 / 84).
     if (!force_mma) {
+        bool taken;
+        rc = run_runs(dtype, bits, G, 1, &w, &s, &b, x, &out, M, &N, K, &taken, lc);
+        if (rc || taken) return rc;
         rc = try_wide(dtype, bits, G, w, s, b, x, out, M, N, K, false, lc);
         if (rc != ERR_UNSUPPORTED) return rc;
     }
@@ -542,8 +576,7 @@ static int op_qmv_batched(int dtype, int bits, uint32_t G, int n, const void* co
 
 // Several weight matrices against the same M activation rows (the prefill siblings of the batched GEMV,
 // crates/metaltile-std/src/ffai/batched_qkv_qmm.rs:49-68, batched_4_qmm.rs:61-85): row m of every output is the
-// GEMV of activation row m. One qmm per matrix, in order on the caller's stream; at prefill sizes a launch is
-// long against its fixed cost, so one grid over all the matrices would buy nothing.
+// GEMV of activation row m. The matrices that the K-run kernel is for go in one launch; the others one qmm each, in order.
 static int op_qmm_batched(int dtype, int bits, uint32_t G, int n, const void* const* w, const void* const* s,
                           const void* const* b, const void* x, void* const* outs, const uint32_t* N, uint32_t M, uint32_t K,
                           bool exact, const LaunchCtx& lc) {
@@ -556,10 +589,20 @@ static int op_qmm_batched(int dtype, int bits, uint32_t G, int n, const void* co
     if (!x) return fail(ERR_BAD_ARG, "null buffer");
     for (int j = 0; j < n; j++)
         if (!w[j] || !s[j] || !b[j] || !outs[j]) return fail(ERR_BAD_ARG, "null buffer");
-    for (int j = 0; j < n; j++) {
+    bool taken[4] = {};
+    if (!exact) {
+        int rc = run_runs(dtype, bits, G, n, w, s, b, x, outs, M, N, K, taken, lc);
+        if (rc) return rc;
+    }
+    int first = 0, last = n - 1;
+    const bool any = taken[0] || taken[1] || taken[2] || taken[3];
+    while (first < n && taken[first]) first++;
+    while (last >= 0 && taken[last]) last--;
+    for (int j = first; j <= last; j++) {
+        if (taken[j]) continue;
         LaunchCtx l2 = lc;
-        if (j) l2.start = nullptr;
-        if (j + 1 < n) l2.stop = nullptr;
+        if (any || j != first) l2.start = nullptr;
+        if (j != last) l2.stop = nullptr;
         // exact: the caller named a reference kernel, whose rows are GEMVs on the exact f32 s*q + b (as mt_qmm's are):
         // the GEMV family at every M; else mtq_qmm's routing, which takes batches to the tiles and their rounded weights
         int rc = exact ? op_qmv(dtype, bits, G, w[j], s[j], b[j], x, outs[j], M, N[j], K, l2)
@@ -1767,6 +1810,11 @@ int mtq_set_option(const char* name, int value) {
         if (value < 0 || value > 2) return fail(ERR_BAD_ARG, "qmv.norm_mfma must be 0 (choose), 1 (never) or 2 (wherever the shape allows)");
         options().qmv_norm_mfma = value;
         return MTQ_OK;
+    }
+    if (!strcmp(name, "qmv.runs")) {
+        if (value < 0 || value > 2) return fail(ERR_BAD_ARG, "qmv.runs must be 0 (choose), 1 (never) or 2 (wherever the shape allows)");
+        options().qmv_runs = value;
+        return ERR_OK;
     }
     if (!strcmp(name, "qmv.wide_kp")) {
         if (value < 0 || value > 16 || (value & (value - 1))) return fail(ERR_BAD_ARG, "qmv.wide_kp must be 0, 1, 2, 4, 8 or 16");

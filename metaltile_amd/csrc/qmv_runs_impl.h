@@ -1,0 +1,328 @@
+// The K-run matrix-core GEMV (see qmv_runs.hip for the routing and the geometry): kernel and argument block.
+#pragma once
+// Batches of a few activation rows (up to 16) against one or several weight matrices of the same row length, f16 / bf16,
+// with exact-dequant arithmetic: out[m][n] = sum_g (s[n][g] * sum_k q[n][k] x[m][k] + b[n][g] * sum_k x[m][k]), the
+// rows of mt_qmm (crates/metaltile-std/src/mlx/quantized.rs:1330-1500) and of the batched projections
+// (crates/metaltile-std/src/ffai/batched_qkv_qmm.rs:49-68, batched_4_qmm.rs:61-85).
+//
+// What bounds such a batch is the stream of weights; what kept the other kernels from it on matrices of 5 - 60 MB were
+// the parts around the stream: a launch per matrix, activations staged in LDS by every workgroup before its first
+// product, or f32 partial tiles of a split K and a second launch that adds them. Here one launch takes all matrices, and
+// its workgroups (one per compute unit) walk their blocks of 16 weight rows. The sixteen waves of a workgroup share a
+// block, each with a run of K / 16 codes of every row, whose activations it reads once, in the operand layout of the
+// 16x16x32 MFMA, and keeps in registers: from then on the only loads are weights, scales and biases, PF blocks ahead.
+// (Vector loads complete in order: activations read along the way, even from the L2, make a wave wait for all weights
+// asked for before them. The same kernel with activations read per block streamed at half the rate.) The sixteen sums of
+// a result meet in LDS. The split of K depends on K alone: a matrix gives the same bits in whatever batch of matrices.
+//
+// A step is 128 codes of a row (64 of 8-bit codes). Lane (j, q) = (lane % 16, lane / 16) loads the 16 bytes of row j at
+// 16 q: 32 codes (16). An MFMA has to stay inside one group of codes, so for groups shorter than a step the four lanes
+// of a row exchange dwords (v_permlane32_swap, and v_permlane16_swap for groups of 32 4-bit codes), and the activations
+// are put in the order that leaves, once. The sums of the activations over each group, which
+// the bias and the offset of the code conversion are multiplied by, come from one more MFMA per activation operand,
+// against ones: its result has the layout of the products and needs no cross-lane step.
+// Every load is a buffer load whose out-of-range offsets read zeros without a memory access: rows past the matrix or
+// the batch, steps past a wave's run and blocks past the last one are given such offsets, so that every wave issues the
+// same loads in the same order.
+#include "mtq_device.h"
+#include "mtq_internal.h"
+
+#include <type_traits>
+
+namespace mtq {
+
+struct QmvRunsArgs {
+    const unsigned char* w[4];
+    const unsigned char* scales[4];
+    const unsigned char* biases[4];
+    uint16_t* out[4];
+    uint32_t N[4];
+    uint32_t block0[4];      // first block of 16 weight rows of each matrix; 0x7FFFFFFF past the last one
+    uint32_t blocks;         // of all matrices
+    const unsigned char* x;
+    uint32_t M, K;
+};
+
+typedef uint32_t kr_u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t kr_u32x2 __attribute__((ext_vector_type(2)));
+typedef float kr_f32x4 __attribute__((ext_vector_type(4)));
+
+template <int DT> __device__ __forceinline__ kr_f32x4 kr_mfma(kr_u32x4 a, kr_u32x4 b, kr_f32x4 c) {
+    if constexpr (DT == DT_BF16) {
+        typedef __attribute__((ext_vector_type(8))) __bf16 v8;
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8, a), __builtin_bit_cast(v8, b), c, 0, 0, 0);
+    } else {
+        typedef __attribute__((ext_vector_type(8))) _Float16 v8;
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8, a), __builtin_bit_cast(v8, b), c, 0, 0, 0);
+    }
+}
+
+template <int B, int E, class F> __device__ __forceinline__ void kr_for(F&& f) {
+    if constexpr (B < E) {
+        f(std::integral_constant<int, B>{});
+        kr_for<B + 1, E>(f);
+    }
+}
+
+constexpr uint32_t KR_OOB = 0x80000000u;   // every buffer is shorter than 2 GiB (host): base + KR_OOB is out of range for any base below 2 GiB
+constexpr int KR_NT = 2;                   // cache policy of the weights: read once
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t kr_rsrc(uint64_t a, uint32_t bytes) {
+    // (the base is the same in every lane: the descriptor is kept in scalar registers)
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a), hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
+    return __builtin_amdgcn_make_buffer_rsrc((void*)(((uint64_t)hi << 32) | lo), 0, __builtin_amdgcn_readfirstlane(bytes), 0x00020000);
+}
+
+template <int DT> __device__ __forceinline__ float kr_elem(uint32_t dw, int odd) {
+    if constexpr (DT == DT_BF16) return __uint_as_float(odd ? (dw & 0xFFFF0000u) : (dw << 16));
+    else return f16_bits_to_f32(odd ? (dw >> 16) : (dw & 0xFFFFu));
+}
+
+// What a code width fixes: the codes a lane loads per step, the MFMAs of a step, the dwords an MFMA's 8 codes per lane
+// come in, and the offset its conversion adds to every code.
+template <int DT, int BITS> struct KrCodes {
+    static constexpr int LANE = 128 / BITS;       // codes in a lane's 16 bytes
+    static constexpr int STEP = 4 * LANE;
+    static constexpr int UNITS = STEP / 32;
+    static constexpr int DPU = BITS / 4;          // dwords per unit
+    static constexpr float MAGIC = BITS == 4 ? (DT == DT_BF16 ? 128.0f : 1024.0f) : (DT == DT_BF16 ? 0.0f : 1024.0f);
+};
+
+// 8 codes -> an MFMA operand of (MAGIC + code). 4-bit pairs come out as codes (0, 4), (1, 5), (2, 6), (3, 7).
+template <int DT, int BITS> __device__ __forceinline__ kr_u32x4 kr_convert(const uint32_t* d, uint32_t kor) {
+    if constexpr (BITS == 4) {
+        const uint32_t m = 0x000F000Fu, v = d[0];
+        return kr_u32x4{(v & m) | kor, ((v >> 4) & m) | kor, ((v >> 8) & m) | kor, ((v >> 12) & m) | kor};
+    } else if constexpr (DT == DT_F16) {
+        // bytes (code, 0x64, code, 0x64)
+        return kr_u32x4{__builtin_amdgcn_perm(kor, d[0], 0x04010400u), __builtin_amdgcn_perm(kor, d[0], 0x04030402u),
+                        __builtin_amdgcn_perm(kor, d[1], 0x04010400u), __builtin_amdgcn_perm(kor, d[1], 0x04030402u)};
+    } else {
+        // integers up to 255 are exact in bf16: the upper halves of their f32 forms
+        kr_u32x4 o;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const uint32_t v = d[i / 2] >> (16 * (i % 2));
+            const uint32_t f0 = __float_as_uint((float)(v & 0xFFu)), f1 = __float_as_uint((float)((v >> 8) & 0xFFu));
+            o[i] = __builtin_amdgcn_perm(f1, f0, 0x07060302u);
+        }
+        return o;
+    }
+}
+
+// DT, BITS (4 or 8), G (32, 64, 128), XS: steps of a wave's run at most, PF: blocks whose
+// weights are in flight ahead of the one that is worked on.
+template <int DT, int BITS, int G, int XS, int PF> __global__ __launch_bounds__(1024) void qmv_runs_kernel(QmvRunsArgs a) {
+    using C = KrCodes<DT, BITS>;
+    constexpr int KP = 16;
+    constexpr int EG = G < C::STEP ? G : C::STEP;   // codes per scale within a step
+    constexpr int GPS = C::STEP / EG;               // scales per step: 1, 2 or 4
+    constexpr int UPG = EG / 32;                    // MFMAs per scale
+    constexpr bool SWAP32 = EG * 2 <= C::STEP, SWAP16 = EG * 4 <= C::STEP;
+    constexpr int SDW = GPS == 4 ? 2 : 1;           // dwords of scales per step and row
+    constexpr int SR = (XS + 3) / 4;                // scale registers: lanes (j, q) hold steps q, q + 4 of row j
+    constexpr bool HOLD = XS * GPS <= 4;       // the activations' sums stay in registers
+    __shared__ float red[2][KP * 256];
+
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t kp = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t j = lane & 15u, q = lane >> 4;
+    const uint32_t K = a.K, wrow_bytes = K / 8u * BITS, gpr = K / (uint32_t)G;
+
+    // this wave's run of steps
+    const uint32_t steps = K / (uint32_t)C::STEP;
+    const uint32_t t0 = steps * kp / KP, cnt = steps * (kp + 1u) / KP - t0;   // cnt <= XS (host)
+
+    const uint32_t wlane = j * wrow_bytes + t0 * 64u + q * 16u;
+    uint32_t slane[SR];
+#pragma unroll
+    for (int i = 0; i < SR; i++) {
+        const uint32_t n = q + 4u * i, at = t0 + n;
+        slane[i] = n < cnt ? j * gpr * 2u + (G > C::STEP ? at / (uint32_t)(G / EG) : at * GPS) * 2u : KR_OOB;
+    }
+    uint32_t step_dead[XS];   // steps past the run
+#pragma unroll
+    for (int n = 0; n < XS; n++) step_dead[n] = (cnt - (uint32_t)(n + 1)) & KR_OOB;
+
+    // The matrix of a block, by sums of masked differences on the scalar unit. (Selections among the arguments become an
+    // indexed read of a copy of them in scratch memory, with a wait for every load in flight.)
+    const uint32_t n_blocks = a.blocks;
+    auto pick = [&](const auto* f, uint32_t blk) {
+        uint64_t v = (uint64_t)f[0];
+#pragma unroll
+        for (int i = 1; i < 4; i++) {
+            const int64_t in = (int32_t)(a.block0[i] - 1u - blk) >> 31;   // all ones from the matrix's first block on
+            v += ((uint64_t)f[i] - (uint64_t)f[i - 1]) & (uint64_t)in;
+        }
+        return v;
+    };
+
+    struct Block {   // a block's weights, scales and biases in flight
+        kr_u32x4 w[XS];
+        uint32_t s[SR][SDW], b[SR][SDW];
+    };
+    auto load_block = [&](Block& d, uint32_t blk) {
+        // (Everything but the lane's own part is worked out on the scalar unit. The offsets are put out of range with the sign of
+        // a difference: from a selection the optimiser makes a branch around the loads, and waits there for all in flight.)
+        const uint32_t at_blk = min(blk, n_blocks - 1u), N = (uint32_t)pick(a.N, at_blk), first = (uint32_t)pick(a.block0, at_blk);
+        const uint32_t row0 = (at_blk - first) * 16u, rows = blk < n_blocks ? N - row0 : 0u;   // (16 or more: a whole block)
+        const __amdgpu_buffer_rsrc_t wr = kr_rsrc(pick(a.w, at_blk), N * wrow_bytes), sr = kr_rsrc(pick(a.scales, at_blk), N * gpr * 2u),
+                                     br = kr_rsrc(pick(a.biases, at_blk), N * gpr * 2u);
+        const uint32_t dead = (rows - 1u - j) & KR_OOB;
+        const uint32_t wo = (wlane + row0 * wrow_bytes) | dead, s0 = row0 * gpr * 2u;
+#pragma unroll
+        for (int i = 0; i < SR; i++) {
+            const uint32_t o = (slane[i] + s0) | dead;
+            if constexpr (GPS == 1) {
+                d.s[i][0] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(sr, (int)o, 0, 0);
+                d.b[i][0] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(br, (int)o, 0, 0);
+            } else if constexpr (GPS == 2) {
+                d.s[i][0] = __builtin_amdgcn_raw_buffer_load_b32(sr, (int)o, 0, 0);
+                d.b[i][0] = __builtin_amdgcn_raw_buffer_load_b32(br, (int)o, 0, 0);
+            } else {
+                const kr_u32x2 sv = __builtin_amdgcn_raw_buffer_load_b64(sr, (int)o, 0, 0), bv = __builtin_amdgcn_raw_buffer_load_b64(br, (int)o, 0, 0);
+                d.s[i][0] = sv.x; d.s[i][1] = sv.y; d.b[i][0] = bv.x; d.b[i][1] = bv.y;
+            }
+        }
+#pragma unroll
+        for (int n = 0; n < XS; n++) d.w[n] = __builtin_amdgcn_raw_buffer_load_b128(wr, (int)((wo + 64u * n) | step_dead[n]), 0, KR_NT);
+    };
+
+    Block ring[PF + 1];
+    kr_for<0, PF>([&](auto p) { load_block(ring[decltype(p)::value], blockIdx.x + gridDim.x * (uint32_t)decltype(p)::value); });
+
+    // ---- the activations of the run. Load k of a step takes pieces 4 k + q of 8 codes: 64 contiguous bytes of every row (read
+    // straight into the operand layout, a load would touch 64 separate lines; at 16 rows that took 3 us more). Unit u's
+    // pieces are 4 u + q where both exchanges are made, and otherwise those of where the lane's codes come from.
+    constexpr bool SWAP_X16 = !SWAP16 && !(BITS == 8 && SWAP32), SWAP_X32 = !SWAP32;
+    kr_u32x4 xop[XS][C::UNITS];
+    {
+        const __amdgpu_buffer_rsrc_t xr = kr_rsrc((uint64_t)a.x, a.M * K * 2u);
+        const uint32_t piece = BITS == 8 && SWAP32 ? (q & 1u) * 2u + (q >> 1) : q;
+#pragma unroll
+        for (int n = 0; n < XS; n++) {
+            const uint32_t o = ((j * K + (t0 + n) * (uint32_t)C::STEP + piece * 8u) * 2u) | ((a.M - 1u - j) & KR_OOB) | step_dead[n];
+#pragma unroll
+            for (int k = 0; k < C::UNITS; k++) xop[n][k] = __builtin_amdgcn_raw_buffer_load_b128(xr, (int)(o + 64u * k), 0, 0);
+        }
+#pragma unroll
+        for (int n = 0; n < XS; n++) {
+            auto swap = [&](int u0, int u1, auto wide) {
+#pragma unroll
+                for (int d = 0; d < 4; d++) {
+                    const uint32_t p = xop[n][u0][d], r = xop[n][u1][d];
+                    const auto t = decltype(wide)::value ? __builtin_amdgcn_permlane32_swap(p, r, false, false) : __builtin_amdgcn_permlane16_swap(p, r, false, false);
+                    xop[n][u0][d] = t[0];
+                    xop[n][u1][d] = t[1];
+                }
+            };
+            if constexpr (BITS == 4) {
+                if constexpr (SWAP_X16) { swap(0, 1, std::false_type{}); swap(2, 3, std::false_type{}); }   // pieces 0 4 2 6 | 1 5 3 7 | 8 12 10 14 | 9 13 11 15
+                if constexpr (SWAP_X32) { swap(0, 2, std::true_type{}); swap(1, 3, std::true_type{}); }     // 0 4 8 12 | 1 5 9 13 | 2 6 10 14 | 3 7 11 15
+#pragma unroll
+                for (int u = 0; u < C::UNITS; u++) {   // in the order the nibble masks deliver the codes
+                    const kr_u32x4 t = xop[n][u];
+                    xop[n][u] = kr_u32x4{__builtin_amdgcn_perm(t.z, t.x, 0x05040100u), __builtin_amdgcn_perm(t.z, t.x, 0x07060302u),
+                                            __builtin_amdgcn_perm(t.w, t.y, 0x05040100u), __builtin_amdgcn_perm(t.w, t.y, 0x07060302u)};
+                }
+            } else if constexpr (SWAP_X32) {
+                swap(0, 1, std::true_type{});    // 0 1 4 5 | 2 3 6 7
+                swap(0, 1, std::false_type{});   // 0 2 4 6 | 1 3 5 7
+            }
+        }
+    }
+    const uint32_t kor = BITS == 8 ? 0x64646464u : magic_or_vgpr<DT>();
+    constexpr uint32_t ONE = DT == DT_BF16 ? 0x3F803F80u : 0x3C003C00u;
+    const kr_u32x4 ones = {ONE, ONE, ONE, ONE};
+    const kr_f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    auto x_sum = [&](int n, int g) {
+        kr_f32x4 s = zero;
+#pragma unroll
+        for (int u = 0; u < UPG; u++) s = kr_mfma<DT>(xop[n][g * UPG + u], ones, s);
+        return s;
+    };
+    kr_f32x4 held[HOLD ? XS : 1][HOLD ? GPS : 1];
+    if constexpr (HOLD) {
+#pragma unroll
+        for (int n = 0; n < XS; n++)
+#pragma unroll
+            for (int g = 0; g < GPS; g++) held[n][g] = x_sum(n, g);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+
+    uint32_t par = 0;
+    uint32_t blk = blockIdx.x;
+    auto turn = [&](auto p_c) {
+        constexpr int p = decltype(p_c)::value;
+        load_block(ring[(p + PF) % (PF + 1)], blk + gridDim.x * (uint32_t)PF);
+        __builtin_amdgcn_sched_barrier(0);
+        Block& d = ring[p];
+        kr_f32x4 tot = zero;
+        kr_for<0, XS>([&](auto n_c) {
+            constexpr int n = decltype(n_c)::value;
+            uint32_t v[4] = {d.w[n].x, d.w[n].y, d.w[n].z, d.w[n].w};
+            if constexpr (SWAP32) {
+#pragma unroll
+                for (int k = 0; k < 2; k++) {
+                    const auto t = __builtin_amdgcn_permlane32_swap(v[k], v[k + 2], false, false);
+                    v[k] = t[0];
+                    v[k + 2] = t[1];
+                }
+            }
+            if constexpr (SWAP16) {
+#pragma unroll
+                for (int k = 0; k < 4; k += 2) {
+                    const auto t = __builtin_amdgcn_permlane16_swap(v[k], v[k + 1], false, false);
+                    v[k] = t[0];
+                    v[k + 1] = t[1];
+                }
+            }
+            const int src = (int)((j + 16u * (n % 4)) * 4u);   // the lane that holds this step's scales of row j
+            kr_for<0, GPS>([&](auto g_c) {
+                constexpr int g = decltype(g_c)::value;
+                kr_f32x4 acc = zero;
+#pragma unroll
+                for (int u = g * UPG; u < (g + 1) * UPG; u++) acc = kr_mfma<DT>(xop[n][u], kr_convert<DT, BITS>(&v[u * C::DPU], kor), acc);
+                const uint32_t sp = (uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)d.s[n / 4][g / 2]);
+                const uint32_t bp = (uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)d.b[n / 4][g / 2]);
+                const float sv = kr_elem<DT>(sp, g % 2), bv = kr_elem<DT>(bp, g % 2);
+                const float bm = C::MAGIC == 0.f ? bv : fmaf(-C::MAGIC, sv, bv);
+                kr_f32x4 xs;
+                if constexpr (HOLD) xs = held[n][g];
+                else xs = x_sum(n, g);
+#pragma unroll
+                for (int r = 0; r < 4; r++) tot[r] = fmaf(bm, xs[r], fmaf(sv, acc[r], tot[r]));
+            });
+        });
+        // The sixteen runs meet in LDS: result r of lane (j, q) is activation row 4 q + r, weight row j. The
+        // other half of the buffer takes the next block, so one barrier per block is enough.
+        float* rd = red[par];
+        par ^= 1u;
+#pragma unroll
+        for (int r = 0; r < 4; r++) rd[(kp * 4u + r) * 64u + lane] = tot[r];
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+        if (tid < 256u) {
+            float s = rd[tid];
+#pragma unroll
+            for (uint32_t o = 1; o < KP; o++) s += rd[o * 256u + tid];
+            __attribute__((address_space(1))) uint16_t* out = (__attribute__((address_space(1))) uint16_t*)pick(a.out, blk);
+            const uint32_t N = (uint32_t)pick(a.N, blk), first = (uint32_t)pick(a.block0, blk);
+            const uint32_t arow = 4u * q + (tid >> 6), wrow = (blk - first) * 16u + j;
+            if (arow < a.M && wrow < N) out[(size_t)arow * N + wrow] = f32_to_elem_bits<DT>(s);
+        }
+        blk += gridDim.x;
+        return blk < n_blocks;   // (the same in every wave of the workgroup)
+    };
+    for (;;) {
+        if (!turn(std::integral_constant<int, 0>{})) break;
+        if (!turn(std::integral_constant<int, 1>{})) break;
+        if constexpr (PF >= 2)
+            if (!turn(std::integral_constant<int, 2>{})) break;
+        if constexpr (PF >= 3)
+            if (!turn(std::integral_constant<int, 3>{})) break;
+    }
+}
+
+}  // namespace mtq
