@@ -261,14 +261,9 @@ static int try_f32_tiles(int bits, uint32_t G, const void* w, const void* s, con
 // Batches of 5..16 rows on the 16-row matrix-core GEMV where the shape allows and it is the fastest kernel;
 // ERR_UNSUPPORTED otherwise. `exact`: the caller's alternative is the GEMV family (passes of up to 8 rows, the
 // same exact-dequant arithmetic); else it is the tile kernel.
-static int try_wide(int dtype, int bits, uint32_t G, const void* w, const void* s, const void* b, const void* x,
-                    void* out, uint32_t M, uint32_t N, uint32_t K, bool exact, const LaunchCtx& lc) {
-    if (M < 5 || M > 16 || options().qmv_wide == 1) return ERR_UNSUPPORTED;
-    QmmParams q;
-    q.dtype = dtype; q.bits = bits; q.group_size = G;
-    q.w = w; q.scales = s; q.biases = b; q.x = x; q.out = out;
-    q.M = M; q.N = N; q.K = K;
-    if (!qmv_wide_takes(q)) return ERR_UNSUPPORTED;
+static bool wide_serves(const QmmParams& q, bool exact) {
+    const uint32_t M = q.M;
+    if (M < 5 || M > 16 || options().qmv_wide == 1 || !qmv_wide_takes(q)) return false;
     // Every workgroup stages its 16 rows of activations (128 KB at K = 4096), which pays once a compute unit streams
     // several times that in weights. us, 5 / 8 / 12 / 16 rows, the other kernels (GEMV passes of up to 8 rows | tiles)
     // against this one: 128256 x 4096 69 66 116 131 | 88 89 90 92 -> 54 53 55 55; 57344 x 4096 31 32 56 62 | 42 43 43
@@ -276,9 +271,17 @@ static int try_wide(int dtype, int bits, uint32_t G, const void* w, const void* 
     // -> 17.5 18.3 19.5 20.3; 8192 x 8192 19 22 32 42 | 17.4 16.9 17.1 17.4 -> 14.8 15.6 17.2 18.3; 14336 x 4096 13.1 13.6
     // 23 27 | 13.5 13.4 13.6 13.7 -> 12.3 12.9 13.8 14.7; 4096 x 14336 23 25 38 50 | 15.2 15.4 15.9 16.0 -> 14.8 15.1 16.2
     // 17.4; 4096 x 4096 7.6 8.3 10.7 12.6 | 9.4 9.6 9.9 10.1 -> 10.1 10.7 11.4 12.1.
-    const uint64_t codes = (uint64_t)N * K;
+    const uint64_t codes = (uint64_t)q.N * q.K;
     const bool pays = M <= 8 ? codes >= 50000000ull : exact ? codes >= (1ull << 25) : codes >= 100000000ull;
-    if (options().qmv_wide != 2 && !pays) return ERR_UNSUPPORTED;
+    return options().qmv_wide == 2 || pays;
+}
+static int try_wide(int dtype, int bits, uint32_t G, const void* w, const void* s, const void* b, const void* x,
+                    void* out, uint32_t M, uint32_t N, uint32_t K, bool exact, const LaunchCtx& lc) {
+    QmmParams q;
+    q.dtype = dtype; q.bits = bits; q.group_size = G;
+    q.w = w; q.scales = s; q.biases = b; q.x = x; q.out = out;
+    q.M = M; q.N = N; q.K = K;
+    if (!wide_serves(q, exact)) return ERR_UNSUPPORTED;
     const size_t need = qmv_wide_scratch_bytes(q);
     if (need) {
         int rc = ensure_scratch(g.scratch_held + need);
@@ -337,6 +340,17 @@ static int op_qmv(int dtype, int bits, uint32_t G, const void* w, const void* s,
     return run_gemv(p, lc);
 }
 
+// 7-bit codes have no GEMV kernel of their own (the reference has no 7-bit kernels either): any
+// number of rows beats the generic kernel on the tile kernel (4096 x 4096: 1 row 28 -> 17 us, 16 rows 236 -> 17).
+// 5..8 rows: rows too long for 8 of them in LDS make the GEMV take two passes, and short, wide
+// matrices leave it few row blocks; the split-K tiles are ahead there (8 rows, GEMV against tiles:
+// 4096 x 14336 26 / 22 us, 1024 x 4096 14 / 10, 8192 x 28672 107 / 62, 28672 x 8192 56 / 39; but
+// 14336 x 4096 12 / 14, 128256 x 4096 70 / 84).
+static bool tiles_serve(int bits, uint32_t M, uint32_t N, uint32_t K) {
+    const bool long_rows = M >= 5 && ((uint64_t)K >= 2 * (uint64_t)N || (K >= 8192 && (uint64_t)N >= 3 * (uint64_t)K));
+    return M >= 9 || long_rows || bits == 7;
+}
+
 // Kernel routing by M, the counterpart of mt_qmm_for
 // (crates/metaltile-std/src/mlx/quantized.rs:5040-5065, which sends M = 16 and the multiples
 // of 32 to its MMA kernels). Here the GEMV family takes 8 activation rows per pass over the
@@ -352,12 +366,6 @@ static int op_qmm(int dtype, int bits, uint32_t G, const void* w, const void* s,
     if (M == 0) return ERR_OK;
     if (!w || !s || !b || !x || !out) return fail(ERR_BAD_ARG, "null buffer");
     if (dtype == DT_F32 && options().qmm_f32_tiles != 1) return op_qmv(dtype, bits, G, w, s, b, x, out, M, N, K, lc);
-    // 7-bit codes have no GEMV kernel of their own (the reference has no 7-bit kernels either): any
-    // number of rows beats the generic kernel on the tile kernel (4096 x 4096: 1 row 28 -> 17 us, 16 rows 236 -> 17).
-    // 5..8 rows: rows too long for 8 of them in LDS make the GEMV take two passes, and short, wide
-    // matrices leave it few row blocks; the split-K tiles are ahead there (8 rows, GEMV against tiles:
-    // 4096 x 14336 26 / 22 us, 1024 x 4096 14 / 10, 8192 x 28672 107 / 62, 28672 x 8192 56 / 39; but
-    // 14336 x 4096 12 / 14, 128256 x 4096 70 / 84).
     if (!force_mma) {
         bool taken;
         rc = run_runs(dtype, bits, G, 1, &w, &s, &b, x, &out, M, &N, K, &taken, lc);
@@ -365,8 +373,7 @@ static int op_qmm(int dtype, int bits, uint32_t G, const void* w, const void* s,
         rc = try_wide(dtype, bits, G, w, s, b, x, out, M, N, K, false, lc);
         if (rc != ERR_UNSUPPORTED) return rc;
     }
-    const bool long_rows = M >= 5 && ((uint64_t)K >= 2 * (uint64_t)N || (K >= 8192 && (uint64_t)N >= 3 * (uint64_t)K));
-    if (M >= 9 || long_rows || force_mma || bits == 7) {
+    if (force_mma || tiles_serve(bits, M, N, K)) {
         QmmParams q;
         q.dtype = dtype; q.bits = bits; q.group_size = G;
         q.w = w; q.scales = s; q.biases = b; q.x = x; q.out = out;
@@ -576,7 +583,8 @@ static int op_qmv_batched(int dtype, int bits, uint32_t G, int n, const void* co
 
 // Several weight matrices against the same M activation rows (the prefill siblings of the batched GEMV,
 // crates/metaltile-std/src/ffai/batched_qkv_qmm.rs:49-68, batched_4_qmm.rs:61-85): row m of every output is the
-// GEMV of activation row m. The matrices that the K-run kernel is for go in one launch; the others one qmm each, in order.
+// GEMV of activation row m. The matrices that the K-run kernel is for go in one launch, those for the tile
+// kernels in as few as their tilings allow, the others one qmm each, in order.
 static int op_qmm_batched(int dtype, int bits, uint32_t G, int n, const void* const* w, const void* const* s,
                           const void* const* b, const void* x, void* const* outs, const uint32_t* N, uint32_t M, uint32_t K,
                           bool exact, const LaunchCtx& lc) {
@@ -594,15 +602,40 @@ static int op_qmm_batched(int dtype, int bits, uint32_t G, int n, const void* co
         int rc = run_runs(dtype, bits, G, n, w, s, b, x, outs, M, N, K, taken, lc);
         if (rc) return rc;
     }
-    int first = 0, last = n - 1;
-    const bool any = taken[0] || taken[1] || taken[2] || taken[3];
-    while (first < n && taken[first]) first++;
-    while (last >= 0 && taken[last]) last--;
-    for (int j = first; j <= last; j++) {
+    // what is left of the batch on the tile kernels goes there together
+    bool started = taken[0] || taken[1] || taken[2] || taken[3];
+    QmmParams tiled[4];
+    int n_tiled = 0, left = 0;
+    bool on_tiles[4] = {};
+    for (int j = 0; j < n; j++) {
         if (taken[j]) continue;
+        QmmParams q;
+        q.dtype = dtype; q.bits = bits; q.group_size = G;
+        q.w = w[j]; q.scales = s[j]; q.biases = b[j]; q.x = x; q.out = outs[j];
+        q.M = M; q.N = N[j]; q.K = K;
+        on_tiles[j] = !exact && dtype != DT_F32 && options().qmm_kernel != 1 && !wide_serves(q, false) && tiles_serve(bits, M, N[j], K) && qmm_direct_takes(q);
+        if (on_tiles[j]) tiled[n_tiled++] = q;
+        else left++;
+    }
+    if (n_tiled) {
+        const size_t need = qmm_direct_batch_scratch_bytes(tiled, n_tiled);
+        if (need) {
+            int rc = ensure_scratch(g.scratch_held + need);
+            if (rc) return rc;
+        }
         LaunchCtx l2 = lc;
-        if (any || j != first) l2.start = nullptr;
-        if (j != last) l2.stop = nullptr;
+        if (started) l2.start = nullptr;
+        if (left) l2.stop = nullptr;
+        int rc = launch_qmm_direct_batch(tiled, n_tiled, l2, need ? (char*)g.scratch_buf + g.scratch_held : nullptr);
+        if (rc) return rc;
+        started = true;
+    }
+    for (int j = 0; j < n; j++) {
+        if (taken[j] || on_tiles[j]) continue;
+        LaunchCtx l2 = lc;
+        if (started) l2.start = nullptr;
+        if (--left) l2.stop = nullptr;
+        started = true;
         // exact: the caller named a reference kernel, whose rows are GEMVs on the exact f32 s*q + b (as mt_qmm's are):
         // the GEMV family at every M; else mtq_qmm's routing, which takes batches to the tiles and their rounded weights
         int rc = exact ? op_qmv(dtype, bits, G, w[j], s[j], b[j], x, outs[j], M, N[j], K, l2)

@@ -29,6 +29,8 @@
 // of N-tiles: its L2 holds its slice of W once and X once.
 #include "qmm_direct_impl.h"
 
+#include <utility>
+
 namespace mtq {
 
 // The kernel itself lives in qmm_direct_impl.h; the instances for 3-, 5-, 6- and 7-bit codes are built in
@@ -43,13 +45,104 @@ static size_t lds_need(uint32_t rows, uint32_t kg, uint32_t gpr, bool sbl) {
     return main_loop > epilogue ? main_loop : epilogue;
 }
 
-// Adds the K splits' partial tiles in split order and rounds to the element type.
-template <int DT> __global__ __launch_bounds__(256) void qmm_split_reduce_kernel(const float* part, void* out, uint32_t total, uint32_t ksplit) {
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+// Adds the K splits' partial tiles in split order and rounds to the element type; VEC results per thread. Up to four
+// matrices of one launch, each from its own first workgroup on.
+struct QmmReduceArgs {
+    const float* part[4];
+    void* out[4];
+    uint32_t total[4];
+    uint32_t first[4];
+    uint32_t ksplit;
+};
+template <int DT, int VEC> __global__ __launch_bounds__(256) void qmm_split_reduce_kernel(QmmReduceArgs a) {
+    const uint32_t m = __builtin_amdgcn_readfirstlane((blockIdx.x >= a.first[1] ? 1u : 0u) + (blockIdx.x >= a.first[2] ? 1u : 0u) + (blockIdx.x >= a.first[3] ? 1u : 0u));
+    const uint32_t i = ((blockIdx.x - a.first[m]) * 256 + threadIdx.x) * VEC, total = a.total[m];
     if (i >= total) return;
-    float r = part[i];
-    for (uint32_t sp = 1; sp < ksplit; sp++) r += part[(size_t)sp * total + i];
-    ((uint16_t*)out)[i] = f32_to_elem_bits<DT>(r);
+    const float* part = a.part[m] + i;
+    float r[VEC];
+    auto load = [&](const float* p, float (&v)[VEC]) {
+        if constexpr (VEC == 4) {
+            const float4 t = *(const float4*)p;
+            v[0] = t.x; v[1] = t.y; v[2] = t.z; v[3] = t.w;
+        } else {
+            v[0] = p[0];
+        }
+    };
+    load(part, r);
+    for (uint32_t sp = 1; sp < a.ksplit; sp++) {
+        float v[VEC];
+        load(part + (size_t)sp * total, v);
+#pragma unroll
+        for (int k = 0; k < VEC; k++) r[k] += v[k];
+    }
+    uint16_t* out = (uint16_t*)a.out[m] + i;
+    uint32_t h[VEC];
+#pragma unroll
+    for (int k = 0; k < VEC; k++) h[k] = f32_to_elem_bits<DT>(r[k]);
+    if constexpr (VEC == 4) *(uint2*)out = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
+    else out[0] = (uint16_t)h[0];
+}
+
+// What one matrix's launch is: the kernel that the tiling picks, its geometry, and whether partial tiles follow.
+struct QmmDLaunch {
+    const void* fn = nullptr;
+    uint32_t grid = 0, block = 0;   // workgroups per K split
+    size_t shmem = 0;
+    bool split = false;
+    QmmDArgs a;
+};
+
+// Launches l[0 .. n): matrices on the same kernel in one launch (at most four), then one addition of their partial tiles.
+static bool qd_same_launch(const QmmDLaunch& p, const QmmDLaunch& q) {
+    return p.fn == q.fn && p.block == q.block && p.split == q.split && p.a.ksplit == q.a.ksplit && p.a.iters_per_split == q.a.iters_per_split && !p.a.tiles && !q.a.tiles;
+}
+static int qd_issue(int dtype, const QmmDLaunch* l, int n, const LaunchCtx& lc) {
+    for (int i = 0, j; i < n; i = j) {
+        QmmDArgs a = l[i].a;
+        QmmDMore more;
+        uint32_t wgs = l[i].grid;
+        size_t shmem = l[i].shmem;
+        for (j = i + 1; j < n && j - i < 4 && qd_same_launch(l[i], l[j]); j++) {
+            const uint32_t k = more.n++;
+            const QmmDArgs& o = l[j].a;
+            more.first[k] = wgs;
+            more.N[k] = o.N; more.n_tiles[k] = o.n_tiles; more.by_m[k] = o.by_m;
+            more.w[k] = o.w; more.scales[k] = o.scales; more.biases[k] = o.biases; more.out[k] = o.out; more.part[k] = o.part;
+            wgs += l[j].grid;
+            if (l[j].shmem > shmem) shmem = l[j].shmem;
+        }
+        hipError_t e = set_max_dynamic_lds(l[i].fn, shmem);
+        if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(max dynamic LDS)");
+        void* args[] = {&a, &more};
+        LaunchCtx l1 = lc, l2 = lc;
+        if (i) l1.start = l2.start = nullptr;
+        if (j < n) l1.stop = l2.stop = nullptr;
+        if (l[i].split) { l1.stop = nullptr; l2.start = nullptr; }
+        e = launch_kernel(l[i].fn, dim3(wgs, l[i].split ? a.ksplit : 1), dim3(l[i].block), args, shmem, l1);
+        if (e != hipSuccess) return hip_fail(e, "qmm tile kernel launch");
+        if (!l[i].split) continue;
+        QmmReduceArgs r;
+        r.ksplit = a.ksplit;
+        bool vec = true;   // four results per thread: their partial sums and outputs are whole vectors
+        for (int k = i; k < j; k++) vec = vec && (uint64_t)l[k].a.M * l[k].a.N % 4 == 0 && (uintptr_t)l[k].a.part % 16 == 0;
+        uint32_t blocks = 0;
+        for (int k = 0; k < 4; k++) {
+            r.first[k] = ~0u;
+            r.part[k] = nullptr; r.out[k] = nullptr; r.total[k] = 0;
+            if (i + k >= j) continue;
+            const QmmDArgs& o = l[i + k].a;
+            r.part[k] = o.part; r.out[k] = o.out; r.total[k] = o.M * o.N;
+            r.first[k] = blocks;
+            const uint32_t per = vec ? 1024 : 256;
+            blocks += (r.total[k] + per - 1) / per;
+        }
+        void* rargs[] = {&r};
+        const void* rf = dtype == DT_BF16 ? (vec ? (const void*)qmm_split_reduce_kernel<DT_BF16, 4> : (const void*)qmm_split_reduce_kernel<DT_BF16, 1>)
+                                          : (vec ? (const void*)qmm_split_reduce_kernel<DT_F16, 4> : (const void*)qmm_split_reduce_kernel<DT_F16, 1>);
+        e = launch_kernel(rf, dim3(blocks), dim3(256), rargs, 0, l2);
+        if (e != hipSuccess) return hip_fail(e, "qmm split reduce kernel launch");
+    }
+    return ERR_OK;
 }
 
 // Shapes the load-to-LDS instances take: 4- or 8-bit codes, 2 K-groups, whole iterations of 128 k, whole 8-element
@@ -88,7 +181,12 @@ static size_t dma_split_lds(int bits, uint32_t rows, uint32_t kgroups, uint32_t 
     return need <= 160 * 1024 ? need : 0;
 }
 
-template <int DT> static int launch_dt(QmmDArgs& a, int bits, uint32_t kgroups, const LaunchCtx& lc, bool grouped = false) {
+// The kernel that a matrix's tiling picks.
+template <int DT> static int choose_dt(const QmmDArgs& a, int bits, uint32_t kgroups, QmmDLaunch& l, bool grouped = false) {
+    l.a = a;
+    l.grid = a.m_tiles * a.n_tiles;
+    l.block = kgroups == 1 ? 256 : 512;
+    l.split = a.ksplit > 1 && !grouped;
     const void* fn = nullptr;
     // 8-bit codes on short rows gain nothing where the launch leaves compute units idle (14336 x 4096, 128 rows:
     // 36.3 against 34.3 us) or on the 4-K-group tiles (4096 x 4096, 16 / 64 rows 11.6 / 15.3 against 10.9 / 14.6;
@@ -97,34 +195,16 @@ template <int DT> static int launch_dt(QmmDArgs& a, int bits, uint32_t kgroups, 
     int dev = 0, cus = 256;
     if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
     if (const size_t shmem = grouped ? 0 : dma_split_lds(bits, a.m_tile_rows, kgroups, a.K, a.gpr, a.iters_per_split, a.ksplit)) {
-        fn = qmm_dma_split_pick(bits, DT, a.m_tile_rows);
-        hipError_t e = set_max_dynamic_lds(fn, shmem);
-        if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(max dynamic LDS)");
-        void* args[] = {&a};
-        LaunchCtx l1 = lc, l2 = lc;
-        l1.stop = nullptr;
-        l2.start = nullptr;
-        e = launch_kernel(fn, dim3(a.m_tiles * a.n_tiles, a.ksplit), dim3(512), args, shmem, l1);
-        if (e != hipSuccess) return hip_fail(e, "qmm load-to-LDS kernel launch");
-        const float* part = a.part;
-        void* out = a.out;
-        uint32_t total = a.M * a.N, ks = a.ksplit;
-        void* rargs[] = {&part, &out, &total, &ks};
-        e = launch_kernel((const void*)qmm_split_reduce_kernel<DT>, dim3((total + 255) / 256), dim3(256), rargs, 0, l2);
-        if (e != hipSuccess) return hip_fail(e, "qmm split reduce kernel launch");
+        l.fn = qmm_dma_split_pick(bits, DT, a.m_tile_rows);
+        l.shmem = shmem;
         return ERR_OK;
     }
     if (a.ksplit <= 1 && dma_fits(bits, a.m_tile_rows, kgroups, a.K, a.gpr) && (!grouped || a.m_tile_rows == 64) &&
         !(b8_short && !grouped && a.m_tile_rows != 256 && (uint64_t)a.m_tiles * a.n_tiles < (uint64_t)cus)) {
         const bool windowed = dma_mode(bits, a.m_tile_rows, kgroups, a.K, a.gpr) == 2;
         const bool shallow = grouped || (uint64_t)a.m_tiles * a.n_tiles > (uint64_t)cus;
-        fn = qmm_dma_pick(bits, DT, a.m_tile_rows, grouped, windowed, shallow);
-        const size_t shmem = qmm_dma_lds_bytes(a.m_tile_rows, a.gpr, windowed, shallow);
-        hipError_t e = set_max_dynamic_lds(fn, (size_t)shmem);
-        if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(max dynamic LDS)");
-        void* args[] = {&a};
-        e = launch_kernel(fn, dim3(a.m_tiles * a.n_tiles), dim3(512), args, shmem, lc);
-        if (e != hipSuccess) return hip_fail(e, "qmm load-to-LDS kernel launch");
+        l.fn = qmm_dma_pick(bits, DT, a.m_tile_rows, grouped, windowed, shallow);
+        l.shmem = qmm_dma_lds_bytes(a.m_tile_rows, a.gpr, windowed, shallow);
         return ERR_OK;
     }
     // The same transport on the 4-K-group tilings of few rows (32 x 64 and 64 x 64 tiles, plain, K-split or grouped
@@ -133,24 +213,8 @@ template <int DT> static int launch_dt(QmmDArgs& a, int bits, uint32_t kgroups, 
     // 17.1 / 20.9 -> 16.3 / 17.1 (64 rows and fewer: the same within 1 %).
     if (options().qmm_dma != 1 && (bits == 4 || bits == 8) && !b8_short && kgroups == 4 && (a.m_tile_rows == 32 || a.m_tile_rows == 64) && a.K % 256 == 0 &&
         a.gpr % 8 == 0 && qmm_dma4_lds_bytes(a.m_tile_rows, a.gpr) <= 160 * 1024 && !(grouped && a.ksplit > 1)) {
-        const bool split = a.ksplit > 1;
-        fn = qmm_dma4_pick(bits, DT, a.m_tile_rows, split, grouped);
-        const size_t shmem = qmm_dma4_lds_bytes(a.m_tile_rows, a.gpr);
-        hipError_t e = set_max_dynamic_lds(fn, (size_t)shmem);
-        if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(max dynamic LDS)");
-        void* args[] = {&a};
-        LaunchCtx l1 = lc, l2 = lc;
-        if (split) { l1.stop = nullptr; l2.start = nullptr; }
-        e = launch_kernel(fn, dim3(a.m_tiles * a.n_tiles, split ? a.ksplit : 1), dim3(512), args, shmem, l1);
-        if (e != hipSuccess) return hip_fail(e, "qmm load-to-LDS kernel launch");
-        if (split) {
-            const float* part = a.part;
-            void* out = a.out;
-            uint32_t total = a.M * a.N, ks = a.ksplit;
-            void* rargs[] = {&part, &out, &total, &ks};
-            e = launch_kernel((const void*)qmm_split_reduce_kernel<DT>, dim3((total + 255) / 256), dim3(256), rargs, 0, l2);
-            if (e != hipSuccess) return hip_fail(e, "qmm split reduce kernel launch");
-        }
+        l.fn = qmm_dma4_pick(bits, DT, a.m_tile_rows, a.ksplit > 1, grouped);
+        l.shmem = qmm_dma4_lds_bytes(a.m_tile_rows, a.gpr);
         return ERR_OK;
     }
     if (a.m_tile_rows == 256) return fail(ERR_UNSUPPORTED, "direct qmm: 256-row tiles need 4- or 8-bit codes, K % 128 == 0 and rows whose scales fit LDS (or, 4-bit codes, groups of 64 or 128 codes)");
@@ -199,25 +263,8 @@ template <int DT> static int launch_dt(QmmDArgs& a, int bits, uint32_t kgroups, 
 #undef QD_G1
 #undef QD_G
     }
-    hipError_t e = set_max_dynamic_lds(fn, (size_t)shmem);
-    if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(max dynamic LDS)");
-    void* args[] = {&a};
-    if (a.ksplit > 1 && !grouped) {
-        LaunchCtx l1 = lc, l2 = lc;
-        l1.stop = nullptr;
-        l2.start = nullptr;
-        e = launch_kernel(fn, dim3(a.m_tiles * a.n_tiles, a.ksplit), dim3(kgroups == 1 ? 256 : 512), args, shmem, l1);
-        if (e != hipSuccess) return hip_fail(e, "qmm direct kernel launch");
-        const float* part = a.part;
-        void* out = a.out;
-        uint32_t total = a.M * a.N, ks = a.ksplit;
-        void* rargs[] = {&part, &out, &total, &ks};
-        e = launch_kernel((const void*)qmm_split_reduce_kernel<DT>, dim3((total + 255) / 256), dim3(256), rargs, 0, l2);
-        if (e != hipSuccess) return hip_fail(e, "qmm split reduce kernel launch");
-        return ERR_OK;
-    }
-    e = launch_kernel(fn, dim3(a.m_tiles * a.n_tiles), dim3(kgroups == 1 ? 256 : 512), args, shmem, lc);
-    if (e != hipSuccess) return hip_fail(e, "qmm direct kernel launch");
+    l.fn = fn;
+    l.shmem = shmem;
     return ERR_OK;
 }
 
@@ -386,7 +433,7 @@ size_t qmm_direct_scratch_bytes(const QmmParams& p) {
     return (size_t)pl.ksplit * p.M * p.N * sizeof(float);
 }
 
-int launch_qmm_direct(const QmmParams& p, const LaunchCtx& lc, void* scratch) {
+static int choose_direct(const QmmParams& p, void* scratch, QmmDLaunch& l) {
     QmmDPlan pl;
     int rc = plan_direct(p, pl);
     if (rc) return rc;
@@ -401,9 +448,8 @@ int launch_qmm_direct(const QmmParams& p, const LaunchCtx& lc, void* scratch) {
     a.M = p.M;
     a.N = p.N;
     a.K = p.K;
-    uint32_t l = 0;
-    while ((1u << l) < G) l++;
-    a.log2g = l;
+    a.log2g = 0;
+    while ((1u << a.log2g) < G) a.log2g++;
     a.gpr = p.K / G;
     a.m_tile_rows = rows;
     // Workgroup ids congruent mod 8 share an XCD and its L2. Whichever operand is smaller is
@@ -421,7 +467,48 @@ int launch_qmm_direct(const QmmParams& p, const LaunchCtx& lc, void* scratch) {
     a.tiles = nullptr;
     a.rowlist = nullptr;
     a.w_expert_bytes = a.sb_expert_elems = 0;
-    return p.dtype == DT_BF16 ? launch_dt<DT_BF16>(a, p.bits, kgroups, lc) : launch_dt<DT_F16>(a, p.bits, kgroups, lc);
+    return p.dtype == DT_BF16 ? choose_dt<DT_BF16>(a, p.bits, kgroups, l) : choose_dt<DT_F16>(a, p.bits, kgroups, l);
+}
+
+int launch_qmm_direct(const QmmParams& p, const LaunchCtx& lc, void* scratch) {
+    QmmDLaunch l;
+    const int rc = choose_direct(p, scratch, l);
+    return rc ? rc : qd_issue(p.dtype, &l, 1, lc);
+}
+
+bool qmm_direct_takes(const QmmParams& p) {
+    QmmDPlan pl;
+    QmmDLaunch l;
+    return plan_direct(p, pl) == ERR_OK && choose_direct(p, const_cast<QmmParams*>(&p), l) == ERR_OK;   // (any address stands for the scratch: nothing is launched)
+}
+
+// Each matrix's tiling, K split and arithmetic are those of its own call, and matrices that so come to the same kernel share
+// its launch: one matrix of a layer is often too few tiles for the chip. us, one launch each -> together: 6-bit codes, 77 rows,
+// (3584 + 2 x 512) x 3584 60.2 -> 22.0, 2 x 18944 x 3584 102 -> 82.7; 4-bit codes, 512 rows, 2 x 1024 x 4096 (K and V, split
+// K, with the additions) 39.2 -> 33.1; 2 x 14336 x 4096 (224 tiles each of 256 compute units) 149.4 -> 149.7.
+size_t qmm_direct_batch_scratch_bytes(const QmmParams* p, int n) {
+    size_t b = 0;
+    for (int i = 0; i < n; i++) b += (qmm_direct_scratch_bytes(p[i]) + 255) & ~(size_t)255;
+    return b;
+}
+
+int launch_qmm_direct_batch(const QmmParams* p, int n, const LaunchCtx& lc, void* scratch) {
+    QmmDLaunch l[4];
+    char* at = (char*)scratch;
+    for (int i = 0; i < n; i++) {
+        const size_t need = qmm_direct_scratch_bytes(p[i]);
+        const int rc = choose_direct(p[i], need ? at : nullptr, l[i]);
+        if (rc) return rc;
+        at += (need + 255) & ~(size_t)255;
+    }
+    // matrices of one kernel side by side
+    for (int i = 0; i + 1 < n; i++)
+        for (int j = i + 1; j < n; j++)
+            if (qd_same_launch(l[i], l[j])) {
+                std::swap(l[i + 1], l[j]);
+                break;
+            }
+    return qd_issue(p[0].dtype, l, n, lc);
 }
 
 // ---- expert-routed rows on the tile kernel ---------------------------------------------------
@@ -595,7 +682,9 @@ int launch_qmm_grouped(const QmmParams& p, const uint32_t* route, bool per_row_i
     a.rowlist = rowlist;
     a.w_expert_bytes = (uint64_t)p.N * p.K * p.bits / 8;
     a.sb_expert_elems = (uint64_t)p.N * a.gpr;
-    return p.dtype == DT_BF16 ? launch_dt<DT_BF16>(a, p.bits, kgroups, last, true) : launch_dt<DT_F16>(a, p.bits, kgroups, last, true);
+    QmmDLaunch ql;
+    rc = p.dtype == DT_BF16 ? choose_dt<DT_BF16>(a, p.bits, kgroups, ql, true) : choose_dt<DT_F16>(a, p.bits, kgroups, ql, true);
+    return rc ? rc : qd_issue(p.dtype, &ql, 1, last);
 }
 
 }  // namespace mtq

@@ -38,6 +38,34 @@ struct QmmDArgs {
     float* part;
 };
 
+// Further matrices of the same launch (the projections of a layer against the same rows): their workgroups (blockIdx.x)
+// follow the first matrix's, on the same tiling, rows, K and K split.
+struct QmmDMore {
+    uint32_t n = 0;                                       // 0..3
+    uint32_t first[3] = {~0u, ~0u, ~0u};                  // first workgroup of each
+    uint32_t N[3] = {}, n_tiles[3] = {}, by_m[3] = {};
+    const unsigned char *w[3] = {}, *scales[3] = {}, *biases[3] = {};
+    void* out[3] = {};
+    float* part[3] = {};
+};
+// Makes `a` this workgroup's matrix; returns the workgroup's number among the matrix's.
+__device__ __forceinline__ uint32_t qd_matrix(QmmDArgs& a, const QmmDMore& more) {
+    uint32_t id = blockIdx.x;
+    if (id >= more.first[0]) {
+        const uint32_t i = __builtin_amdgcn_readfirstlane((id >= more.first[1] ? 1u : 0u) + (id >= more.first[2] ? 1u : 0u));
+        a.w = more.w[i];
+        a.scales = more.scales[i];
+        a.biases = more.biases[i];
+        a.out = more.out[i];
+        a.part = more.part[i];
+        a.N = more.N[i];
+        a.n_tiles = more.n_tiles[i];
+        a.by_m = more.by_m[i];
+        id -= more.first[i];
+    }
+    return id;
+}
+
 
 // MB = 32-row activation blocks per wave (tile height DBM = 32*MB): every
 // converted weight fragment feeds MB MFMAs, so the conversion cost per MFMA
@@ -54,7 +82,7 @@ struct QmmDArgs {
 // 64 k per iteration and no partial sums to combine. Two such workgroups share a compute unit
 // and are not in step with each other, so one's LDS traffic runs under the other's MFMAs.
 template <int DT, int BITS, int PD, int MB, bool SBL, int KG, bool GR = false, bool SP = false>
-__global__ __launch_bounds__(KG == 1 ? 256 : 512) void qmm_direct_kernel(QmmDArgs a) {
+__global__ __launch_bounds__(KG == 1 ? 256 : 512) void qmm_direct_kernel(QmmDArgs a, QmmDMore more) {
     constexpr int NW = KG == 1 ? 4 : 8;      // waves
     constexpr int NT = 64 * NW;              // threads
     constexpr int NWV = NW / KG;             // N-waves
@@ -72,9 +100,10 @@ __global__ __launch_bounds__(KG == 1 ? 256 : 512) void qmm_direct_kernel(QmmDArg
     const uint32_t kg = wave / NWV, wn = wave % NWV;
     const uint32_t fr = lane & 31u, fh = lane >> 5;
 
-    const uint32_t total = a.m_tiles * a.n_tiles;
     uint32_t vid = blockIdx.x;
-    if (!GR && total % 8 == 0) vid = (blockIdx.x & 7u) * (total / 8) + (blockIdx.x >> 3);
+    if constexpr (!GR) vid = qd_matrix(a, more);
+    const uint32_t total = a.m_tiles * a.n_tiles;
+    if (!GR && total % 8 == 0) vid = (vid & 7u) * (total / 8) + (vid >> 3);
     uint32_t nt = a.by_m ? vid % a.n_tiles : vid / a.m_tiles, mt = a.by_m ? vid / a.n_tiles : vid % a.m_tiles;
     // rows of this tile: row j of the tile is row (row_first + j) of the row order, j < row_count
     uint32_t row_first = mt * DBM, row_count = a.M > row_first ? min((uint32_t)DBM, a.M - row_first) : 0u;

@@ -163,3 +163,30 @@ def test_argument_errors():
             ops.qmm_batched(dt, 4, G, [one] * n, [one] * n, [one] * n, one, [one] * n, Ns, M, K)
     ops.qmm_batched(dt, 4, 64, four[:2], four[:2], four[:2], one, four[:2], [8, 8], 0, 512)   # no rows: nothing to do
     one.free()
+
+
+@pytest.mark.parametrize("dt,bits,M,K,Ns", [
+    (DType.F16, 6, 77, 1024, (520, 136, 8, 4096)),      # one tiling, ragged last tiles, one launch
+    (DType.BF16, 4, 130, 4096, (1024, 256, 256)),       # split K: partial tiles of all in one addition
+    (DType.BF16, 4, 33, 4096, (130, 34, 2)),            # results that are not whole vectors of four
+    (DType.F16, 8, 200, 8192, (128, 1024, 128)),        # two tilings in turn
+], ids=str)
+def test_tiled_batch_shares_launches(dt, bits, M, K, Ns):
+    """Matrices whose tilings come to the same kernel share its launch; the bits are those of single calls (whose values
+    the tiling tests hold to the oracle)."""
+    print(f"[case] tiled batch {dt.name} b{bits} M{M} K{K} N={Ns}", flush=True)
+    G = 64
+    cases = [make_case(3300 + j + M, dt, bits, G, M, N, K, bias_rule="midpoint") for j, N in enumerate(Ns)]
+    xb = GpuBuffer.from_bytes(cases[0].x_bytes)
+    ws, ss, bs = ([GpuBuffer.from_bytes(v) for v in part] for part in zip(*((c.w.tobytes(), c.scales_bytes, c.biases_bytes) for c in cases)))
+    guard = b"\xcd" * 64
+    outs = [GpuBuffer.from_bytes(b"\xff" * (M * N * 2) + guard) for N in Ns]
+    single = GpuBuffer(M * max(Ns) * 2)
+    ops.qmm_batched(dt, bits, G, ws, ss, bs, xb, outs, list(Ns), M, K)
+    for j, N in enumerate(Ns):
+        raw = outs[j].read_bytes(M * N * 2 + 64)
+        ops.qmm(dt, bits, G, ws[j], ss[j], bs[j], xb, single, M, N, K)
+        assert raw[-64:] == guard and raw[:-64] == single.read_bytes(M * N * 2), j
+        assert np.all(np.isfinite(unpack_f32(raw[:-64], dt))), j
+    for b in [xb, single] + ws + ss + bs + outs:
+        b.free()
