@@ -54,20 +54,22 @@ template <int BITS> struct AffineGeom {
     static constexpr int NW = EPL * BITS / 32;  // packed words per lane
 };
 
-// EPL consecutive elements -> f32
+// EPL consecutive elements -> f32. What is quantised is read once: as a stream past the caches (14336 x 4096 f32, 4-bit codes,
+// quantised and read back, 118.6 -> 97.2 us; quantising alone 70 -> 49, 5.5 TB/s).
 template <int DT, int EPL> __device__ __forceinline__ void load_elems(const void* p, uint64_t i0, float (&v)[EPL]) {
     if constexpr (DT == DT_F32) {
-        const float4* s = (const float4*)((const float*)p + i0);
+        typedef float a_f32x4 __attribute__((ext_vector_type(4)));
+        const a_f32x4* s = (const a_f32x4*)((const float*)p + i0);
 #pragma unroll
         for (int j = 0; j < EPL / 4; j++) {
-            const float4 t = s[j];
+            const a_f32x4 t = __builtin_nontemporal_load(s + j);
             v[4 * j] = t.x; v[4 * j + 1] = t.y; v[4 * j + 2] = t.z; v[4 * j + 3] = t.w;
         }
     } else {
         const a_u32x4* s = (const a_u32x4*)((const uint16_t*)p + i0);
 #pragma unroll
         for (int j = 0; j < EPL / 8; j++) {
-            const a_u32x4 t = s[j];
+            const a_u32x4 t = __builtin_nontemporal_load(s + j);
 #pragma unroll
             for (int d = 0; d < 4; d++) {
                 if constexpr (DT == DT_BF16) {
