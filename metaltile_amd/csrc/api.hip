@@ -645,6 +645,15 @@ static int op_qmm_batched(int dtype, int bits, uint32_t G, int n, const void* co
     return ERR_OK;
 }
 
+static int run_wide_gather(const QmvParams& p, const LaunchCtx& lc) {
+    const size_t need = qmv_wide_gather_scratch_bytes(p);
+    if (need) {
+        int rc = ensure_scratch(g.scratch_held + need);
+        if (rc) return rc;
+    }
+    return launch_qmv_wide_gather(p, lc, need ? (char*)g.scratch_buf + g.scratch_held : nullptr);
+}
+
 static int op_gather(int mode, int dtype, int bits, uint32_t G, const void* x, const void* w,
                      const void* s, const void* b, const uint32_t* route, void* out, uint32_t T,
                      uint32_t N, uint32_t K, uint32_t E, const LaunchCtx& lc, bool exact_only = false) {
@@ -683,7 +692,7 @@ static int op_gather(int mode, int dtype, int bits, uint32_t G, const void* x, c
     // (mt_moe_gather_qmm_int4* / _b*, crates/metaltile-std/src/ffai/moe.rs:358-433); the tile kernel rounds
     // that value to the element type first, so such a name stays on the GEMV kernels at any routing density.
     if (dtype != DT_F32 && mode != GATHER_SINGLE && options().gather_wide == 2) {
-        rc = launch_qmv_wide_gather(p, lc);
+        rc = run_wide_gather(p, lc);
         if (rc != ERR_UNSUPPORTED) return rc;
     }
     if (dtype != DT_F32 && mode != GATHER_SINGLE && gopt != 1 && (gopt == 2 || (!exact_only && (uint64_t)T > (uint64_t)8 * (E < T ? E : T)))) {
@@ -701,10 +710,11 @@ static int op_gather(int mode, int dtype, int bits, uint32_t G, const void* x, c
     // exact: the 16-row matrix-core GEMV, 16 rows of an expert per pass. 8 experts x 14336 x 4096, rows by random ids,
     // us, 8-row passes of the GEMV family -> this: 32 rows 58.6 -> 54.5 (CSR 63 -> 60), 64 rows 113 -> 56, 128 rows
     // 197 -> 105, 256 rows 345 -> 152 (the tiles, rounded weights: 82 and 99 at 128 and 256 rows). It loses below (16 rows
-    // 53 -> 54.5: a workgroup stages 16 rows whatever the expert has) and on small experts.
+    // 53 -> 54.5: a workgroup stages 16 rows whatever the expert has) and on small experts. Long rows (CSR) in K slices:
+    // 8 x 4096 x 14336, 32 rows by a router, 110 us on the GEMV family -> 73, the addition of the slices' partial rows included.
     if (dtype != DT_F32 && mode != GATHER_SINGLE && options().gather_wide == 0 && (uint64_t)N * K >= (1ull << 24) &&
         (uint64_t)T >= (uint64_t)4 * (E < T ? E : T)) {
-        rc = launch_qmv_wide_gather(p, lc);
+        rc = run_wide_gather(p, lc);
         if (rc != ERR_UNSUPPORTED) return rc;
     }
     return run_gemv(p, lc);

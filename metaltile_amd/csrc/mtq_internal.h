@@ -189,7 +189,9 @@ bool qmv_wide_takes(const QmmParams& p);
 size_t qmv_wide_scratch_bytes(const QmmParams& p);
 int launch_qmv_wide(const QmmParams& p, const LaunchCtx& lc, void* scratch);
 // The same kernel on expert-routed rows (p.gather = GATHER_CSR / GATHER_INDICES), 16 rows of an expert per pass.
-int launch_qmv_wide_gather(const QmvParams& p, const LaunchCtx& lc);
+// scratch: qmv_wide_gather_scratch_bytes(p) bytes (0 when K is not split: then scratch may be null).
+size_t qmv_wide_gather_scratch_bytes(const QmvParams& p);
+int launch_qmv_wide_gather(const QmvParams& p, const LaunchCtx& lc, void* scratch);
 // K-run matrix-core GEMV (qmv_runs.hip): up to 16 activation rows (p.M, p.x, dtype, bits, group size, K; b: the matrices, 1..4
 // of them in one launch), f16 / bf16, 4- and 8-bit codes, K % 128 == 0. A matrix gives the same bits alone and in a batch.
 bool qmv_runs_takes(const QmvParams& p, const QmvBatch& b);

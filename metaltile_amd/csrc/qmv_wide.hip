@@ -13,6 +13,13 @@ template <int DT> __global__ __launch_bounds__(256) void qmv_wide_reduce_kernel(
     ((uint16_t*)out)[i] = f32_to_elem_bits<DT>(r);
 }
 
+static int wide_reduce(int dtype, const float* part, void* out, uint32_t total, uint32_t ks, const LaunchCtx& lc) {
+    void* args[] = {&part, &out, &total, &ks};
+    const void* fn = dtype == DT_BF16 ? (const void*)qmv_wide_reduce_kernel<DT_BF16> : (const void*)qmv_wide_reduce_kernel<DT_F16>;
+    hipError_t e = launch_kernel(fn, dim3((total + 255) / 256), dim3(256), args, 0, lc);
+    return e == hipSuccess ? ERR_OK : hip_fail(e, "wide qmv reduce kernel launch");
+}
+
 struct QmvWPlan {
     uint32_t kslice, ksplit, nb, kp, log2kp, tpk, sets, grid_x;
     size_t lds;
@@ -134,43 +141,51 @@ int launch_qmv_wide(const QmmParams& p, const LaunchCtx& lc, void* scratch) {
     if (pl.ksplit > 1) { l1.stop = nullptr; l2.start = nullptr; }
     e = launch_kernel(fn, dim3(pl.grid_x, pl.ksplit), dim3(1024), args, pl.lds, l1);
     if (e != hipSuccess) return hip_fail(e, "wide qmv kernel launch");
-    if (pl.ksplit > 1) {
-        const float* part = a.part;
-        void* out = a.out;
-        uint32_t total = p.M * p.N, ks = pl.ksplit;
-        void* rargs[] = {&part, &out, &total, &ks};
-        const void* rf = p.dtype == DT_BF16 ? (const void*)qmv_wide_reduce_kernel<DT_BF16> : (const void*)qmv_wide_reduce_kernel<DT_F16>;
-        e = launch_kernel(rf, dim3((total + 255) / 256), dim3(256), rargs, 0, l2);
-        if (e != hipSuccess) return hip_fail(e, "wide qmv reduce kernel launch");
-    }
-    return ERR_OK;
+    return pl.ksplit > 1 ? wide_reduce(p.dtype, a.part, a.out, p.M * p.N, pl.ksplit, l2) : ERR_OK;
 }
 
 // Expert-routed rows (CSR offsets or one expert id per row) on the same kernel: blockIdx.y is the expert, whose rows
 // are worked 16 per pass. Replaces mt_moe_gather_qmm_int4* (crates/metaltile-std/src/ffai/moe.rs:358-433) and the
-// decode side of the per-row-id gathers with the same exact-dequant arithmetic as the GEMV family. Groups of 64 codes,
-// rows of at most 4608 codes (no K slices: their partial rows would need the routing on the host).
+// decode side of the per-row-id gathers with the same exact-dequant arithmetic as the GEMV family. Groups of 64 codes.
+// Rows of more than 4608 codes (a down projection) go in K slices (blockIdx.z), whose f32 partial rows a second launch
+// adds: by CSR offsets only, where every row of the call has an expert and so a sum to be written, and for up to 256 rows.
 const void* qmv_wide_gather_pick(int dtype, int mode, uint32_t nb, uint32_t sets);
 
-int launch_qmv_wide_gather(const QmvParams& p, const LaunchCtx& lc) {
+static int plan_wide_gather(const QmvParams& p, QmvWPlan& pl) {
     const uint32_t G = p.group_size;
     if (p.gather != GATHER_CSR && p.gather != GATHER_INDICES) return fail(ERR_UNSUPPORTED, "wide gather: routing view");
     if ((p.dtype != DT_F16 && p.dtype != DT_BF16) || p.bits != 4 || G != 64) return fail(ERR_UNSUPPORTED, "wide gather: 4-bit g64 f16 / bf16");
     if (p.N == 0 || p.K == 0 || p.K % 512 || p.E == 0 || p.T == 0 || !p.route) return fail(ERR_UNSUPPORTED, "wide gather: shape");
     if ((uintptr_t)p.w % 16 || (uintptr_t)p.x % 16 || (uintptr_t)p.scales % 16 || (uintptr_t)p.biases % 16) return fail(ERR_UNSUPPORTED, "wide gather: alignment");
     if ((uint64_t)p.N * p.K / 2 >= (1ull << 32) || (uint64_t)p.E >= 65536) return fail(ERR_UNSUPPORTED, "wide gather: size");
-    const uint32_t per_turn = wide_bytes_per_turn(G), turns = p.K / 512u;
-    if (turns > (160u * 1024u - 64u) / per_turn) return fail(ERR_UNSUPPORTED, "wide gather: rows too long for one slice");
-    QmvWPlan pl;
-    pl.kslice = p.K;
-    pl.ksplit = 1;
-    pl.lds = (size_t)turns * per_turn;
+    const uint32_t per_turn = wide_bytes_per_turn(G), turns = p.K / 512u, max_turns = (160u * 1024u - 64u) / per_turn;
+    uint32_t ks = (turns + max_turns - 1) / max_turns;
+    if (ks > 1 && (p.gather != GATHER_CSR || p.T > 256 || ks > 16 || (uint64_t)p.T * p.N >= (1ull << 31))) return fail(ERR_UNSUPPORTED, "wide gather: rows too long for one slice");
+    const uint32_t tps = (turns + ks - 1) / ks;
+    ks = (turns + tps - 1) / tps;
+    pl.kslice = tps * 512u;
+    pl.ksplit = ks;
+    pl.lds = (size_t)tps * per_turn;
     const uint32_t e_eff = p.E < p.T ? p.E : p.T;
-    const uint32_t cus = (uint32_t)wide_cus(), want = cus / e_eff > 0 ? cus / e_eff : 1u;
-    if (!wide_geometry(G, turns, (p.N + 15u) / 16u, want, pl)) return fail(ERR_UNSUPPORTED, "wide gather: geometry");
+    const uint32_t cus = (uint32_t)wide_cus(), want = cus / (e_eff * ks) > 0 ? cus / (e_eff * ks) : 1u;
+    if (!wide_geometry(G, tps, (p.N + 15u) / 16u, want, pl)) return fail(ERR_UNSUPPORTED, "wide gather: geometry");
     if (p.gather == GATHER_INDICES) pl.lds += (size_t)p.T * 4;
     // (the kernel's statically allocated row counter shares the 160 KB with the dynamic part)
     if (pl.lds + 64 > 160 * 1024) return fail(ERR_UNSUPPORTED, "wide gather: the row list does not fit LDS");
+    return ERR_OK;
+}
+
+size_t qmv_wide_gather_scratch_bytes(const QmvParams& p) {
+    QmvWPlan pl;
+    return plan_wide_gather(p, pl) == ERR_OK && pl.ksplit > 1 ? (size_t)pl.ksplit * p.T * p.N * sizeof(float) : 0;
+}
+
+int launch_qmv_wide_gather(const QmvParams& p, const LaunchCtx& lc, void* scratch) {
+    const uint32_t G = p.group_size;
+    QmvWPlan pl;
+    const int rc = plan_wide_gather(p, pl);
+    if (rc) return rc;
+    if (pl.ksplit > 1 && !scratch) return fail(ERR_BAD_ARG, "wide gather: K slices without a scratch buffer");
     const void* fn = qmv_wide_gather_pick(p.dtype, p.gather, pl.nb, pl.sets);
     if (!fn) return fail(ERR_UNSUPPORTED, "wide gather: geometry not built");
     QmvWArgs a;
@@ -179,7 +194,7 @@ int launch_qmv_wide_gather(const QmvParams& p, const LaunchCtx& lc) {
     a.biases = (const uint16_t*)p.biases;
     a.x = (const uint16_t*)p.x;
     a.out = p.out;
-    a.part = nullptr;
+    a.part = (float*)scratch;
     a.M = p.T;
     a.N = p.N;
     a.K = p.K;
@@ -194,9 +209,11 @@ int launch_qmv_wide_gather(const QmvParams& p, const LaunchCtx& lc) {
     hipError_t e = set_max_dynamic_lds(fn, pl.lds);
     if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(max dynamic LDS)");
     void* args[] = {&a};
-    e = launch_kernel(fn, dim3(pl.grid_x, p.E), dim3(1024), args, pl.lds, lc);
+    LaunchCtx l1 = lc, l2 = lc;
+    if (pl.ksplit > 1) { l1.stop = nullptr; l2.start = nullptr; }
+    e = launch_kernel(fn, dim3(pl.grid_x, p.E, pl.ksplit), dim3(1024), args, pl.lds, l1);
     if (e != hipSuccess) return hip_fail(e, "wide gather kernel launch");
-    return ERR_OK;
+    return pl.ksplit > 1 ? wide_reduce(p.dtype, a.part, p.out, p.T * p.N, pl.ksplit, l2) : ERR_OK;
 }
 
 }  // namespace mtq

@@ -37,9 +37,9 @@ struct QmvWArgs {
     const uint16_t* biases;
     const uint16_t* x;
     void* out;
-    float* part;          // [ksplit][M][N] when gridDim.y > 1
+    float* part;          // [ksplit][M][N] when K is cut into slices (gridDim.y, of gathers gridDim.z, > 1)
     uint32_t M, N, K, gpr;
-    uint32_t kslice;      // codes per K slice (blockIdx.y), a multiple of 512
+    uint32_t kslice;      // codes per K slice (blockIdx.y, of gathers blockIdx.z), a multiple of 512
     uint32_t kp, log2kp;  // waves that share a wave's row blocks, each with a run of the slice's turns (a power of two)
     uint32_t tpk;         // turns per such wave
     const uint32_t* route;   // gathers: CSR offsets [E + 1] or one expert id per row [T]; blockIdx.y is the expert
@@ -140,7 +140,7 @@ template <int DT, int G, int NB, int SETS, int MODE = GATHER_NONE> __global__ __
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t j = lane & 15u, q = lane >> 4;
     constexpr bool GATHER = MODE != GATHER_NONE;
-    const uint32_t k0 = GATHER ? 0u : blockIdx.y * a.kslice, klen = min(a.kslice, a.K - k0);
+    const uint32_t k0 = (GATHER ? blockIdx.z : blockIdx.y) * a.kslice, klen = min(a.kslice, a.K - k0);
     const uint32_t turns = klen / 512u, ng = klen / (uint32_t)G;
     qw_u32x4* XL = (qw_u32x4*)lds;                                   // [klen / 8 pieces][16 rows]
     float* XG = (float*)(lds + (size_t)(klen / 8u) * 256u);          // [ng][16 rows]
@@ -490,7 +490,7 @@ template <int DT, int G, int NB, int SETS, int MODE = GATHER_NONE> __global__ __
             for (int i = 0; i < NB; i++) {
                 const uint32_t wrow = (rb0 + i) * 16u + jp;   // (worked out again: one register fewer across the stream)
                 if (wrow >= a.N) continue;
-                if (!GATHER && gridDim.y > 1) a.part[((size_t)blockIdx.y * a.M + orow) * a.N + wrow] = tot[i][r];
+                if ((GATHER ? gridDim.z : gridDim.y) > 1) a.part[((size_t)(GATHER ? blockIdx.z : blockIdx.y) * a.M + orow) * a.N + wrow] = tot[i][r];
                 else ((uint16_t*)a.out)[(size_t)orow * a.N + wrow] = f32_to_elem_bits<DT>(tot[i][r]);
             }
         }

@@ -143,3 +143,26 @@ def test_wide_gather(oracle, wide_gather, dt, N, K, counts, kp, nb):
     assert rel_err(got[1:].reshape(-1), exp[perm][1:].reshape(-1)) <= 1e-2, "permuted ids"
     for buf in (w, s, b, x, xb, r, out):
         buf.free()
+
+
+@pytest.mark.parametrize("dt", [DType.F16, DType.BF16], ids=lambda d: d.name)
+@pytest.mark.parametrize("N,K,counts,tail", [(144, 5120, (3, 0, 17, 1), 0), (40, 14336, (0, 16, 2), 5), (4096, 9216, (20, 12, 0), 0)])
+def test_wide_gather_in_k_slices(oracle, wide_gather, dt, N, K, counts, tail):
+    """Rows longer than one slice, by CSR offsets: partial rows of every slice, an expert without rows, more than 16 rows, rows
+    past the last offset (expert 0's), against the f64-accumulated oracle: 1e-2, the bound of the exact-dequant kernels."""
+    bits, G, E, T = 4, 64, len(counts), sum(counts) + tail
+    wide_gather(0, 0)
+    offsets = np.concatenate([[0], np.cumsum(counts)]).astype("<u4")
+    c = make_case(77, dt, bits, G, T, N, K, E=E)
+    print(f"[case] wide gather in K slices {dt.name} N{N} K{K} counts={counts} tail={tail}", flush=True)
+    rc, launches, scratch, _ = ops.plan("gather_csr", dt, bits, G, 1, N, K, E, T)
+    assert rc == 0 and "qmv_wide_kernel" in launches[0][0] and launches[0][1][2] > 1 and "qmv_wide_reduce" in launches[1][0]
+    assert scratch >= launches[0][1][2] * T * N * 4
+    bufs = [GpuBuffer.from_bytes(v) for v in (c.x_bytes, c.w.tobytes(), c.scales_bytes, c.biases_bytes, offsets.tobytes())]
+    out = GpuBuffer.from_bytes(b"\xff" * (T * N * 2) + b"\xcd" * 64)
+    ops.gather_qmv_csr(dt, bits, G, *bufs, out, T, N, K, E)
+    raw = out.read_bytes(T * N * 2 + 64)
+    exp = oracle.gather_qmm(c.x_f, c.w, c.scales_f, c.biases_f, T, K, N, E, bits, G, expert_offsets=offsets, f64=True, threads=8)
+    assert raw[-64:] == b"\xcd" * 64 and rel_err(unpack_f32(raw[:-64], dt), exp) <= 1e-2
+    for b in bufs + [out]:
+        b.free()
