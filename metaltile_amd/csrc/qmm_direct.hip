@@ -96,13 +96,24 @@ struct QmmDLaunch {
 static bool qd_same_launch(const QmmDLaunch& p, const QmmDLaunch& q) {
     return p.fn == q.fn && p.block == q.block && p.split == q.split && p.a.ksplit == q.a.ksplit && p.a.iters_per_split == q.a.iters_per_split && !p.a.tiles && !q.a.tiles;
 }
+// Whether a matrix of `more` workgroups behind `have` of them comes in under fewer rounds than in a launch of its own. The 8-wave
+// workgroups have a compute unit each, and full rounds cost the same in either (16640 x 7680 twice, 72 rows, 130 tiles each:
+// 1 % slower together, with the clock down and four tiles in a round of their own); the 4-wave ones share compute units.
+static bool qd_saves_round(const QmmDLaunch& l, uint32_t have, uint32_t more) {
+    if (l.block != 512) return true;
+    int dev = 0, cus = 256;
+    if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    const uint64_t ks = l.split ? l.a.ksplit : 1, c = (uint64_t)cus;
+    auto rounds = [&](uint64_t wgs) { return (wgs * ks + c - 1) / c; };
+    return rounds((uint64_t)have + more) < rounds(have) + rounds(more);
+}
 static int qd_issue(int dtype, const QmmDLaunch* l, int n, const LaunchCtx& lc) {
     for (int i = 0, j; i < n; i = j) {
         QmmDArgs a = l[i].a;
-        QmmDMore more;
+        QmmDMore& more = a.more;
         uint32_t wgs = l[i].grid;
         size_t shmem = l[i].shmem;
-        for (j = i + 1; j < n && j - i < 4 && qd_same_launch(l[i], l[j]); j++) {
+        for (j = i + 1; j < n && j - i < 4 && qd_same_launch(l[i], l[j]) && qd_saves_round(l[i], wgs, l[j].grid); j++) {
             const uint32_t k = more.n++;
             const QmmDArgs& o = l[j].a;
             more.first[k] = wgs;
@@ -113,7 +124,7 @@ static int qd_issue(int dtype, const QmmDLaunch* l, int n, const LaunchCtx& lc) 
         }
         hipError_t e = set_max_dynamic_lds(l[i].fn, shmem);
         if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(max dynamic LDS)");
-        void* args[] = {&a, &more};
+        void* args[] = {&a};
         LaunchCtx l1 = lc, l2 = lc;
         if (i) l1.start = l2.start = nullptr;
         if (j < n) l1.stop = l2.stop = nullptr;
@@ -375,6 +386,10 @@ static int plan_direct(const QmmParams& p, QmmDPlan& pl) {
         }
         if (dma_ks) { rows = 128; kgroups = 2; }
     }
+    // The bit-stream widths are bound by the conversion of codes: at 65..128 rows a 64-row tile converts every weight twice.
+    // Long rows take 128-row tiles, K split to fill the chip (us, 64 x 64 tiles -> these: 3584 x 18944, 6-bit codes, 77 / 128
+    // rows 70.6 / 72.8 -> 47.3 / 49.5, 3-bit, 100 rows 58.4 -> 42.5; at K = 8192 they lose, 2048 columns 19.7 -> 23.8).
+    if (odd_bits && p.M > 64 && p.M <= 128 && p.K > 8192 && tall_wide >= 24 && tall_wide * 2 <= (uint64_t)cus) { rows = 128; kgroups = 1; }
     if (options().qmm_tile_rows) rows = (uint32_t)options().qmm_tile_rows;
     if (options().qmm_kgroups) kgroups = (uint32_t)options().qmm_kgroups;
     // An iteration covers 64 k per K-group: K must be a multiple of 64 * K-groups (an odd number of
@@ -407,6 +422,12 @@ static int plan_direct(const QmmParams& p, QmmDPlan& pl) {
         // tall tiles on long rows: splits to about two 4-wave workgroups per compute unit, rounded
         ks = (uint32_t)((4 * (uint64_t)cus / tiles + 1) / 2);
         if (ks > 8) ks = 8;
+        if (ks > iters / 16) ks = iters / 16;
+    } else if (options().qmm_ksplit == 0 && odd_bits && rows == 128 && kgroups == 1 && p.M <= 128 && tiles < (uint64_t)cus && tiles * 2 > (uint64_t)cus) {
+        // a 4-wave workgroup converting codes keeps a compute unit busy by itself: fewer of them than compute units are
+        // split in K (18944 x 3584, 148 tiles, 1 / 2 / 3 / 4 splits, 6-bit codes: 77 rows 50.9 / 49.3 / 41.4 / 46.6 us, 128
+        // rows 49.9 / 52.3 / 45.8 / 53.0; 3-bit, 100 rows 40.6 / 43.2 / 38.8 / 44.0)
+        ks = (uint32_t)(7 * (uint64_t)cus / (4 * tiles));
         if (ks > iters / 16) ks = iters / 16;
     } else if (options().qmm_ksplit == 0 && kgroups != 2 && tiles * 2 <= (uint64_t)cus && iters >= QMM_SPLIT_MIN_ITERS) {
         // one workgroup per compute unit, at least 4 iterations each (measured optimum: 4096 x 14336,
@@ -485,7 +506,7 @@ bool qmm_direct_takes(const QmmParams& p) {
 // Each matrix's tiling, K split and arithmetic are those of its own call, and matrices that so come to the same kernel share
 // its launch: one matrix of a layer is often too few tiles for the chip. us, one launch each -> together: 6-bit codes, 77 rows,
 // (3584 + 2 x 512) x 3584 60.2 -> 22.0, 2 x 18944 x 3584 102 -> 82.7; 4-bit codes, 512 rows, 2 x 1024 x 4096 (K and V, split
-// K, with the additions) 39.2 -> 33.1; 2 x 14336 x 4096 (224 tiles each of 256 compute units) 149.4 -> 149.7.
+// K, with the additions) 39.2 -> 33.1; 2 x 14336 x 4096 (224 tiles each of 256 compute units) 149.4 -> 149.7: left apart.
 size_t qmm_direct_batch_scratch_bytes(const QmmParams* p, int n) {
     size_t b = 0;
     for (int i = 0; i < n; i++) b += (qmm_direct_scratch_bytes(p[i]) + 255) & ~(size_t)255;

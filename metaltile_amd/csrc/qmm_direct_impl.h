@@ -15,7 +15,7 @@ namespace mtq {
         __builtin_amdgcn_sched_barrier(0);  \
     } while (0)
 
-struct QmmDArgs {
+struct QmmDBase {
     const unsigned char* w;
     const unsigned char* scales;
     const unsigned char* biases;
@@ -48,8 +48,11 @@ struct QmmDMore {
     void* out[3] = {};
     float* part[3] = {};
 };
+struct QmmDArgs : QmmDBase {
+    QmmDMore more;
+};
 // Makes `a` this workgroup's matrix; returns the workgroup's number among the matrix's.
-__device__ __forceinline__ uint32_t qd_matrix(QmmDArgs& a, const QmmDMore& more) {
+__device__ __forceinline__ uint32_t qd_matrix(QmmDBase& a, const QmmDMore& more) {
     uint32_t id = blockIdx.x;
     if (id >= more.first[0]) {
         const uint32_t i = __builtin_amdgcn_readfirstlane((id >= more.first[1] ? 1u : 0u) + (id >= more.first[2] ? 1u : 0u));
@@ -82,7 +85,8 @@ __device__ __forceinline__ uint32_t qd_matrix(QmmDArgs& a, const QmmDMore& more)
 // 64 k per iteration and no partial sums to combine. Two such workgroups share a compute unit
 // and are not in step with each other, so one's LDS traffic runs under the other's MFMAs.
 template <int DT, int BITS, int PD, int MB, bool SBL, int KG, bool GR = false, bool SP = false>
-__global__ __launch_bounds__(KG == 1 ? 256 : 512) void qmm_direct_kernel(QmmDArgs a, QmmDMore more) {
+__global__ __launch_bounds__(KG == 1 ? 256 : 512) void qmm_direct_kernel(QmmDArgs args) {
+    QmmDBase a = args;
     constexpr int NW = KG == 1 ? 4 : 8;      // waves
     constexpr int NT = 64 * NW;              // threads
     constexpr int NWV = NW / KG;             // N-waves
@@ -101,7 +105,7 @@ __global__ __launch_bounds__(KG == 1 ? 256 : 512) void qmm_direct_kernel(QmmDArg
     const uint32_t fr = lane & 31u, fh = lane >> 5;
 
     uint32_t vid = blockIdx.x;
-    if constexpr (!GR) vid = qd_matrix(a, more);
+    if constexpr (!GR) vid = qd_matrix(a, args.more);
     const uint32_t total = a.m_tiles * a.n_tiles;
     if (!GR && total % 8 == 0) vid = (vid & 7u) * (total / 8) + (vid >> 3);
     uint32_t nt = a.by_m ? vid % a.n_tiles : vid / a.m_tiles, mt = a.by_m ? vid / a.n_tiles : vid % a.m_tiles;

@@ -130,7 +130,8 @@ template <int NBUF, int WSN, int IPW, int NWL, int NSB> struct QmmDmaWaits {
 // BITS: 4, or 8 (a lane's 32 codes are then 32 bytes: two 16-byte loads per iteration, bytes converted with the
 // byte-select converts; everything else alike).
 template <int DT, int MB, int KG, int NW, int NB = 0, bool GR = false, bool SP = false, bool WIN = false, int BITS = 4>
-__global__ __launch_bounds__(64 * NW) void qmm_dma_kernel(QmmDArgs a, QmmDMore more) {
+__global__ __launch_bounds__(64 * NW) void qmm_dma_kernel(QmmDArgs args) {
+    QmmDBase a = args;
     static_assert(NW == 8 || NW == 16, "two or four waves per SIMD");
     static_assert(KG == 2 || KG == 4, "2 or 4 K-groups");
     static_assert(MB == 1 || MB == 2 || MB == 4 || MB == 8, "32 to 256 rows");
@@ -160,7 +161,7 @@ __global__ __launch_bounds__(64 * NW) void qmm_dma_kernel(QmmDArgs a, QmmDMore m
     const uint32_t fr = lane & 31u, fh = lane >> 5;
 
     uint32_t vid = blockIdx.x;
-    if constexpr (!GR) vid = qd_matrix(a, more);
+    if constexpr (!GR) vid = qd_matrix(a, args.more);
     const uint32_t total = a.m_tiles * a.n_tiles;
     if (!GR && total % 8 == 0) vid = (vid & 7u) * (total / 8) + (vid >> 3);
     uint32_t nt = a.by_m ? vid % a.n_tiles : vid / a.m_tiles, mt = a.by_m ? vid / a.n_tiles : vid % a.m_tiles;

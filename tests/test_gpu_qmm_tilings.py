@@ -421,3 +421,30 @@ def test_load_to_lds_tiles_with_k_split(oracle, options, dt, M, N, K, G, bits):
                 assert float(np.abs(got[ksplit] - got[1]).max()) <= (2.0 ** -7 if dt == DType.BF16 else 2.0 ** -10) * scale * 2
     for buf in (w, s, b, x):
         buf.free()
+
+
+@pytest.mark.parametrize("dt,bits,M,N,K,ksplit", [
+    (DType.F16, 6, 65, 3080, 8512, 8), (DType.BF16, 3, 128, 3200, 8320, 8),      # long rows: 128-row tiles, K split
+    (DType.F16, 5, 77, 17000, 2048, 2), (DType.BF16, 6, 128, 16520, 3136, 3),    # fewer 4-wave workgroups than compute units
+], ids=str)
+def test_bit_stream_widths_at_65_to_128_rows(oracle, dt, bits, M, N, K, ksplit):
+    """The tilings the 3-, 5- and 6-bit codes take at 65..128 rows, ragged last tiles and splits: 2e-2 against the oracle's
+    mt_qmm_mma arithmetic (rounded weights), on the first, last and some other columns."""
+    G, odt = 64, {DType.F16: 1, DType.BF16: 2}[dt]
+    print(f"[case] qmm {dt.name} b{bits} M{M} N{N} K{K}", flush=True)
+    rc, launches, _, _ = ops.plan("qmm", dt, bits, G, M, N, K)
+    assert rc == 0 and "4, " in launches[0][0] and launches[0][1][1] == ksplit and launches[0][2][0] == 256, launches
+    c = make_case(4400 + M, dt, bits, G, M, N, K, bias_rule="midpoint")
+    bufs = [GpuBuffer.from_bytes(v) for v in (c.w.tobytes(), c.scales_bytes, c.biases_bytes, c.x_bytes)]
+    out = GpuBuffer.from_bytes(b"\xff" * (M * N * 2) + b"\xcd" * 64)
+    ops.qmm(dt, bits, G, *bufs, out, M, N, K)
+    raw = out.read_bytes(M * N * 2 + 64)
+    got = unpack_f32(raw[:-64], dt).reshape(M, N)
+    assert raw[-64:] == b"\xcd" * 64 and np.all(np.isfinite(got))
+    for lo, hi in ((0, 160), (N // 2, N // 2 + 64), (N - 150, N)):
+        w = c.w.reshape(N, -1)[lo:hi].reshape(-1).copy()
+        s, b = (v.reshape(N, -1)[lo:hi].reshape(-1).copy() for v in (c.scales_f, c.biases_f))
+        exp = oracle.qmm_mma(w, s, b, c.x_f, M, hi - lo, K, bits, G, odt, threads=8).reshape(-1)
+        assert rel_err(got[:, lo:hi].reshape(-1), oracle.round_through(exp.astype(np.float32), odt)) <= 2e-2, (lo, hi)
+    for b in bufs + [out]:
+        b.free()
