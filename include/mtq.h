@@ -433,7 +433,8 @@ MTQ_API int mtq_flush_cache(void);
  *   "qmv.norm_mfma"        mtq_rms_norm_qmv with the norm applied inside the matrix-core GEMV (4-bit codes, f16 / bf16):
  *                          0 = where it is faster than the streaming kernel's fused form, 1 = never, 2 = wherever the
  *                          shape allows
- *   "gather.wide"          expert-routed rows on the 16-row matrix-core GEMV (4-bit g64 f16 / bf16, K <= 4608): 0 = where
+ *   "gather.wide"          expert-routed rows on the 16-row matrix-core GEMV (4-bit g64 f16 / bf16, K <= 4608; by CSR
+ *                          offsets longer rows too, in K slices, up to 256 rows of x): 0 = where
  *                          it is the fastest kernel (large experts, at least 4 rows per expert, below the tile
  *                          kernel's crossover or under an exact-dequant name), 1 = never, 2 = wherever the shape allows
  *   "qmv.runs"             K-run matrix-core GEMV for batches of up to 16 rows (4- and 8-bit codes, f16 / bf16, K % 128 == 0,
