@@ -7,7 +7,7 @@ about 2^-24 * 1024 * sqrt(K) * scale (0.1) = 6e-4 absolute. max |a-e| / max(|e|,
 import numpy as np
 import pytest
 
-from metaltile_amd import DType, GpuBuffer, ops, unpack_f32
+from metaltile_amd import DType, GpuBuffer, ops, pack_f32, unpack_f32
 from metaltile_amd.runtime import _ensure_init
 from metaltile_amd.synth import make_case
 from tests.parity import rel_err
@@ -66,3 +66,50 @@ def test_mixed_batch_keeps_bits():
         assert got == singles[j].read_bytes(M * N * 2) and np.any(unpack_f32(got, dt) != 0.0), j
     for b in [x] + ws + ss + bs + outs + singles:
         b.free()
+
+
+@pytest.mark.parametrize("dt", [DType.F16, DType.BF16], ids=lambda d: d.name)
+@pytest.mark.parametrize("bits,G,M,N,K", [(4, 64, 16, 272, 4096), (4, 128, 9, 33, 5120), (4, 32, 3, 48, 2048), (8, 64, 12, 100, 3584), (8, 32, 5, 20, 1152)])
+def test_infinite_and_huge_activations(dt, bits, G, M, N, K):
+    """One infinite activation in a row makes its results infinities of the weight's sign, as a product with the weights does, and
+    a bf16 one of 1e37 (which the conversion's offset would carry past the f32 range) stays a number: the roundings of the weights
+    (2^-9 |w|, |w| about 0.08: 6e-3 rms on a sum of 4096) and of the result, to 3e-2. A NaN stays one. Rows without such a value
+    keep their bits."""
+    print(f"[case] K-run qmv, infinities {dt.name} b{bits} g{G} M{M} N{N} K{K}", flush=True)
+    lib = _ensure_init()
+    c = make_case(970 + M, dt, bits, G, M, N, K, bias_rule="midpoint")
+    plain = c.x_f.reshape(M, K).astype(np.float32)
+    x = plain.copy()
+    if dt == DType.BF16:
+        x[0, K - 1] = 1e37
+    x[1, K // 3] = np.inf
+    x[2, 5] = -np.inf
+    if M > 3:
+        x[M - 1, K // 2] = np.nan
+    codes = ((c.w.reshape(N, -1, 1) >> np.arange(0, 32, bits, dtype=np.uint32)) & ((1 << bits) - 1)).reshape(N, K).astype(np.float32)
+    s, b = (np.repeat(v.reshape(N, K // G), G, axis=1).astype(np.float32) for v in (c.scales_f, c.biases_f))
+    w = unpack_f32(pack_f32((codes * s + b).reshape(-1), dt), dt).reshape(N, K).astype(np.float64)
+    bufs = [GpuBuffer.from_bytes(v) for v in (c.w.tobytes(), c.scales_bytes, c.biases_bytes)]
+    got = []
+    try:
+        assert lib.mtq_set_option(b"qmv.runs", 2) == 0
+        assert "qmv_runs_kernel" in ops.plan("qmm", dt, bits, G, M, N, K)[1][0][0]
+        for v in (x, plain):
+            xb, out = GpuBuffer.from_bytes(pack_f32(v.reshape(-1), dt)), GpuBuffer(M * N * 2)
+            ops.qmm(dt, bits, G, *bufs, xb, out, M, N, K)
+            got.append(np.frombuffer(out.read_bytes(M * N * 2), dtype="<u2").reshape(M, N).copy())
+            xb.free()
+            out.free()
+    finally:
+        lib.mtq_set_option(b"qmv.runs", 0)
+        for v in bufs:
+            v.free()
+    values = unpack_f32(got[0].tobytes(), dt).reshape(M, N)
+    assert rel_err(values[0], w @ unpack_f32(pack_f32(x[0], dt), dt).astype(np.float64)) <= 3e-2
+    with np.errstate(invalid="ignore"):
+        for row, k in ((1, K // 3), (2, 5)):
+            np.testing.assert_array_equal(values[row], (w[:, k] * np.float64(x[row, k])).astype(np.float32))
+    rest = [m for m in range(M) if np.array_equal(x[m], plain[m])]
+    np.testing.assert_array_equal(got[0][rest], got[1][rest])
+    if M > 3:
+        assert np.all(np.isnan(values[M - 1]))
