@@ -102,6 +102,8 @@ struct State {
     void* scratch_buf = nullptr;     // library-owned scratch: normalised rows, qvm partial sums
     size_t scratch_bytes = 0;
     size_t scratch_held = 0;         // bytes at the front of scratch_buf that the running op keeps for itself
+    bool scratch_captured = false;   // a captured launch has scratch_buf's address: it lives until mtq_shutdown
+    std::vector<void*> scratch_old;  // earlier buffers that graphs still write to
     size_t flush_bytes = 0;
     uint64_t* probe_buf = nullptr;   // four u64 written by the clock probe
     hipDeviceProp_t prop;
@@ -379,10 +381,10 @@ static int op_qmm(int dtype, int bits, uint32_t G, const void* w, const void* s,
         q.w = w; q.scales = s; q.biases = b; q.x = x; q.out = out;
         q.M = M; q.N = N; q.K = K;
         if (options().qmm_kernel != 1) {
-            const size_t need = qmm_direct_scratch_bytes(q);  // f32 partial tiles when K is split
-            if (need) {
-                rc = ensure_scratch(g.scratch_held + need);
-                if (rc) return rc;
+            size_t need = qmm_direct_scratch_bytes(q);  // f32 partial tiles when K is split
+            if (need && ensure_scratch(g.scratch_held + need)) {
+                q.unsplit = true;   // no memory for them
+                need = 0;
             }
             rc = launch_qmm_direct(q, lc, need ? (char*)g.scratch_buf + g.scratch_held : nullptr);
             if (rc != ERR_UNSUPPORTED) return rc;
@@ -393,22 +395,40 @@ static int op_qmm(int dtype, int bits, uint32_t G, const void* w, const void* s,
     return op_qmv(dtype, bits, G, w, s, b, x, out, M, N, K, lc);
 }
 
-// Library-owned device scratch (normalised rows, qvm partial sums): grown on demand, never shrunk.
+// Library-owned device scratch (normalised rows, qvm partial sums, partial tiles): grown on demand, never shrunk. A buffer
+// that a captured launch was given stays allocated, since the graph writes to it at every replay; and while the stream is
+// being captured nothing is waited for or freed, and the allocation is made in the relaxed capture mode, in which it is
+// allowed. Every buffer that replaces a kept one is at least twice as large: those kept are less than the last one in all.
 static int ensure_scratch(size_t need) {
     if (g_plan.on) {  // mtq_plan has put a stand-in address into scratch_buf; nothing is allocated
         plan_note_scratch(need);
         return ERR_OK;
     }
-    if (g.scratch_bytes >= need) return ERR_OK;
-    if (g.scratch_buf) {
-        MTQ_HIP(hipStreamSynchronize(g.stream));  // earlier launches may still use the old buffer
-        MTQ_HIP(hipFree(g.scratch_buf));
-        g.scratch_buf = nullptr;
-        g.scratch_bytes = 0;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    MTQ_HIP(hipStreamIsCapturing(g.stream, &st));
+    const bool capturing = st != hipStreamCaptureStatusNone;
+    if (g.scratch_bytes < need) {
+        size_t cap = need < 65536 ? 65536 : need;
+        const bool keep = g.scratch_buf && (capturing || g.scratch_captured);
+        if (keep && cap < 2 * g.scratch_bytes) cap = 2 * g.scratch_bytes;
+        if (g.scratch_buf && !keep) {
+            MTQ_HIP(hipStreamSynchronize(g.stream));  // earlier launches may still use the old buffer
+            MTQ_HIP(hipFree(g.scratch_buf));
+            g.scratch_buf = nullptr;
+            g.scratch_bytes = 0;
+        }
+        void* p = nullptr;
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        if (capturing) MTQ_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+        const hipError_t e = hipMalloc(&p, cap);
+        if (capturing) MTQ_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+        if (e != hipSuccess) return hip_fail(e, "hipMalloc(scratch)");
+        if (keep) g.scratch_old.push_back(g.scratch_buf);
+        g.scratch_buf = p;
+        g.scratch_bytes = cap;
+        g.scratch_captured = false;
     }
-    const size_t cap = need < 65536 ? 65536 : need;
-    MTQ_HIP(hipMalloc(&g.scratch_buf, cap));
-    g.scratch_bytes = cap;
+    if (capturing) g.scratch_captured = true;
     return ERR_OK;
 }
 
@@ -617,12 +637,13 @@ static int op_qmm_batched(int dtype, int bits, uint32_t G, int n, const void* co
         if (on_tiles[j]) tiled[n_tiled++] = q;
         else left++;
     }
+    const size_t need = qmm_direct_batch_scratch_bytes(tiled, n_tiled);
+    if (need && ensure_scratch(g.scratch_held + need)) {   // no memory for all partial tiles at once: one matrix after the other
+        for (int j = 0; j < n; j++) on_tiles[j] = false;
+        left += n_tiled;
+        n_tiled = 0;
+    }
     if (n_tiled) {
-        const size_t need = qmm_direct_batch_scratch_bytes(tiled, n_tiled);
-        if (need) {
-            int rc = ensure_scratch(g.scratch_held + need);
-            if (rc) return rc;
-        }
         LaunchCtx l2 = lc;
         if (started) l2.start = nullptr;
         if (left) l2.stop = nullptr;
@@ -647,10 +668,7 @@ static int op_qmm_batched(int dtype, int bits, uint32_t G, int n, const void* co
 
 static int run_wide_gather(const QmvParams& p, const LaunchCtx& lc) {
     const size_t need = qmv_wide_gather_scratch_bytes(p);
-    if (need) {
-        int rc = ensure_scratch(g.scratch_held + need);
-        if (rc) return rc;
-    }
+    if (need && ensure_scratch(g.scratch_held + need)) return ERR_UNSUPPORTED;   // no memory for the partial rows: the GEMV family needs none
     return launch_qmv_wide_gather(p, lc, need ? (char*)g.scratch_buf + g.scratch_held : nullptr);
 }
 
@@ -1205,8 +1223,7 @@ int mtq_shutdown(void) {
     if (g.flush_buf) (void)hipFree(g.flush_buf);
     if (g.probe_buf) (void)hipFree(g.probe_buf);
     if (g.scratch_buf) (void)hipFree(g.scratch_buf);
-    g.scratch_buf = nullptr;
-    g.scratch_bytes = 0;
+    for (void* p : g.scratch_old) (void)hipFree(p);
     if (g.ev_start) (void)hipEventDestroy(g.ev_start);
     if (g.ev_stop) (void)hipEventDestroy(g.ev_stop);
     if (g.own_stream) (void)hipStreamDestroy(g.own_stream);

@@ -172,6 +172,7 @@ struct QmmParams {
     const void* x = nullptr;  // T [M][K]
     void* out = nullptr;      // T [M][N]
     uint32_t M = 0, N = 0, K = 0;
+    bool unsplit = false;     // no K split, and so no scratch
 };
 // Tiled MFMA GEMM with weights dequantised into LDS (qmm.hip).
 int launch_qmm_mfma(const QmmParams& p, const LaunchCtx& lc);

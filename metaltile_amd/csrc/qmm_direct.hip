@@ -293,6 +293,7 @@ struct QmmDPlan {
 
 // Checks the shape and picks the tile, the K-groups and the K split.
 static int plan_direct(const QmmParams& p, QmmDPlan& pl) {
+    const int ksplit_option = p.unsplit ? 1 : options().qmm_ksplit;
     if (p.dtype != DT_F16 && p.dtype != DT_BF16)
         return fail(ERR_UNSUPPORTED, "direct qmm: f16 / bf16 activations only");
     if (p.bits < 2 || p.bits > 8) return fail(ERR_UNSUPPORTED, "direct qmm: bits must be in 2..8");
@@ -376,7 +377,7 @@ static int plan_direct(const QmmParams& p, QmmDPlan& pl) {
     // 31.3 / 40.4 / 48.4 (128 rows lose, 22.0 -> 24.3); 5120 x 13824, 128 / 256 / 384 rows 47.9 / 70.7 / 92.2 -> 37.4 /
     // 55.6 / 75.9; 8192 x 28672 (a split's scales fit LDS from 4 splits on), 128 / 256 rows 163.5 / 184.4 -> 84.7 / 156.7.
     uint32_t dma_ks = 0;
-    if (!options().qmm_tile_rows && !options().qmm_kgroups && options().qmm_ksplit == 0 && p.K >= 8192 &&
+    if (!options().qmm_tile_rows && !options().qmm_kgroups && ksplit_option == 0 && p.K >= 8192 &&
         (p.M > 128 || (p.M > 96 && p.K > 8192)) && tall_wide * 2 <= (uint64_t)cus && (uint64_t)p.M * p.N < (1ull << 31)) {
         uint32_t ks = (uint32_t)((uint64_t)cus / tall_wide);
         ks = ks > 8 ? 8 : ks;
@@ -416,20 +417,20 @@ static int plan_direct(const QmmParams& p, QmmDPlan& pl) {
     const uint64_t tiles = (uint64_t)((p.M + rows - 1) / rows) * ((p.N + tile_cols - 1) / tile_cols);
     const uint32_t iters = p.K / (64 * kgroups);
     uint32_t ks = 1;
-    if (options().qmm_ksplit > 1) ks = (uint32_t)options().qmm_ksplit;
+    if (ksplit_option > 1) ks = (uint32_t)ksplit_option;
     else if (dma_ks) ks = dma_ks;
-    else if (options().qmm_ksplit == 0 && rows == 128 && kgroups == 1 && p.K >= 8192 && tiles < 2 * (uint64_t)cus) {
+    else if (ksplit_option == 0 && rows == 128 && kgroups == 1 && p.K >= 8192 && tiles < 2 * (uint64_t)cus) {
         // tall tiles on long rows: splits to about two 4-wave workgroups per compute unit, rounded
         ks = (uint32_t)((4 * (uint64_t)cus / tiles + 1) / 2);
         if (ks > 8) ks = 8;
         if (ks > iters / 16) ks = iters / 16;
-    } else if (options().qmm_ksplit == 0 && odd_bits && rows == 128 && kgroups == 1 && p.M <= 128 && tiles < (uint64_t)cus && tiles * 2 > (uint64_t)cus) {
+    } else if (ksplit_option == 0 && odd_bits && rows == 128 && kgroups == 1 && p.M <= 128 && tiles < (uint64_t)cus && tiles * 2 > (uint64_t)cus) {
         // a 4-wave workgroup converting codes keeps a compute unit busy by itself: fewer of them than compute units are
         // split in K (18944 x 3584, 148 tiles, 1 / 2 / 3 / 4 splits, 6-bit codes: 77 rows 50.9 / 49.3 / 41.4 / 46.6 us, 128
         // rows 49.9 / 52.3 / 45.8 / 53.0; 3-bit, 100 rows 40.6 / 43.2 / 38.8 / 44.0)
         ks = (uint32_t)(7 * (uint64_t)cus / (4 * tiles));
         if (ks > iters / 16) ks = iters / 16;
-    } else if (options().qmm_ksplit == 0 && kgroups != 2 && tiles * 2 <= (uint64_t)cus && iters >= QMM_SPLIT_MIN_ITERS) {
+    } else if (ksplit_option == 0 && kgroups != 2 && tiles * 2 <= (uint64_t)cus && iters >= QMM_SPLIT_MIN_ITERS) {
         // one workgroup per compute unit, at least 4 iterations each (measured optimum: 4096 x 14336,
         // 32 rows, 64 tiles: 1 / 2 / 4 / 8 / 16 splits 57 / 34 / 23 / 27 / 32 us; 2048 x 8192, 32 tiles:
         // 23 / 17 / 12 / 11 / 12 us; 8192 x 28672, 128 tiles: 108 / 63 / 62 / 66 / 80 us)
