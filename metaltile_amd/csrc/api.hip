@@ -17,6 +17,7 @@
 #include "../../include/mtq.h"
 #include "../../include/mtq_measure.h"
 #include "mtq_internal.h"
+#include "qmm_direct_plan.h"
 
 namespace mtq {
 
@@ -381,12 +382,13 @@ static int op_qmm(int dtype, int bits, uint32_t G, const void* w, const void* s,
         q.w = w; q.scales = s; q.biases = b; q.x = x; q.out = out;
         q.M = M; q.N = N; q.K = K;
         if (options().qmm_kernel != 1) {
-            size_t need = qmm_direct_scratch_bytes(q);  // f32 partial tiles when K is split
-            if (need && ensure_scratch(g.scratch_held + need)) {
-                q.unsplit = true;   // no memory for them
-                need = 0;
+            QmmDLaunch l;
+            rc = plan_qmm_direct(q, l);
+            if (rc == ERR_OK && l.scratch && ensure_scratch(g.scratch_held + l.scratch)) {
+                q.unsplit = true;   // no memory for the partial tiles
+                rc = plan_qmm_direct(q, l);
             }
-            rc = launch_qmm_direct(q, lc, need ? (char*)g.scratch_buf + g.scratch_held : nullptr);
+            if (rc == ERR_OK) rc = launch_qmm_direct(&l, 1, l.scratch ? (char*)g.scratch_buf + g.scratch_held : nullptr, lc);
             if (rc != ERR_UNSUPPORTED) return rc;
         }
         rc = launch_qmm_mfma(q, lc);
@@ -624,7 +626,8 @@ static int op_qmm_batched(int dtype, int bits, uint32_t G, int n, const void* co
     }
     // what is left of the batch on the tile kernels goes there together
     bool started = taken[0] || taken[1] || taken[2] || taken[3];
-    QmmParams tiled[4];
+    QmmDLaunch tiled[4];
+    size_t need = 0;   // bytes of their partial tiles
     int n_tiled = 0, left = 0;
     bool on_tiles[4] = {};
     for (int j = 0; j < n; j++) {
@@ -633,11 +636,11 @@ static int op_qmm_batched(int dtype, int bits, uint32_t G, int n, const void* co
         q.dtype = dtype; q.bits = bits; q.group_size = G;
         q.w = w[j]; q.scales = s[j]; q.biases = b[j]; q.x = x; q.out = outs[j];
         q.M = M; q.N = N[j]; q.K = K;
-        on_tiles[j] = !exact && dtype != DT_F32 && options().qmm_kernel != 1 && !wide_serves(q, false) && tiles_serve(bits, M, N[j], K) && qmm_direct_takes(q);
-        if (on_tiles[j]) tiled[n_tiled++] = q;
+        on_tiles[j] = !exact && dtype != DT_F32 && options().qmm_kernel != 1 && !wide_serves(q, false) && tiles_serve(bits, M, N[j], K) &&
+                      plan_qmm_direct(q, tiled[n_tiled]) == ERR_OK;
+        if (on_tiles[j]) need += tiled[n_tiled++].scratch;
         else left++;
     }
-    const size_t need = qmm_direct_batch_scratch_bytes(tiled, n_tiled);
     if (need && ensure_scratch(g.scratch_held + need)) {   // no memory for all partial tiles at once: one matrix after the other
         for (int j = 0; j < n; j++) on_tiles[j] = false;
         left += n_tiled;
@@ -647,7 +650,7 @@ static int op_qmm_batched(int dtype, int bits, uint32_t G, int n, const void* co
         LaunchCtx l2 = lc;
         if (started) l2.start = nullptr;
         if (left) l2.stop = nullptr;
-        int rc = launch_qmm_direct_batch(tiled, n_tiled, l2, need ? (char*)g.scratch_buf + g.scratch_held : nullptr);
+        int rc = launch_qmm_direct(tiled, n_tiled, need ? (char*)g.scratch_buf + g.scratch_held : nullptr, l2);
         if (rc) return rc;
         started = true;
     }

@@ -176,14 +176,6 @@ struct QmmParams {
 };
 // Tiled MFMA GEMM with weights dequantised into LDS (qmm.hip).
 int launch_qmm_mfma(const QmmParams& p, const LaunchCtx& lc);
-// 64x128 tiles, weights converted in MFMA operand registers, activations through LDS (qmm_direct.hip).
-// scratch: qmm_direct_scratch_bytes(p) bytes (0 when K is not split: then scratch may be null).
-size_t qmm_direct_scratch_bytes(const QmmParams& p);
-int launch_qmm_direct(const QmmParams& p, const LaunchCtx& lc, void* scratch);
-bool qmm_direct_takes(const QmmParams& p);
-// The same for up to four matrices against the same rows: those whose tilings come to the same kernel share a launch.
-size_t qmm_direct_batch_scratch_bytes(const QmmParams* p, int n);
-int launch_qmm_direct_batch(const QmmParams* p, int n, const LaunchCtx& lc, void* scratch);
 // 16-row matrix-core GEMV (qmv_wide.hip): 4-bit codes, f16 / bf16, at most 16 rows, K % 512 == 0.
 // scratch: qmv_wide_scratch_bytes(p) bytes (0 when K is not split: then scratch may be null).
 bool qmv_wide_takes(const QmmParams& p);

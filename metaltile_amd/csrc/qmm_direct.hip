@@ -83,15 +83,6 @@ template <int DT, int VEC> __global__ __launch_bounds__(256) void qmm_split_redu
     else out[0] = (uint16_t)h[0];
 }
 
-// What one matrix's launch is: the kernel that the tiling picks, its geometry, and whether partial tiles follow.
-struct QmmDLaunch {
-    const void* fn = nullptr;
-    uint32_t grid = 0, block = 0;   // workgroups per K split
-    size_t shmem = 0;
-    bool split = false;
-    QmmDArgs a;
-};
-
 // Launches l[0 .. n): matrices on the same kernel in one launch (at most four), then one addition of their partial tiles.
 static bool qd_same_launch(const QmmDLaunch& p, const QmmDLaunch& q) {
     return p.fn == q.fn && p.block == q.block && p.split == q.split && p.a.ksplit == q.a.ksplit && p.a.iters_per_split == q.a.iters_per_split && !p.a.tiles && !q.a.tiles;
@@ -101,13 +92,11 @@ static bool qd_same_launch(const QmmDLaunch& p, const QmmDLaunch& q) {
 // 1 % slower together, with the clock down and four tiles in a round of their own); the 4-wave ones share compute units.
 static bool qd_saves_round(const QmmDLaunch& l, uint32_t have, uint32_t more) {
     if (l.block != 512) return true;
-    int dev = 0, cus = 256;
-    if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    const uint64_t ks = l.split ? l.a.ksplit : 1, c = (uint64_t)cus;
+    const uint64_t ks = l.split ? l.a.ksplit : 1, c = l.cus;
     auto rounds = [&](uint64_t wgs) { return (wgs * ks + c - 1) / c; };
     return rounds((uint64_t)have + more) < rounds(have) + rounds(more);
 }
-static int qd_issue(int dtype, const QmmDLaunch* l, int n, const LaunchCtx& lc) {
+static int qd_issue(const QmmDLaunch* l, int n, const LaunchCtx& lc) {
     for (int i = 0, j; i < n; i = j) {
         QmmDArgs a = l[i].a;
         QmmDMore& more = a.more;
@@ -148,7 +137,7 @@ static int qd_issue(int dtype, const QmmDLaunch* l, int n, const LaunchCtx& lc) 
             blocks += (r.total[k] + per - 1) / per;
         }
         void* rargs[] = {&r};
-        const void* rf = dtype == DT_BF16 ? (vec ? (const void*)qmm_split_reduce_kernel<DT_BF16, 4> : (const void*)qmm_split_reduce_kernel<DT_BF16, 1>)
+        const void* rf = l[i].dtype == DT_BF16 ? (vec ? (const void*)qmm_split_reduce_kernel<DT_BF16, 4> : (const void*)qmm_split_reduce_kernel<DT_BF16, 1>)
                                           : (vec ? (const void*)qmm_split_reduce_kernel<DT_F16, 4> : (const void*)qmm_split_reduce_kernel<DT_F16, 1>);
         e = launch_kernel(rf, dim3(blocks), dim3(256), rargs, 0, l2);
         if (e != hipSuccess) return hip_fail(e, "qmm split reduce kernel launch");
@@ -193,8 +182,10 @@ static size_t dma_split_lds(int bits, uint32_t rows, uint32_t kgroups, uint32_t 
 }
 
 // The kernel that a matrix's tiling picks.
-template <int DT> static int choose_dt(const QmmDArgs& a, int bits, uint32_t kgroups, QmmDLaunch& l, bool grouped = false) {
-    l.a = a;
+template <int DT> static int choose_dt(int bits, uint32_t kgroups, QmmDLaunch& l, bool grouped = false) {
+    const QmmDArgs& a = l.a;
+    const uint64_t cus = l.cus;
+    l.dtype = DT;
     l.grid = a.m_tiles * a.n_tiles;
     l.block = kgroups == 1 ? 256 : 512;
     l.split = a.ksplit > 1 && !grouped;
@@ -203,17 +194,15 @@ template <int DT> static int choose_dt(const QmmDArgs& a, int bits, uint32_t kgr
     // 36.3 against 34.3 us) or on the 4-K-group tiles (4096 x 4096, 16 / 64 rows 11.6 / 15.3 against 10.9 / 14.6;
     // 4096 x 14336 20.2 / 28.7 against 31.6 / 37.4): those stay on the register-staged instances
     const bool b8_short = bits == 8 && a.K < 8192 && options().qmm_dma < 2;
-    int dev = 0, cus = 256;
-    if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
     if (const size_t shmem = grouped ? 0 : dma_split_lds(bits, a.m_tile_rows, kgroups, a.K, a.gpr, a.iters_per_split, a.ksplit)) {
         l.fn = qmm_dma_split_pick(bits, DT, a.m_tile_rows);
         l.shmem = shmem;
         return ERR_OK;
     }
     if (a.ksplit <= 1 && dma_fits(bits, a.m_tile_rows, kgroups, a.K, a.gpr) && (!grouped || a.m_tile_rows == 64) &&
-        !(b8_short && !grouped && a.m_tile_rows != 256 && (uint64_t)a.m_tiles * a.n_tiles < (uint64_t)cus)) {
+        !(b8_short && !grouped && a.m_tile_rows != 256 && (uint64_t)a.m_tiles * a.n_tiles < cus)) {
         const bool windowed = dma_mode(bits, a.m_tile_rows, kgroups, a.K, a.gpr) == 2;
-        const bool shallow = grouped || (uint64_t)a.m_tiles * a.n_tiles > (uint64_t)cus;
+        const bool shallow = grouped || (uint64_t)a.m_tiles * a.n_tiles > cus;
         l.fn = qmm_dma_pick(bits, DT, a.m_tile_rows, grouped, windowed, shallow);
         l.shmem = qmm_dma_lds_bytes(a.m_tile_rows, a.gpr, windowed, shallow);
         return ERR_OK;
@@ -288,7 +277,7 @@ static bool qmm_direct_split_built(uint32_t rows, uint32_t kgroups) {
 }
 
 struct QmmDPlan {
-    uint32_t rows, kgroups, ksplit, iters_per_split;
+    uint32_t rows, kgroups, ksplit, iters_per_split, cus;
 };
 
 // Checks the shape and picks the tile, the K-groups and the K split.
@@ -311,6 +300,7 @@ static int plan_direct(const QmmParams& p, QmmDPlan& pl) {
     // half the chip idle, 64 x 64 tiles on 4 K-groups (M = 128: 18.6 us against 26).
     int dev = 0, cus = 256;
     if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    pl.cus = (uint32_t)cus;
     const uint64_t tall_wide = (uint64_t)((p.M + 127) / 128) * ((p.N + 127) / 128);
     const uint64_t short_wide = (uint64_t)((p.M + 63) / 64) * ((p.N + 127) / 128);
     uint32_t rows = 64, kgroups = 2;
@@ -449,19 +439,14 @@ static int plan_direct(const QmmParams& p, QmmDPlan& pl) {
     return ERR_OK;
 }
 
-size_t qmm_direct_scratch_bytes(const QmmParams& p) {
-    QmmDPlan pl;
-    if (plan_direct(p, pl) != ERR_OK || pl.ksplit <= 1) return 0;
-    return (size_t)pl.ksplit * p.M * p.N * sizeof(float);
-}
-
-static int choose_direct(const QmmParams& p, void* scratch, QmmDLaunch& l) {
+int plan_qmm_direct(const QmmParams& p, QmmDLaunch& l) {
     QmmDPlan pl;
     int rc = plan_direct(p, pl);
     if (rc) return rc;
     const uint32_t G = p.group_size, rows = pl.rows, kgroups = pl.kgroups;
-    if (pl.ksplit > 1 && !scratch) return fail(ERR_BAD_ARG, "direct qmm: K split without a scratch buffer");
-    QmmDArgs a;
+    l.cus = pl.cus;
+    l.scratch = pl.ksplit > 1 ? ((size_t)pl.ksplit * p.M * p.N * sizeof(float) + 255) & ~(size_t)255 : 0;
+    QmmDArgs& a = l.a;
     a.w = (const unsigned char*)p.w;
     a.scales = (const unsigned char*)p.scales;
     a.biases = (const unsigned char*)p.biases;
@@ -485,43 +470,24 @@ static int choose_direct(const QmmParams& p, void* scratch, QmmDLaunch& l) {
     a.iters = p.K / (64 * kgroups);
     a.ksplit = pl.ksplit;
     a.iters_per_split = pl.iters_per_split;
-    a.part = (float*)scratch;
+    a.part = nullptr;   // (launch_qmm_direct)
     a.tiles = nullptr;
     a.rowlist = nullptr;
     a.w_expert_bytes = a.sb_expert_elems = 0;
-    return p.dtype == DT_BF16 ? choose_dt<DT_BF16>(a, p.bits, kgroups, l) : choose_dt<DT_F16>(a, p.bits, kgroups, l);
-}
-
-int launch_qmm_direct(const QmmParams& p, const LaunchCtx& lc, void* scratch) {
-    QmmDLaunch l;
-    const int rc = choose_direct(p, scratch, l);
-    return rc ? rc : qd_issue(p.dtype, &l, 1, lc);
-}
-
-bool qmm_direct_takes(const QmmParams& p) {
-    QmmDPlan pl;
-    QmmDLaunch l;
-    return plan_direct(p, pl) == ERR_OK && choose_direct(p, const_cast<QmmParams*>(&p), l) == ERR_OK;   // (any address stands for the scratch: nothing is launched)
+    return p.dtype == DT_BF16 ? choose_dt<DT_BF16>(p.bits, kgroups, l) : choose_dt<DT_F16>(p.bits, kgroups, l);
 }
 
 // Each matrix's tiling, K split and arithmetic are those of its own call, and matrices that so come to the same kernel share
 // its launch: one matrix of a layer is often too few tiles for the chip. us, one launch each -> together: 6-bit codes, 77 rows,
 // (3584 + 2 x 512) x 3584 60.2 -> 22.0, 2 x 18944 x 3584 102 -> 82.7; 4-bit codes, 512 rows, 2 x 1024 x 4096 (K and V, split
 // K, with the additions) 39.2 -> 33.1; 2 x 14336 x 4096 (224 tiles each of 256 compute units) 149.4 -> 149.7: left apart.
-size_t qmm_direct_batch_scratch_bytes(const QmmParams* p, int n) {
-    size_t b = 0;
-    for (int i = 0; i < n; i++) b += (qmm_direct_scratch_bytes(p[i]) + 255) & ~(size_t)255;
-    return b;
-}
-
-int launch_qmm_direct_batch(const QmmParams* p, int n, const LaunchCtx& lc, void* scratch) {
-    QmmDLaunch l[4];
+int launch_qmm_direct(QmmDLaunch* l, int n, void* scratch, const LaunchCtx& lc) {
     char* at = (char*)scratch;
     for (int i = 0; i < n; i++) {
-        const size_t need = qmm_direct_scratch_bytes(p[i]);
-        const int rc = choose_direct(p[i], need ? at : nullptr, l[i]);
-        if (rc) return rc;
-        at += (need + 255) & ~(size_t)255;
+        if (!l[i].scratch) continue;
+        if (!scratch) return fail(ERR_BAD_ARG, "direct qmm: K split without a scratch buffer");
+        l[i].a.part = (float*)at;
+        at += l[i].scratch;
     }
     // matrices of one kernel side by side
     for (int i = 0; i + 1 < n; i++)
@@ -530,7 +496,7 @@ int launch_qmm_direct_batch(const QmmParams* p, int n, const LaunchCtx& lc, void
                 std::swap(l[i + 1], l[j]);
                 break;
             }
-    return qd_issue(p[0].dtype, l, n, lc);
+    return qd_issue(l, n, lc);
 }
 
 // ---- expert-routed rows on the tile kernel ---------------------------------------------------
@@ -671,7 +637,8 @@ int launch_qmm_grouped(const QmmParams& p, const uint32_t* route, bool per_row_i
     const uint32_t* rowlist = gt.rowlist;
     const LaunchCtx& last = gt.last;
 
-    QmmDArgs a;
+    QmmDLaunch ql;
+    QmmDArgs& a = ql.a;
     a.w = (const unsigned char*)p.w;
     a.scales = (const unsigned char*)p.scales;
     a.biases = (const unsigned char*)p.biases;
@@ -689,6 +656,7 @@ int launch_qmm_grouped(const QmmParams& p, const uint32_t* route, bool per_row_i
     // 64 x 128 tiles; 64 x 64 on 4 K-groups when that still leaves fewer tiles than compute units. Row
     // tiles: every expert's last tile is partial, half an expert's worth on average (128 experts x
     // 768 x 2048, 10 rows each: 68 us on 4 K-groups, 44 us on 2).
+    ql.cus = (uint32_t)cus;
     const uint64_t row_tiles = (uint64_t)(T + 63) / 64 + (E < T ? E : T) / 2;
     uint32_t kgroups = (row_tiles * ((p.N + 127) / 128) * 2 <= (uint64_t)cus && p.K % 256 == 0) ? 4 : 2;
     if (tile_rows == 32) kgroups = 4;
@@ -704,9 +672,8 @@ int launch_qmm_grouped(const QmmParams& p, const uint32_t* route, bool per_row_i
     a.rowlist = rowlist;
     a.w_expert_bytes = (uint64_t)p.N * p.K * p.bits / 8;
     a.sb_expert_elems = (uint64_t)p.N * a.gpr;
-    QmmDLaunch ql;
-    rc = p.dtype == DT_BF16 ? choose_dt<DT_BF16>(a, p.bits, kgroups, ql, true) : choose_dt<DT_F16>(a, p.bits, kgroups, ql, true);
-    return rc ? rc : qd_issue(p.dtype, &ql, 1, last);
+    rc = p.dtype == DT_BF16 ? choose_dt<DT_BF16>(p.bits, kgroups, ql, true) : choose_dt<DT_F16>(p.bits, kgroups, ql, true);
+    return rc ? rc : qd_issue(&ql, 1, last);
 }
 
 }  // namespace mtq

@@ -3,6 +3,7 @@
 #pragma once
 #include "mtq_internal.h"
 #include "qmm_common.h"
+#include "qmm_direct_plan.h"
 
 namespace mtq {
 
@@ -15,42 +16,6 @@ namespace mtq {
         __builtin_amdgcn_sched_barrier(0);  \
     } while (0)
 
-struct QmmDBase {
-    const unsigned char* w;
-    const unsigned char* scales;
-    const unsigned char* biases;
-    const unsigned char* x;
-    void* out;
-    uint32_t M, N, K;
-    uint32_t log2g, gpr;
-    uint32_t m_tiles, n_tiles, iters;
-    uint32_t m_tile_rows;  // 32 (4 K-groups only), 64 or 128
-    uint32_t by_m;         // consecutive workgroup ids walk the N-tiles of one M-tile (else the M-tiles of one N-tile)
-    // grouped mode (expert-routed rows): tiles[0] = number of row tiles, then one uint4 per tile
-    // (expert, first row of the tile in the row order, rows in the tile, 0); rowlist maps the row
-    // order to rows of x / out (null: the identity). w / scales / biases are the stacked experts'.
-    const uint32_t* tiles;
-    const uint32_t* rowlist;
-    uint64_t w_expert_bytes, sb_expert_elems;
-    // split K (few tiles, long rows): workgroup (x, y) works iterations [y * iters_per_split, +iters_per_split)
-    // of tile x and writes its f32 partial tile to part[y][M][N]; a second kernel adds the splits in order.
-    uint32_t ksplit, iters_per_split;
-    float* part;
-};
-
-// Further matrices of the same launch (the projections of a layer against the same rows): their workgroups (blockIdx.x)
-// follow the first matrix's, on the same tiling, rows, K and K split.
-struct QmmDMore {
-    uint32_t n = 0;                                       // 0..3
-    uint32_t first[3] = {~0u, ~0u, ~0u};                  // first workgroup of each
-    uint32_t N[3] = {}, n_tiles[3] = {}, by_m[3] = {};
-    const unsigned char *w[3] = {}, *scales[3] = {}, *biases[3] = {};
-    void* out[3] = {};
-    float* part[3] = {};
-};
-struct QmmDArgs : QmmDBase {
-    QmmDMore more;
-};
 // Makes `a` this workgroup's matrix; returns the workgroup's number among the matrix's.
 __device__ __forceinline__ uint32_t qd_matrix(QmmDBase& a, const QmmDMore& more) {
     uint32_t id = blockIdx.x;
