@@ -1,9 +1,9 @@
 """The K-run matrix-core GEMV (mtq_qmm and mtq_qmm_batched at 2..16 rows): the edges of its blocks of 16 weight rows, of its
 steps of 128 (64) codes over sixteen waves, of its groups and of the batch, against the f64-accumulated oracle.
 
-Bound: exact-dequant arithmetic, so what is left is the rounding of the result (2^-9 of it in bf16, 2^-12 in f16) and f32
-sums; the conversion adds up to 1024 to a code and takes it out again, which for K = 8192 and |x| up to 5 leaves at most
-about 2^-24 * 1024 * sqrt(K) * scale (0.1) = 6e-4 absolute. max |a-e| / max(|e|, 1) <= 1e-2 (bf16), 3e-3 (f16)."""
+Bound: exact-dequant arithmetic, so what is left is the rounding of the result (half a unit in its last place: at
+most 2^-8 of it in bf16, 2^-11 in f16) and f32 sums; the conversion adds up to 1024 to a code and takes it out again, which
+for K = 8192 and |x| up to 5 leaves at most about 2^-24 * 1024 * sqrt(K) * scale (0.1) = 6e-4 absolute. max |a-e| / max(|e|, 1) <= 1e-2 (bf16), 3e-3 (f16)."""
 import numpy as np
 import pytest
 
@@ -44,6 +44,39 @@ def test_edges(oracle, dt, bits, G, M, K, Ns):
             ops.qmm(dt, bits, G, ws[j], ss[j], bs[j], x, single, M, N, K)
             assert single.read_bytes(M * N * 2) == raw[:-64], j
             single.free()
+    finally:
+        lib.mtq_set_option(b"qmv.runs", 0)
+        for b in [x] + ws + ss + bs + outs:
+            b.free()
+
+
+@pytest.mark.parametrize("dt,bits,G,M,K,Ns,instance", [
+    (DType.BF16, 4, 64, 16, 1024, (14000, 9001, 1600), "1, 3"), (DType.F16, 4, 32, 6, 384, (24601,), "1, 3"),
+    (DType.F16, 4, 128, 9, 2176, (9001, 7600), "2, 2"), (DType.BF16, 8, 64, 16, 1152, (9001, 8000), "2, 2"),
+    (DType.BF16, 4, 64, 5, 5120, (7001, 6000), "3, 1"), (DType.F16, 4, 32, 16, 6272, (7001, 5400), "4, 1"),
+    (DType.BF16, 8, 128, 7, 3072, (7001, 6000), "4, 1"), (DType.F16, 8, 32, 3, 4224, (12401,), "5, 1"),
+])
+def test_many_blocks_per_workgroup(oracle, dt, bits, G, M, K, Ns, instance):
+    """The walk: with PF blocks in flight ahead, every workgroup of the 256 has PF + 2 blocks of 16 weight rows or more, so
+    every slot of the ring and both halves of the sums' buffer are used again. A matrix begins inside the wrap, and the last block
+    of each is ragged. (The instances' last two numbers are the steps of a run and PF.)"""
+    print(f"[case] K-run qmv walk {dt.name} b{bits} g{G} M{M} K{K} N={Ns}", flush=True)
+    assert sum(-(-N // 16) for N in Ns) >= 256 * (int(instance[-1]) + 2)
+    lib = _ensure_init()
+    cases = [make_case(930 + j + M, dt, bits, G, M, N, K, bias_rule="midpoint") for j, N in enumerate(Ns)]
+    x = GpuBuffer.from_bytes(cases[0].x_bytes)
+    ws, ss, bs = ([GpuBuffer.from_bytes(v) for v in part] for part in zip(*((c.w.tobytes(), c.scales_bytes, c.biases_bytes) for c in cases)))
+    guard = b"\xcd" * 64
+    outs = [GpuBuffer.from_bytes(b"\xff" * (M * N * 2) + guard) for N in Ns]
+    try:
+        assert lib.mtq_set_option(b"qmv.runs", 2) == 0
+        assert f"{bits}, {G}, {instance}>" in ops.plan("qmm", dt, bits, G, M, Ns[0], K)[1][0][0]
+        ops.qmm_batched(dt, bits, G, ws, ss, bs, x, outs, list(Ns), M, K)
+        for j, (c, N) in enumerate(zip(cases, Ns)):
+            raw = outs[j].read_bytes(M * N * 2 + 64)
+            assert raw[-64:] == guard
+            exp = oracle.qmm_f64(c.w, c.scales_f, c.biases_f, cases[0].x_f, M, N, K, bits, G, threads=8).reshape(-1)
+            assert rel_err(unpack_f32(raw[:-64], dt), exp) <= TOL[dt], j
     finally:
         lib.mtq_set_option(b"qmv.runs", 0)
         for b in [x] + ws + ss + bs + outs:
@@ -113,3 +146,29 @@ def test_infinite_and_huge_activations(dt, bits, G, M, N, K):
     np.testing.assert_array_equal(got[0][rest], got[1][rest])
     if M > 3:
         assert np.all(np.isnan(values[M - 1]))
+
+
+@pytest.mark.parametrize("which", ["w", "scales", "biases", "x", "out"])
+def test_operands_off_16_bytes(oracle, which):
+    """An operand at 8 bytes past a multiple of 16 (a slice of a larger buffer): the loads of 16 bytes are not for it, so another
+    kernel takes the call (the K-run kernel's stores are of single elements: `out` may lie anywhere). f16, K = 512: those that round the weight to
+    the element type first add about 2^-12 * |w| (0.1 rms) * sqrt(K) * |x| = 6e-4 rms; 1e-2."""
+    dt, bits, G, M, N, K = DType.F16, 4, 64, 16, 72, 512
+    print(f"[case] K-run qmv, {which} off 16 bytes", flush=True)
+    c = make_case(990, dt, bits, G, M, N, K, bias_rule="midpoint")
+    off = {n: 8 if n == which else 0 for n in ("w", "scales", "biases", "x", "out")}
+    data = dict(w=c.w.tobytes(), scales=c.scales_bytes, biases=c.biases_bytes, x=c.x_bytes, out=b"\xff" * (M * N * 2))
+    bufs = {n: GpuBuffer.from_bytes(b"\xcd" * off[n] + v + b"\xcd" * 64) for n, v in data.items()}
+    at = {n: bufs[n].ptr + off[n] for n in bufs}
+    exp = oracle.qmm_f64(c.w, c.scales_f, c.biases_f, c.x_f, M, N, K, bits, G).reshape(-1)
+    for batch in (False, True):
+        bufs["out"].upload(np.full(off["out"] + M * N * 2 + 64, 0xCD, np.uint8))
+        if batch:
+            ops.qmm_batched(dt, bits, G, [at["w"]], [at["scales"]], [at["biases"]], at["x"], [at["out"]], [N], M, K)
+        else:
+            ops.qmm(dt, bits, G, at["w"], at["scales"], at["biases"], at["x"], at["out"], M, N, K)
+        raw = bufs["out"].read_bytes(off["out"] + M * N * 2 + 64)
+        assert raw[:off["out"]] == b"\xcd" * off["out"] and raw[-64:] == b"\xcd" * 64
+        assert rel_err(unpack_f32(raw[off["out"]:-64], dt), exp) <= 1e-2, batch
+    for b in bufs.values():
+        b.free()

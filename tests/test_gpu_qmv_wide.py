@@ -146,9 +146,10 @@ def test_wide_gather(oracle, wide_gather, dt, N, K, counts, kp, nb):
 
 
 @pytest.mark.parametrize("dt", [DType.F16, DType.BF16], ids=lambda d: d.name)
-@pytest.mark.parametrize("N,K,counts,tail", [(144, 5120, (3, 0, 17, 1), 0), (40, 14336, (0, 16, 2), 5), (4096, 9216, (20, 12, 0), 0)])
+@pytest.mark.parametrize("N,K,counts,tail", [(144, 5120, (3, 0, 17, 1), 0), (40, 14336, (0, 16, 2), 5), (4096, 9216, (20, 12, 0), 0),
+                                               (200, 5632, (5, 0, 18), 2), (1040, 9728, (17, 3), 0), (72, 18944, (2, 16), 1)])   # a shorter last slice
 def test_wide_gather_in_k_slices(oracle, wide_gather, dt, N, K, counts, tail):
-    """Rows longer than one slice, by CSR offsets: partial rows of every slice, an expert without rows, more than 16 rows, rows
+    """Rows longer than one slice, by CSR offsets: partial rows of every slice, a last slice that is shorter than the others, an expert without rows, more than 16 rows, rows
     past the last offset (expert 0's), against the f64-accumulated oracle: 1e-2, the bound of the exact-dequant kernels."""
     bits, G, E, T = 4, 64, len(counts), sum(counts) + tail
     wide_gather(0, 0)
