@@ -17,6 +17,7 @@ import pytest
 
 from metaltile_amd import DType, GpuBuffer, MtqError, ops, pack_f32, unpack_f32
 from metaltile_amd.synth import make_case
+from tests.hip_graph import Graph
 from tests.parity import rel_err
 from tests.test_gpu_batched import REF_TOL, _quantize_int4, _ref_err, _source
 
@@ -165,17 +166,24 @@ def test_argument_errors():
     one.free()
 
 
-@pytest.mark.parametrize("dt,bits,M,K,Ns", [
-    (DType.F16, 6, 77, 1024, (520, 136, 8, 4096)),      # one tiling, ragged last tiles, one launch
-    (DType.BF16, 4, 130, 4096, (1024, 256, 256)),       # split K: partial tiles of all in one addition
-    (DType.BF16, 4, 33, 4096, (130, 34, 2)),            # results that are not whole vectors of four
-    (DType.F16, 8, 200, 8192, (128, 1024, 128)),        # two tilings in turn
+@pytest.mark.parametrize("dt,bits,M,K,Ns,kinds,launches", [
+    (DType.F16, 6, 77, 1024, (520, 136, 8, 4096), 1, 1),      # one tiling, ragged last tiles, one launch
+    (DType.BF16, 4, 130, 4096, (1024, 256, 256), 1, 4),       # split K: partial tiles of two in one addition; the third would begin a second round
+    (DType.BF16, 4, 33, 4096, (130, 34, 2), 1, 2),            # results that are not whole vectors of four
+    (DType.F16, 8, 200, 8192, (128, 1024, 128), 1, 2),        # 8-bit codes, split K
+    (DType.BF16, 4, 200, 8192, (128, 4096, 128), 2, 4),       # two K splits in turn: the first and the last together, each pair with partial tiles of its own
+    (DType.BF16, 4, 200, 2048, (256, 8192, 320), 2, 2),       # two tilings in turn, unsplit
+    (DType.BF16, 4, 200, 8192, (128, 3000, 4096, 1024), 3, 6),   # three K splits: the first and the last together
+    (DType.BF16, 4, 130, 512, (12000, 12000), 1, 2),          # 188 tiles each of 256 compute units: no round saved, left apart
 ], ids=str)
-def test_tiled_batch_shares_launches(dt, bits, M, K, Ns):
-    """Matrices whose tilings come to the same kernel share its launch; the bits are those of single calls (whose values
-    the tiling tests hold to the oracle)."""
+def test_tiled_batch_shares_launches(dt, bits, M, K, Ns, kinds, launches):
+    """Matrices whose tilings come to the same kernel share its launch, wherever in the batch they stand; the bits are those of
+    single calls (whose values the tiling tests hold to the oracle). kinds: kernels and K splits that the matrices plan to;
+    launches: what the batch comes to, additions of partial tiles included."""
     print(f"[case] tiled batch {dt.name} b{bits} M{M} K{K} N={Ns}", flush=True)
     G = 64
+    plans = [ops.plan("qmm", dt, bits, G, M, N, K)[1] for N in Ns]
+    assert len({(p[0][0], p[0][1][1]) for p in plans}) == kinds
     cases = [make_case(3300 + j + M, dt, bits, G, M, N, K, bias_rule="midpoint") for j, N in enumerate(Ns)]
     xb = GpuBuffer.from_bytes(cases[0].x_bytes)
     ws, ss, bs = ([GpuBuffer.from_bytes(v) for v in part] for part in zip(*((c.w.tobytes(), c.scales_bytes, c.biases_bytes) for c in cases)))
@@ -188,5 +196,12 @@ def test_tiled_batch_shares_launches(dt, bits, M, K, Ns):
         ops.qmm(dt, bits, G, ws[j], ss[j], bs[j], xb, single, M, N, K)
         assert raw[-64:] == guard and raw[:-64] == single.read_bytes(M * N * 2), j
         assert np.all(np.isfinite(unpack_f32(raw[:-64], dt))), j
+    g = Graph()
+    try:
+        with g:
+            ops.qmm_batched(dt, bits, G, ws, ss, bs, xb, outs, list(Ns), M, K)
+        assert g.nodes == launches
+    finally:
+        g.close()
     for b in [xb, single] + ws + ss + bs + outs:
         b.free()
