@@ -45,8 +45,19 @@ static size_t lds_need(uint32_t rows, uint32_t kg, uint32_t gpr, bool sbl) {
     return main_loop > epilogue ? main_loop : epilogue;
 }
 
-// Adds the K splits' partial tiles in split order and rounds to the element type; VEC results per thread. Up to four
-// matrices of one launch, each from its own first workgroup on.
+// Adds the K splits' partial tiles in split order and rounds to the element type. One result per thread: the partial tiles lie
+// in other dies' caches, and few threads of four results each wait longer for them (2048 x 8192, 8 splits, 32 rows, the whole
+// product: 9.9 -> 12.7 us).
+template <int DT> __device__ __forceinline__ void split_reduce(const float* part, void* out, uint32_t total, uint32_t ksplit, uint32_t i) {
+    if (i >= total) return;
+    float r = part[i];
+    for (uint32_t sp = 1; sp < ksplit; sp++) r += part[(size_t)sp * total + i];
+    ((uint16_t*)out)[i] = f32_to_elem_bits<DT>(r);
+}
+template <int DT> __global__ __launch_bounds__(256) void qmm_split_reduce_kernel(const float* part, void* out, uint32_t total, uint32_t ksplit) {
+    split_reduce<DT>(part, out, total, ksplit, blockIdx.x * 256 + threadIdx.x);
+}
+// The same for up to four matrices of one launch, each from its own first workgroup on.
 struct QmmReduceArgs {
     const float* part[4];
     void* out[4];
@@ -54,33 +65,9 @@ struct QmmReduceArgs {
     uint32_t first[4];
     uint32_t ksplit;
 };
-template <int DT, int VEC> __global__ __launch_bounds__(256) void qmm_split_reduce_kernel(QmmReduceArgs a) {
+template <int DT> __global__ __launch_bounds__(256) void qmm_split_reduce_batch_kernel(QmmReduceArgs a) {
     const uint32_t m = __builtin_amdgcn_readfirstlane((blockIdx.x >= a.first[1] ? 1u : 0u) + (blockIdx.x >= a.first[2] ? 1u : 0u) + (blockIdx.x >= a.first[3] ? 1u : 0u));
-    const uint32_t i = ((blockIdx.x - a.first[m]) * 256 + threadIdx.x) * VEC, total = a.total[m];
-    if (i >= total) return;
-    const float* part = a.part[m] + i;
-    float r[VEC];
-    auto load = [&](const float* p, float (&v)[VEC]) {
-        if constexpr (VEC == 4) {
-            const float4 t = *(const float4*)p;
-            v[0] = t.x; v[1] = t.y; v[2] = t.z; v[3] = t.w;
-        } else {
-            v[0] = p[0];
-        }
-    };
-    load(part, r);
-    for (uint32_t sp = 1; sp < a.ksplit; sp++) {
-        float v[VEC];
-        load(part + (size_t)sp * total, v);
-#pragma unroll
-        for (int k = 0; k < VEC; k++) r[k] += v[k];
-    }
-    uint16_t* out = (uint16_t*)a.out[m] + i;
-    uint32_t h[VEC];
-#pragma unroll
-    for (int k = 0; k < VEC; k++) h[k] = f32_to_elem_bits<DT>(r[k]);
-    if constexpr (VEC == 4) *(uint2*)out = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
-    else out[0] = (uint16_t)h[0];
+    split_reduce<DT>(a.part[m], a.out[m], a.total[m], a.ksplit, (blockIdx.x - a.first[m]) * 256 + threadIdx.x);
 }
 
 // Launches l[0 .. n): matrices on the same kernel in one launch (at most four), then one addition of their partial tiles.
@@ -96,9 +83,14 @@ static bool qd_saves_round(const QmmDLaunch& l, uint32_t have, uint32_t more) {
     auto rounds = [&](uint64_t wgs) { return (wgs * ks + c - 1) / c; };
     return rounds((uint64_t)have + more) < rounds(have) + rounds(more);
 }
-static int qd_issue(const QmmDLaunch* l, int n, const LaunchCtx& lc) {
+// The partial tiles of each launch begin at `scratch`: the launches follow one another, and what the last one left in the caches
+// is written over (2 x 2048 x 8192, 8 splits, 64 rows, each launch with memory of its own 25.2 us, the same memory 23.2).
+static int qd_issue(const QmmDLaunch* l, int n, void* scratch, const LaunchCtx& lc) {
     for (int i = 0, j; i < n; i = j) {
         QmmDArgs a = l[i].a;
+        a.part = l[i].split ? (float*)scratch : nullptr;
+        const float* part[4] = {a.part};
+        char* at = (char*)scratch + l[i].scratch;
         QmmDMore& more = a.more;
         uint32_t wgs = l[i].grid;
         size_t shmem = l[i].shmem;
@@ -107,7 +99,9 @@ static int qd_issue(const QmmDLaunch* l, int n, const LaunchCtx& lc) {
             const QmmDArgs& o = l[j].a;
             more.first[k] = wgs;
             more.N[k] = o.N; more.n_tiles[k] = o.n_tiles; more.by_m[k] = o.by_m;
-            more.w[k] = o.w; more.scales[k] = o.scales; more.biases[k] = o.biases; more.out[k] = o.out; more.part[k] = o.part;
+            more.w[k] = o.w; more.scales[k] = o.scales; more.biases[k] = o.biases; more.out[k] = o.out;
+            if (l[j].split) part[k + 1] = more.part[k] = (float*)at;
+            at += l[j].scratch;
             wgs += l[j].grid;
             if (l[j].shmem > shmem) shmem = l[j].shmem;
         }
@@ -121,25 +115,26 @@ static int qd_issue(const QmmDLaunch* l, int n, const LaunchCtx& lc) {
         e = launch_kernel(l[i].fn, dim3(wgs, l[i].split ? a.ksplit : 1), dim3(l[i].block), args, shmem, l1);
         if (e != hipSuccess) return hip_fail(e, "qmm tile kernel launch");
         if (!l[i].split) continue;
-        QmmReduceArgs r;
-        r.ksplit = a.ksplit;
-        bool vec = true;   // four results per thread: their partial sums and outputs are whole vectors
-        for (int k = i; k < j; k++) vec = vec && (uint64_t)l[k].a.M * l[k].a.N % 4 == 0 && (uintptr_t)l[k].a.part % 16 == 0;
-        uint32_t blocks = 0;
-        for (int k = 0; k < 4; k++) {
-            r.first[k] = ~0u;
-            r.part[k] = nullptr; r.out[k] = nullptr; r.total[k] = 0;
-            if (i + k >= j) continue;
-            const QmmDArgs& o = l[i + k].a;
-            r.part[k] = o.part; r.out[k] = o.out; r.total[k] = o.M * o.N;
-            r.first[k] = blocks;
-            const uint32_t per = vec ? 1024 : 256;
-            blocks += (r.total[k] + per - 1) / per;
+        const bool bf16 = l[i].dtype == DT_BF16;
+        if (j == i + 1) {
+            uint32_t total = a.M * a.N;
+            void* rargs[] = {&a.part, &a.out, &total, &a.ksplit};
+            e = launch_kernel(bf16 ? (const void*)qmm_split_reduce_kernel<DT_BF16> : (const void*)qmm_split_reduce_kernel<DT_F16>, dim3((total + 255) / 256), dim3(256), rargs, 0, l2);
+        } else {
+            QmmReduceArgs r{};
+            r.ksplit = a.ksplit;
+            uint32_t blocks = 0;
+            for (int k = 0; k < 4; k++) {
+                r.first[k] = ~0u;
+                if (i + k >= j) continue;
+                const QmmDArgs& o = l[i + k].a;
+                r.part[k] = part[k]; r.out[k] = o.out; r.total[k] = o.M * o.N;
+                r.first[k] = blocks;
+                blocks += (r.total[k] + 255) / 256;
+            }
+            void* rargs[] = {&r};
+            e = launch_kernel(bf16 ? (const void*)qmm_split_reduce_batch_kernel<DT_BF16> : (const void*)qmm_split_reduce_batch_kernel<DT_F16>, dim3(blocks), dim3(256), rargs, 0, l2);
         }
-        void* rargs[] = {&r};
-        const void* rf = l[i].dtype == DT_BF16 ? (vec ? (const void*)qmm_split_reduce_kernel<DT_BF16, 4> : (const void*)qmm_split_reduce_kernel<DT_BF16, 1>)
-                                          : (vec ? (const void*)qmm_split_reduce_kernel<DT_F16, 4> : (const void*)qmm_split_reduce_kernel<DT_F16, 1>);
-        e = launch_kernel(rf, dim3(blocks), dim3(256), rargs, 0, l2);
         if (e != hipSuccess) return hip_fail(e, "qmm split reduce kernel launch");
     }
     return ERR_OK;
@@ -470,7 +465,7 @@ int plan_qmm_direct(const QmmParams& p, QmmDLaunch& l) {
     a.iters = p.K / (64 * kgroups);
     a.ksplit = pl.ksplit;
     a.iters_per_split = pl.iters_per_split;
-    a.part = nullptr;   // (launch_qmm_direct)
+    a.part = nullptr;   // (qd_issue)
     a.tiles = nullptr;
     a.rowlist = nullptr;
     a.w_expert_bytes = a.sb_expert_elems = 0;
@@ -482,13 +477,8 @@ int plan_qmm_direct(const QmmParams& p, QmmDLaunch& l) {
 // (3584 + 2 x 512) x 3584 60.2 -> 22.0, 2 x 18944 x 3584 102 -> 82.7; 4-bit codes, 512 rows, 2 x 1024 x 4096 (K and V, split
 // K, with the additions) 39.2 -> 33.1; 2 x 14336 x 4096 (224 tiles each of 256 compute units) 149.4 -> 149.7: left apart.
 int launch_qmm_direct(QmmDLaunch* l, int n, void* scratch, const LaunchCtx& lc) {
-    char* at = (char*)scratch;
-    for (int i = 0; i < n; i++) {
-        if (!l[i].scratch) continue;
-        if (!scratch) return fail(ERR_BAD_ARG, "direct qmm: K split without a scratch buffer");
-        l[i].a.part = (float*)at;
-        at += l[i].scratch;
-    }
+    for (int i = 0; i < n; i++)
+        if (l[i].scratch && !scratch) return fail(ERR_BAD_ARG, "direct qmm: K split without a scratch buffer");
     // matrices of one kernel side by side
     for (int i = 0; i + 1 < n; i++)
         for (int j = i + 1; j < n; j++)
@@ -496,7 +486,7 @@ int launch_qmm_direct(QmmDLaunch* l, int n, void* scratch, const LaunchCtx& lc) 
                 std::swap(l[i + 1], l[j]);
                 break;
             }
-    return qd_issue(l, n, lc);
+    return qd_issue(l, n, scratch, lc);
 }
 
 // ---- expert-routed rows on the tile kernel ---------------------------------------------------
@@ -673,7 +663,7 @@ int launch_qmm_grouped(const QmmParams& p, const uint32_t* route, bool per_row_i
     a.w_expert_bytes = (uint64_t)p.N * p.K * p.bits / 8;
     a.sb_expert_elems = (uint64_t)p.N * a.gpr;
     rc = p.dtype == DT_BF16 ? choose_dt<DT_BF16>(p.bits, kgroups, ql, true) : choose_dt<DT_F16>(p.bits, kgroups, ql, true);
-    return rc ? rc : qd_issue(&ql, 1, last);
+    return rc ? rc : qd_issue(&ql, 1, nullptr, last);
 }
 
 }  // namespace mtq

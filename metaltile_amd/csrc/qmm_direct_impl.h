@@ -16,10 +16,14 @@ namespace mtq {
         __builtin_amdgcn_sched_barrier(0);  \
     } while (0)
 
-// Makes `a` this workgroup's matrix; returns the workgroup's number among the matrix's.
+// Makes `a` this workgroup's matrix; returns the workgroup's number among the matrix's. The first matrix's arguments are
+// loaded ahead of the branch, all at once: left to itself the compiler chooses between the two addresses of each and loads where
+// it is used, a trip to memory after the other (0.4 - 0.8 us of every launch, of one matrix too: 4096 x 4096, 17 rows 10.3 -> 11.1).
 __device__ __forceinline__ uint32_t qd_matrix(QmmDBase& a, const QmmDMore& more) {
     uint32_t id = blockIdx.x;
-    if (id >= more.first[0]) {
+    const uint32_t second = more.first[0];
+    asm volatile("" ::"s"(a.w), "s"(a.scales), "s"(a.biases), "s"(a.x), "s"(a.out), "s"(a.part), "s"(a.N), "s"(a.n_tiles), "s"(a.by_m), "s"(second));
+    if (id >= second) {
         const uint32_t i = __builtin_amdgcn_readfirstlane((id >= more.first[1] ? 1u : 0u) + (id >= more.first[2] ? 1u : 0u));
         a.w = more.w[i];
         a.scales = more.scales[i];

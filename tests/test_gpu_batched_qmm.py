@@ -169,7 +169,7 @@ def test_argument_errors():
 @pytest.mark.parametrize("dt,bits,M,K,Ns,kinds,launches", [
     (DType.F16, 6, 77, 1024, (520, 136, 8, 4096), 1, 1),      # one tiling, ragged last tiles, one launch
     (DType.BF16, 4, 130, 4096, (1024, 256, 256), 1, 4),       # split K: partial tiles of two in one addition; the third would begin a second round
-    (DType.BF16, 4, 33, 4096, (130, 34, 2), 1, 2),            # results that are not whole vectors of four
+    (DType.BF16, 4, 33, 4096, (130, 34, 2), 1, 2),            # ragged results, split K
     (DType.F16, 8, 200, 8192, (128, 1024, 128), 1, 2),        # 8-bit codes, split K
     (DType.BF16, 4, 200, 8192, (128, 4096, 128), 2, 4),       # two K splits in turn: the first and the last together, each pair with partial tiles of its own
     (DType.BF16, 4, 200, 2048, (256, 8192, 320), 2, 2),       # two tilings in turn, unsplit
