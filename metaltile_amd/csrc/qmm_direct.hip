@@ -70,6 +70,11 @@ template <int DT> __global__ __launch_bounds__(256) void qmm_split_reduce_batch_
     split_reduce<DT>(a.part[m], a.out[m], a.total[m], a.ksplit, (blockIdx.x - a.first[m]) * 256 + threadIdx.x);
 }
 
+// Whether a tile of dbn weight rows has its scales and biases staged in LDS, once for the whole of K.
+static bool stages_scales(uint32_t dbn, uint32_t gpr) {
+    return gpr % 8 == 0 && (size_t)2 * dbn * (gpr + 2) * 2 <= 48 * 1024;
+}
+
 // Launches l[0 .. n): matrices on the same kernel in one launch (at most four), then one addition of their partial tiles.
 static bool qd_same_launch(const QmmDLaunch& p, const QmmDLaunch& q) {
     return p.fn == q.fn && p.block == q.block && p.split == q.split && p.a.ksplit == q.a.ksplit && p.a.iters_per_split == q.a.iters_per_split && !p.a.tiles && !q.a.tiles;
@@ -216,7 +221,7 @@ template <int DT> static int choose_dt(int bits, uint32_t kgroups, QmmDLaunch& l
     const bool tall = a.m_tile_rows == 128;
     const uint32_t dbn = kgroups == 1 ? 128 : 32 * (8 / kgroups);
     // scales and biases of the tile's rows in LDS when they fit beside the activation tiles
-    const bool sbl = a.gpr % 8 == 0 && (size_t)2 * dbn * (a.gpr + 2) * 2 <= 48 * 1024;
+    const bool sbl = stages_scales(dbn, a.gpr);
     const size_t shmem = lds_need(a.m_tile_rows, kgroups, a.gpr, sbl);
     if (shmem > 160 * 1024) return fail(ERR_UNSUPPORTED, "direct qmm: tile does not fit in LDS");
 #define QD_PICK3(B, MBv, KGv) (sbl ? (const void*)qmm_direct_kernel<DT, B, 2, MBv, true, KGv> : (const void*)qmm_direct_kernel<DT, B, 2, MBv, false, KGv>)
@@ -372,10 +377,14 @@ static int plan_direct(const QmmParams& p, QmmDPlan& pl) {
         }
         if (dma_ks) { rows = 128; kgroups = 2; }
     }
-    // The bit-stream widths are bound by the conversion of codes: at 65..128 rows a 64-row tile converts every weight twice.
-    // Long rows take 128-row tiles, K split to fill the chip (us, 64 x 64 tiles -> these: 3584 x 18944, 6-bit codes, 77 / 128
-    // rows 70.6 / 72.8 -> 47.3 / 49.5, 3-bit, 100 rows 58.4 -> 42.5; at K = 8192 they lose, 2048 columns 19.7 -> 23.8).
-    if (odd_bits && p.M > 64 && p.M <= 128 && p.K > 8192 && tall_wide >= 24 && tall_wide * 2 <= (uint64_t)cus) { rows = 128; kgroups = 1; }
+    // The bit-stream widths convert more per weight than they multiply: at 65..128 rows a 64-row tile converts every weight twice.
+    // Long rows take 128-row tiles, K split to fill the chip. us, 64-row tiles -> these, 6-bit codes, 66 / 100 / 128 rows (5- and
+    // 7-bit as 6-bit, 3-bit half as much), groups of 64: 3584 x 18944 69 / 71 / 73 -> 46 / 47 / 49, 5120 x 14336 97 / 103 / 107 -> 63 /
+    // 66 / 69, 16384 x 9216 110 / 112 / 113 -> 80 / 84 / 89, 3072 x 8256 117 / 119 / 120 -> 29 / 30 / 31. Not with fewer than 24 of
+    // them (2048 x 14336 33 -> 34), nor with 33..64 where the 64 x 64 tiles on 4 K-groups are one round of the chip and have their
+    // scales in LDS (8192 x 9216 45 / 45 / 52 -> 48 / 51 / 54, 8192 x 12288 in groups of 128 60 / 59 / 66 -> 61 / 64 / 65).
+    const bool one_round = tall_wide > 32 && tall_wide <= 64 && p.K % 256 == 0 && stages_scales(64, p.K / G);
+    if (odd_bits && p.M > 64 && p.M <= 128 && p.K > 8192 && tall_wide >= 24 && tall_wide * 2 <= (uint64_t)cus && !one_round) { rows = 128; kgroups = 1; }
     if (options().qmm_tile_rows) rows = (uint32_t)options().qmm_tile_rows;
     if (options().qmm_kgroups) kgroups = (uint32_t)options().qmm_kgroups;
     // An iteration covers 64 k per K-group: K must be a multiple of 64 * K-groups (an odd number of
@@ -409,12 +418,15 @@ static int plan_direct(const QmmParams& p, QmmDPlan& pl) {
         ks = (uint32_t)((4 * (uint64_t)cus / tiles + 1) / 2);
         if (ks > 8) ks = 8;
         if (ks > iters / 16) ks = iters / 16;
-    } else if (ksplit_option == 0 && odd_bits && rows == 128 && kgroups == 1 && p.M <= 128 && tiles < (uint64_t)cus && tiles * 2 > (uint64_t)cus) {
-        // a 4-wave workgroup converting codes keeps a compute unit busy by itself: fewer of them than compute units are
-        // split in K (18944 x 3584, 148 tiles, 1 / 2 / 3 / 4 splits, 6-bit codes: 77 rows 50.9 / 49.3 / 41.4 / 46.6 us, 128
-        // rows 49.9 / 52.3 / 45.8 / 53.0; 3-bit, 100 rows 40.6 / 43.2 / 38.8 / 44.0)
-        ks = (uint32_t)(7 * (uint64_t)cus / (4 * tiles));
-        if (ks > iters / 16) ks = iters / 16;
+    } else if (ksplit_option == 0 && odd_bits && rows == 128 && kgroups == 1 && p.M <= 128 && tiles * 2 > (uint64_t)cus && tiles * 3 <= 2 * (uint64_t)cus && iters >= 48) {
+        // Two 4-wave workgroups share a compute unit: three splits of a tile come in beside each other up to two thirds of a tile
+        // per compute unit; a fourth split, or one tile more, begins a second round, and two splits fill the chip no better than
+        // one tile each. us, 6-bit codes, 1 / 2 / 3 / 4 splits, 77 rows: 16512 x 3584 (129 tiles) 48.8 / 49.8 / 39.7 / 46.4, 19200 x
+        // 3584 (150) 48.9 / 49.0 / 41.3 / 47.1, 22016 x 3584 (172) 49.5 / 50.4 / 55.8 / 49.1; 128 rows: 18944 x 3584 49.5 / 53.2 / 45.6 /
+        // 53.0. 1 / 3 splits at 170 tiles, 66 / 100 / 128 rows: 21760 x 4096 56.6 / 57.2 / 57.5 -> 46.4 / 49.9 / 51.7, 21760 x 3072
+        // 42.8 / 43.3 / 43.7 -> 37.3 / 40.7 / 42.7 (3-bit codes 36.7 / 37.2 / 37.8 -> 34.1 / 37.3 / 39.3). Shorter rows gain nothing
+        // (18944 x 2048, 77 / 128 rows 29.9 / 30.7 -> 29.9 / 33.9).
+        ks = 3;
     } else if (ksplit_option == 0 && kgroups != 2 && tiles * 2 <= (uint64_t)cus && iters >= QMM_SPLIT_MIN_ITERS) {
         // one workgroup per compute unit, at least 4 iterations each (measured optimum: 4096 x 14336,
         // 32 rows, 64 tiles: 1 / 2 / 4 / 8 / 16 splits 57 / 34 / 23 / 27 / 32 us; 2048 x 8192, 32 tiles:

@@ -425,10 +425,12 @@ def test_load_to_lds_tiles_with_k_split(oracle, options, dt, M, N, K, G, bits):
 
 @pytest.mark.parametrize("dt,bits,M,N,K,ksplit", [
     (DType.F16, 6, 65, 3080, 8512, 8), (DType.BF16, 3, 128, 3200, 8320, 8),      # long rows: 128-row tiles, K split
-    (DType.F16, 5, 77, 17000, 2048, 2), (DType.BF16, 6, 128, 16520, 3136, 3),    # fewer 4-wave workgroups than compute units
+    (DType.BF16, 7, 100, 4100, 9280, 8),
+    (DType.F16, 5, 77, 17000, 2048, 1), (DType.BF16, 6, 128, 16520, 3136, 3),    # fewer 4-wave workgroups than compute units
+    (DType.BF16, 7, 66, 21700, 3072, 3),
 ], ids=str)
 def test_bit_stream_widths_at_65_to_128_rows(oracle, dt, bits, M, N, K, ksplit):
-    """The tilings the 3-, 5- and 6-bit codes take at 65..128 rows, ragged last tiles and splits: 2e-2 against the oracle's
+    """The tilings the 3-, 5-, 6- and 7-bit codes take at 65..128 rows, ragged last tiles and splits: 2e-2 against the oracle's
     mt_qmm_mma arithmetic (rounded weights), on the first, last and some other columns."""
     G, odt = 64, {DType.F16: 1, DType.BF16: 2}[dt]
     print(f"[case] qmm {dt.name} b{bits} M{M} N{N} K{K}", flush=True)

@@ -217,3 +217,19 @@ def test_benchmark_configurations_are_routed_as_documented():
         for G in (32, 64, 128):
             ks, _ = kernels("qmv", DType.F16, bits, G, M, 8192, 8192)
             assert "generic" not in ks[0], (bits, G, M, ks)
+
+
+@pytest.mark.parametrize("bits,M,N,K,G,tile,ksplit", [
+    (6, 77, 16512, 3584, 64, 128, 3), (7, 128, 21760, 3072, 64, 128, 3),       # 129 and 170 of 256 compute units: three splits are one round
+    (6, 77, 21888, 3584, 64, 128, 1), (3, 128, 28672, 8128, 64, 128, 1),       # 171 tiles and more: unsplit
+    (5, 100, 18944, 2048, 64, 128, 1), (6, 66, 16384, 3584, 64, 64, 1),        # short rows; no more than half the chip
+    (6, 100, 3584, 18944, 64, 128, 8), (7, 66, 4096, 9216, 64, 128, 8),        # long rows: tall tiles
+    (6, 100, 8192, 9216, 64, 64, 1), (3, 66, 5120, 14336, 128, 64, 1),         # ... but not for one round of 64 x 64 tiles with staged scales
+    (6, 100, 8192, 11008, 64, 128, 8), (6, 100, 8192, 8256, 64, 128, 8), (6, 100, 2048, 18944, 64, 64, 4),
+])
+def test_bit_stream_tiles_at_65_to_128_rows(bits, M, N, K, G, tile, ksplit):
+    """The tile height and the K split of the 3-, 5-, 6- and 7-bit codes, on both sides of each line."""
+    rc, launches, _, _ = ops.plan("qmm", DType.F16, bits, G, M, N, K)
+    assert rc == 0
+    args = launches[0][0].split("<")[1].split(", ")
+    assert int(args[3]) * 32 == tile and launches[0][1][1] == ksplit, launches
