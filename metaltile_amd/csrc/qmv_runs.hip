@@ -43,25 +43,38 @@ bool qmv_runs_takes(const QmvParams& p, const QmvBatch& b) {
     return true;
 }
 
-// Where the kernel stands against the others, us, bf16 / f16, weights from memory (others -> this; a single matrix, and the
-// projections that a layer has in one call):
-//                              4 rows         8 rows         16 rows               8-bit codes: 4 rows, 8 rows, 16 rows
-//   1024 x 4096               8.4 ->  6.8    9.1 ->  7.7    9.3 ->  8.7          8.3 ->  8.1   9.7 ->  8.9  10.0 -> 10.2
-//   4096 x 4096               6.5 ->  7.2    8.6 ->  7.8   10.5 ->  9.0          7.9 ->  9.2   9.3 ->  9.4  11.5 -> 10.6
-//   5120 x 5120               9.6 -> 11.1   12.3 -> 11.9   11.7 -> 13.8         10.6 -> 14.5  17.0 -> 15.5  14.7 -> 17.6
-//   14336 x 4096             10.2 -> 13.7   13.3 -> 14.3   13.8 -> 15.7         15.2 -> 18.7  18.6 -> 19.4  18.4 -> 20.8
-//   128256 x 4096              55 -> 65       55 -> 66       57 -> 68             91 -> 116    105 -> 121    128 -> 126
-//   4096 + 2 x 1024 x 4096   23.6 -> 10.0   26.2 -> 10.7   28.5 -> 11.7         24.4 -> 12.2  28.7 -> 12.7  32.4 -> 14.1
-//   3 x 5120 x 5120          27.2 -> 16.7   36.4 -> 17.6   34.4 -> 19.2         31.5 -> 24.4  50.5 -> 25.5  43.4 -> 27.7
-//   2 x 14336 x 4096         19.8 -> 18.9   25.7 -> 19.6   27.2 -> 21.0         30.0 -> 30.4  36.8 -> 31.5  36.2 -> 33.1
-// A matrix's route cannot depend on whether it comes in a batch (it would not have the same bits), so the line lies where
-// a layer gains: from 5 rows up to 75 M codes (60 M of 8 bits), where a long matrix alone loses 1 - 2 us to the 16-row
-// kernel and the tiles and a batch of them gains 6 and more; below 5 rows, where those kernels keep up on all but the
-// shortest matrices (the K and V projections of grouped-query attention), up to 4.5 M.
+// Where the kernel stands against the others. A matrix's route cannot depend on whether it comes in a batch (it would not have
+// the same bits), so a call of one matrix pays for what the projections of a layer gain in one call. The lines lie where two
+// matrices of a size together gain more than one alone loses. us, bf16, groups of 64, weights from memory, others -> this, one
+// matrix | two in a batch, 5, 9 and 16 rows:
+//   2048 x 2048     5.6  8.1  8.1 ->  5.3  5.5  6.1 | 11.4 16.0 16.1 ->  5.6  5.6  6.2
+//   4096 x 4096     7.9 10.0 10.0 ->  7.0  7.6  8.8 | 15.4 19.6 20.1 ->  9.9 10.4 11.7     8 bits 17.1 21.9 22.7 -> 12.7 13.2 14.5
+//   5120 x 5120    11.4 11.1 11.5 -> 11.3 12.1 13.8 | 22.7 22.1 22.8 -> 14.2 15.0 16.7     8 bits 33.1 28.1 29.1 -> 20.7 21.4 23.3
+//   16384 x 2048    8.8  9.2  9.3 -> 10.0 10.4 11.1 | 17.7 18.4 18.5 -> 14.3 14.7 15.4     8 bits 23.3 22.3 22.8 -> 19.2 19.3 20.0
+//   14336 x 4096   12.3 13.5 13.6 -> 13.8 14.4 15.8 | 24.8 26.9 27.1 -> 19.7 20.1 21.5     8 bits 37.8 36.9 37.5 -> 31.6 32.0 33.9
+//   13824 x 5120   16.3 16.0 16.6 -> 17.0 17.8 19.5 | 32.6 32.1 32.9 -> 25.6 26.3 28.3     (70.8 M codes; 16384 x 5120, 84 M, 16 rows 17.0 -> 19.9 | 34.1 -> 31.5;
+//   28672 x 4096, 117 M, 5 rows 19.3 -> 19.9 | 35.9 -> 34.4; 8 bits 16384 x 5120, 16 rows 24.3 -> 28.6 | 48.7 -> 48.9)
+//   7168 x 7168    13.9 14.8 15.0 -> 15.6 16.6 18.9 | 27.9 29.6 29.9 -> 23.6 24.5 27.0
+//   1024 x 8192     9.9  9.8 10.2 -> 10.2 11.4 13.8 | 19.6 19.7 20.7 -> 10.8 12.0 14.5
+//   2048 x 8192     9.4  9.4  9.5 -> 10.8 11.8 14.4 | 18.7 18.7 18.9 -> 11.7 12.7 15.3
+//   16384 x 512     7.9  5.8  5.8 ->  8.4  8.2  8.3 | 15.7 11.6 11.6 -> 12.2 12.3 12.4
+// and 2, 3 and 4 rows:
+//   512 x 3584      5.9  7.1  7.6 ->  5.9  6.0  6.1 | 11.7 14.2 15.2 ->  6.1  6.1  6.3
+//   1024 x 4096     5.9  7.2  8.2 ->  6.2  6.3  6.5 | 12.2 14.7 16.8 ->  6.4  6.6  6.9     8 bits 12.7 14.9 16.8 -> 7.8 8.2 8.4
+//   768 x 3072      5.3  6.5  7.1 ->  5.9  6.0  6.1 | 10.7 13.2 14.2 ->  6.1  6.2  6.3     8 bits 4.4 5.1 5.6 -> 6.7 6.9 7.0 | 8.7 10.1 11.1 -> 6.9 7.1 7.3
+//   1280 x 5120     5.1  5.5  5.7 ->  7.5  7.7  8.0 | 10.0 10.9 11.1 ->  7.7  7.9  8.0
+//   512 x 8192      6.3  7.6  8.8 ->  9.5  9.9 10.3 | 13.0 15.5 17.9 ->  9.8 10.2 10.6
+//   4096 x 1024     3.6  3.8  3.8 ->  5.3  5.3  5.4 |  7.1  7.4  7.4 ->  6.4  6.4  6.5
+// So: below 5 rows short matrices against rows of 2048 to 4096 codes (the K and V projections of grouped-query attention; 8-bit
+// codes from 3 rows); from 5 rows up to 75 M codes (60 M of 8 bits), and from 9 rows, where the others take tiles, no more than
+// 1024 weight rows of more than 6144 codes (four steps a run, whose registers leave one block in flight) and no more than 8192 of
+// fewer than 2048 (some of the sixteen waves have no step, and a workgroup has more than two blocks to walk).
 bool qmv_runs_preferred(int bits, uint32_t M, uint32_t N, uint32_t K) {
     if (M < 2 || M > 16) return false;
     const uint64_t codes = (uint64_t)N * K;
-    return codes <= (M < 5 ? 4500000ull : bits == 4 ? 75000000ull : 60000000ull);
+    if (M < 5) return K >= 2048 && K <= 4096 && (uint64_t)N * 2 <= K && codes <= 4500000ull && (bits == 4 || M > 2);
+    if (M > 8 && ((K > 6144 && N > 1024) || (K < 2048 && N > 8192))) return false;
+    return codes <= (bits == 4 ? 75000000ull : 60000000ull);
 }
 
 static uint32_t runs_cus() {

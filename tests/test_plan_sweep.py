@@ -233,3 +233,15 @@ def test_bit_stream_tiles_at_65_to_128_rows(bits, M, N, K, G, tile, ksplit):
     assert rc == 0
     args = launches[0][0].split("<")[1].split(", ")
     assert int(args[3]) * 32 == tile and launches[0][1][1] == ksplit, launches
+
+
+@pytest.mark.parametrize("bits,M,N,K,runs", [
+    (4, 2, 1024, 4096, True), (8, 2, 1024, 4096, False), (8, 3, 1024, 4096, True), (4, 4, 1024, 1024, False), (4, 4, 512, 2048, True), (4, 4, 2048, 2048, False),
+    (4, 3, 512, 8192, False), (4, 2, 4096, 1024, False), (4, 5, 8192, 8192, True), (4, 9, 8192, 8192, False), (4, 16, 1024, 8192, True), (4, 9, 1025, 8192, False),
+    (4, 9, 1040, 6144, True), (4, 16, 8192, 512, True), (4, 16, 8208, 512, False), (4, 8, 16384, 512, True), (8, 16, 16384, 2048, True), (4, 16, 13824, 5120, True),
+    (4, 16, 16384, 5120, False), (8, 16, 14336, 4096, True), (8, 16, 16384, 4096, False), (4, 1, 1024, 4096, False), (4, 17, 1024, 4096, False),
+])
+def test_k_run_lines(bits, M, N, K, runs):
+    """Which matrices the K-run kernel is for, on both sides of each line."""
+    rc, launches, _, _ = ops.plan("qmm", DType.BF16, bits, 64, M, N, K)
+    assert rc == 0 and ("qmv_runs_kernel" in launches[0][0]) == runs, launches[0][0]
