@@ -120,12 +120,20 @@ MTQ_API int mtq_qmv(int dtype, int bits, uint32_t group_size, const void *w, con
                     uint32_t K);
 
 /* qmm: same product for any M; routes by M like mt_qmm_for
- * (crates/metaltile-std/src/mlx/quantized.rs:5040-5065): from 9 rows (from 5 where the
- * rows are long) the MFMA tile kernel (replaces mt_qmm_mma / _m16 / _int8 / _int2 / _b3 /
+ * (crates/metaltile-std/src/mlx/quantized.rs:5040-5065). 5 to 16 rows on a 4- or 8-bit f16 /
+ * bf16 matrix of up to 75 M codes (60 M of 8 bits), K % 128 == 0, K <= 8192 (5120 of 8 bits;
+ * from 9 rows with K > 6144 only N <= 1024, with K < 2048 only N <= 8192), and 2 to 4 rows on
+ * short ones (2048 <= K <= 4096, 2 N <= K, 4.5 M codes; 8 bits from 3 rows) run on the K-run
+ * kernel: exact w_hat; an activation that takes its sums past the f32 range is multiplied with
+ * w_hat rounded to the element type. 5 to 8 rows on a 4-bit matrix of 50 M codes or more, 9 to
+ * 16 on one of 100 M, run on the 16-row kernel (exact w_hat). Else from 9 rows (from 5 where
+ * the rows are long) the MFMA tile kernel (replaces mt_qmm_mma / _m16 / _int8 / _int2 / _b3 /
  * _b5 / _b6, quantized.rs:2106, 2408, 2731, 3330, 3560-3900; w_hat rounded to the element
- * type before the multiply, as there), below that the qmv family (exact w_hat). MTQ_F32
- * batches run on the f32 matrix cores from 5 rows. Short, wide matrices split K over
- * workgroups through a library-owned buffer (allocated on first use). */
+ * type before the multiply, as there), below that the qmv family (exact w_hat). A matrix takes
+ * the same kernel here and in mtq_qmm_batched, whose launch the K-run kernel shares: a single
+ * call is up to 4 us slower for it than it could be (8192 x 8192, 8 rows 15.5 -> 17.9 us, a
+ * pair 30.7 -> 26.3). MTQ_F32 batches run on the f32 matrix cores from 5 rows. Short, wide
+ * matrices split K over workgroups through a library-owned buffer (allocated on first use). */
 MTQ_API int mtq_qmm(int dtype, int bits, uint32_t group_size, const void *w, const void *scales,
                     const void *biases, const void *x, void *out, uint32_t M, uint32_t N,
                     uint32_t K);

@@ -356,8 +356,10 @@ static bool tiles_serve(int bits, uint32_t M, uint32_t N, uint32_t K) {
 
 // Kernel routing by M, the counterpart of mt_qmm_for
 // (crates/metaltile-std/src/mlx/quantized.rs:5040-5065, which sends M = 16 and the multiples
-// of 32 to its MMA kernels). Here the GEMV family takes 8 activation rows per pass over the
-// weights, so it serves up to 8 rows; from 9 rows the MFMA tile kernel takes over: a second GEMV
+// of 32 to its MMA kernels). Here the K-run kernel (qmv_runs_preferred) and the 16-row GEMV
+// (wide_serves) take the batches of up to 16 rows that they are fastest with. Of the others, the
+// GEMV family takes 8 activation rows per pass over the weights, so it serves up to 8 rows; from 9
+// rows the MFMA tile kernel takes over: a second GEMV
 // pass always loses to 32-row tiles once short matrices split K over workgroups (16 rows, GEMV
 // against tiles: 4096 x 14336 50 / 23 us, 2048 x 8192 21 / 11, 1024 x 4096 24 / 11, 14336 x 4096
 // 25 / 15, 128256 x 4096 134 / 98).
@@ -732,7 +734,9 @@ static int op_gather(int mode, int dtype, int bits, uint32_t G, const void* x, c
     // us, 8-row passes of the GEMV family -> this: 32 rows 58.6 -> 54.5 (CSR 63 -> 60), 64 rows 113 -> 56, 128 rows
     // 197 -> 105, 256 rows 345 -> 152 (the tiles, rounded weights: 82 and 99 at 128 and 256 rows). It loses below (16 rows
     // 53 -> 54.5: a workgroup stages 16 rows whatever the expert has) and on small experts. Long rows (CSR) in K slices:
-    // 8 x 4096 x 14336, 32 rows by a router, 110 us on the GEMV family -> 73, the addition of the slices' partial rows included.
+    // 8 x 4096 x 14336, 32 / 64 rows by a router, 101 / 149 us on the GEMV family -> 54 / 56, the addition of the slices' partial
+    // rows included; 64 x 4096 x 5632, 256 rows 279 -> 173, 4 x 2048 x 8192, 16 rows 17.9 -> 15.1. (These rows' limit, 256, bounds
+    // the partial results; beyond it, and below 4 rows per expert, long rows stay on the GEMV family, not because it is faster.)
     if (dtype != DT_F32 && mode != GATHER_SINGLE && options().gather_wide == 0 && (uint64_t)N * K >= (1ull << 24) &&
         (uint64_t)T >= (uint64_t)4 * (E < T ? E : T)) {
         rc = run_wide_gather(p, lc);
