@@ -54,22 +54,21 @@ template <int BITS> struct AffineGeom {
     static constexpr int NW = EPL * BITS / 32;  // packed words per lane
 };
 
-// EPL consecutive elements -> f32. What is quantised is read once: as a stream past the caches (14336 x 4096 f32, 4-bit codes,
-// quantised and read back, 118.6 -> 97.2 us; quantising alone 70 -> 49, 5.5 TB/s).
-template <int DT, int EPL> __device__ __forceinline__ void load_elems(const void* p, uint64_t i0, float (&v)[EPL]) {
+// EPL consecutive elements -> f32; STREAM: read past the caches (affine_streams).
+template <int DT, int EPL, bool STREAM> __device__ __forceinline__ void load_elems(const void* p, uint64_t i0, float (&v)[EPL]) {
     if constexpr (DT == DT_F32) {
         typedef float a_f32x4 __attribute__((ext_vector_type(4)));
         const a_f32x4* s = (const a_f32x4*)((const float*)p + i0);
 #pragma unroll
         for (int j = 0; j < EPL / 4; j++) {
-            const a_f32x4 t = __builtin_nontemporal_load(s + j);
+            const a_f32x4 t = STREAM ? __builtin_nontemporal_load(s + j) : s[j];
             v[4 * j] = t.x; v[4 * j + 1] = t.y; v[4 * j + 2] = t.z; v[4 * j + 3] = t.w;
         }
     } else {
         const a_u32x4* s = (const a_u32x4*)((const uint16_t*)p + i0);
 #pragma unroll
         for (int j = 0; j < EPL / 8; j++) {
-            const a_u32x4 t = __builtin_nontemporal_load(s + j);
+            const a_u32x4 t = STREAM ? __builtin_nontemporal_load(s + j) : s[j];
 #pragma unroll
             for (int d = 0; d < 4; d++) {
                 if constexpr (DT == DT_BF16) {
@@ -109,7 +108,7 @@ template <int BITS> struct AffineUnroll {
     static constexpr int U = AffineGeom<BITS>::EPL == 8 ? 4 : (AffineGeom<BITS>::EPL == 16 ? 2 : 1);
 };
 
-template <int DT, int BITS>
+template <int DT, int BITS, bool STREAM>
 __global__ __launch_bounds__(256) void affine_quantize_kernel(AffineArgs a) {
 #pragma clang fp contract(off)
     constexpr int EPL = AffineGeom<BITS>::EPL, NW = AffineGeom<BITS>::NW, U = AffineUnroll<BITS>::U;
@@ -121,7 +120,7 @@ __global__ __launch_bounds__(256) void affine_quantize_kernel(AffineArgs a) {
     for (int u = 0; u < U; u++) {
         t[u] = ((uint64_t)blockIdx.x * U + u) * 256u + threadIdx.x;
         live[u] = t[u] < n_lanes;  // the lanes of a group are live or not together (256 is a multiple of their count)
-        load_elems<DT, EPL>(a.in, (live[u] ? t[u] : n_lanes - 1) * EPL, v[u]);
+        load_elems<DT, EPL, STREAM>(a.in, (live[u] ? t[u] : n_lanes - 1) * EPL, v[u]);
     }
 #pragma unroll
     for (int u = 0; u < U; u++) {
@@ -227,6 +226,15 @@ __global__ __launch_bounds__(256) void affine_dequantize_kernel(AffineArgs a) {
     }
 }
 
+// A matrix that the last-level cache cannot hold beside what it becomes (256 MB) only drives that out of it: such an input is
+// read past the caches. f32, 4-bit codes, quantised and read back, us, caches used -> passed by: 14336 x 4096 (235 MB) 117.8 -> 96.4,
+// 8-bit 143.6 -> 107.0; 8192 x 4096 (134 MB), read before 57.3 -> 57.8, 8-bit 62.0 -> 62.8; 4096 x 4096 32.9 -> 33.9, 8-bit 34.9 -> 36.5. A
+// lane of the other widths has 64 or 128 bytes to itself, a line that its loads share only through a cache: 14336 x 4096, 2 / 3 /
+// 6 bits 133 / 136 / 143 -> 139 / 177 / 183. 16-bit elements gain nothing (14336 x 4096, 4-bit codes 57.1 -> 58.9).
+static bool affine_streams(uint64_t n_elem) {
+    return n_elem * sizeof(float) > (192ull << 20);
+}
+
 template <int DT, int BITS> static int launch_one(bool quantize, AffineArgs& a, const LaunchCtx& lc) {
     constexpr int EPL = AffineGeom<BITS>::EPL;
     if (a.group_size % EPL) return fail(ERR_UNSUPPORTED, "affine: group_size must be a multiple of the lane's run (8, 16 or 32 elements)");
@@ -240,7 +248,10 @@ template <int DT, int BITS> static int launch_one(bool quantize, AffineArgs& a, 
     const uint64_t blocks = (lanes + per_block - 1) / per_block;
     if (blocks == 0) return ERR_OK;
     if (blocks > 0x7FFFFFFFull) return fail(ERR_SHAPE, "affine: too many elements for one launch");
-    const void* fn = quantize ? (const void*)affine_quantize_kernel<DT, BITS> : (const void*)affine_dequantize_kernel<DT, BITS>;
+    const void* fn = !quantize ? (const void*)affine_dequantize_kernel<DT, BITS> : (const void*)affine_quantize_kernel<DT, BITS, false>;
+    if constexpr (DT == DT_F32 && EPL == 8) {
+        if (quantize && affine_streams(a.n_elem)) fn = (const void*)affine_quantize_kernel<DT, BITS, true>;
+    }
     void* args[] = {&a};
     hipError_t e = launch_kernel(fn, dim3((uint32_t)blocks), dim3(256), args, 0, lc);
     if (e != hipSuccess) return hip_fail(e, "affine kernel launch");

@@ -147,3 +147,28 @@ def test_affine_rejects_bad_shapes():
         ops.affine_dequantize(DType.F32, 4, 12, a, a, a, a, 120)    # group not a multiple of the lane's run
     ops.affine_quantize(DType.F32, 4, 64, a, a, a, a, 0)            # nothing to do
     a.free()
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+def test_matrix_larger_than_the_caches(bits):
+    """f32 matrices above 192 MiB are read past the caches: their codes, scales and biases are the bits that the same elements
+    give in two calls below that line, and nothing is written behind them. The last group ends within a workgroup."""
+    G = 64
+    n = (192 << 18) + 64 * 37          # 201 MB
+    half = n // 2 // G * G
+    v = np.random.default_rng(bits).standard_normal(n, dtype=np.float32)
+    print(f"[case] affine_quantize f32 b{bits} n={n}", flush=True)
+    w = GpuBuffer.from_bytes(v.tobytes())
+    got, exp = [], []
+    for parts, res in (([(0, n)], got), ([(0, half), (half, n - half)], exp)):
+        sizes = (n * bits // 8, n // G * 4, n // G * 4)
+        bufs = [GpuBuffer.from_bytes(b"\xcd" * (k + 64)) for k in sizes]
+        for at, count in parts:
+            ops.affine_quantize(DType.F32, bits, G, w.ptr + at * 4, bufs[0].ptr + at * bits // 8, bufs[1].ptr + at // G * 4, bufs[2].ptr + at // G * 4, count)
+        for b, k in zip(bufs, sizes):
+            raw = b.read_bytes(k + 64)
+            assert raw[-64:] == b"\xcd" * 64
+            res.append(raw)
+            b.free()
+    w.free()
+    assert got == exp
