@@ -293,16 +293,37 @@ static int try_wide(int dtype, int bits, uint32_t G, const void* w, const void* 
     return launch_qmv_wide(q, lc, need ? (char*)g.scratch_buf + g.scratch_held : nullptr);
 }
 
+// Whether a route of another kernel that the caller has asked for stands against the K-run kernels.
+static bool runs_barred() {
+    const Options& o = options();
+    return o.qmv_runs == 1 || (o.qmv_runs == 0 && (o.qmv_wide == 2 || o.qmv_mfma == 2 || o.qmv_kernel || o.qmm_kernel || o.qmm_kgroups || o.qmm_ksplit ||
+                                                   o.qmm_tile_rows || o.qmm_dma || o.qmm_splits));
+}
+
+// A batch on long rows, on the K-run kernel in slices of K.
+static bool slices_serve(const QmmParams& q) {
+    if (runs_barred() || options().qmv_runs == 2 || !qmv_slices_takes(q)) return false;
+    return options().qmv_runs == 3 || qmv_slices_preferred(q.bits, q.group_size, q.M, q.N, q.K);
+}
+static int try_slices(int dtype, int bits, uint32_t G, const void* w, const void* s, const void* b, const void* x, void* out,
+                      uint32_t M, uint32_t N, uint32_t K, const LaunchCtx& lc) {
+    QmmParams q;
+    q.dtype = dtype; q.bits = bits; q.group_size = G;
+    q.w = w; q.scales = s; q.biases = b; q.x = x; q.out = out;
+    q.M = M; q.N = N; q.K = K;
+    if (!slices_serve(q)) return ERR_UNSUPPORTED;
+    int rc = ensure_scratch(g.scratch_held + qmv_slices_scratch_bytes(q));
+    if (rc) return rc;
+    return launch_qmv_slices(q, lc, (char*)g.scratch_buf + g.scratch_held);
+}
+
 // The matrices of a batch that the K-run kernel is for, in one launch: taken[j] says which those are. The rule looks at one
 // matrix at a time, so that a matrix gives the same bits alone and in a batch.
 static int run_runs(int dtype, int bits, uint32_t G, int n, const void* const* w, const void* const* s, const void* const* b,
                     const void* x, void* const* outs, uint32_t M, const uint32_t* N, uint32_t K, bool* taken, const LaunchCtx& lc) {
     const Options& o = options();
     for (int j = 0; j < n; j++) taken[j] = false;
-    // a route of another kernel that the caller has asked for stands
-    if (o.qmv_runs == 1 || (o.qmv_runs == 0 && (o.qmv_wide == 2 || o.qmv_mfma == 2 || o.qmv_kernel || o.qmm_kernel || o.qmm_kgroups || o.qmm_ksplit ||
-                                                o.qmm_tile_rows || o.qmm_dma || o.qmm_splits)))
-        return ERR_OK;
+    if (runs_barred() || o.qmv_runs == 3) return ERR_OK;
     QmvParams p;
     p.dtype = dtype; p.bits = bits; p.group_size = G; p.x = x; p.M = M; p.K = K;
     QmvBatch all;
@@ -375,6 +396,8 @@ static int op_qmm(int dtype, int bits, uint32_t G, const void* w, const void* s,
         bool taken;
         rc = run_runs(dtype, bits, G, 1, &w, &s, &b, x, &out, M, &N, K, &taken, lc);
         if (rc || taken) return rc;
+        rc = try_slices(dtype, bits, G, w, s, b, x, out, M, N, K, lc);
+        if (rc != ERR_UNSUPPORTED) return rc;
         rc = try_wide(dtype, bits, G, w, s, b, x, out, M, N, K, false, lc);
         if (rc != ERR_UNSUPPORTED) return rc;
     }
@@ -638,7 +661,7 @@ static int op_qmm_batched(int dtype, int bits, uint32_t G, int n, const void* co
         q.dtype = dtype; q.bits = bits; q.group_size = G;
         q.w = w[j]; q.scales = s[j]; q.biases = b[j]; q.x = x; q.out = outs[j];
         q.M = M; q.N = N[j]; q.K = K;
-        on_tiles[j] = !exact && dtype != DT_F32 && options().qmm_kernel != 1 && !wide_serves(q, false) && tiles_serve(bits, M, N[j], K) &&
+        on_tiles[j] = !exact && dtype != DT_F32 && options().qmm_kernel != 1 && !slices_serve(q) && !wide_serves(q, false) && tiles_serve(bits, M, N[j], K) &&
                       plan_qmm_direct(q, tiled[n_tiled]) == ERR_OK;
         if (on_tiles[j]) need += tiled[n_tiled++].scratch;
         else left++;
@@ -1879,7 +1902,7 @@ int mtq_set_option(const char* name, int value) {
         return MTQ_OK;
     }
     if (!strcmp(name, "qmv.runs")) {
-        if (value < 0 || value > 2) return fail(ERR_BAD_ARG, "qmv.runs must be 0 (choose), 1 (never) or 2 (wherever the shape allows)");
+        if (value < 0 || value > 3) return fail(ERR_BAD_ARG, "qmv.runs must be 0 (choose), 1 (never), 2 (wherever the shape allows) or 3 (in slices of K wherever the shape allows)");
         options().qmv_runs = value;
         return ERR_OK;
     }

@@ -118,7 +118,7 @@ struct Options {
     int qmv_wide_kp = 0;          // 16-row matrix-core GEMV: waves sharing a row block (0 = choose; 1, 2, 4, 8, 16)
     int qmv_wide_nb = 0;          // 16-row matrix-core GEMV: row blocks per wave (0 = choose; 1, 2)
     int gather_wide = 0;          // expert-routed rows on the 16-row matrix-core GEMV: 0 = choose, 1 = never, 2 = wherever the shape allows
-    int qmv_runs = 0;             // K-run matrix-core GEMV for batches of up to 16 rows: 0 = choose per shape, 1 = never, 2 = wherever the shape allows
+    int qmv_runs = 0;             // K-run matrix-core GEMV for batches of up to 16 rows: 0 = choose per shape, 1 = never, 2 = wherever the shape allows, 3 = the K-sliced form wherever the shape allows
     int qmv_wide = 0;             // 16-row matrix-core GEMV for batches of 5..16 rows: 0 = choose per shape, 1 = never, 2 = wherever the shape allows
 };
 Options& options();
@@ -190,6 +190,13 @@ int launch_qmv_wide_gather(const QmvParams& p, const LaunchCtx& lc, void* scratc
 bool qmv_runs_takes(const QmvParams& p, const QmvBatch& b);
 bool qmv_runs_preferred(int bits, uint32_t M, uint32_t N, uint32_t K);   // one matrix's sizes
 int launch_qmv_runs(const QmvParams& p, const QmvBatch& b, const LaunchCtx& lc);
+// The same walk on slices of K: one matrix of longer rows. scratch: qmv_slices_scratch_bytes(p) bytes.
+bool qmv_slices_takes(const QmmParams& p);
+bool qmv_slices_preferred(int bits, uint32_t G, uint32_t M, uint32_t N, uint32_t K);
+size_t qmv_slices_scratch_bytes(const QmmParams& p);
+int launch_qmv_slices(const QmmParams& p, const LaunchCtx& lc, void* scratch);
+// Adds f32 partial results [slices][total] in slice order and rounds to the element type (qmv_wide.hip).
+int add_slices(int dtype, const float* part, void* out, uint32_t total, uint32_t slices, const LaunchCtx& lc);
 // f32 operands on the f32 matrix cores, any code width (qmm_f32.hip).
 // scratch: qmm_f32_scratch_bytes(p) bytes (0 when K is not split: then scratch may be null).
 size_t qmm_f32_scratch_bytes(const QmmParams& p);

@@ -20,20 +20,11 @@ static bool runs_aligned(const void* w, const void* s, const void* b, const void
     return (uintptr_t)w % 16 == 0 && (uintptr_t)s % 16 == 0 && (uintptr_t)b % 16 == 0 && (uintptr_t)x % 16 == 0;
 }
 
-// Blocks in flight: as many as the registers of sixteen waves hold beside the activations.
-template <int DT, int BITS, int G> static const void* runs_pick_steps(uint32_t xs) {
-    if constexpr (BITS == 4)
-        return xs <= 1 ? (const void*)qmv_runs_kernel<DT, 4, G, 1, 3> : xs == 2 ? (const void*)qmv_runs_kernel<DT, 4, G, 2, 2> :
-               xs == 3 ? (const void*)qmv_runs_kernel<DT, 4, G, 3, 1> : (const void*)qmv_runs_kernel<DT, 4, G, 4, 1>;
-    else
-        return xs <= 2 ? (const void*)qmv_runs_kernel<DT, 8, G, 2, 2> : xs <= 4 ? (const void*)qmv_runs_kernel<DT, 8, G, 4, 1> : (const void*)qmv_runs_kernel<DT, 8, G, 5, 1>;
-}
-template <int DT, int BITS> static const void* runs_pick_g(uint32_t G, uint32_t xs) {
-    return G == 32 ? runs_pick_steps<DT, BITS, 32>(xs) : G == 64 ? runs_pick_steps<DT, BITS, 64>(xs) : runs_pick_steps<DT, BITS, 128>(xs);
-}
-static const void* runs_pick(int dtype, int bits, uint32_t G, uint32_t xs) {
-    if (dtype == DT_BF16) return bits == 4 ? runs_pick_g<DT_BF16, 4>(G, xs) : runs_pick_g<DT_BF16, 8>(G, xs);
-    return bits == 4 ? runs_pick_g<DT_F16, 4>(G, xs) : runs_pick_g<DT_F16, 8>(G, xs);
+// (instances: qmv_runs_pick.h, one translation unit per element type)
+const void* qmv_runs_pick_f16(int bits, uint32_t G, bool sliced, uint32_t xs);
+const void* qmv_runs_pick_bf16(int bits, uint32_t G, bool sliced, uint32_t xs);
+static const void* runs_pick(int dtype, int bits, uint32_t G, bool sliced, uint32_t xs) {
+    return dtype == DT_BF16 ? qmv_runs_pick_bf16(bits, G, sliced, xs) : qmv_runs_pick_f16(bits, G, sliced, xs);
 }
 
 bool qmv_runs_takes(const QmvParams& p, const QmvBatch& b) {
@@ -65,16 +56,41 @@ bool qmv_runs_takes(const QmvParams& p, const QmvBatch& b) {
 //   1280 x 5120     5.1  5.5  5.7 ->  7.5  7.7  8.0 | 10.0 10.9 11.1 ->  7.7  7.9  8.0
 //   512 x 8192      6.3  7.6  8.8 ->  9.5  9.9 10.3 | 13.0 15.5 17.9 ->  9.8 10.2 10.6
 //   4096 x 1024     3.6  3.8  3.8 ->  5.3  5.3  5.4 |  7.1  7.4  7.4 ->  6.4  6.4  6.5
-// So: below 5 rows short matrices against rows of 2048 to 4096 codes (the K and V projections of grouped-query attention; 8-bit
+// Four rows on matrices of 16 to 76 M codes in rows of 2049 to 5120 (not 4096 of 8192 or more weight rows, which have a kernel of
+// their own, qmv_rows_few.hip): 4096 x 4096 6.2 -> 7.8 | 12.4 -> 9.1; 5120 x 5120 8.9 -> 9.8 | 17.9 -> 12.9; 18944 x 3584 13.7 -> 14.1 | 27.2 -> 21.8;
+// 13824 x 5120 12.9 -> 14.6 | 25.5 -> 22.6; 8 bits 5120 x 5120 11.1 -> 13.1 | 22.2 -> 18.6; 18944 x 3584 18.3 -> 19.1 | 36.4 -> 32.1.
+// So: below 5 rows those, and short matrices against rows of 2048 to 4096 codes (the K and V projections of grouped-query attention; 8-bit
 // codes from 3 rows); from 5 rows up to 75 M codes (60 M of 8 bits), and from 9 rows, where the others take tiles, no more than
 // 1024 weight rows of more than 6144 codes (four steps a run, whose registers leave one block in flight) and no more than 8192 of
 // fewer than 2048 (some of the sixteen waves have no step, and a workgroup has more than two blocks to walk).
 bool qmv_runs_preferred(int bits, uint32_t M, uint32_t N, uint32_t K) {
     if (M < 2 || M > 16) return false;
     const uint64_t codes = (uint64_t)N * K;
+    if (M == 4 && K > 2048 && K <= 5120 && codes >= 16000000ull && codes <= 76000000ull && !(bits == 4 && K == 4096 && N >= 8192)) return true;
     if (M < 5) return K >= 2048 && K <= 4096 && (uint64_t)N * 2 <= K && codes <= 4500000ull && (bits == 4 || M > 2);
     if (M > 8 && ((K > 6144 && N > 1024) || (K < 2048 && N > 8192))) return false;
     return codes <= (bits == 4 ? 75000000ull : 60000000ull);
+}
+
+// The K-sliced form against the others; it pays a second launch (about 5 us with its gap), so it is for what they are slow at.
+// us, groups of 64 where nothing else is said, others -> this:
+//   3, 4 rows of more than 18432 codes (four rows do not fit the LDS of the matrix-core GEMV, which reads the weights twice):
+//     3584 x 18944 24.4 -> 19.8, 8 bits 34.3 -> 23.2; 8192 x 28672 53.9 -> 42.9, 8 bits 88.8 -> 60.4; 1024 x 18688 16.0 -> 12.6
+//     (at 14336 codes 12.8 -> 19.1)
+//   K no multiple of 256 (no K split on the tiles): 4096 x 9344 in groups of 128, 5 / 16 rows 79.7 / 80.2 -> 13.6 / 14.0; 7168 x
+//     18560 165 -> 25
+//   4-bit rows whose scales are not whole 16-byte vectors (register-staged tiles): 5120 x 13824 in groups of 128, 9 / 16 rows
+//     24.4 / 24.8 -> 17.8 / 18.0; 4096 x 11008, 5 / 16 rows 18.1 / 19.0 -> 17.8 / 17.9; but 2048 x 8960 in groups of 128 10.9 -> 11.4, and
+//     up to 8 rows, where the 16-row kernel takes it, 5120 x 13824 15.6 -> 17.9
+//   8 bits, 5..8 rows on less than twice as many codes as weight rows (two passes of the GEMV): 8192 x 10240 36.2 -> 24.9; and from
+//     230 M codes: 8192 x 28672, 16 rows 96.8 -> 64.5 (16384 x 12288, 201 M: 51.9 -> 55.0)
+bool qmv_slices_preferred(int bits, uint32_t G, uint32_t M, uint32_t N, uint32_t K) {
+    if (M < 3 || M > 16 || K <= 8192) return false;
+    if (M <= 4) return K > 18432;
+    if (K % 256) return true;
+    const uint64_t codes = (uint64_t)N * K;
+    if (bits == 8) return codes >= 230000000ull || (M <= 8 && K < 2 * (uint64_t)N);
+    return K / G % 8u != 0 && N >= 4096 && !(M <= 8 && codes >= 50000000ull && K % 512 == 0);
 }
 
 static uint32_t runs_cus() {
@@ -100,12 +116,52 @@ int launch_qmv_runs(const QmvParams& p, const QmvBatch& b, const LaunchCtx& lc) 
     a.x = (const unsigned char*)p.x;
     a.M = p.M;
     a.K = p.K;
-    const uint32_t cus = runs_cus(), wgs = a.blocks < cus ? a.blocks : cus;
-    const void* fn = runs_pick(p.dtype, p.bits, p.group_size, runs_steps(p.bits, p.K));
+    a.slices = 1;
+    const uint32_t cus = runs_cus(), wgs = a.blocks < cus ? a.blocks : cus, xs = runs_steps(p.bits, p.K);
+    const void* fn = runs_pick(p.dtype, p.bits, p.group_size, false, xs);
     void* args[] = {&a};
-    hipError_t e = launch_kernel(fn, dim3(wgs), dim3(1024), args, 0, lc);
+    hipError_t e = launch_kernel(fn, dim3(wgs), dim3(p.bits == 4 && (xs <= 1 || xs == 4) ? 512 : 1024), args, 0, lc);
     if (e != hipSuccess) return hip_fail(e, "K-run qmv kernel launch");
     return ERR_OK;
+}
+
+// Rows too long for the registers of one workgroup, in slices of up to 5120 codes: each workgroup works on one slice, f32 sums
+// of the slices go to scratch and a second launch adds them in slice order.
+static uint32_t slices_of(uint32_t K) { return (K + 5119u) / 5120u; }
+
+bool qmv_slices_takes(const QmmParams& p) {
+    const uint32_t G = p.group_size, M = p.M, N = p.N, K = p.K;
+    if ((p.dtype != DT_F16 && p.dtype != DT_BF16) || (p.bits != 4 && p.bits != 8) || (G != 32 && G != 64 && G != 128)) return false;
+    if (M == 0 || M > 16 || N == 0 || K % 128 || K % G || K <= 5120 || slices_of(K) > 16u) return false;
+    if (!runs_aligned(p.w, p.scales, p.biases, p.x) || (uint64_t)slices_of(K) * M * N >= (1ull << 31)) return false;
+    return (uint64_t)N * K * p.bits / 8 < (1ull << 31) && (uint64_t)M * K * 2 < (1ull << 31) && (uint64_t)N * (K / G) * 2 < (1ull << 31);
+}
+
+size_t qmv_slices_scratch_bytes(const QmmParams& p) { return (size_t)slices_of(p.K) * p.M * p.N * sizeof(float); }
+
+int launch_qmv_slices(const QmmParams& p, const LaunchCtx& lc, void* scratch) {
+    if (!qmv_slices_takes(p) || !scratch) return fail(ERR_UNSUPPORTED, "K-sliced qmv: shape not taken");
+    QmvRunsArgs a{};
+    for (int j = 1; j < 4; j++) a.block0[j] = 0x7FFFFFFFu;
+    a.w[0] = (const unsigned char*)p.w;
+    a.scales[0] = (const unsigned char*)p.scales;
+    a.biases[0] = (const unsigned char*)p.biases;
+    a.out[0] = (uint16_t*)p.out;
+    a.part[0] = (float*)scratch;
+    a.N[0] = p.N;
+    a.blocks = (p.N + 15u) / 16u;
+    a.x = (const unsigned char*)p.x;
+    a.M = p.M;
+    a.K = p.K;
+    a.slices = slices_of(p.K);
+    const uint32_t per = runs_cus() / a.slices > 0 ? runs_cus() / a.slices : 1u, wgs = (a.blocks < per ? a.blocks : per) * a.slices;
+    void* args[] = {&a};
+    LaunchCtx l1 = lc, l2 = lc;
+    l1.stop = nullptr;
+    l2.start = nullptr;
+    hipError_t e = launch_kernel(runs_pick(p.dtype, p.bits, p.group_size, true, 0), dim3(wgs), dim3(512), args, 0, l1);
+    if (e != hipSuccess) return hip_fail(e, "K-sliced qmv kernel launch");
+    return add_slices(p.dtype, (const float*)scratch, p.out, p.M * p.N, a.slices, l2);
 }
 
 }  // namespace mtq

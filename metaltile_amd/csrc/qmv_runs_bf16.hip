@@ -1,0 +1,8 @@
+// The K-run matrix-core GEMV, bf16 instances.
+#include "qmv_runs_pick.h"
+
+namespace mtq {
+
+const void* qmv_runs_pick_bf16(int bits, uint32_t G, bool sliced, uint32_t xs) { return runs_pick_type<DT_BF16>(bits, G, sliced, xs); }
+
+}  // namespace mtq

@@ -8,15 +8,19 @@
 // What bounds such a batch is the stream of weights; what kept the other kernels from it on matrices of 5 - 60 MB were
 // the parts around the stream: a launch per matrix, activations staged in LDS by every workgroup before its first
 // product, or f32 partial tiles of a split K and a second launch that adds them. Here one launch takes all matrices, and
-// its workgroups (one per compute unit) walk their blocks of 16 weight rows. The sixteen waves of a workgroup share a
-// block, each with a run of K / 16 codes of every row, whose activations it reads once, in the operand layout of the
-// 16x16x32 MFMA, and keeps in registers: from then on the only loads are weights, scales and biases, PF blocks ahead.
+// its workgroups (one per compute unit) walk their blocks of 16 weight rows. The waves of a workgroup (KP: sixteen, or eight) share a
+// block, each with a run of K / KP codes of every row, whose activations it reads once, turns into the operand layout of the
+// 16x16x32 MFMA and keeps in registers: from then on the only loads are weights, scales and biases, PF blocks ahead.
 // (Vector loads complete in order: activations read along the way, even from the L2, make a wave wait for all weights
-// asked for before them. The same kernel with activations read per block streamed at half the rate.) The sixteen sums of
+// asked for before them. The same kernel with activations read per block streamed at half the rate.) The KP sums of
 // a result meet in LDS. The split of K depends on K alone: a matrix gives the same bits in whatever batch of matrices.
 //
-// A step is 128 codes of a row (64 of 8-bit codes). Lane (j, q) = (lane % 16, lane / 16) loads the 16 bytes of row j at
-// 16 q: 32 codes (16). An MFMA has to stay inside one group of codes, so for groups shorter than a step the four lanes
+// A step is 128 codes of a row (64 of 8-bit codes), 64 bytes, of which lane (j, q) = (lane % 16, lane / 16) multiplies the 16 bytes
+// of row j at 16 q: 32 codes (16). What bounded the kernel was finding the lines: with neighbouring lanes in sixteen different rows
+// a load of 1 KB occupies the compute unit's address path four times as long as with four neighbours in one row, about 64 clk
+// against 16, and that was all of a block's 5000 clk at 16 rows (64 weight and scale loads of it). So four neighbours load a row's
+// step, and the pieces are turned in LDS (one write and one read of 16 bytes, conflict-free). 16 rows, us, groups of 128, before ->
+// after, with the activations first and turned alike: 3 x 5120 x 5120 17.2 -> 13.5, 5120 x 5120 12.4 -> 8.9, 2 x 13824 x 5120 24.2 -> 21.0. An MFMA has to stay inside one group of codes, so for groups shorter than a step the four lanes
 // of a row exchange dwords (v_permlane32_swap, and v_permlane16_swap for groups of 32 4-bit codes), and the activations
 // are put in the order that leaves, once. The sums of the activations over each group, which
 // the bias and the offset of the code conversion are multiplied by, come from one more MFMA per activation operand,
@@ -41,6 +45,8 @@ struct QmvRunsArgs {
     uint32_t blocks;         // of all matrices
     const unsigned char* x;
     uint32_t M, K;
+    uint32_t slices;         // of K, for the sliced kernel: workgroup i works on slice i % slices
+    float* part[4];          // and its f32 sums [slice][M][N]
 };
 
 typedef uint32_t kr_u32x4 __attribute__((ext_vector_type(4)));
@@ -62,6 +68,13 @@ template <int B, int E, class F> __device__ __forceinline__ void kr_for(F&& f) {
         f(std::integral_constant<int, B>{});
         kr_for<B + 1, E>(f);
     }
+}
+
+// Between a wave's writes to its own LDS and its reads of what other lanes wrote (LDS operations of a wave complete in order: no wait).
+__device__ __forceinline__ void kr_turned() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
 }
 
 constexpr uint32_t KR_OOB = 0x80000000u;   // every buffer is shorter than 2 GiB (host): base + KR_OOB is out of range for any base below 2 GiB
@@ -124,17 +137,20 @@ template <int DT, int BITS> __device__ __forceinline__ kr_u32x4 kr_weights(const
 
 // DT, BITS (4 or 8), G (32, 64, 128), XS: steps of a wave's run at most, PF: blocks whose
 // weights are in flight ahead of the one that is worked on.
-template <int DT, int BITS, int G, int XS, int PF> __global__ __launch_bounds__(1024) void qmv_runs_kernel(QmvRunsArgs a) {
+template <int KP, bool SLICED, int DT, int BITS, int G, int XS, int PF> __device__ __forceinline__ void qmv_runs_body(const QmvRunsArgs& a) {
     using C = KrCodes<DT, BITS>;
-    constexpr int KP = 16;
     constexpr int EG = G < C::STEP ? G : C::STEP;   // codes per scale within a step
     constexpr int GPS = C::STEP / EG;               // scales per step: 1, 2 or 4
     constexpr int UPG = EG / 32;                    // MFMAs per scale
     constexpr bool SWAP32 = EG * 2 <= C::STEP, SWAP16 = EG * 4 <= C::STEP;
     constexpr int SDW = GPS == 4 ? 2 : 1;           // dwords of scales per step and row
     constexpr int SR = (XS + 3) / 4;                // scale registers: lanes (j, q) hold steps q, q + 4 of row j
-    constexpr bool HOLD = XS * GPS <= 4;       // the activations' sums stay in registers
+    constexpr bool HOLD = XS * GPS <= (KP == 16 ? 4 : 5);   // the activations' sums stay in registers
+    constexpr bool SUMS = !HOLD && KP != 16;                // or in LDS
+    constexpr int SLOTS = C::UNITS;                         // KB of LDS in which a wave turns a step's weights, or its activations
     __shared__ float red[2][KP * 256];
+    __shared__ kr_u32x4 turned[KP * SLOTS * 64];
+    __shared__ __attribute__((aligned(16))) float sums[SUMS ? KP * XS * GPS * 16 : 4];
 
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t kp = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -142,15 +158,30 @@ template <int DT, int BITS, int G, int XS, int PF> __global__ __launch_bounds__(
     const uint32_t K = a.K, wrow_bytes = K / 8u * BITS, gpr = K / (uint32_t)G;
 
     // this wave's run of steps
-    const uint32_t steps = K / (uint32_t)C::STEP;
-    const uint32_t t0 = steps * kp / KP, cnt = steps * (kp + 1u) / KP - t0;   // cnt <= XS (host)
+    const uint32_t all_steps = K / (uint32_t)C::STEP;
+    uint32_t first_step = 0, steps = all_steps, slice = 0, wg = blockIdx.x, wgs = gridDim.x;
+    if constexpr (SLICED) {
+        // (the grid is a whole number of workgroups per slice)
+        wg = blockIdx.x / a.slices;
+        slice = blockIdx.x - wg * a.slices;
+        wgs = gridDim.x / a.slices;
+        first_step = all_steps * slice / a.slices;
+        steps = all_steps * (slice + 1u) / a.slices - first_step;
+    }
+    const uint32_t t_in = steps * kp / KP, t0 = first_step + t_in, cnt = steps * (kp + 1u) / KP - t_in;   // cnt <= XS (host)
 
-    const uint32_t wlane = j * wrow_bytes + t0 * 64u + q * 16u;
+    // What a lane loads: slot ls of row lr, of the four 16-byte pieces that a step has of a row; the pieces of a row are dealt to
+    // its slots so that the sixteen rows' reads from LDS do not meet in a bank.
+    const uint32_t lr = lane >> 2, ls = lane & 3u, lpiece = (ls ^ (lr >> 1)) & 3u;
+    const uint32_t my_row = j * 4u, my_turn = (j >> 1) & 3u;   // (row j, piece p) lies in slot my_row + (p ^ my_turn)
+    kr_u32x4* const swap_lds = turned + kp * (uint32_t)(SLOTS * 64);
+
+    const uint32_t wlane = lr * wrow_bytes + t0 * 64u + lpiece * 16u;
     uint32_t slane[SR];
 #pragma unroll
     for (int i = 0; i < SR; i++) {
-        const uint32_t n = q + 4u * i, at = t0 + n;
-        slane[i] = n < cnt ? j * gpr * 2u + (G > C::STEP ? at / (uint32_t)(G / EG) : at * GPS) * 2u : KR_OOB;
+        const uint32_t n = ls + 4u * i, at = t0 + n;
+        slane[i] = n < cnt ? lr * gpr * 2u + (G > C::STEP ? at / (uint32_t)(G / EG) : at * GPS) * 2u : KR_OOB;
     }
     uint32_t step_dead[XS];   // steps past the run
 #pragma unroll
@@ -180,7 +211,7 @@ template <int DT, int BITS, int G, int XS, int PF> __global__ __launch_bounds__(
         const uint32_t row0 = (at_blk - first) * 16u, rows = blk < n_blocks ? N - row0 : 0u;   // (16 or more: a whole block)
         const __amdgpu_buffer_rsrc_t wr = kr_rsrc(pick(a.w, at_blk), N * wrow_bytes), sr = kr_rsrc(pick(a.scales, at_blk), N * gpr * 2u),
                                      br = kr_rsrc(pick(a.biases, at_blk), N * gpr * 2u);
-        const uint32_t dead = (rows - 1u - j) & KR_OOB;
+        const uint32_t dead = (rows - 1u - lr) & KR_OOB;
         const uint32_t wo = (wlane + row0 * wrow_bytes) | dead, s0 = row0 * gpr * 2u;
 #pragma unroll
         for (int i = 0; i < SR; i++) {
@@ -201,46 +232,44 @@ template <int DT, int BITS, int G, int XS, int PF> __global__ __launch_bounds__(
     };
 
     Block ring[PF + 1];
-    kr_for<0, PF>([&](auto p) { load_block(ring[decltype(p)::value], blockIdx.x + gridDim.x * (uint32_t)decltype(p)::value); });
 
-    // ---- the activations of the run. Load k of a step takes pieces 4 k + q of 8 codes: 64 contiguous bytes of every row (read
-    // straight into the operand layout, a load touches 64 separate lines: 5120 x 5120 in groups of 128, 16 rows 14.5 us, so 12.5). Unit u's
-    // pieces are 4 u + q where both exchanges are made, and otherwise those of where the lane's codes come from.
-    constexpr bool SWAP_X16 = !SWAP16 && !(BITS == 8 && SWAP32), SWAP_X32 = !SWAP32;
+    // ---- the activations of the run, ahead of the first weights (loads complete in order, over the whole compute unit: behind
+    // weights from memory they came late, 5120 x 5120 in groups of 128, 16 rows 11.6 us, so 10.1). They are turned in LDS: four neighbouring lanes read 64
+    // contiguous bytes (read straight into the operand layout, 16 rows next to each other, a load of 1 KB took four times as long
+    // to find its lines: 12.4 us, so 10.9), and unit u of lane (j, q) takes the piece of 8 codes that its weights will be.
     kr_u32x4 xop[XS][C::UNITS];
     {
         const __amdgpu_buffer_rsrc_t xr = kr_rsrc((uint64_t)a.x, a.M * K * 2u);
-        const uint32_t piece = BITS == 8 && SWAP32 ? (q & 1u) * 2u + (q >> 1) : q;
+        const uint32_t xo = ((lr * K + t0 * (uint32_t)C::STEP + lpiece * 8u) * 2u) | ((a.M - 1u - lr) & KR_OOB);
 #pragma unroll
-        for (int n = 0; n < XS; n++) {
-            const uint32_t o = ((j * K + (t0 + n) * (uint32_t)C::STEP + piece * 8u) * 2u) | ((a.M - 1u - j) & KR_OOB) | step_dead[n];
+        for (int n = 0; n < XS; n++)
 #pragma unroll
-            for (int k = 0; k < C::UNITS; k++) xop[n][k] = __builtin_amdgcn_raw_buffer_load_b128(xr, (int)(o + 64u * k), 0, 0);
+            for (int k = 0; k < C::UNITS; k++) xop[n][k] = __builtin_amdgcn_raw_buffer_load_b128(xr, (int)((xo + (uint32_t)(n * C::STEP * 2 + k * 64)) | step_dead[n]), 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_barrier();   // no wave's weights ahead of another's activations
+        kr_for<0, PF>([&](auto p) { load_block(ring[decltype(p)::value], wg + wgs * (uint32_t)decltype(p)::value); });
+        __builtin_amdgcn_sched_barrier(0);
+        uint32_t from[C::UNITS];
+#pragma unroll
+        for (uint32_t u = 0; u < C::UNITS; u++) {
+            const uint32_t p = BITS == 4 ? (SWAP16 ? 4u * u + q : SWAP32 ? (u >> 1) * 8u + (u & 1u) + (q & 1u) * 4u + (q >> 1) * 2u : 4u * q + u)
+                                         : (SWAP32 ? 4u * u + (q & 1u) * 2u + (q >> 1) : 2u * q + u);
+            from[u] = p / 4u * 64u + my_row + ((p ^ my_turn) & 3u);
         }
 #pragma unroll
         for (int n = 0; n < XS; n++) {
-            auto swap = [&](int u0, int u1, auto wide) {
 #pragma unroll
-                for (int d = 0; d < 4; d++) {
-                    const uint32_t p = xop[n][u0][d], r = xop[n][u1][d];
-                    const auto t = decltype(wide)::value ? __builtin_amdgcn_permlane32_swap(p, r, false, false) : __builtin_amdgcn_permlane16_swap(p, r, false, false);
-                    xop[n][u0][d] = t[0];
-                    xop[n][u1][d] = t[1];
-                }
-            };
-            if constexpr (BITS == 4) {
-                if constexpr (SWAP_X16) { swap(0, 1, std::false_type{}); swap(2, 3, std::false_type{}); }   // pieces 0 4 2 6 | 1 5 3 7 | 8 12 10 14 | 9 13 11 15
-                if constexpr (SWAP_X32) { swap(0, 2, std::true_type{}); swap(1, 3, std::true_type{}); }     // 0 4 8 12 | 1 5 9 13 | 2 6 10 14 | 3 7 11 15
+            for (int k = 0; k < C::UNITS; k++) swap_lds[k * 64 + lane] = xop[n][k];
+            kr_turned();
 #pragma unroll
-                for (int u = 0; u < C::UNITS; u++) {   // in the order the nibble masks deliver the codes
-                    const kr_u32x4 t = xop[n][u];
+            for (int u = 0; u < C::UNITS; u++) {
+                const kr_u32x4 t = swap_lds[from[u]];
+                if constexpr (BITS == 4)   // in the order the nibble masks deliver the codes
                     xop[n][u] = kr_u32x4{__builtin_amdgcn_perm(t.z, t.x, 0x05040100u), __builtin_amdgcn_perm(t.z, t.x, 0x07060302u),
-                                            __builtin_amdgcn_perm(t.w, t.y, 0x05040100u), __builtin_amdgcn_perm(t.w, t.y, 0x07060302u)};
-                }
-            } else if constexpr (SWAP_X32) {
-                swap(0, 1, std::true_type{});    // 0 1 4 5 | 2 3 6 7
-                swap(0, 1, std::false_type{});   // 0 2 4 6 | 1 3 5 7
+                                         __builtin_amdgcn_perm(t.w, t.y, 0x05040100u), __builtin_amdgcn_perm(t.w, t.y, 0x07060302u)};
+                else xop[n][u] = t;
             }
+            kr_turned();
         }
     }
     const uint32_t kor = BITS == 8 ? 0x64646464u : magic_or_vgpr<DT>();
@@ -259,6 +288,17 @@ template <int DT, int BITS, int G, int XS, int PF> __global__ __launch_bounds__(
         for (int n = 0; n < XS; n++)
 #pragma unroll
             for (int g = 0; g < GPS; g++) held[n][g] = x_sum(n, g);
+    }
+    if constexpr (SUMS) {
+        // [step][group][activation row], a wave's own: every column of the product is the same
+#pragma unroll
+        for (int n = 0; n < XS; n++)
+#pragma unroll
+            for (int g = 0; g < GPS; g++) {
+                const kr_f32x4 s = x_sum(n, g);
+                if (j == 0) *(kr_f32x4*)&sums[((kp * XS + n) * GPS + g) * 16 + 4 * q] = s;
+            }
+        kr_turned();
     }
     __builtin_amdgcn_sched_barrier(0);
 
@@ -283,18 +323,23 @@ template <int DT, int BITS, int G, int XS, int PF> __global__ __launch_bounds__(
         }
     };
     uint32_t par = 0;
-    uint32_t blk = blockIdx.x;
+    uint32_t blk = wg;
     auto turn = [&](auto p_c) {
         constexpr int p = decltype(p_c)::value;
-        load_block(ring[(p + PF) % (PF + 1)], blk + gridDim.x * (uint32_t)PF);
+        load_block(ring[(p + PF) % (PF + 1)], blk + wgs * (uint32_t)PF);
         __builtin_amdgcn_sched_barrier(0);
+        const uint32_t now = blk;
+        blk += wgs;
+        if (now >= n_blocks) return;   // (the same in every wave of the workgroup)
         Block& d = ring[p];
         kr_f32x4 tot = zero;
         kr_for<0, XS>([&](auto n_c) {
             constexpr int n = decltype(n_c)::value;
             uint32_t v[4];
-            codes_of(d.w[n], v);
-            const int src = (int)((j + 16u * (n % 4)) * 4u);   // the lane that holds this step's scales of row j
+            swap_lds[n % SLOTS * 64 + lane] = d.w[n];
+            kr_turned();
+            codes_of(swap_lds[n % SLOTS * 64 + my_row + (q ^ my_turn)], v);
+            const int src = (int)((my_row + (n % 4)) * 4u);   // the lane that holds this step's scales of row j
             kr_for<0, GPS>([&](auto g_c) {
                 constexpr int g = decltype(g_c)::value;
                 kr_f32x4 acc = zero;
@@ -306,39 +351,40 @@ template <int DT, int BITS, int G, int XS, int PF> __global__ __launch_bounds__(
                 const float bm = C::MAGIC == 0.f ? bv : fmaf(-C::MAGIC, sv, bv);
                 kr_f32x4 xs;
                 if constexpr (HOLD) xs = held[n][g];
+                else if constexpr (SUMS) xs = *(const kr_f32x4*)&sums[((kp * XS + n) * GPS + g) * 16 + 4 * q];
                 else xs = x_sum(n, g);
 #pragma unroll
                 for (int r = 0; r < 4; r++) tot[r] = fmaf(bm, xs[r], fmaf(sv, acc[r], tot[r]));
             });
         });
         // With an infinite activation, or one that the offset or the codes carry past the f32 range, the two halves of the
-        // formula are infinities of either sign and their sum no number. Such sums are worked out again, from the
-        // registers, with the weights themselves as operands, rounded to the element type as in the tile kernels.
+        // formula are infinities of either sign and their sum no number. Such sums are worked out again
+        // with the weights themselves as operands, rounded to the element type as in the tile kernels.
         // (What the look at the sums costs: 13824 x 5120, 16 rows 19.0 -> 19.3 us, 4096 x 4096 8.9 -> 9.0.)
         if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(__builtin_isfinite(tot[0]) && __builtin_isfinite(tot[1]) && __builtin_isfinite(tot[2]) && __builtin_isfinite(tot[3]))) != 0, 0)) {
+            // (From memory and in a rolled loop: the copies of the turn stay short. In the registers' order and unrolled the
+            // code was three times as long.)
             kr_f32x4 plain = zero;
-            kr_for<0, XS>([&](auto n_c) {
-                constexpr int n = decltype(n_c)::value;
-                kr_u32x4 w = d.w[n];
-                int src = (int)((j + 16u * (n % 4)) * 4u);
-                asm volatile("" : "+v"(w), "+v"(src));   // (nothing of the first pass is kept in registers for this one)
-                uint32_t v[4];
-                codes_of(w, v);
-                kr_for<0, GPS>([&](auto g_c) {
-                    constexpr int g = decltype(g_c)::value;
-                    const float sv = kr_elem<DT>((uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)d.s[n / 4][g / 2]), g % 2);
-                    const float bv = kr_elem<DT>((uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)d.b[n / 4][g / 2]), g % 2);
-#pragma unroll
-                    for (int u = g * UPG; u < (g + 1) * UPG; u++) {
-                        plain = kr_mfma<DT>(xop[n][u], kr_weights<DT, BITS>(&v[u * C::DPU], sv, bv), plain);
-                        __builtin_amdgcn_sched_barrier(0);
-                    }
-                });
-            });
+            const uint32_t at_blk = now, N = (uint32_t)pick(a.N, at_blk), row0 = (at_blk - (uint32_t)pick(a.block0, at_blk)) * 16u;
+            const __amdgpu_buffer_rsrc_t wr = kr_rsrc(pick(a.w, at_blk), N * wrow_bytes), sr = kr_rsrc(pick(a.scales, at_blk), N * gpr * 2u),
+                                         br = kr_rsrc(pick(a.biases, at_blk), N * gpr * 2u), xr = kr_rsrc((uint64_t)a.x, a.M * K * 2u);
+#pragma unroll 1
+            for (uint32_t k0 = t0 * (uint32_t)C::STEP, end = k0 + cnt * (uint32_t)C::STEP; k0 < end; k0 += 32u) {
+                const uint32_t k = k0 + 8u * q, wo = (row0 + j) * wrow_bytes + k / 8u * BITS, so = ((row0 + j) * gpr + k / (uint32_t)G) * 2u;   // rows past the last: zeros
+                uint32_t d[2] = {};
+                d[0] = __builtin_amdgcn_raw_buffer_load_b32(wr, (int)wo, 0, 0);
+                if constexpr (BITS == 8) d[1] = __builtin_amdgcn_raw_buffer_load_b32(wr, (int)wo + 4, 0, 0);
+                const uint32_t sp = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(sr, (int)so, 0, 0), bp = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(br, (int)so, 0, 0);
+                kr_u32x4 xv = __builtin_amdgcn_raw_buffer_load_b128(xr, (int)(((j * K + k) * 2u) | ((a.M - 1u - j) & KR_OOB)), 0, 0);
+                if constexpr (BITS == 4)   // in the order of kr_weights
+                    xv = kr_u32x4{__builtin_amdgcn_perm(xv.z, xv.x, 0x05040100u), __builtin_amdgcn_perm(xv.z, xv.x, 0x07060302u),
+                                  __builtin_amdgcn_perm(xv.w, xv.y, 0x05040100u), __builtin_amdgcn_perm(xv.w, xv.y, 0x07060302u)};
+                plain = kr_mfma<DT>(xv, kr_weights<DT, BITS>(d, kr_elem<DT>(sp, 0), kr_elem<DT>(bp, 0)), plain);
+            }
 #pragma unroll
             for (int r = 0; r < 4; r++) tot[r] = __builtin_isfinite(tot[r]) ? tot[r] : plain[r];
         }
-        // The sixteen runs meet in LDS: result r of lane (j, q) is activation row 4 q + r, weight row j. The
+        // The runs meet in LDS: result r of lane (j, q) is activation row 4 q + r, weight row j. The
         // other half of the buffer takes the next block, so one barrier per block is enough.
         float* rd = red[par];
         par ^= 1u;
@@ -351,22 +397,33 @@ template <int DT, int BITS, int G, int XS, int PF> __global__ __launch_bounds__(
             float s = rd[tid];
 #pragma unroll
             for (uint32_t o = 1; o < KP; o++) s += rd[o * 256u + tid];
-            __attribute__((address_space(1))) uint16_t* out = (__attribute__((address_space(1))) uint16_t*)pick(a.out, blk);
-            const uint32_t N = (uint32_t)pick(a.N, blk), first = (uint32_t)pick(a.block0, blk);
-            const uint32_t arow = 4u * q + (tid >> 6), wrow = (blk - first) * 16u + j;
-            if (arow < a.M && wrow < N) out[(size_t)arow * N + wrow] = f32_to_elem_bits<DT>(s);
+            __attribute__((address_space(1))) uint16_t* out = (__attribute__((address_space(1))) uint16_t*)pick(a.out, now);
+            const uint32_t N = (uint32_t)pick(a.N, now), first = (uint32_t)pick(a.block0, now);
+            const uint32_t arow = 4u * q + (tid >> 6), wrow = (now - first) * 16u + j;
+            if (arow < a.M && wrow < N) {
+                if constexpr (SLICED) {
+                    __attribute__((address_space(1))) float* part = (__attribute__((address_space(1))) float*)pick(a.part, now);
+                    part[((size_t)slice * a.M + arow) * N + wrow] = s;
+                } else {
+                    out[(size_t)arow * N + wrow] = f32_to_elem_bits<DT>(s);
+                }
+            }
         }
-        blk += gridDim.x;
-        return blk < n_blocks;   // (the same in every wave of the workgroup)
     };
-    for (;;) {
-        if (!turn(std::integral_constant<int, 0>{})) break;
-        if (!turn(std::integral_constant<int, 1>{})) break;
-        if constexpr (PF >= 2)
-            if (!turn(std::integral_constant<int, 2>{})) break;
-        if constexpr (PF >= 3)
-            if (!turn(std::integral_constant<int, 3>{})) break;
-    }
+    // (The way out lies behind the last turn only. From breaks between the turns the compiler makes one edge back to the loop's
+    // head, on which it takes the loads of any turn to be still in flight, and waits at the head for all of them: with one block
+    // ahead, none was in flight at every second turn.)
+    do kr_for<0, PF + 1>(turn);
+    while (blk < n_blocks);
+}
+
+// XS: steps of a sixteenth of K at most.
+template <int KP, int DT, int BITS, int G, int XS, int PF> __global__ __launch_bounds__(KP * 64) void qmv_runs_kernel(QmvRunsArgs a) {
+    qmv_runs_body<KP, false, DT, BITS, G, XS * 16 / KP, PF>(a);
+}
+// On one of a.slices slices of K, whose sums a second launch adds; XS: steps of an eighth of a slice at most.
+template <int DT, int BITS, int G, int XS, int PF> __global__ __launch_bounds__(512) void qmv_slices_kernel(QmvRunsArgs a) {
+    qmv_runs_body<8, true, DT, BITS, G, XS, PF>(a);
 }
 
 }  // namespace mtq

@@ -13,7 +13,7 @@ template <int DT> __global__ __launch_bounds__(256) void qmv_wide_reduce_kernel(
     ((uint16_t*)out)[i] = f32_to_elem_bits<DT>(r);
 }
 
-static int wide_reduce(int dtype, const float* part, void* out, uint32_t total, uint32_t ks, const LaunchCtx& lc) {
+int add_slices(int dtype, const float* part, void* out, uint32_t total, uint32_t ks, const LaunchCtx& lc) {
     void* args[] = {&part, &out, &total, &ks};
     const void* fn = dtype == DT_BF16 ? (const void*)qmv_wide_reduce_kernel<DT_BF16> : (const void*)qmv_wide_reduce_kernel<DT_F16>;
     hipError_t e = launch_kernel(fn, dim3((total + 255) / 256), dim3(256), args, 0, lc);
@@ -141,7 +141,7 @@ int launch_qmv_wide(const QmmParams& p, const LaunchCtx& lc, void* scratch) {
     if (pl.ksplit > 1) { l1.stop = nullptr; l2.start = nullptr; }
     e = launch_kernel(fn, dim3(pl.grid_x, pl.ksplit), dim3(1024), args, pl.lds, l1);
     if (e != hipSuccess) return hip_fail(e, "wide qmv kernel launch");
-    return pl.ksplit > 1 ? wide_reduce(p.dtype, a.part, a.out, p.M * p.N, pl.ksplit, l2) : ERR_OK;
+    return pl.ksplit > 1 ? add_slices(p.dtype, a.part, a.out, p.M * p.N, pl.ksplit, l2) : ERR_OK;
 }
 
 // Expert-routed rows (CSR offsets or one expert id per row) on the same kernel: blockIdx.y is the expert, whose rows
@@ -213,7 +213,7 @@ int launch_qmv_wide_gather(const QmvParams& p, const LaunchCtx& lc, void* scratc
     if (pl.ksplit > 1) { l1.stop = nullptr; l2.start = nullptr; }
     e = launch_kernel(fn, dim3(pl.grid_x, p.E, pl.ksplit), dim3(1024), args, pl.lds, l1);
     if (e != hipSuccess) return hip_fail(e, "wide gather kernel launch");
-    return pl.ksplit > 1 ? wide_reduce(p.dtype, a.part, p.out, p.T * p.N, pl.ksplit, l2) : ERR_OK;
+    return pl.ksplit > 1 ? add_slices(p.dtype, a.part, p.out, p.T * p.N, pl.ksplit, l2) : ERR_OK;
 }
 
 }  // namespace mtq
