@@ -168,28 +168,56 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(SortArgs a) {
     for (uint32_t x = after + tid; x <= a.n_experts; x += 1024) a.expert_offsets[x] = a.n;
 }
 
-// Counting sort, stable, for up to 2048 experts and any number of entries. The 16 waves of one
-// workgroup own consecutive segments of the entries. Pass 1: per-wave histograms in LDS. Pass 2: the
-// experts' CSR offsets (scan over experts) and, per wave and expert, where that wave's first entry
-// of the expert goes. Pass 3: each wave walks its segment 64 entries at a time; an entry's place is
+// Counting sort, stable, for up to 2048 experts and any number of entries. Each workgroup places `share` consecutive
+// entries, its 16 waves consecutive segments of them, and counts all entries for itself: those before its share, those of
+// each of its segments, those after it. So no workgroup waits for another, and reading 64 KB of ids once per workgroup costs
+// less than a second launch. Pass 2: the experts' CSR offsets (scan over experts) and, per wave and expert, where that
+// wave's first entry of the expert goes. Pass 3: each wave walks its segment 64 entries at a time; an entry's place is
 // its wave's cursor for the expert plus its rank among the equal entries of the 64 (the lanes with the
 // same expert are found with one ballot per bit of the expert id), and the cursors move on. Waves never wait for each other after pass 2.
-__global__ __launch_bounds__(1024) void moe_count_sort_kernel(SortArgs a) {
+// What bounds it is the scattered stores and the chain of each 64 entries, which one compute unit had to do for all of them:
+// 16384 entries of 128 experts 21.6 -> 6.3 us, 4096 of 8 experts 4.6 us.
+struct CountSortArgs {
+    SortArgs s;
+    uint32_t share;   // entries a workgroup places, a multiple of 1024
+    uint32_t wide;    // the ids begin on 16 bytes
+};
+__global__ __launch_bounds__(1024) void moe_count_sort_kernel(CountSortArgs c) {
+    const SortArgs& a = c.s;
     extern __shared__ uint32_t tab[];            // [16][E] counts, then cursors
     const uint32_t E = a.n_experts, W = 16;
-    uint32_t* offs = tab + W * E;                // [E] totals, then exclusive offsets
+    uint32_t* before = tab + W * E;              // [E] entries ahead of this workgroup's
+    uint32_t* offs = before + E;                 // [E] entries behind them, then totals, then exclusive offsets
     const uint32_t tid = threadIdx.x, lane = tid & 63u, w = tid >> 6;
-    const uint32_t seg = ((a.n + W - 1) / W + 63u) & ~63u;
-    const uint32_t lo = min(a.n, w * seg), hi = min(a.n, lo + seg);
-    for (uint32_t i = tid; i < W * E; i += 1024) tab[i] = 0;
+    const uint32_t seg = c.share / W;
+    const uint32_t first = min(a.n, blockIdx.x * c.share), last = min(a.n, first + c.share);
+    const uint32_t lo = min(last, first + w * seg), hi = min(last, lo + seg);
+    for (uint32_t i = tid; i < (W + 2) * E; i += 1024) tab[i] = 0;
     __syncthreads();
-    for (uint32_t base = lo; base < hi; base += 64) {
-        const uint32_t i = base + lane;
-        if (i < hi) atomicAdd(&tab[w * E + min(a.indices[i], E - 1)], 1u);
+    auto count = [&](uint32_t i, uint32_t id) {
+        const uint32_t e = min(id, E - 1);
+        atomicAdd(i < first ? before + e : i < last ? tab + ((i - first) / seg) * E + e : offs + e, 1u);
+    };
+    const uint32_t n4 = c.wide ? a.n / 4 : 0u;
+    for (uint32_t v0 = tid; v0 < n4; v0 += 4 * 1024) {  // four loads in flight
+        uint4 v[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) v[u] = ((const uint4*)a.indices)[min(v0 + u * 1024, n4 - 1)];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const uint32_t q = v0 + u * 1024;
+            if (q >= n4) continue;
+            count(4 * q, v[u].x);
+            count(4 * q + 1, v[u].y);
+            count(4 * q + 2, v[u].z);
+            count(4 * q + 3, v[u].w);
+        }
     }
+    for (uint32_t i = 4 * n4 + tid; i < a.n; i += 1024) count(i, a.indices[i]);
     __syncthreads();
     for (uint32_t e = tid; e < E; e += 1024) {
-        uint32_t t = 0;
+        uint32_t t = before[e] + offs[e];
+#pragma unroll
         for (uint32_t v = 0; v < W; v++) t += tab[v * E + e];
         offs[e] = t;
     }
@@ -214,14 +242,18 @@ __global__ __launch_bounds__(1024) void moe_count_sort_kernel(SortArgs a) {
     __syncthreads();
     for (uint32_t e = tid; e < E; e += 1024) {
         uint32_t run = offs[e];
-        a.expert_offsets[e] = run;
+        if (blockIdx.x == 0) a.expert_offsets[e] = run;
+        run += before[e];
+        uint32_t n_of[W];
+#pragma unroll
+        for (uint32_t v = 0; v < W; v++) n_of[v] = tab[v * E + e];
+#pragma unroll
         for (uint32_t v = 0; v < W; v++) {
-            const uint32_t c = tab[v * E + e];
             tab[v * E + e] = run;
-            run += c;
+            run += n_of[v];
         }
     }
-    if (tid == 0) a.expert_offsets[E] = a.n;
+    if (blockIdx.x == 0 && tid == 0) a.expert_offsets[E] = a.n;
     __syncthreads();
     uint32_t* cur = tab + w * E;
     uint32_t nbits = 0;
@@ -256,14 +288,20 @@ int launch_moe_sort(const uint32_t* indices, uint32_t n_tokens, uint32_t k, uint
     if (n_experts <= 2048 && n64 > 128 && options().moe_sort != 1) {
         // counting sort: no limit on the entries held in LDS, 10 x faster than the network at 32768 entries
         if (n64 >= (1ull << 31)) return fail(ERR_UNSUPPORTED, "expert sort: too many entries");
-        SortArgs a{indices, sort_token_idx, inv_perm, expert_offsets, (uint32_t)n64, 0, k, n_experts};
-        const size_t shmem = (size_t)17 * n_experts * 4;
+        // One wave step (64 entries) per wave up to 65536 entries. Ids sorted in place of their own inverse: one workgroup, which
+        // alone reads an id before it writes that place.
+        const uint32_t n = (uint32_t)n64;
+        const bool in_place = (uintptr_t)inv_perm < (uintptr_t)(indices + n) && (uintptr_t)indices < (uintptr_t)(inv_perm + n);
+        const uint32_t most = in_place ? 1u : 64u;
+        const uint32_t share = ((n + most - 1) / most + 1023u) & ~1023u;
+        CountSortArgs a{{indices, sort_token_idx, inv_perm, expert_offsets, n, 0, k, n_experts}, share, (uintptr_t)indices % 16 == 0 ? 1u : 0u};
+        const size_t shmem = (size_t)18 * n_experts * 4;
         if (shmem > 48 * 1024) {
             hipError_t e = set_max_dynamic_lds((const void*)moe_count_sort_kernel, (size_t)shmem);
             if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(max dynamic LDS)");
         }
         void* args[] = {&a};
-        hipError_t e = launch_kernel((const void*)moe_count_sort_kernel, dim3(1), dim3(1024), args, shmem, lc);
+        hipError_t e = launch_kernel((const void*)moe_count_sort_kernel, dim3((n + share - 1) / share), dim3(1024), args, shmem, lc);
         if (e != hipSuccess) return hip_fail(e, "expert sort kernel launch");
         return ERR_OK;
     }

@@ -109,6 +109,36 @@ def test_sort_by_expert(oracle, T, k, E):
         b.free()
 
 
+@pytest.mark.parametrize("T,k,E", [(128, 8, 16), (1025, 1, 128), (2047, 1, 3), (65536, 1, 64), (65537, 1, 64), (200001, 1, 2048), (40001, 5, 60)])
+@pytest.mark.parametrize("shift", [0, 1], ids=["aligned", "off 16 bytes"])
+def test_sort_over_many_workgroups(oracle, T, k, E, shift):
+    """Around the shares of entries that a workgroup places (1024, and more than 64 shares of it), a last vector of ids that is not
+    whole, ids past the last expert, one expert taking most entries, ids that begin 4 bytes behind a 16-byte line."""
+    print(f"[case] moe_sort over workgroups T={T} k={k} E={E} shift={shift}", flush=True)
+    rng = np.random.default_rng(T + E)
+    idx = np.where(rng.random(T * k) < 0.5, E // 2, rng.integers(0, E + 1, T * k)).astype("<u4")
+    rsti, rinv, roffs = oracle.moe_sort_by_expert(np.minimum(idx, E - 1), T, k, E)
+    di = GpuBuffer.from_bytes(b"\0" * (4 * shift) + idx.tobytes())
+    sti, inv, offs = GpuBuffer(T * k * 4), GpuBuffer(T * k * 4), GpuBuffer.from_bytes(b"\xff" * ((E + 1) * 4))
+    ops.moe_sort_by_expert(di.ptr + 4 * shift, T, k, E, sti, inv, offs)
+    assert np.array_equal(_u32(sti, T * k), rsti)
+    assert np.array_equal(_u32(inv, T * k), rinv)
+    assert np.array_equal(_u32(offs, E + 1), roffs)
+    for b in (di, sti, inv, offs):
+        b.free()
+
+
+def test_sort_with_the_inverse_in_place_of_the_ids(oracle):
+    T, k, E = 5000, 1, 37
+    idx = np.random.default_rng(6).integers(0, E, T * k).astype("<u4")
+    rsti, rinv, roffs = oracle.moe_sort_by_expert(idx, T, k, E)
+    di, sti, offs = GpuBuffer.from_bytes(idx.tobytes()), GpuBuffer(T * 4), GpuBuffer((E + 1) * 4)
+    ops.moe_sort_by_expert(di, T, k, E, sti, di, offs)
+    assert np.array_equal(_u32(sti, T), rsti) and np.array_equal(_u32(di, T), rinv) and np.array_equal(_u32(offs, E + 1), roffs)
+    for b in (di, sti, offs):
+        b.free()
+
+
 def test_sort_network_equals_counting_sort(oracle):
     """Both device sorts give the oracle's permutation (the counting sort serves up to 2048 experts,
     the network up to 32768 entries)."""
