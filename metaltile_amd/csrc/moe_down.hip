@@ -4,9 +4,14 @@
 // crates/metaltile-std/src/ffai/moe_down_swiglu_accum.rs:146-282).
 //
 // A workgroup stages slot_w[k] * silu(gate_k) * up_k for every slot in LDS as f32 (the
-// reference keeps the activation in f32 too), then each of its four waves takes output rows:
+// reference keeps the activation in f32 too), then each of its eight waves takes output rows:
 // the 64 lanes split the (slot, 16-byte weight chunk) pairs of a row between them, so one
 // wave-wide load covers whole 16-byte pieces of up to eight different experts' rows.
+// What bounds it: a chain of the staging (every compute unit works out every activation), the weights' trip to memory and the
+// dot products out of LDS. So there is one workgroup per compute unit where the rows allow, a row's first weights are asked for
+// ahead of the staging and the next ones ahead of the dot products, and the staged quads are swizzled: neighbouring lanes read
+// 128 bytes apart, which met 8 of the 64 banks. 8 slots of
+// 768 codes, 2048 rows, bf16: 10.9 -> 8.7 us (two workgroups of four waves per compute unit before).
 #include "mtq_device.h"
 #include "mtq_internal.h"
 
@@ -24,11 +29,38 @@ struct MoeDownArgs {
     uint32_t in_dim, out_dim, log2g, n_experts, n_slots, rows_per_wg, wide_acts;
 };
 
-template <int DT> __global__ __launch_bounds__(256) void moe_down_swiglu_kernel(MoeDownArgs a) {
-    extern __shared__ __align__(16) float inner[];  // [n_slots][in_dim]
-    __shared__ uint32_t expert_of[8];
+// Place of 16-byte quad Q of the staged activations: the eight quads of a 32-code chunk are turned by the chunk's number.
+__device__ __forceinline__ uint32_t down_quad(uint32_t Q) { return Q ^ ((Q >> 3) & 7u); }
+
+constexpr int DOWN_THREADS = 512, DOWN_WAVES = DOWN_THREADS / 64;
+
+template <int DT> __global__ __launch_bounds__(DOWN_THREADS) void moe_down_swiglu_kernel(MoeDownArgs a) {
+    extern __shared__ __align__(16) float inner[];  // [n_slots][in_dim], quads at down_quad
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-    if (tid < a.n_slots) expert_of[tid] = min(a.experts[tid], a.n_experts - 1);
+    const uint32_t chunks = a.in_dim / 32;      // 16-byte pieces of a 4-bit row
+    const uint32_t items = a.n_slots * chunks;
+    const uint32_t ng = a.in_dim >> a.log2g;
+    const uint32_t row0 = blockIdx.x * a.rows_per_wg, rows = min(a.rows_per_wg, a.out_dim - row0);
+    // up to four items of a row per lane: their weights, scales and biases
+    struct Set {
+        uint4 w[4];
+        float sc[4], bi[4];
+    };
+    auto load_set = [&](Set& s, uint32_t r, uint32_t base) {
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const uint32_t it = base + u * 64 + lane;
+            if (it >= items) continue;
+            const uint32_t k = it / chunks, c = it - k * chunks;
+            const size_t erow = (size_t)min(a.experts[k], a.n_experts - 1) * a.out_dim + row0 + r;
+            s.w[u] = *(const uint4*)(a.w + erow * (a.in_dim / 8) + c * 4);
+            const size_t g = erow * ng + ((c * 32) >> a.log2g);
+            s.sc[u] = load_elem<DT>(a.scales, g);
+            s.bi[u] = load_elem<DT>(a.biases, g);
+        }
+    };
+    Set cur = {};
+    if (wave < rows) load_set(cur, wave, 0);
     // Every (slot, 16-byte piece) of the gate / up rows is one item; a thread issues the loads of
     // up to four items before it touches any of them, so the staging costs one memory round trip.
     // Pointers are picked with compare-selects: an indexed read of the argument arrays would go
@@ -45,12 +77,12 @@ template <int DT> __global__ __launch_bounds__(256) void moe_down_swiglu_kernel(
     if (a.wide_acts) {
         constexpr int V = DT == DT_F32 ? 4 : 8;  // elements per 16-byte load (in_dim % 32 == 0)
         const uint32_t per_slot = a.in_dim / V, total = a.n_slots * per_slot;
-        for (uint32_t base = 0; base < total; base += 1024) {
+        for (uint32_t base = 0; base < total; base += 4 * DOWN_THREADS) {
             uint4 gv[4], uv[4];
             float sw[4];
 #pragma unroll
             for (int u = 0; u < 4; u++) {
-                const uint32_t it = min(base + u * 256 + tid, total - 1);
+                const uint32_t it = min(base + u * DOWN_THREADS + tid, total - 1);
                 const uint32_t k = it / per_slot, d = (it - k * per_slot) * V;
                 gv[u] = *(const uint4*)((const elem_t*)gate_of(k) + d);
                 uv[u] = *(const uint4*)((const elem_t*)up_of(k) + d);
@@ -58,60 +90,61 @@ template <int DT> __global__ __launch_bounds__(256) void moe_down_swiglu_kernel(
             }
 #pragma unroll
             for (int u = 0; u < 4; u++) {
-                const uint32_t it = base + u * 256 + tid;
+                const uint32_t it = base + u * DOWN_THREADS + tid;   // (slots lie one behind the other: item `it` is elements V it ..)
                 if (it >= total) break;
-                const uint32_t k = it / per_slot, d = (it - k * per_slot) * V;
+                float4 q[V / 4];
 #pragma unroll
                 for (int i = 0; i < V; i++) {
                     const float g = load_elem<DT>(&gv[u], i), up = load_elem<DT>(&uv[u], i);
                     const float silu = g / (1.0f + expf(0.0f - g));
-                    inner[k * a.in_dim + d + i] = sw[u] * (silu * up);
+                    ((float*)q)[i] = sw[u] * (silu * up);
                 }
+#pragma unroll
+                for (int i = 0; i < V / 4; i++) ((float4*)inner)[down_quad(it * (V / 4) + i)] = q[i];
             }
         }
     } else {
-        for (uint32_t it = tid; it < a.n_slots * a.in_dim; it += 256) {
+        for (uint32_t it = tid; it < a.n_slots * a.in_dim; it += DOWN_THREADS) {
             const uint32_t k = it / a.in_dim, d = it - k * a.in_dim;
             const float g = load_elem<DT>(gate_of(k), d), up = load_elem<DT>(up_of(k), d);
             const float silu = g / (1.0f + expf(0.0f - g));
-            inner[it] = load_elem<DT>(a.slot_w, k) * (silu * up);
+            inner[down_quad(it >> 2) * 4 + (it & 3u)] = load_elem<DT>(a.slot_w, k) * (silu * up);
         }
     }
     __syncthreads();
-    const uint32_t chunks = a.in_dim / 32;      // 16-byte pieces of a 4-bit row
-    const uint32_t items = a.n_slots * chunks;
-    const uint32_t ng = a.in_dim >> a.log2g;
-    for (uint32_t r = wave; r < a.rows_per_wg; r += 4) {
-        const uint32_t row = blockIdx.x * a.rows_per_wg + r;
-        if (row >= a.out_dim) break;  // uniform per wave
+    for (uint32_t r = wave; r < rows; r += DOWN_WAVES) {
         float acc = 0.f;
-        for (uint32_t it = lane; it < items; it += 64) {
-            const uint32_t k = it / chunks, c = it - k * chunks;
-            const size_t erow = (size_t)expert_of[k] * a.out_dim + row;
-            const uint4 wv = *(const uint4*)(a.w + erow * (a.in_dim / 8) + c * 4);
-            const uint32_t g = (c * 32) >> a.log2g;
-            const float sc = load_elem<DT>(a.scales, erow * ng + g), bi = load_elem<DT>(a.biases, erow * ng + g);
-            const float4* xv = (const float4*)(inner + k * a.in_dim + c * 32);
-            const uint32_t wd[4] = {wv.x, wv.y, wv.z, wv.w};
-            float dot = 0.f, xs = 0.f;
+        for (uint32_t base = 0; base < items; base += 256) {
+            const bool more = base + 256 < items;
+            Set next = {};
+            if (more || r + DOWN_WAVES < rows) load_set(next, more ? r : r + DOWN_WAVES, more ? base + 256 : 0u);
 #pragma unroll
-            for (int d = 0; d < 4; d++) {
-                const float4 x0 = xv[2 * d], x1 = xv[2 * d + 1];
-                const uint32_t q = wd[d];
-                dot = fmaf((float)(q & 15u), x0.x, dot);
-                dot = fmaf((float)((q >> 4) & 15u), x0.y, dot);
-                dot = fmaf((float)((q >> 8) & 15u), x0.z, dot);
-                dot = fmaf((float)((q >> 12) & 15u), x0.w, dot);
-                dot = fmaf((float)((q >> 16) & 15u), x1.x, dot);
-                dot = fmaf((float)((q >> 20) & 15u), x1.y, dot);
-                dot = fmaf((float)((q >> 24) & 15u), x1.z, dot);
-                dot = fmaf((float)(q >> 28), x1.w, dot);
-                xs += (x0.x + x0.y) + (x0.z + x0.w) + (x1.x + x1.y) + (x1.z + x1.w);
+            for (int u = 0; u < 4; u++) {
+                const uint32_t it = base + u * 64 + lane;
+                if (it >= items) continue;
+                const float4* xv = (const float4*)inner + it * 8;
+                const uint32_t wd[4] = {cur.w[u].x, cur.w[u].y, cur.w[u].z, cur.w[u].w};
+                float dot = 0.f, xs = 0.f;
+#pragma unroll
+                for (int d = 0; d < 4; d++) {
+                    const float4 x0 = xv[(2 * d) ^ (it & 7u)], x1 = xv[(2 * d + 1) ^ (it & 7u)];
+                    const uint32_t q = wd[d];
+                    dot = fmaf((float)(q & 15u), x0.x, dot);
+                    dot = fmaf((float)((q >> 4) & 15u), x0.y, dot);
+                    dot = fmaf((float)((q >> 8) & 15u), x0.z, dot);
+                    dot = fmaf((float)((q >> 12) & 15u), x0.w, dot);
+                    dot = fmaf((float)((q >> 16) & 15u), x1.x, dot);
+                    dot = fmaf((float)((q >> 20) & 15u), x1.y, dot);
+                    dot = fmaf((float)((q >> 24) & 15u), x1.z, dot);
+                    dot = fmaf((float)(q >> 28), x1.w, dot);
+                    xs += (x0.x + x0.y) + (x0.z + x0.w) + (x1.x + x1.y) + (x1.z + x1.w);
+                }
+                acc += cur.sc[u] * dot + cur.bi[u] * xs;
             }
-            acc += sc * dot + bi * xs;
+            cur = next;
         }
         acc = seg_allreduce(acc, 64);
-        if (lane == 0) store_elem<DT>(a.out, row, acc);
+        if (lane == 0) store_elem<DT>(a.out, row0 + r, acc);
     }
 }
 
@@ -148,13 +181,13 @@ int launch_moe_down_swiglu(int dtype, uint32_t group_size, uint32_t n_slots, con
     a.log2g = lg;
     a.n_experts = n_experts;
     a.n_slots = n_slots;
-    // about two workgroups per CU: the SwiGLU staging is repeated by every workgroup
+    // about one workgroup per CU: the SwiGLU staging is repeated by every workgroup
     int dev = 0, n_cu = 0;
     if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n_cu <= 0)
         n_cu = 256;
     const uint32_t cus = (uint32_t)n_cu;
-    uint32_t rpw = (out_dim + 2 * cus - 1) / (2 * cus);
-    rpw = (rpw + 3) / 4 * 4;
+    uint32_t rpw = (out_dim + cus - 1) / cus;
+    rpw = (rpw + DOWN_WAVES - 1) / DOWN_WAVES * DOWN_WAVES;
     a.rows_per_wg = rpw;
     const size_t shmem = (size_t)n_slots * in_dim * sizeof(float);
     const void* fn;
@@ -169,7 +202,7 @@ int launch_moe_down_swiglu(int dtype, uint32_t group_size, uint32_t n_slots, con
         if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(max dynamic LDS)");
     }
     void* args[] = {&a};
-    hipError_t e = launch_kernel(fn, dim3((out_dim + rpw - 1) / rpw), dim3(256), args, shmem, lc);
+    hipError_t e = launch_kernel(fn, dim3((out_dim + rpw - 1) / rpw), dim3(DOWN_THREADS), args, shmem, lc);
     if (e != hipSuccess) return hip_fail(e, "moe down + swiglu kernel launch");
     return ERR_OK;
 }

@@ -78,6 +78,36 @@ def test_shapes(oracle, dt, slots, K, N, G, E):
         buf.free()
 
 
+@pytest.mark.parametrize("off", [0, 8], ids=["aligned", "off 16 bytes"])
+@pytest.mark.parametrize("slots,K,N,G,E", [(8, 4096, 24, 128, 3), (7, 1184, 9, 32, 5), (8, 1056, 2049, 32, 2), (2, 96, 4200, 32, 3), (1, 32, 1, 32, 1)])
+def test_more_items_than_one_set_and_more_rows_than_waves(oracle, slots, K, N, G, E, off):
+    """Rows of one to four sets of 256 (slot, 32-code) items and what is left, workgroups of one to three rows per wave with a last
+    one that is short, a single item; gate and up rows off the 16 bytes that the wide staging asks for. Bounds as above."""
+    print(f"[case] moe_down_swiglu sets slots={slots} K={K} N={N} g{G} E={E} off={off}", flush=True)
+    dt = DType.BF16
+    rng = np.random.default_rng(K + N + slots)
+    rt = lambda v: oracle.round_through(np.asarray(v, dtype=np.float32), ODT[dt])
+    gates, ups = rt(rng.standard_normal((slots, K)) * 1.5).reshape(slots, K), rt(rng.standard_normal((slots, K))).reshape(slots, K)
+    experts = rng.integers(0, E, slots).astype("<u4")
+    sw = rt(rng.random(slots))
+    w, s, b = _quantize_int4(((rng.random(E * N * K, dtype=np.float32) - 0.5) * 0.5).astype(np.float32), E * N, K, G)
+    s, b = rt(s), rt(b)
+    _, exp64 = oracle.moe_down_swiglu_accum(gates, ups, experts, sw, w, s, b, K, N, G)
+    exp = oracle.round_through(exp64.astype(np.float32), ODT[dt])
+    gb = [GpuBuffer.from_bytes(b"\0" * off + pack_f32(gates[k], dt)) for k in range(slots)]
+    ub = [GpuBuffer.from_bytes(b"\0" * off + pack_f32(ups[k], dt)) for k in range(slots)]
+    bufs = [GpuBuffer.from_bytes(v) for v in (experts.tobytes(), pack_f32(sw, dt), w.tobytes(), pack_f32(s, dt), pack_f32(b, dt))]
+    out = GpuBuffer.from_bytes(b"\xff" * (N * 2 + 64))
+    ops.moe_down_swiglu_accum(dt, G, [x.ptr + off for x in gb], [x.ptr + off for x in ub], *bufs, out, K, N, E)
+    raw = out.read_bytes()
+    assert raw[N * 2:] == b"\xff" * 64
+    got = unpack_f32(raw[:N * 2], dt)
+    assert np.isfinite(got).all()
+    assert rel_err(got, exp) <= 1e-2
+    for buf in gb + ub + bufs + [out]:
+        buf.free()
+
+
 def test_rejects_unsupported_shapes():
     b = GpuBuffer(1 << 16)
     for K, G, slots in ((100, 64, 8), (8192, 64, 8), (768, 48, 8), (768, 64, 9), (768, 64, 0)):
