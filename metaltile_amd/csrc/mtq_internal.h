@@ -208,7 +208,7 @@ size_t qmm_grouped_scratch_bytes(uint32_t T, uint32_t E, bool sort_rows, uint32_
 int launch_qmm_grouped(const QmmParams& p, const uint32_t* route, bool per_row_ids, uint32_t T, uint32_t E, void* scratch,
                        const LaunchCtx& lc);
 // The table of row tiles behind both grouped launchers: tiles[0] = count, tiles[1 + i] = (expert,
-// first row in the row order, rows, 0); rowlist maps the row order to rows of x / out (null: identity).
+// first row in the row order, rows, place in its run | run length << 16); rowlist maps the row order to rows of x / out (null: identity).
 struct GatherTiles {
     uint32_t* tiles = nullptr;
     const uint32_t* rowlist = nullptr;

@@ -186,7 +186,7 @@ template <int DT> static int choose_dt(int bits, uint32_t kgroups, QmmDLaunch& l
     const QmmDArgs& a = l.a;
     const uint64_t cus = l.cus;
     l.dtype = DT;
-    l.grid = a.m_tiles * a.n_tiles;
+    l.grid = grouped ? (a.m_tiles * a.n_tiles + 7) & ~7u : a.m_tiles * a.n_tiles;   // (expert-routed rows: eight even shares)
     l.block = kgroups == 1 ? 256 : 512;
     l.split = a.ksplit > 1 && !grouped;
     const void* fn = nullptr;
@@ -523,7 +523,11 @@ __global__ __launch_bounds__(64) void gather_tiles_kernel(TileTabArgs a) {
     uint4* tab = (uint4*)a.tiles + 1;
     auto emit = [&](uint32_t first, uint32_t e, uint32_t lo, uint32_t hi) {
         uint32_t i = first;
-        for (uint32_t r = lo; r < hi && i < a.max_tiles; r += a.tile_rows, i++) tab[i] = make_uint4(e, r, min(a.tile_rows, hi - r), 0u);
+        const uint32_t cnt = (hi - lo + a.tile_rows - 1) / a.tile_rows;
+        for (uint32_t j = 0, r = lo; r < hi && i < a.max_tiles; r += a.tile_rows, i++, j++) {
+            const uint32_t in_run = j % QD_RUN, run = min(QD_RUN, cnt - (j - in_run));
+            tab[i] = make_uint4(e, r, min(a.tile_rows, hi - r), in_run | run << 16);
+        }
     };
     for (uint32_t base = 0; base < a.E; base += 64) {
         const uint32_t e = base + lane;

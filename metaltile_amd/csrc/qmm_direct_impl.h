@@ -38,6 +38,23 @@ __device__ __forceinline__ uint32_t qd_matrix(QmmDBase& a, const QmmDMore& more)
     return id;
 }
 
+// Expert-routed rows: this workgroup's row tile and column tile; false past the last one. Workgroups congruent mod 8 share an
+// XCD and its L2: each XCD takes an even share of consecutive tiles, and inside it the row tiles of one run (up to QD_RUN of one
+// expert) stand side by side at each column tile, so that a run's weights cross the fabric once and its activations stay in
+// that L2. In launch order over all XCDs every XCD fetched all activations and each row tile its weights again
+// (128 experts of 768 x 2048, 128 rows each 108 -> 98.5 us; of 2048 x 768 133 -> 128.7).
+__device__ __forceinline__ bool qd_routed_tile(const uint32_t* tiles, uint32_t n_tiles, uint4& t, uint32_t& nt) {
+    const uint32_t total = tiles[0] * n_tiles, share = (total + 7) / 8, at = blockIdx.x >> 3;
+    const uint32_t vid = (blockIdx.x & 7u) * share + at;
+    if (at >= share || vid >= total) return false;
+    const uint4* tab = (const uint4*)tiles + 1;
+    uint32_t mt = vid / n_tiles;
+    const uint32_t run = tab[mt].w, first = mt - (run & 0xFFFFu), len = run >> 16, in_run = vid - first * n_tiles;
+    nt = in_run / len;
+    mt = first + in_run - nt * len;
+    t = tab[mt];
+    return true;
+}
 
 // MB = 32-row activation blocks per wave (tile height DBM = 32*MB): every
 // converted weight fragment feeds MB MFMAs, so the conversion cost per MFMA
@@ -81,10 +98,8 @@ __global__ __launch_bounds__(KG == 1 ? 256 : 512) void qmm_direct_kernel(QmmDArg
     // rows of this tile: row j of the tile is row (row_first + j) of the row order, j < row_count
     uint32_t row_first = mt * DBM, row_count = a.M > row_first ? min((uint32_t)DBM, a.M - row_first) : 0u;
     if constexpr (GR) {
-        nt = blockIdx.x % a.n_tiles;
-        mt = blockIdx.x / a.n_tiles;
-        if (mt >= a.tiles[0]) return;  // the grid is sized for the worst routing
-        const uint4 t = ((const uint4*)a.tiles)[1 + mt];
+        uint4 t;
+        if (!qd_routed_tile(a.tiles, a.n_tiles, t, nt)) return;  // the grid is sized for the worst routing
         row_first = t.y;
         row_count = t.z;
         a.w += (size_t)t.x * a.w_expert_bytes;

@@ -4,6 +4,8 @@
 
 namespace mtq {
 
+constexpr uint32_t QD_RUN = 8;   // row tiles of an expert that go through its column tiles together
+
 struct QmmDBase {
     const unsigned char* w;
     const unsigned char* scales;
@@ -16,8 +18,9 @@ struct QmmDBase {
     uint32_t m_tile_rows;  // 32 (4 K-groups only), 64 or 128
     uint32_t by_m;         // consecutive workgroup ids walk the N-tiles of one M-tile (else the M-tiles of one N-tile)
     // grouped mode (expert-routed rows): tiles[0] = number of row tiles, then one uint4 per tile
-    // (expert, first row of the tile in the row order, rows in the tile, 0); rowlist maps the row
-    // order to rows of x / out (null: the identity). w / scales / biases are the stacked experts'.
+    // (expert, first row of the tile in the row order, rows in the tile, its place in its run of at most QD_RUN row tiles of the
+    // expert | the run's length << 16); rowlist maps the row order to rows of x / out (null: the identity). w / scales / biases
+    // are the stacked experts'.
     const uint32_t* tiles;
     const uint32_t* rowlist;
     uint64_t w_expert_bytes, sb_expert_elems;

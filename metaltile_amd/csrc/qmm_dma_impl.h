@@ -167,10 +167,8 @@ __global__ __launch_bounds__(64 * NW) void qmm_dma_kernel(QmmDArgs args) {
     uint32_t nt = a.by_m ? vid % a.n_tiles : vid / a.m_tiles, mt = a.by_m ? vid / a.n_tiles : vid % a.m_tiles;
     uint32_t row_first = mt * DBM, row_count = a.M > row_first ? min((uint32_t)DBM, a.M - row_first) : 0u;
     if constexpr (GR) {
-        nt = blockIdx.x % a.n_tiles;
-        mt = blockIdx.x / a.n_tiles;
-        if (mt >= a.tiles[0]) return;  // the grid is sized for the worst routing
-        const uint4 t = ((const uint4*)a.tiles)[1 + mt];
+        uint4 t;
+        if (!qd_routed_tile(a.tiles, a.n_tiles, t, nt)) return;  // the grid is sized for the worst routing
         row_first = t.y;
         row_count = t.z;
         a.w += (size_t)t.x * a.w_expert_bytes;

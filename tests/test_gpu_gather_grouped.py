@@ -246,3 +246,32 @@ def test_names_keep_their_arithmetic(runner, oracle, bits):
         lib.mtq_set_option(b"gather.names_exact", 0)
     for buf in (w, s, b, x, off, idx, out):
         buf.free()
+
+@pytest.mark.parametrize("bits,N,K,G,counts", [
+    (4, 128, 256, 64, [513, 0, 1, 1100, 64]),      # 9 + 1 + 18 + 1 row tiles of one column tile: runs of 8 and of what is left
+    (4, 640, 512, 64, [65, 128, 0, 512, 3]),       # column tiles that are no power of two
+    (8, 264, 256, 32, [600, 30]),                  # a ragged last column tile
+    (6, 384, 256, 64, [577, 0, 130]),              # the register-staged kernel
+    (4, 128, 256, 64, [1, 0, 0]),                  # one tile: most shares are empty
+], ids=str)
+def test_grouped_gather_runs_of_row_tiles(oracle, grouped, bits, N, K, G, counts):
+    """Every tile of every expert is worked on once, whatever the number of row tiles, column tiles and their product; rows of
+    unsorted ids too. Bound: one rounding of a bf16 result (2^-9 of its value, 2e-2 as in the tests above)."""
+    dt, E, T = DType.BF16, len(counts), sum(counts)
+    c = make_case(7700 + N + K, dt, bits, G, T, N, K, E=E)
+    ids_sorted = np.repeat(np.arange(E), counts).astype("<u4")
+    offsets = np.concatenate([[0], np.cumsum(counts)]).astype("<u4")
+    ids_shuffled = ids_sorted[np.random.default_rng(8).permutation(T)]
+    w, s, b, x = (GpuBuffer.from_bytes(v) for v in (c.w.tobytes(), c.scales_bytes, c.biases_bytes, c.x_bytes))
+    grouped(2)
+    for view, route, fn, ids in (("csr", offsets, ops.gather_qmv_csr, ids_sorted), ("indices", ids_shuffled, ops.gather_qmv_indices, ids_shuffled)):
+        print(f"[case] runs of row tiles {view} b{bits} N={N} K={K} {counts}", flush=True)
+        out = GpuBuffer.from_bytes(np.full(T * N + 1024, 0x7B7B, np.uint16).tobytes())
+        r = GpuBuffer.from_bytes(route.tobytes())
+        fn(dt, bits, G, x, w, s, b, r, out, T, N, K, E)
+        raw = np.frombuffer(out.read_bytes(), np.uint16)
+        out.free(); r.free()
+        assert np.all(raw[T * N:] == 0x7B7B), view
+        assert rel_err(unpack_f32(raw[:T * N].tobytes(), dt), _expected(oracle, c, ids, T, N, K, E, bits, G, dt)) <= 2e-2, view
+    for buf in (w, s, b, x):
+        buf.free()
