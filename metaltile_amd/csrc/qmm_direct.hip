@@ -161,6 +161,14 @@ static int dma_mode(int bits, uint32_t rows, uint32_t kgroups, uint32_t K, uint3
 }
 static bool dma_fits(int bits, uint32_t rows, uint32_t kgroups, uint32_t K, uint32_t gpr) { return dma_mode(bits, rows, kgroups, K, gpr) != 0; }
 
+// The same for the tall tiles of expert-routed rows, which take any even number of groups.
+static int routed_mode(int bits, uint32_t K, uint32_t gpr) {
+    if (options().qmm_dma == 1 || (bits != 4 && bits != 8) || K % 128 || gpr % 2) return 0;
+    if (options().qmm_dma != 2 && qmm_dma_routed_lds_bytes(gpr, false) <= 160 * 1024) return 1;
+    const uint32_t G = K / gpr;
+    return (G == 64 || G == 128) && gpr >= 32 ? 2 : 0;
+}
+
 // K-split load-to-LDS instances on 2 K-groups (64 x 128 and 128 x 128 tiles): every split stages its own share of
 // the tile's scales and biases (whole 8-group vectors, or pairs of groups where rows are not whole vectors) beside the
 // ring of three tiles. Returns the LDS bytes, or 0
@@ -197,6 +205,12 @@ template <int DT> static int choose_dt(int bits, uint32_t kgroups, QmmDLaunch& l
     if (const size_t shmem = grouped ? 0 : dma_split_lds(bits, a.m_tile_rows, kgroups, a.K, a.gpr, a.iters_per_split, a.ksplit)) {
         l.fn = qmm_dma_split_pick(bits, DT, a.m_tile_rows);
         l.shmem = shmem;
+        return ERR_OK;
+    }
+    if (grouped && a.m_tile_rows == QD_ROUTED_ROWS) {
+        const bool windowed = routed_mode(bits, a.K, a.gpr) == 2;
+        l.fn = qmm_dma_routed_pick(bits, DT, windowed);
+        l.shmem = qmm_dma_routed_lds_bytes(a.gpr, windowed);
         return ERR_OK;
     }
     if (a.ksplit <= 1 && dma_fits(bits, a.m_tile_rows, kgroups, a.K, a.gpr) && (!grouped || a.m_tile_rows == 64) &&
@@ -523,10 +537,10 @@ __global__ __launch_bounds__(64) void gather_tiles_kernel(TileTabArgs a) {
     uint4* tab = (uint4*)a.tiles + 1;
     auto emit = [&](uint32_t first, uint32_t e, uint32_t lo, uint32_t hi) {
         uint32_t i = first;
-        const uint32_t cnt = (hi - lo + a.tile_rows - 1) / a.tile_rows;
-        for (uint32_t j = 0, r = lo; r < hi && i < a.max_tiles; r += a.tile_rows, i++, j++) {
+        const uint32_t cnt = (hi - lo + a.tile_rows - 1) / a.tile_rows, per = (hi - lo + cnt - 1) / cnt;   // even pieces
+        for (uint32_t j = 0, r = lo; r < hi && i < a.max_tiles; r += per, i++, j++) {
             const uint32_t in_run = j % QD_RUN, run = min(QD_RUN, cnt - (j - in_run));
-            tab[i] = make_uint4(e, r, min(a.tile_rows, hi - r), in_run | run << 16);
+            tab[i] = make_uint4(e, r, min(per, hi - r), in_run | run << 16);
         }
     };
     for (uint32_t base = 0; base < a.E; base += 64) {
@@ -569,6 +583,14 @@ __global__ __launch_bounds__(64) void gather_tiles_kernel(TileTabArgs a) {
 // against 36 / 43). With more rows, or many small experts, the 32-row tiles lose (every weight is converted
 // once per 32 rows instead of 64: 128 x 2048 x 768, 48 rows each: 75 against 137 us).
 static uint32_t grouped_tile_rows(const QmmParams& p, uint32_t T, uint32_t E) {
+    // Tall row tiles from 64 rows per expert on (64-row tiles -> these, us: 128 x 768 x 2048, 55 / 64 / 96 rows each 60.7 / 74.8 /
+    // 89.8 -> 62.0 / 62.9 / 75.9; 128 x 2048 x 768 67.7 / 83.4 / 109.6 -> 77.4 / 81.9 / 99.9; 8 x 14336 x 4096, 50 / 64 / 256 rows 98.8 /
+    // 139 / 354 -> 114.5 / 125.5 / 311), where they are tiles for half the chip at least. Not on short rows where an expert's rows
+    // are two pieces of about 96 (128 x 2048 x 768, 192 rows each: 181.8 -> 185.8; 256 rows 232 -> 216).
+    const uint64_t hit = E < T ? E : T, pieces = (T + QD_ROUTED_ROWS - 1) / QD_ROUTED_ROWS, tall = pieces > hit ? pieces : hit;
+    const bool short_halves = p.K < 1024 && (uint64_t)T > 160 * hit && (uint64_t)T < 224 * hit;
+    if (routed_mode(p.bits, p.K, p.K / p.group_size) && !options().qmm_tile_rows && (uint64_t)T >= 64 * hit && !short_halves && tall * ((p.N + 127) / 128) >= 128)
+        return QD_ROUTED_ROWS;
     if (p.K % 256 || (p.bits != 2 && p.bits != 4 && p.bits != 8)) return 64u;
     if (options().qmm_tile_rows == 32) return 32u;
     if (options().qmm_tile_rows == 64) return 64u;
@@ -666,6 +688,7 @@ int launch_qmm_grouped(const QmmParams& p, const uint32_t* route, bool per_row_i
     const uint64_t row_tiles = (uint64_t)(T + 63) / 64 + (E < T ? E : T) / 2;
     uint32_t kgroups = (row_tiles * ((p.N + 127) / 128) * 2 <= (uint64_t)cus && p.K % 256 == 0) ? 4 : 2;
     if (tile_rows == 32) kgroups = 4;
+    if (tile_rows == QD_ROUTED_ROWS) kgroups = 2;
     a.m_tile_rows = tile_rows;
     a.m_tiles = max_tiles;
     a.n_tiles = (p.N + 32 * (8 / kgroups) - 1) / (32 * (8 / kgroups));

@@ -42,7 +42,7 @@ __device__ __forceinline__ uint32_t qd_matrix(QmmDBase& a, const QmmDMore& more)
 // XCD and its L2: each XCD takes an even share of consecutive tiles, and inside it the row tiles of one run (up to QD_RUN of one
 // expert) stand side by side at each column tile, so that a run's weights cross the fabric once and its activations stay in
 // that L2. In launch order over all XCDs every XCD fetched all activations and each row tile its weights again
-// (128 experts of 768 x 2048, 128 rows each 108 -> 98.5 us; of 2048 x 768 133 -> 128.7).
+// (128 experts of 768 x 2048, 128 rows each, 64-row tiles in runs of 8 108 -> 98.5 us; of 2048 x 768 133 -> 128.7).
 __device__ __forceinline__ bool qd_routed_tile(const uint32_t* tiles, uint32_t n_tiles, uint4& t, uint32_t& nt) {
     const uint32_t total = tiles[0] * n_tiles, share = (total + 7) / 8, at = blockIdx.x >> 3;
     const uint32_t vid = (blockIdx.x & 7u) * share + at;
@@ -371,6 +371,9 @@ size_t qmm_dma_lds_bytes(uint32_t tile_rows, uint32_t gpr, bool windowed, bool s
 size_t qmm_dma_split_lds_bytes(uint32_t tile_rows, uint32_t groups);
 const void* qmm_dma_split_pick(int bits, int dtype, uint32_t tile_rows);
 const void* qmm_dma4_pick(int bits, int dtype, uint32_t tile_rows, bool split, bool grouped);
+// Expert-routed rows on row tiles of up to QD_ROUTED_ROWS rows (4- and 8-bit codes).
+const void* qmm_dma_routed_pick(int bits, int dtype, bool windowed);
+size_t qmm_dma_routed_lds_bytes(uint32_t gpr, bool windowed);
 size_t qmm_dma4_lds_bytes(uint32_t tile_rows, uint32_t gpr);
 
 }  // namespace mtq

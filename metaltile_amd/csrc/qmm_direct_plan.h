@@ -4,7 +4,8 @@
 
 namespace mtq {
 
-constexpr uint32_t QD_RUN = 8;   // row tiles of an expert that go through its column tiles together
+constexpr uint32_t QD_ROUTED_ROWS = 160;   // the tall row tiles of expert-routed rows
+constexpr uint32_t QD_RUN = 4;   // row tiles of an expert that go through its column tiles together
 
 struct QmmDBase {
     const unsigned char* w;
@@ -15,7 +16,7 @@ struct QmmDBase {
     uint32_t M, N, K;
     uint32_t log2g, gpr;
     uint32_t m_tiles, n_tiles, iters;
-    uint32_t m_tile_rows;  // 32 (4 K-groups only), 64 or 128
+    uint32_t m_tile_rows;  // 32 (4 K-groups only), 64, 128 or 256; 160 for expert-routed rows (at most)
     uint32_t by_m;         // consecutive workgroup ids walk the N-tiles of one M-tile (else the M-tiles of one N-tile)
     // grouped mode (expert-routed rows): tiles[0] = number of row tiles, then one uint4 per tile
     // (expert, first row of the tile in the row order, rows in the tile, its place in its run of at most QD_RUN row tiles of the

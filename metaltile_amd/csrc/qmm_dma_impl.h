@@ -129,12 +129,13 @@ template <int NBUF, int WSN, int IPW, int NWL, int NSB> struct QmmDmaWaits {
 // 64 and 128 codes), as one more hand-counted load per iteration. The LDS footprint no longer depends on K.
 // BITS: 4, or 8 (a lane's 32 codes are then 32 bytes: two 16-byte loads per iteration, bytes converted with the
 // byte-select converts; everything else alike).
-template <int DT, int MB, int KG, int NW, int NB = 0, bool GR = false, bool SP = false, bool WIN = false, int BITS = 4>
-__global__ __launch_bounds__(64 * NW) void qmm_dma_kernel(QmmDArgs args) {
+// routed, routed_nt (GR): the row tile and the column tile.
+template <int DT, int MB, int KG, int NW, int NB, bool GR, bool SP, bool WIN, int BITS>
+__device__ __forceinline__ void qmm_dma_tile(const QmmDArgs& args, const uint4 routed, const uint32_t routed_nt) {
     QmmDBase a = args;
     static_assert(NW == 8 || NW == 16, "two or four waves per SIMD");
     static_assert(KG == 2 || KG == 4, "2 or 4 K-groups");
-    static_assert(MB == 1 || MB == 2 || MB == 4 || MB == 8, "32 to 256 rows");
+    static_assert((MB >= 1 && MB <= 5) || MB == 8, "32 to 256 rows");
     static_assert(BITS == 4 || BITS == 8, "4- or 8-bit codes");
     constexpr int NWL = BITS / 4;              // 16-byte weight loads per lane and iteration
     constexpr float KSCALE = BITS == 4 ? 512.f : 1.f;   // 4-bit codes are read as fp8 = code / 512
@@ -167,13 +168,12 @@ __global__ __launch_bounds__(64 * NW) void qmm_dma_kernel(QmmDArgs args) {
     uint32_t nt = a.by_m ? vid % a.n_tiles : vid / a.m_tiles, mt = a.by_m ? vid / a.n_tiles : vid % a.m_tiles;
     uint32_t row_first = mt * DBM, row_count = a.M > row_first ? min((uint32_t)DBM, a.M - row_first) : 0u;
     if constexpr (GR) {
-        uint4 t;
-        if (!qd_routed_tile(a.tiles, a.n_tiles, t, nt)) return;  // the grid is sized for the worst routing
-        row_first = t.y;
-        row_count = t.z;
-        a.w += (size_t)t.x * a.w_expert_bytes;
-        a.scales += (size_t)t.x * a.sb_expert_elems * 2;
-        a.biases += (size_t)t.x * a.sb_expert_elems * 2;
+        nt = routed_nt;
+        row_first = routed.y;
+        row_count = routed.z;
+        a.w += (size_t)routed.x * a.w_expert_bytes;
+        a.scales += (size_t)routed.x * a.sb_expert_elems * 2;
+        a.biases += (size_t)routed.x * a.sb_expert_elems * 2;
     }
     auto row_of = [&](uint32_t j) -> uint32_t {  // j < row_count
         if constexpr (GR) return a.rowlist ? a.rowlist[row_first + j] : row_first + j;
@@ -530,6 +530,32 @@ __global__ __launch_bounds__(64 * NW) void qmm_dma_kernel(QmmDArgs args) {
             }
         }
     });
+}
+
+template <int DT, int MB, int KG, int NW, int NB = 0, bool GR = false, bool SP = false, bool WIN = false, int BITS = 4>
+__global__ __launch_bounds__(64 * NW) void qmm_dma_kernel(QmmDArgs args) {
+    uint4 t = make_uint4(0, 0, 0, 0);
+    uint32_t nt = 0;
+    if constexpr (GR) {
+        if (!qd_routed_tile(args.tiles, args.n_tiles, t, nt)) return;  // the grid is sized for the worst routing
+    }
+    qmm_dma_tile<DT, MB, KG, NW, NB, GR, SP, WIN, BITS>(args, t, nt);
+}
+
+// Many rows per expert: row tiles of up to 160 rows, each on as many 32-row blocks as it has. An expert's rows are cut into even
+// pieces, so that 128 rows or a few more are one tile and each weight is converted once for them (64-row tiles: two or three
+// times, the last one nearly empty). 160 rows are what three buffers and the scales leave room for in LDS. us, the whole gather with
+// its table, bf16, 64-row tiles -> these: 128 experts of 768 x 2048, 128 rows each 108 -> 95 (8-bit codes 173 -> 120), of 2048 x 768
+// 133 -> 117; 8 experts of 14336 x 4096, 512 rows each 666 -> 603, of 4096 x 14336, 64 / 128 rows each 172 / 261 -> 118 / 165.
+// What is left is the start and end of each tile (about 7 us of 22 at 2048 codes): one workgroup fills a compute unit's registers.
+template <int DT, bool WIN, int BITS> __global__ __launch_bounds__(512) void qmm_dma_routed_kernel(QmmDArgs args) {
+    uint4 t;
+    uint32_t nt;
+    if (!qd_routed_tile(args.tiles, args.n_tiles, t, nt)) return;
+    if (t.z <= 64) qmm_dma_tile<DT, 2, 2, 8, 0, true, false, WIN, BITS>(args, t, nt);
+    else if (t.z <= 96) qmm_dma_tile<DT, 3, 2, 8, 0, true, false, WIN, BITS>(args, t, nt);
+    else if (t.z <= 128) qmm_dma_tile<DT, 4, 2, 8, 0, true, false, WIN, BITS>(args, t, nt);
+    else qmm_dma_tile<DT, 5, 2, 8, 0, true, false, WIN, BITS>(args, t, nt);
 }
 
 }  // namespace mtq

@@ -275,3 +275,49 @@ def test_grouped_gather_runs_of_row_tiles(oracle, grouped, bits, N, K, G, counts
         assert rel_err(unpack_f32(raw[:T * N].tobytes(), dt), _expected(oracle, c, ids, T, N, K, E, bits, G, dt)) <= 2e-2, view
     for buf in (w, s, b, x):
         buf.free()
+
+
+@pytest.mark.parametrize("dt,bits,N,K,G,counts", [
+    (DType.BF16, 4, 8192, 768, 64, [161, 0, 64, 65, 96, 97]),       # every height; rows of 12 groups
+    (DType.F16, 4, 8264, 256, 32, [128, 129, 160, 1]),               # a ragged last column tile
+    (DType.BF16, 8, 8192, 128, 64, [700, 150]),                     # five even pieces, a single iteration
+    (DType.BF16, 4, 8192, 5760, 64, [130, 100]),                    # scales in two windows
+    (DType.F16, 8, 8192, 5760, 64, [81, 159]),
+], ids=str)
+def test_grouped_gather_on_tall_row_tiles(oracle, dt, bits, N, K, G, counts):
+    """Row tiles of up to 160 rows, chosen by the rows per expert, against the 64-row tiles: the same products added in the same
+    order by the same instructions, so the same bits; and those against the oracle on a sample of columns (2e-2 as above)."""
+    lib = _lib.load()
+    E, T = len(counts), sum(counts)
+    c = make_case(7900 + N + K, dt, bits, G, T, N, K, E=E)
+    ids_sorted = np.repeat(np.arange(E), counts).astype("<u4")
+    offsets = np.concatenate([[0], np.cumsum(counts)]).astype("<u4")
+    ids_shuffled = ids_sorted[np.random.default_rng(8).permutation(T)]
+    w, s, b, x = (GpuBuffer.from_bytes(v) for v in (c.w.tobytes(), c.scales_bytes, c.biases_bytes, c.x_bytes))
+    try:
+        for view, route, fn, ids in (("csr", offsets, ops.gather_qmv_csr, ids_sorted), ("indices", ids_shuffled, ops.gather_qmv_indices, ids_shuffled)):
+            r, got = GpuBuffer.from_bytes(route.tobytes()), []
+            for rows in (0, 64):
+                print(f"[case] tall row tiles {view} {dt.name} b{bits} N={N} K={K} {counts} rows={rows}", flush=True)
+                assert lib.mtq_set_option(b"qmm.tile_rows", rows) == 0
+                out = GpuBuffer.from_bytes(np.full(T * N + 1024, 0x7B7B, np.uint16).tobytes())
+                fn(dt, bits, G, x, w, s, b, r, out, T, N, K, E)
+                got.append(np.frombuffer(out.read_bytes(), np.uint16))
+                out.free()
+            r.free()
+            assert np.all(got[0][T * N:] == 0x7B7B), view
+            assert np.array_equal(got[0], got[1]), view
+            some = [0, 33, N - 1]   # columns
+            wpr, spr = K * bits // 32, K // G
+            for e in range(E):
+                rows = np.nonzero(ids == e)[0]
+                if rows.size == 0:
+                    continue
+                wc, sc, bc = (np.concatenate([v[(e * N + n) * m:(e * N + n + 1) * m] for n in some]) for v, m in ((c.w, wpr), (c.scales_f, spr), (c.biases_f, spr)))
+                exp = oracle.qmm_mma(wc, sc, bc, np.ascontiguousarray(c.x_f.reshape(T, K)[rows]).reshape(-1), rows.size, len(some), K, bits, G, ODT[dt], threads=8)
+                mine = unpack_f32(np.ascontiguousarray(got[0][:T * N].reshape(T, N)[rows][:, some]).tobytes(), dt)
+                assert rel_err(mine, oracle.round_through(exp.reshape(-1), ODT[dt])) <= 2e-2, view
+    finally:
+        lib.mtq_set_option(b"qmm.tile_rows", 0)
+    for buf in (w, s, b, x):
+        buf.free()
