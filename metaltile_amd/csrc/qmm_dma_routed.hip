@@ -6,8 +6,8 @@
 namespace mtq {
 
 template <int BITS> static const void* routed_t(int dtype, bool windowed) {
-    if (dtype == DT_BF16) return windowed ? (const void*)qmm_dma_routed_kernel<DT_BF16, true, BITS> : (const void*)qmm_dma_routed_kernel<DT_BF16, false, BITS>;
-    if (dtype == DT_F16) return windowed ? (const void*)qmm_dma_routed_kernel<DT_F16, true, BITS> : (const void*)qmm_dma_routed_kernel<DT_F16, false, BITS>;
+    if (dtype == DT_BF16) return windowed ? (const void*)tall::qmm_dma_kernel<DT_BF16, 2, 2, 8, 2, true, false, true, BITS> : (const void*)tall::qmm_dma_kernel<DT_BF16, 2, 2, 8, 2, true, false, false, BITS>;
+    if (dtype == DT_F16) return windowed ? (const void*)tall::qmm_dma_kernel<DT_F16, 2, 2, 8, 2, true, false, true, BITS> : (const void*)tall::qmm_dma_kernel<DT_F16, 2, 2, 8, 2, true, false, false, BITS>;
     return nullptr;
 }
 

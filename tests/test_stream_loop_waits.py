@@ -207,3 +207,23 @@ int main() { return 0; }
         text = open(os.path.join(CSRC, header)).read()
         assert re.search(r"static_assert\(\s*(Waits|" + name + r"<[^>]*>)::holds\(\)", text), header
         assert "qm_wait_vm<(" not in text and "qw_wait<2" not in text, f"{header}: a wait count written as a literal expression"
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc is needed to produce the assembly")
+def test_tall_routed_kernels_wait_only_where_written():
+    """The kernel of expert-routed rows holds the tile's code at four heights, one behind the other: waits that the source does not
+    hold may stand between two heights' MFMAs (the end of one, the start of the next) and nowhere else, and scratch memory nowhere."""
+    with tempfile.TemporaryDirectory() as tmp:
+        outs = [_assembly(s, os.path.join(tmp, s + ".s")) for s in ("qmm_dma_routed.hip", "qmm_dma_routed_b8.hip")]
+    n = 0
+    for lines in outs:
+        starts = [(i, l.split(":")[0]) for i, l in enumerate(lines) if "14qmm_dma_kernel" in l and l.startswith("_ZN3mtq4tall") and "; @" in l]
+        starts.append((len(lines), ""))
+        for (s0, name), (s1, _) in zip(starts, starts[1:]):
+            body = lines[s0:s1]
+            mf = [i for i, l in enumerate(body) if "v_mfma" in l]
+            gaps = sum(any("s_waitcnt vmcnt" in body[i] and "ASMSTART" not in body[i - 1] for i in range(a, b)) for a, b in zip(mf, mf[1:]))
+            assert mf and gaps <= 3, f"{name}: {gaps} pairs of MFMAs with waits between them that the source does not hold"
+            assert not any("scratch_" in l for l in body), f"{name}: scratch memory touched"
+            n += 1
+    assert n == 8
