@@ -164,7 +164,7 @@ __device__ __forceinline__ void qmm_dma_tile(const QmmDArgs& args, const uint4 r
     uint32_t vid = blockIdx.x;
     if constexpr (!GR) vid = qd_matrix(a, args.more);
     const uint32_t total = a.m_tiles * a.n_tiles;
-    if (!GR && total % 8 == 0) vid = (vid & 7u) * (total / 8) + (vid >> 3);
+    if constexpr (!GR) vid = qd_xcd_share(vid, total);
     uint32_t nt = a.by_m ? vid % a.n_tiles : vid / a.m_tiles, mt = a.by_m ? vid / a.n_tiles : vid % a.m_tiles;
     uint32_t row_first = mt * DBM, row_count = a.M > row_first ? min((uint32_t)DBM, a.M - row_first) : 0u;
     if constexpr (GR) {
