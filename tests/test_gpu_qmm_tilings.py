@@ -136,6 +136,31 @@ def test_tile_kernel_on_ragged_n(oracle, options, N, tiling):
     assert rel_err(got, exp) <= 2e-2
 
 
+@pytest.mark.parametrize("dma", [0, 1])
+@pytest.mark.parametrize("rows,cols", [(1, 1), (7, 1), (2, 4), (3, 3), (3, 5), (1, 17), (5, 5)])
+def test_tile_counts_that_are_no_multiple_of_8(oracle, options, rows, cols, dma):
+    """Tiles are dealt to the XCDs in eight shares that may differ by one: every tile is worked on once, whichever operand is
+    walked first, with and without direct loads to LDS. Against the mma-semantics oracle, 2e-2 as for the prefill configuration."""
+    M, N, K, G, bits, dt = 64 * rows - 3, 128 * cols, 512, 64, 4, DType.BF16
+    print(f"[case] qmm of {rows} x {cols} tiles, qmm.dma={dma}", flush=True)
+    c = make_case(5700 + 20 * rows + cols, dt, bits, G, M, N, K)
+    exp = oracle.qmm_mma(c.w, c.scales_f, c.biases_f, c.x_f, M, N, K, bits, G, ODT[dt], threads=8)
+    exp = oracle.round_through(exp.astype(np.float32), ODT[dt])
+    bufs = [GpuBuffer.from_bytes(v) for v in (c.w.tobytes(), c.scales_bytes, c.biases_bytes, c.x_bytes)]
+    for name, value in (("qmm.tile_rows", 64), ("qmm.kgroups", 2), ("qmm.kernel", 2), ("qmm.dma", dma), ("qmm.ksplit", 1)):
+        options(name, value)
+    for by_m in (1, 2):
+        options("qmm.by_m", by_m)
+        out = GpuBuffer.from_bytes(np.full(M * N, 0x7FC0, np.uint16).tobytes())
+        ops.qmm(dt, bits, G, *bufs, out, M, N, K)
+        got = unpack_f32(out.read_bytes(), dt)
+        out.free()
+        assert not np.isnan(got).any()
+        assert rel_err(got, exp) <= 2e-2
+    for buf in bufs:
+        buf.free()
+
+
 @pytest.mark.parametrize("dt", [DType.BF16, DType.F16], ids=lambda d: d.name)
 @pytest.mark.parametrize("bits", [3, 5, 6, 7])
 def test_direct_qmm_bit_stream_widths(oracle, options, bits, dt):
