@@ -473,6 +473,8 @@ MTQ_API int mtq_flush_cache(void);
  *   "gather.names_exact"   the exact-dequant gather names of mtq_dispatch (mt_moe_gather_qmm_int4, _m8, _m16, _m32, _b3 ..
  *                          _b8): 0 = always on the GEMV kernels (exact s*q + b, as those reference kernels compute), 1 = grouped
  *                          on the tile kernel above 8 rows per expert like the typed entry points (w_hat rounded to T first)
+ *   "scratch.most_kb"      largest library-owned scratch buffer in KB, 0 = no limit: a call that wants more goes the way it goes
+ *                          where that memory cannot be allocated
  *   "qvm.wgs"              qvm: workgroups to aim for when K is sliced, 0 = choose
  *   "moe.sort"             expert sort: 0 = choose by size, 1 = always the bitonic network
  *   "moe_down.rows"        fused MoE down projection: output rows per workgroup, 0 = choose

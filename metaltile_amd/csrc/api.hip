@@ -252,12 +252,9 @@ static int try_f32_tiles(int bits, uint32_t G, const void* w, const void* s, con
     q.w = w; q.scales = s; q.biases = b; q.x = x; q.out = out;
     q.M = M; q.N = N; q.K = K;
     const size_t need = qmm_f32_scratch_bytes(q);  // f32 partial tiles when K is split
-    if (need) {
-        // behind whatever the calling op holds at the front of the buffer (a normalised row)
-        int rc = ensure_scratch(g.scratch_held + need);
-        if (rc) return rc;
-    }
-    return launch_qmm_f32(q, lc, need ? (char*)g.scratch_buf + g.scratch_held : nullptr);
+    // behind whatever the calling op holds at the front of the buffer (a normalised row); unsplit where there is no memory
+    const bool split = need && ensure_scratch(g.scratch_held + need) == ERR_OK;
+    return launch_qmm_f32(q, lc, split ? (char*)g.scratch_buf + g.scratch_held : nullptr);
 }
 
 
@@ -286,10 +283,7 @@ static int try_wide(int dtype, int bits, uint32_t G, const void* w, const void* 
     q.M = M; q.N = N; q.K = K;
     if (!wide_serves(q, exact)) return ERR_UNSUPPORTED;
     const size_t need = qmv_wide_scratch_bytes(q);
-    if (need) {
-        int rc = ensure_scratch(g.scratch_held + need);
-        if (rc) return rc;
-    }
+    if (need && ensure_scratch(g.scratch_held + need)) return ERR_UNSUPPORTED;   // no memory for the partial rows: the caller's other kernels do without
     return launch_qmv_wide(q, lc, need ? (char*)g.scratch_buf + g.scratch_held : nullptr);
 }
 
@@ -311,9 +305,7 @@ static int try_slices(int dtype, int bits, uint32_t G, const void* w, const void
     q.dtype = dtype; q.bits = bits; q.group_size = G;
     q.w = w; q.scales = s; q.biases = b; q.x = x; q.out = out;
     q.M = M; q.N = N; q.K = K;
-    if (!slices_serve(q)) return ERR_UNSUPPORTED;
-    int rc = ensure_scratch(g.scratch_held + qmv_slices_scratch_bytes(q));
-    if (rc) return rc;
+    if (!slices_serve(q) || ensure_scratch(g.scratch_held + qmv_slices_scratch_bytes(q))) return ERR_UNSUPPORTED;   // (no memory for the sums: as above)
     return launch_qmv_slices(q, lc, (char*)g.scratch_buf + g.scratch_held);
 }
 
@@ -427,6 +419,7 @@ static int op_qmm(int dtype, int bits, uint32_t G, const void* w, const void* s,
 // being captured nothing is waited for or freed, and the allocation is made in the relaxed capture mode, in which it is
 // allowed. Every buffer that replaces a kept one is at least twice as large: those kept are less than the last one in all.
 static int ensure_scratch(size_t need) {
+    if (options().scratch_most_kb && need > (size_t)options().scratch_most_kb * 1024) return fail(ERR_HIP, "library scratch: more than scratch.most_kb");
     if (g_plan.on) {  // mtq_plan has put a stand-in address into scratch_buf; nothing is allocated
         plan_note_scratch(need);
         return ERR_OK;
@@ -1900,6 +1893,11 @@ int mtq_set_option(const char* name, int value) {
         if (value < 0 || value > 2) return fail(ERR_BAD_ARG, "qmv.norm_mfma must be 0 (choose), 1 (never) or 2 (wherever the shape allows)");
         options().qmv_norm_mfma = value;
         return MTQ_OK;
+    }
+    if (!strcmp(name, "scratch.most_kb")) {
+        if (value < 0) return fail(ERR_BAD_ARG, "scratch.most_kb must be 0 (no limit) or a size in KB");
+        options().scratch_most_kb = value;
+        return ERR_OK;
     }
     if (!strcmp(name, "qmv.runs")) {
         if (value < 0 || value > 3) return fail(ERR_BAD_ARG, "qmv.runs must be 0 (choose), 1 (never), 2 (wherever the shape allows) or 3 (in slices of K wherever the shape allows)");

@@ -119,6 +119,7 @@ struct Options {
     int qmv_wide_nb = 0;          // 16-row matrix-core GEMV: row blocks per wave (0 = choose; 1, 2)
     int gather_wide = 0;          // expert-routed rows on the 16-row matrix-core GEMV: 0 = choose, 1 = never, 2 = wherever the shape allows
     int qmv_runs = 0;             // K-run matrix-core GEMV for batches of up to 16 rows: 0 = choose per shape, 1 = never, 2 = wherever the shape allows, 3 = the K-sliced form wherever the shape allows
+    int scratch_most_kb = 0;      // largest library-owned scratch buffer (0 = no limit): a call that needs more finds no memory
     int qmv_wide = 0;             // 16-row matrix-core GEMV for batches of 5..16 rows: 0 = choose per shape, 1 = never, 2 = wherever the shape allows
 };
 Options& options();

@@ -3,7 +3,7 @@ replayed after later calls that need more. Every replay gives the bits of the ea
 import numpy as np
 import pytest
 
-from metaltile_amd import DType, GpuBuffer, _lib, ops
+from metaltile_amd import DType, GpuBuffer, _lib, ops, unpack_f32
 from metaltile_amd.runtime import _ensure_init
 from metaltile_amd.synth import make_case
 from tests.hip_graph import Graph
@@ -47,7 +47,16 @@ def _batch(dt):
     return [b for o in ops_of for b in (*o[0], o[1])], out, 2 * M * N * 2, lambda: ops.qmm_batched(dt, 4, 64, ws, ss, bs, x, outs, [N, N], M, K)
 
 
-@pytest.mark.parametrize("make", [_gather, _bit_stream, _batch], ids=lambda f: f.__name__[1:])
+def _slices(dt):
+    """Four rows of more than 18432 codes: f32 sums of slices of K."""
+    M, N, K = 4, 1024, 18688
+    assert "qmv_slices_kernel" in ops.plan("qmm", dt, 4, 64, M, N, K)[1][0][0]
+    wsb, x = _operands(8, dt, 4, M, N, K)
+    out = GpuBuffer(M * N * 2)
+    return [x, *wsb], out, M * N * 2, lambda: ops.qmm(dt, 4, 64, *wsb, x, out, M, N, K)
+
+
+@pytest.mark.parametrize("make", [_gather, _bit_stream, _batch, _slices], ids=lambda f: f.__name__[1:])
 def test_captured_first_and_replayed_after_growth(make):
     dt = DType.BF16
     print(f"[case] scratch under capture, {make.__name__}", flush=True)
@@ -80,3 +89,27 @@ def test_captured_first_and_replayed_after_growth(make):
         g.close()
         for b in bufs + [out, big_out, big[1], *big[0]]:
             b.free()
+
+
+@pytest.mark.parametrize("bits,G,M,N,K", [(4, 64, 4, 1024, 18688), (8, 64, 3, 272, 18944), (4, 128, 16, 4096, 9344), (8, 64, 8, 8192, 10240)])
+def test_slices_without_memory(oracle, bits, G, M, N, K):
+    """Where the K slices' sums find no memory the call is served by the kernels that need none, alone and in a batch. Bound,
+    2-norm over 2-norm: the roundings to bf16 of the result and, on the tiles, of the weights, each up to 2^-9 of a value: 4e-3."""
+    dt = DType.BF16
+    print(f"[case] K-sliced qmv without memory b{bits} g{G} M{M} N{N} K{K}", flush=True)
+    lib = _ensure_init()
+    c = make_case(890 + M, dt, bits, G, M, N, K, bias_rule="midpoint")
+    bufs = [GpuBuffer.from_bytes(v) for v in (c.w.tobytes(), c.scales_bytes, c.biases_bytes, c.x_bytes)]
+    outs = [GpuBuffer.from_bytes(b"\xff" * (M * N * 2)) for _ in range(2)]
+    try:
+        assert lib.mtq_set_option(b"scratch.most_kb", 1) == 0
+        ops.qmm(dt, bits, G, *bufs, outs[0], M, N, K)
+        ops.qmm_batched(dt, bits, G, [bufs[0]], [bufs[1]], [bufs[2]], bufs[3], [outs[1]], [N], M, K)
+        got = [o.read_bytes(M * N * 2) for o in outs]
+    finally:
+        lib.mtq_set_option(b"scratch.most_kb", 0)
+    exp = oracle.qmm_f64(c.w, c.scales_f, c.biases_f, c.x_f, M, N, K, bits, G, threads=8).reshape(-1)
+    assert got[0] == got[1]
+    assert np.linalg.norm(unpack_f32(got[0], dt) - exp) <= 4e-3 * np.linalg.norm(exp)
+    for b in bufs + outs:
+        b.free()

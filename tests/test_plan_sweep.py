@@ -11,7 +11,7 @@ import itertools
 
 import pytest
 
-from metaltile_amd import DType, ops
+from metaltile_amd import DType, _lib, ops
 
 OK, BAD_ARG, SHAPE, UNSUPPORTED = 0, -2, -3, -7
 LDS_MAX = 160 * 1024
@@ -245,3 +245,27 @@ def test_k_run_lines(bits, M, N, K, runs):
     """Which matrices the K-run kernel is for, on both sides of each line."""
     rc, launches, _, _ = ops.plan("qmm", DType.BF16, bits, 64, M, N, K)
     assert rc == 0 and ("qmv_runs_kernel" in launches[0][0]) == runs, launches[0][0]
+
+
+@pytest.mark.parametrize("dt,bits,G,M,N,K,first", [
+    (DType.BF16, 4, 64, 4, 1024, 18688, "qmv_mfma_kernel"),          # K slices; two passes of two rows
+    (DType.BF16, 8, 64, 3, 3584, 18944, "qmv_mfma_kernel"),
+    (DType.F16, 4, 128, 16, 4096, 9344, "qmm_d"),                    # K slices; K no multiple of 256: the tiles
+    (DType.BF16, 8, 64, 8, 8192, 10240, "qmv_mfma_kernel"),
+    (DType.BF16, 4, 64, 8, 4096, 14336, "qmm_d"),                    # the 16-row GEMV with K split, or split tiles
+    (DType.BF16, 4, 64, 512, 4096, 14336, "qmm_d"),                  # split tiles
+    (DType.F32, 4, 64, 32, 4096, 4096, "qmm_f32_kernel"),
+])
+def test_products_without_scratch_memory(dt, bits, G, M, N, K, first):
+    """A product that writes partial results into the library's buffer runs on a kernel that needs none where the buffer cannot
+    be allocated."""
+    lib = _lib.load()
+    rc, launches, scratch, _ = ops.plan("qmm", dt, bits, G, M, N, K)
+    assert rc == OK and scratch > 1024
+    try:
+        assert lib.mtq_set_option(b"scratch.most_kb", 1) == OK
+        rc, launches, scratch, n = ops.plan("qmm", dt, bits, G, M, N, K)
+        assert rc == OK and scratch == 0 and first in launches[0][0], (rc, launches)
+        assert not any("reduce" in l[0] for l in launches)
+    finally:
+        lib.mtq_set_option(b"scratch.most_kb", 0)
