@@ -457,7 +457,8 @@ MTQ_API int mtq_flush_cache(void);
  *                          kernel with the weights converted in registers
  *   "qmm.kgroups"          register-operand tile kernel: K-groups per workgroup, 0 = choose, or 1 / 2 / 4
  *   "qmm.tile_rows"        activation rows per tile, 0 = choose, or 32 (4 K-groups only) / 64 / 128 / 256 (4- and 8-bit
- *                          codes on 2 K-groups only)
+ *                          codes on 2 K-groups only) / 160 (expert-routed rows of 4- and 8-bit codes: up to 160 rows a tile,
+ *                          wherever the shape allows)
  *   "qmm.dma"              tile instances that bring the activation tile in by load-to-LDS instructions (4- and 8-bit
  *                          codes): 0 = where the shape allows and it pays (8-bit codes: rows of 8192 codes and more, or
  *                          launches that fill the chip), 1 = never (the register-staged instances; same results bit for

@@ -740,7 +740,7 @@ static int op_gather(int mode, int dtype, int bits, uint32_t G, const void* x, c
         q.w = w; q.scales = s; q.biases = b; q.x = x; q.out = out;
         q.M = T; q.N = N; q.K = K;
         const bool ids = mode == GATHER_INDICES;
-        rc = ensure_scratch(qmm_grouped_scratch_bytes(T, E, ids, 32));  // sized for the smaller tile height: more tiles
+        rc = ensure_scratch(qmm_grouped_scratch_bytes(q, T, E, ids));
         if (rc) return rc;
         rc = launch_qmm_grouped(q, route, ids, T, E, g.scratch_buf, lc);
         if (rc != ERR_UNSUPPORTED) return rc;
@@ -1972,7 +1972,8 @@ int mtq_set_option(const char* name, int value) {
         return MTQ_OK;
     }
     if (!strcmp(name, "qmm.tile_rows")) {
-        if (value != 0 && value != 32 && value != 64 && value != 128 && value != 256) return fail(ERR_BAD_ARG, "qmm.tile_rows must be 0, 32, 64, 128 or 256");
+        if (value != 0 && value != 32 && value != 64 && value != 128 && value != 160 && value != 256)
+            return fail(ERR_BAD_ARG, "qmm.tile_rows must be 0, 32, 64, 128, 160 or 256");
         options().qmm_tile_rows = value;
         return MTQ_OK;
     }

@@ -106,7 +106,7 @@ struct Options {
     int gather_names_exact = 0;   // name-keyed exact-dequant gathers (mt_moe_gather_qmm_int4*, _b*): 0 = never on the rounding tile kernel, 1 = by rows per expert
     int qmm_ksplit = 0;           // direct qmm: 0 = choose, 1 = never split K, n = n splits
     int qmm_f32_tiles = 0;        // f32 batches on the f32 matrix cores: 0 = choose by rows, 1 = never, 2 = always
-    int qmm_tile_rows = 0;        // direct qmm: activation rows per tile (0 = choose; 32, 64, 128, 256)
+    int qmm_tile_rows = 0;        // direct qmm: activation rows per tile (0 = choose; 32, 64, 128, 256; 160: expert-routed rows)
     int qmm_dma = 0;              // direct qmm: activation tiles by load-to-LDS instructions: 0 = where it pays, 1 = never, 2 = with the scales in windows even where whole rows fit, 3 = wherever the shape allows
     int qmv_mfma = 0;             // matrix-core qmv: 0 auto, 1 never, 2 whenever the shape fits
     int qmv_mfma_kp = 0;          // matrix-core qmv: K parts per row block
@@ -205,10 +205,11 @@ int launch_qmm_f32(const QmmParams& p, const LaunchCtx& lc, void* scratch);
 // Expert-routed rows on the same kernel (many rows per expert): p holds one expert's shapes (N, K),
 // x [T][K], out [T][N], w / scales / biases the stacked experts. `route` = CSR offsets [E + 1], or one
 // expert id per row when per_row_ids. scratch: qmm_grouped_scratch_bytes() bytes.
-size_t qmm_grouped_scratch_bytes(uint32_t T, uint32_t E, bool sort_rows, uint32_t tile_rows = 64);
+size_t qmm_grouped_scratch_bytes(const QmmParams& p, uint32_t T, uint32_t E, bool sort_rows);
+size_t qmm_grouped_scratch_bytes(uint32_t T, uint32_t E, bool sort_rows, uint32_t tile_rows);
 int launch_qmm_grouped(const QmmParams& p, const uint32_t* route, bool per_row_ids, uint32_t T, uint32_t E, void* scratch,
                        const LaunchCtx& lc);
-// The table of row tiles behind both grouped launchers: tiles[0] = count, tiles[1 + i] = (expert,
+// The table of row tiles behind both grouped launchers (qmm_direct_plan.h); 32-row tiles: tiles[0] = count, tiles + 4 + 4 i = (expert,
 // first row in the row order, rows, place in its run | run length << 16); rowlist maps the row order to rows of x / out (null: identity).
 struct GatherTiles {
     uint32_t* tiles = nullptr;

@@ -161,6 +161,9 @@ static int dma_mode(int bits, uint32_t rows, uint32_t kgroups, uint32_t K, uint3
 }
 static bool dma_fits(int bits, uint32_t rows, uint32_t kgroups, uint32_t K, uint32_t gpr) { return dma_mode(bits, rows, kgroups, K, gpr) != 0; }
 
+// "qmm.tile_rows" for matrices that are not routed (160 is for expert-routed rows alone).
+static int tile_rows_option() { return options().qmm_tile_rows == (int)QD_ROUTED_ROWS ? 0 : options().qmm_tile_rows; }
+
 // The same for the tall tiles of expert-routed rows, which take any even number of groups.
 static int routed_mode(int bits, uint32_t K, uint32_t gpr) {
     if (options().qmm_dma == 1 || (bits != 4 && bits != 8) || K % 128 || gpr % 2) return 0;
@@ -354,7 +357,7 @@ static int plan_direct(const QmmParams& p, QmmDPlan& pl) {
     // (long rows that leave even the 64-row tiles short of one per compute unit keep the K-split tall tiles chosen
     // above: 300 rows, 4096 x 11008 63 us against 68, 4096 x 14336 79 against 81)
     const bool underfilled_long = p.M >= 256 && p.K > 8192 && short_wide < (uint64_t)cus;   // (at K = 8192 the 64-row tiles win: 300 rows 38 us against 49)
-    if (p.M > 64 && short_wide * 2 > (uint64_t)cus && !underfilled_long && !options().qmm_tile_rows && !options().qmm_kgroups) {
+    if (p.M > 64 && short_wide * 2 > (uint64_t)cus && !underfilled_long && !tile_rows_option() && !options().qmm_kgroups) {
         static const uint32_t heights[3] = {64, 128, 256};
         static const double base[3] = {20.6, 28.0, 48.5}, full[3] = {0.16, 0.35, 0.45}, more[3] = {1.15, 1.10, 1.0};
         double best = 0.0;
@@ -381,7 +384,7 @@ static int plan_direct(const QmmParams& p, QmmDPlan& pl) {
     // 31.3 / 40.4 / 48.4 (128 rows lose, 22.0 -> 24.3); 5120 x 13824, 128 / 256 / 384 rows 47.9 / 70.7 / 92.2 -> 37.4 /
     // 55.6 / 75.9; 8192 x 28672 (a split's scales fit LDS from 4 splits on), 128 / 256 rows 163.5 / 184.4 -> 84.7 / 156.7.
     uint32_t dma_ks = 0;
-    if (!options().qmm_tile_rows && !options().qmm_kgroups && ksplit_option == 0 && p.K >= 8192 &&
+    if (!tile_rows_option() && !options().qmm_kgroups && ksplit_option == 0 && p.K >= 8192 &&
         (p.M > 128 || (p.M > 96 && p.K > 8192)) && tall_wide * 2 <= (uint64_t)cus && (uint64_t)p.M * p.N < (1ull << 31)) {
         uint32_t ks = (uint32_t)((uint64_t)cus / tall_wide);
         ks = ks > 8 ? 8 : ks;
@@ -399,7 +402,7 @@ static int plan_direct(const QmmParams& p, QmmDPlan& pl) {
     // scales in LDS (8192 x 9216 45 / 45 / 52 -> 48 / 51 / 54, 8192 x 12288 in groups of 128 60 / 59 / 66 -> 61 / 64 / 65).
     const bool one_round = tall_wide > 32 && tall_wide <= 64 && p.K % 256 == 0 && stages_scales(64, p.K / G);
     if (odd_bits && p.M > 64 && p.M <= 128 && p.K > 8192 && tall_wide >= 24 && tall_wide * 2 <= (uint64_t)cus && !one_round) { rows = 128; kgroups = 1; }
-    if (options().qmm_tile_rows) rows = (uint32_t)options().qmm_tile_rows;
+    if (tile_rows_option()) rows = (uint32_t)tile_rows_option();
     if (options().qmm_kgroups) kgroups = (uint32_t)options().qmm_kgroups;
     // An iteration covers 64 k per K-group: K must be a multiple of 64 * K-groups (an odd number of
     // iterations is fine). Rows that are not (K = 11008 = 43 * 256 is, 11072 = 173 * 64 is not for 2 or
@@ -413,7 +416,7 @@ static int plan_direct(const QmmParams& p, QmmDPlan& pl) {
     if (rows == 256 && !dma_fits(p.bits, 256, kgroups, p.K, p.K / G))
         return fail(ERR_BAD_ARG, "qmm.tile_rows 256 needs 4- or 8-bit codes, 2 K-groups, K % 128 == 0 and rows whose scales fit LDS (or, 4-bit codes, groups of 64 or 128 codes)");
     if (rows == 32 && kgroups != 4) {
-        if (options().qmm_tile_rows) return fail(ERR_BAD_ARG, "qmm.tile_rows 32 needs 4 K-groups");
+        if (tile_rows_option()) return fail(ERR_BAD_ARG, "qmm.tile_rows 32 needs 4 K-groups");
         rows = 64;
     }
     pl.rows = rows;
@@ -524,20 +527,27 @@ int launch_qmm_direct(QmmDLaunch* l, int n, void* scratch, const LaunchCtx& lc) 
 // whose id names no expert: they get no tile, so their output rows stay untouched.
 struct TileTabArgs {
     const uint32_t* off;  // [E + 1]
-    uint32_t* tiles;      // [4 + 4 * max_tiles]
+    uint32_t* tiles;      // [4 + 4 * max_tiles], by height [4 + 16 * max_tiles]
     uint32_t E, T, tile_rows, max_tiles, tail_to_0;
 };
-__global__ __launch_bounds__(64) void gather_tiles_kernel(TileTabArgs a) {
+// BY_HEIGHT: a table for each height class (routed_deal.h), else one, in expert order; tiles[0 .. 3] their lengths.
+template <bool BY_HEIGHT> __global__ __launch_bounds__(64) void gather_tiles_kernel(TileTabArgs a) {
     // One wave, 64 experts at a time: lane l takes expert base + l. The rule needs, per expert, the
-    // largest offset before it (a running maximum) and the number of tiles before it (a running sum);
-    // both are wave scans, carried from one batch of 64 to the next, so the table comes out in expert
+    // largest offset before it (a running maximum) and the number of tiles of its class before it (running sums);
+    // both are wave scans, carried from one batch of 64 to the next, so a table comes out in expert
     // order exactly as a serial walk would write it, without a chain of dependent loads.
+    constexpr uint32_t NH = BY_HEIGHT ? QD_HEIGHTS : 1;
     const uint32_t lane = threadIdx.x;
-    uint32_t n = 0, mx = 0;  // carried: tiles so far, largest offset so far (wave-uniform)
-    uint4* tab = (uint4*)a.tiles + 1;
-    auto emit = [&](uint32_t first, uint32_t e, uint32_t lo, uint32_t hi) {
+    uint32_t n[NH] = {}, mx = 0;  // carried: tiles so far, largest offset so far (wave-uniform)
+    auto pieces = [&](uint32_t rows) { return (rows + a.tile_rows - 1) / a.tile_rows; };
+    auto height = [&](uint32_t rows, uint32_t cnt) -> uint32_t {   // class of an expert's tiles: 32-row blocks 5, 4, 3, up to 2
+        if constexpr (!BY_HEIGHT) return 0u;
+        return cnt ? QD_HEIGHTS + 1 - max(2u, ((rows + cnt - 1) / cnt + 31u) / 32u) : 0u;
+    };
+    auto emit = [&](uint32_t h, uint32_t first, uint32_t e, uint32_t lo, uint32_t hi) {
+        uint4* tab = (uint4*)a.tiles + 1 + (size_t)h * a.max_tiles;
         uint32_t i = first;
-        const uint32_t cnt = (hi - lo + a.tile_rows - 1) / a.tile_rows, per = (hi - lo + cnt - 1) / cnt;   // even pieces
+        const uint32_t cnt = pieces(hi - lo), per = (hi - lo + cnt - 1) / cnt;   // even pieces
         for (uint32_t j = 0, r = lo; r < hi && i < a.max_tiles; r += per, i++, j++) {
             const uint32_t in_run = j % QD_RUN, run = min(QD_RUN, cnt - (j - in_run));
             tab[i] = make_uint4(e, r, min(per, hi - r), in_run | run << 16);
@@ -556,24 +566,37 @@ __global__ __launch_bounds__(64) void gather_tiles_kernel(TileTabArgs a) {
         uint32_t before = __shfl_up(pm, 1, 64);  // largest offset of the earlier lanes of this batch
         before = lane == 0 ? mx : max(mx, before);
         const uint32_t lo = min(before, a.T), hi = min(o1, a.T);
-        const uint32_t cnt = (e < a.E && hi > lo) ? (hi - lo + a.tile_rows - 1) / a.tile_rows : 0u;
-        uint32_t ps = cnt;  // inclusive running sum of tile counts
+        const uint32_t cnt = (e < a.E && hi > lo) ? pieces(hi - lo) : 0u, mine = height(hi - lo, cnt);
+        uint32_t ps[NH], at = 0;  // inclusive running sums of tile counts
 #pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const uint32_t t = __shfl_up(ps, d, 64);
-            if (lane >= (uint32_t)d) ps += t;
+        for (uint32_t h = 0; h < NH; h++) ps[h] = mine == h ? cnt : 0u;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1)
+#pragma unroll
+            for (uint32_t h = 0; h < NH; h++) {
+                const uint32_t t = __shfl_up(ps[h], d, 64);
+                if (lane >= (uint32_t)d) ps[h] += t;
+            }
+#pragma unroll
+        for (uint32_t h = 0; h < NH; h++) {
+            if (mine == h) at = n[h] + ps[h] - cnt;
+            n[h] += __shfl(ps[h], 63, 64);
         }
-        if (cnt) emit(n + ps - cnt, e, lo, hi);
-        n += __shfl(ps, 63, 64);
+        if (cnt) emit(mine, at, e, lo, hi);
         mx = max(mx, __shfl(pm, 63, 64));
     }
     if (lane == 0) {
         if (a.tail_to_0 && mx < a.T) {
-            const uint32_t cnt = (a.T - mx + a.tile_rows - 1) / a.tile_rows;
-            emit(n, 0u, mx, a.T);
-            n += cnt;
+            const uint32_t cnt = pieces(a.T - mx), mine = height(a.T - mx, cnt);
+#pragma unroll
+            for (uint32_t h = 0; h < NH; h++)
+                if (mine == h) {
+                    emit(h, n[h], 0u, mx, a.T);
+                    n[h] += cnt;
+                }
         }
-        a.tiles[0] = min(n, a.max_tiles);
+#pragma unroll
+        for (uint32_t h = 0; h < QD_HEIGHTS; h++) a.tiles[h] = h < NH ? min(n[h < NH ? h : 0], a.max_tiles) : 0u;
     }
 }
 
@@ -583,25 +606,38 @@ __global__ __launch_bounds__(64) void gather_tiles_kernel(TileTabArgs a) {
 // against 36 / 43). With more rows, or many small experts, the 32-row tiles lose (every weight is converted
 // once per 32 rows instead of 64: 128 x 2048 x 768, 48 rows each: 75 against 137 us).
 static uint32_t grouped_tile_rows(const QmmParams& p, uint32_t T, uint32_t E) {
-    // Tall row tiles from 64 rows per expert on (64-row tiles -> these, us: 128 x 768 x 2048, 55 / 64 / 96 rows each 60.7 / 74.8 /
-    // 89.8 -> 62.0 / 62.9 / 75.9; 128 x 2048 x 768 67.7 / 83.4 / 109.6 -> 77.4 / 81.9 / 99.9; 8 x 14336 x 4096, 50 / 64 / 256 rows 98.8 /
-    // 139 / 354 -> 114.5 / 125.5 / 311), where they are tiles for half the chip at least. Not on short rows where an expert's rows
-    // are two pieces of about 96 (128 x 2048 x 768, 192 rows each: 181.8 -> 185.8; 256 rows 232 -> 216).
-    const uint64_t hit = E < T ? E : T, pieces = (T + QD_ROUTED_ROWS - 1) / QD_ROUTED_ROWS, tall = pieces > hit ? pieces : hit;
-    const bool short_halves = p.K < 1024 && (uint64_t)T > 160 * hit && (uint64_t)T < 224 * hit;
-    if (routed_mode(p.bits, p.K, p.K / p.group_size) && !options().qmm_tile_rows && (uint64_t)T >= 64 * hit && !short_halves && tall * ((p.N + 127) / 128) >= 128)
+    // Tall row tiles from 64 rows per expert on. us, bf16, the whole gather, 64-row tiles -> these, rows by even / random / skewed
+    // routing (an expert's share as 1 / rank):
+    //   128 x 768 x 2048, 64 rows per expert 48.8 67.4 67.5 -> 56.7 60.6 72.1, 128 77.7 96.6 102 -> 70.8 75.9 94.9; 8 bits, 64 rows
+    //     63.1 89.4 92.6 -> 60.6 64.5 79.2
+    //   64 x 1408 x 2048, 64 rows 42.8 61.7 62.4 -> 47.3 51.6 61.8, 256 133 152 155 -> 120 131 130; 16 x 6400 x 4096, 64 rows 89.5 109 109 ->
+    //     99.9 104 106; 8 x 14336 x 4096, 512 rows 620 648 621 -> 526 562 548 (8 bits 979 1041 1003 -> 661 679 669)
+    // A tile's start and end outweigh the loop on short rows, so 4-bit codes from 96 rows there: 128 x 2048 x 768, 64 rows 52.9 74.9
+    // 77.5 -> 68.4 72.9 88.2, 96 rows 92.2 91.8 99.0 -> 80.3 83.7 102, 128 rows 95.1 113 117 -> 92.2 97.5 115; 192 rows, two pieces of 96,
+    // 137 154 161 -> 146 150 151 (8 bits, 64 rows 80.8 113 117 -> 85.3 87.5 103). One tile has a compute unit to itself: fewer
+    // than two for each are one round or two, as the routing falls, and 4-bit codes go there from 128 rows: 8 x 4096 x 14336, 64 rows
+    // 106 153 148 -> 101 111 174, 96 rows 167 166 168 -> 119 134 181, 128 rows 170 240 238 -> 141 158 203 (8 bits, 64 rows 154
+    // 279 277 -> 146 153 248). At least tiles for half the chip.
+    const uint64_t hit = E < T ? E : T, pieces = (T + QD_ROUTED_ROWS - 1) / QD_ROUTED_ROWS, tiles = (pieces > hit ? pieces : hit) * ((p.N + 127) / 128);
+    const uint32_t from = p.bits == 8 ? 64 : tiles < 512 ? 128 : p.K < 1024 ? 96 : 64;
+    const bool pays = (uint64_t)T >= from * hit && tiles >= 128;
+    if (routed_mode(p.bits, p.K, p.K / p.group_size) && (options().qmm_tile_rows == (int)QD_ROUTED_ROWS || (options().qmm_tile_rows == 0 && pays)))
         return QD_ROUTED_ROWS;
     if (p.K % 256 || (p.bits != 2 && p.bits != 4 && p.bits != 8)) return 64u;
-    if (options().qmm_tile_rows == 32) return 32u;
-    if (options().qmm_tile_rows == 64) return 64u;
+    if (tile_rows_option() == 32) return 32u;
+    if (tile_rows_option() == 64) return 64u;
     return ((uint64_t)T <= 24ull * E && (uint64_t)p.N * p.K >= (1ull << 24)) ? 32u : 64u;
 }
 
 size_t qmm_grouped_scratch_bytes(uint32_t T, uint32_t E, bool sort_rows, uint32_t tile_rows) {
     const size_t max_tiles = (size_t)(T + tile_rows - 1) / tile_rows + E + 1;
-    size_t b = 16 + max_tiles * 16;
+    size_t b = 16 + max_tiles * 16 * (tile_rows == QD_ROUTED_ROWS ? QD_HEIGHTS : 1);
     if (sort_rows) b += ((size_t)2 * T + E + 2 + 3) / 4 * 16;  // sorted row list, inverse permutation, offsets of E + 1 buckets
     return b;
+}
+
+size_t qmm_grouped_scratch_bytes(const QmmParams& p, uint32_t T, uint32_t E, bool sort_rows) {
+    return qmm_grouped_scratch_bytes(T, E, sort_rows, grouped_tile_rows(p, T, E));
 }
 
 // Sorts per-row ids by expert where needed and launches the tile table kernel into `scratch`
@@ -621,7 +657,7 @@ int build_gather_tiles(const uint32_t* route, bool per_row_ids, uint32_t T, uint
     out.last.start = nullptr;
     bool started = false;
     if (per_row_ids) {
-        uint32_t* sorted = tiles + 4 + (size_t)max_tiles * 4;
+        uint32_t* sorted = tiles + 4 + (size_t)max_tiles * 4 * (tile_rows == QD_ROUTED_ROWS ? QD_HEIGHTS : 1);
         uint32_t* inv = sorted + T;
         uint32_t* offs = inv + T;
         // one bucket more than experts: the sort clamps ids to its last bucket, which so collects the
@@ -634,7 +670,8 @@ int build_gather_tiles(const uint32_t* route, bool per_row_ids, uint32_t T, uint
     }
     TileTabArgs ta{off, tiles, E, T, tile_rows, max_tiles, per_row_ids ? 0u : 1u};
     void* targs[] = {&ta};
-    hipError_t e = launch_kernel((const void*)gather_tiles_kernel, dim3(1), dim3(64), targs, 0, started ? mid : first);
+    const void* fn = tile_rows == QD_ROUTED_ROWS ? (const void*)gather_tiles_kernel<true> : (const void*)gather_tiles_kernel<false>;
+    hipError_t e = launch_kernel(fn, dim3(1), dim3(64), targs, 0, started ? mid : first);
     if (e != hipSuccess) return hip_fail(e, "gather tile table kernel launch");
     out.tiles = tiles;
     out.rowlist = rowlist;

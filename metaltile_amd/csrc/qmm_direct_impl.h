@@ -47,19 +47,22 @@ __device__ __forceinline__ uint32_t qd_xcd_share(uint32_t id, uint32_t total) {
 }
 
 // Expert-routed rows: this workgroup's row tile and column tile; false past the last one. Workgroups congruent mod 8 share an
-// XCD and its L2: each XCD takes an even share of consecutive tiles, and inside it the row tiles of one run (up to QD_RUN of one
-// expert) stand side by side at each column tile, so that a run's weights cross the fabric once and its activations stay in
-// that L2. In launch order over all XCDs every XCD fetched all activations and each row tile its weights again
-// (128 experts of 768 x 2048, 128 rows each, 64-row tiles in runs of 8 108 -> 98.5 us; of 2048 x 768 133 -> 128.7).
-__device__ __forceinline__ bool qd_routed_tile(const uint32_t* tiles, uint32_t n_tiles, uint4& t, uint32_t& nt) {
-    const uint32_t total = tiles[0] * n_tiles, share = (total + 7) / 8, at = blockIdx.x >> 3;
-    const uint32_t vid = (blockIdx.x & 7u) * share + at;
-    if (at >= share || vid >= total) return false;
+// XCD and its L2: each XCD takes an even share of consecutive tiles of every height class, and inside it the row tiles of one run (up to
+// QD_RUN of one expert) stand side by side at each column tile, so that a run's weights cross the fabric once and its activations stay in
+// that L2 (in launch order over all XCDs every XCD fetched all activations and each row tile its weights again). us, 16384 rows on 128
+// experts of 2048 x 768, even / half of the rows with one expert, one sequence of tiles cut into eight -> even shares of each height
+// 90 / 139 -> 93 / 110 (64-row tiles in launch order 96 / 106); 4096 rows on 64 experts of 1408 x 2048, random / shares as 1 / rank 52 / 91
+// -> 52 / 63 (56 / 65).
+__device__ __forceinline__ bool qd_routed_tile(const uint32_t* tiles, uint32_t m_tiles, uint32_t n_tiles, uint4& t, uint32_t& nt) {
     const uint4* tab = (const uint4*)tiles + 1;
+    const uint4 head = ((const uint4*)tiles)[0];
+    const uint32_t count[QD_HEIGHTS] = {head.x, head.y, head.z, head.w};
+    const uint32_t vid = routed_deal(count, m_tiles, n_tiles, blockIdx.x & 7u, blockIdx.x >> 3);
+    if (vid == 0xFFFFFFFFu) return false;
     uint32_t mt = vid / n_tiles;
-    const uint32_t run = tab[mt].w, first = mt - (run & 0xFFFFu), len = run >> 16, in_run = vid - first * n_tiles;
+    const uint32_t run = tab[mt].w, run0 = mt - (run & 0xFFFFu), len = run >> 16, in_run = vid - run0 * n_tiles;
     nt = in_run / len;
-    mt = first + in_run - nt * len;
+    mt = run0 + in_run - nt * len;
     t = tab[mt];
     return true;
 }
@@ -107,7 +110,7 @@ __global__ __launch_bounds__(KG == 1 ? 256 : 512) void qmm_direct_kernel(QmmDArg
     uint32_t row_first = mt * DBM, row_count = a.M > row_first ? min((uint32_t)DBM, a.M - row_first) : 0u;
     if constexpr (GR) {
         uint4 t;
-        if (!qd_routed_tile(a.tiles, a.n_tiles, t, nt)) return;  // the grid is sized for the worst routing
+        if (!qd_routed_tile(a.tiles, a.m_tiles, a.n_tiles, t, nt)) return;  // the grid is sized for the worst routing
         row_first = t.y;
         row_count = t.z;
         a.w += (size_t)t.x * a.w_expert_bytes;

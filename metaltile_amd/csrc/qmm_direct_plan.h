@@ -1,6 +1,7 @@
 // What a launch of the tile kernels (qmm_direct.hip) is: their argument block, and one matrix's kernel and geometry.
 #pragma once
 #include "mtq_internal.h"
+#include "routed_deal.h"
 
 namespace mtq {
 
@@ -18,9 +19,10 @@ struct QmmDBase {
     uint32_t m_tiles, n_tiles, iters;
     uint32_t m_tile_rows;  // 32 (4 K-groups only), 64, 128 or 256; 160 for expert-routed rows (at most)
     uint32_t by_m;         // consecutive workgroup ids walk the N-tiles of one M-tile (else the M-tiles of one N-tile)
-    // grouped mode (expert-routed rows): tiles[0] = number of row tiles, then one uint4 per tile
+    // grouped mode (expert-routed rows): tiles[0 .. 3] = number of row tiles of each height class, then a table of m_tiles slots for
+    // each class (one class and table but for the tall tiles) with one uint4 per tile
     // (expert, first row of the tile in the row order, rows in the tile, its place in its run of at most QD_RUN row tiles of the
-    // expert | the run's length << 16); rowlist maps the row order to rows of x / out (null: the identity). w / scales / biases
+    // expert | the run's length << 16); rowlist maps the row order to rows of x / out (null: identity). w / scales / biases
     // are the stacked experts'.
     const uint32_t* tiles;
     const uint32_t* rowlist;

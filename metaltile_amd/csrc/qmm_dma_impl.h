@@ -537,7 +537,7 @@ __global__ __launch_bounds__(64 * NW) void qmm_dma_kernel(QmmDArgs args) {
     uint4 t = make_uint4(0, 0, 0, 0);
     uint32_t nt = 0;
     if constexpr (GR) {
-        if (!qd_routed_tile(args.tiles, args.n_tiles, t, nt)) return;  // the grid is sized for the worst routing
+        if (!qd_routed_tile(args.tiles, args.m_tiles, args.n_tiles, t, nt)) return;  // the grid is sized for the worst routing
     }
     qmm_dma_tile<DT, MB, KG, NW, NB, GR, SP, WIN, BITS>(args, t, nt);
 }
@@ -554,7 +554,7 @@ template <int DT, int MB, int KG, int NW, int NB, bool GR, bool SP, bool WIN, in
     static_assert(MB == 2 && GR && !SP, "expert-routed rows, 64 rows and more");
     uint4 t;
     uint32_t nt;
-    if (!qd_routed_tile(args.tiles, args.n_tiles, t, nt)) return;
+    if (!qd_routed_tile(args.tiles, args.m_tiles, args.n_tiles, t, nt)) return;
     if (t.z <= 64) qmm_dma_tile<DT, 2, KG, NW, 0, true, false, WIN, BITS>(args, t, nt);
     else if (t.z <= 96) qmm_dma_tile<DT, 3, KG, NW, 0, true, false, WIN, BITS>(args, t, nt);
     else if (t.z <= 128) qmm_dma_tile<DT, 4, KG, NW, 0, true, false, WIN, BITS>(args, t, nt);

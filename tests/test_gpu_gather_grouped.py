@@ -248,7 +248,7 @@ def test_names_keep_their_arithmetic(runner, oracle, bits):
         buf.free()
 
 @pytest.mark.parametrize("bits,N,K,G,counts", [
-    (4, 128, 256, 64, [513, 0, 1, 1100, 64]),      # 9 + 1 + 18 + 1 row tiles of one column tile: runs of 8 and of what is left
+    (4, 128, 256, 64, [513, 0, 1, 1100, 64]),      # 9 + 1 + 18 + 1 row tiles of one column tile: runs of 4 and of what is left
     (4, 640, 512, 64, [65, 128, 0, 512, 3]),       # column tiles that are no power of two
     (8, 264, 256, 32, [600, 30]),                  # a ragged last column tile
     (6, 384, 256, 64, [577, 0, 130]),              # the register-staged kernel
@@ -283,9 +283,10 @@ def test_grouped_gather_runs_of_row_tiles(oracle, grouped, bits, N, K, G, counts
     (DType.BF16, 8, 8192, 128, 64, [700, 150]),                     # five even pieces, a single iteration
     (DType.BF16, 4, 8192, 5760, 64, [130, 100]),                    # scales in two windows
     (DType.F16, 8, 8192, 5760, 64, [81, 159]),
+    (DType.BF16, 4, 384, 512, 64, [2, 700, 33, 0, 150, 9] + [70] * 70),   # experts over two batches of lanes, more than 8 tiles of each height
 ], ids=str)
 def test_grouped_gather_on_tall_row_tiles(oracle, dt, bits, N, K, G, counts):
-    """Row tiles of up to 160 rows, chosen by the rows per expert, against the 64-row tiles: the same products added in the same
+    """Row tiles of up to 160 rows, in tables by height and dealt by height, against the 64-row tiles: the same products added in the same
     order by the same instructions, so the same bits; and those against the oracle on a sample of columns (2e-2 as above)."""
     lib = _lib.load()
     E, T = len(counts), sum(counts)
@@ -297,9 +298,11 @@ def test_grouped_gather_on_tall_row_tiles(oracle, dt, bits, N, K, G, counts):
     try:
         for view, route, fn, ids in (("csr", offsets, ops.gather_qmv_csr, ids_sorted), ("indices", ids_shuffled, ops.gather_qmv_indices, ids_shuffled)):
             r, got = GpuBuffer.from_bytes(route.tobytes()), []
-            for rows in (0, 64):
+            for rows in (160, 64):
                 print(f"[case] tall row tiles {view} {dt.name} b{bits} N={N} K={K} {counts} rows={rows}", flush=True)
                 assert lib.mtq_set_option(b"qmm.tile_rows", rows) == 0
+                kernel = ops.plan(f"gather_{view}", dt, bits, G, 1, N, K, E, T)[1][-1][0]
+                assert ("tall::" in kernel) == (rows == 160), kernel
                 out = GpuBuffer.from_bytes(np.full(T * N + 1024, 0x7B7B, np.uint16).tobytes())
                 fn(dt, bits, G, x, w, s, b, r, out, T, N, K, E)
                 got.append(np.frombuffer(out.read_bytes(), np.uint16))

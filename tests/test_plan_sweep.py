@@ -269,3 +269,20 @@ def test_products_without_scratch_memory(dt, bits, G, M, N, K, first):
         assert not any("reduce" in l[0] for l in launches)
     finally:
         lib.mtq_set_option(b"scratch.most_kb", 0)
+
+
+@pytest.mark.parametrize("bits,E,N,K,per,tall", [
+    (4, 128, 768, 2048, 64, True), (4, 128, 768, 2048, 63, False), (8, 128, 768, 2048, 64, True), (8, 128, 768, 2048, 63, False),
+    (4, 128, 2048, 768, 96, True), (4, 128, 2048, 768, 95, False), (8, 128, 2048, 768, 64, True), (4, 128, 2048, 768, 192, True),   # short rows
+    (4, 8, 4096, 14336, 128, True), (4, 8, 4096, 14336, 127, False), (8, 8, 4096, 14336, 64, True),   # fewer than two tiles a compute unit
+    (4, 8, 8192, 4096, 64, True), (4, 8, 8064, 4096, 64, False),
+    (8, 2, 8192, 4096, 64, True), (8, 2, 8064, 4096, 64, False),     # tiles for half the chip
+    (6, 128, 768, 2048, 128, False), (4, 128, 768, 2080, 128, False),
+])
+def test_tall_routed_lines(bits, E, N, K, per, tall):
+    """Where expert-routed rows run on tiles of up to 160 rows, on both sides of each line; the scratch holds their four tables."""
+    rc, launches, scratch, _ = ops.plan("gather_csr", DType.BF16, bits, 32 if K % 64 else 64, 1, N, K, E, per * E)
+    assert rc == OK and ("tall::" in launches[-1][0]) == tall, launches
+    rows = 160 if tall else 64
+    if bits != 6:
+        assert scratch == 16 + (-(-per * E // rows) + E + 1) * 16 * (4 if tall else 1)
