@@ -325,7 +325,7 @@ static int run_runs(int dtype, int bits, uint32_t G, int n, const void* const* w
         QmvBatch one;
         one.n = 1;
         one.w[0] = w[j]; one.scales[0] = s[j]; one.biases[0] = b[j]; one.out[0] = outs[j]; one.N[0] = N[j];
-        if ((o.qmv_runs != 2 && !qmv_runs_preferred(bits, M, N[j], K)) || !qmv_runs_takes(p, one)) continue;
+        if ((o.qmv_runs != 2 && !qmv_runs_preferred(bits, G, M, N[j], K)) || !qmv_runs_takes(p, one)) continue;
         taken[j] = true;
         left--;
         const int i = all.n++;

@@ -189,7 +189,7 @@ int launch_qmv_wide_gather(const QmvParams& p, const LaunchCtx& lc, void* scratc
 // K-run matrix-core GEMV (qmv_runs.hip): up to 16 activation rows (p.M, p.x, dtype, bits, group size, K; b: the matrices, 1..4
 // of them in one launch), f16 / bf16, 4- and 8-bit codes, K % 128 == 0. A matrix gives the same bits alone and in a batch.
 bool qmv_runs_takes(const QmvParams& p, const QmvBatch& b);
-bool qmv_runs_preferred(int bits, uint32_t M, uint32_t N, uint32_t K);   // one matrix's sizes
+bool qmv_runs_preferred(int bits, uint32_t G, uint32_t M, uint32_t N, uint32_t K);   // one matrix's sizes
 int launch_qmv_runs(const QmvParams& p, const QmvBatch& b, const LaunchCtx& lc);
 // The same walk on slices of K: one matrix of longer rows. scratch: qmv_slices_scratch_bytes(p) bytes.
 bool qmv_slices_takes(const QmmParams& p);

@@ -56,18 +56,30 @@ bool qmv_runs_takes(const QmvParams& p, const QmvBatch& b) {
 //   1280 x 5120     5.1  5.5  5.7 ->  7.5  7.7  8.0 | 10.0 10.9 11.1 ->  7.7  7.9  8.0
 //   512 x 8192      6.3  7.6  8.8 ->  9.5  9.9 10.3 | 13.0 15.5 17.9 ->  9.8 10.2 10.6
 //   4096 x 1024     3.6  3.8  3.8 ->  5.3  5.3  5.4 |  7.1  7.4  7.4 ->  6.4  6.4  6.5
-// Four rows on matrices of 16 to 76 M codes in rows of 2049 to 5120 (not 4096 of 8192 or more weight rows, which have a kernel of
-// their own, qmv_rows_few.hip): 4096 x 4096 6.2 -> 7.8 | 12.4 -> 9.1; 5120 x 5120 8.9 -> 9.8 | 17.9 -> 12.9; 18944 x 3584 13.7 -> 14.1 | 27.2 -> 21.8;
-// 13824 x 5120 12.9 -> 14.6 | 25.5 -> 22.6; 8 bits 5120 x 5120 11.1 -> 13.1 | 22.2 -> 18.6; 18944 x 3584 18.3 -> 19.1 | 36.4 -> 32.1.
-// So: below 5 rows those, and short matrices against rows of 2048 to 4096 codes (the K and V projections of grouped-query attention; 8-bit
-// codes from 3 rows); from 5 rows up to 75 M codes (60 M of 8 bits), and from 9 rows, where the others take tiles, no more than
+// 2 to 4 rows on more than 16384 weight rows: the GEMV's 256 workgroups of sixteen waves hold four rows a wave at once, past that
+// every one walks a second block of them (bf16, 2 | 3 | 4 rows alone, then a pair at 4 rows; groups of 64):
+//   16384 x 3584    9.7 | 10.0 | 10.0 -> 13.3 | 13.4 | 13.4, 20.0 -> 19.4        8 bits 14.8 | 15.5 | 15.9 -> 16.7 | 16.7 | 16.7, 32.0 -> 28.7
+//   16512 x 3584   13.5 | 13.9 | 13.9 -> 14.0 | 14.1 | 14.0, 27.9 -> 20.3        8 bits 17.9 | 18.8 | 19.1 -> 19.2 | 19.1 | 19.2, 38.0 -> 31.1
+//   18944 x 3584   13.7 | 14.1 | 14.0 -> 14.5 | 14.6 | 14.4, 28.2 -> 23.0        8 bits 18.4 | 19.2 | 19.6 -> 19.9 | 20.0 | 20.0, 39.2 -> 34.1
+//   16512 x 2048    9.6 | 10.2 | 10.3 -> 10.3 | 10.3 | 10.5, 20.5 -> 15.0        8 bits 13.5 | 14.2 | 14.2 -> 12.7 | 12.7 | 12.6, 28.5 -> 18.7
+//   24576 x 3072   13.9 | 14.4 | 14.4 -> 14.7 | 14.8 | 14.8, 28.8 -> 24.0        8 bits 17.7 | 19.8 | 19.9 -> 20.7 | 21.0 | 20.8, 39.9 -> 37.3
+//   28672 x 2560   13.8 | 14.3 | 14.3 -> 16.3 | 16.4 | 16.4, 28.4 -> 26.3 (seven blocks of 4096 rows each on a workgroup: past six, no)
+//   16512 x 4096   15.0 | 15.2 | 15.0 -> 14.5 | 14.7 | 14.6, 30.4 -> 21.3        8 bits 20.2 | 21.0 | 21.2 -> 23.4 | 22.7 | 23.2, 42.5 -> 38.4
+// Not in groups of 32, whose scales weigh more here (18944 x 3584, 4 rows 13.7 -> 16.9 | 27.5 -> 27.9), and not with 8 bits at 2 rows
+// (24576 x 3072 17.7 -> 20.7 | a pair 35.3 -> 37.4). Fewer weight rows lose more alone than they are sure to gain: 4096 x 4096, 4 rows
+// 6.0 -> 7.3 | 12.0 -> 9.3, 8192 x 4096 7.4 -> 9.2 | 14.9 -> 14.2; 5120 x 5120, 3 rows 8.5 -> 9.7 | 17.1 -> 13.1.
+// So: below 5 rows the gate and up projections of more than 16384 (to 24576) rows of 2048 to 4096 codes, and short matrices against such rows (the
+// K and V projections of grouped-query attention), both with 8-bit codes from 3 rows; from 5 rows up to 75 M codes (60 M of 8 bits), and from 9 rows, where the others take tiles, no more than
 // 1024 weight rows of more than 6144 codes (four steps a run, whose registers leave one block in flight) and no more than 8192 of
 // fewer than 2048 (some of the sixteen waves have no step, and a workgroup has more than two blocks to walk).
-bool qmv_runs_preferred(int bits, uint32_t M, uint32_t N, uint32_t K) {
+bool qmv_runs_preferred(int bits, uint32_t G, uint32_t M, uint32_t N, uint32_t K) {
     if (M < 2 || M > 16) return false;
     const uint64_t codes = (uint64_t)N * K;
-    if (M == 4 && K > 2048 && K <= 5120 && codes >= 16000000ull && codes <= 76000000ull && !(bits == 4 && K == 4096 && N >= 8192)) return true;
-    if (M < 5) return K >= 2048 && K <= 4096 && (uint64_t)N * 2 <= K && codes <= 4500000ull && (bits == 4 || M > 2);
+    if (M < 5) {
+        if (K < 2048 || K > 4096 || (bits == 8 && M == 2)) return false;
+        const bool tall = N > 16384 && N <= 24576 && codes <= 75000000ull && G >= 64;
+        return tall || ((uint64_t)N * 2 <= K && codes <= 4500000ull);
+    }
     if (M > 8 && ((K > 6144 && N > 1024) || (K < 2048 && N > 8192))) return false;
     return codes <= (bits == 4 ? 75000000ull : 60000000ull);
 }

@@ -247,6 +247,17 @@ def test_k_run_lines(bits, M, N, K, runs):
     assert rc == 0 and ("qmv_runs_kernel" in launches[0][0]) == runs, launches[0][0]
 
 
+@pytest.mark.parametrize("bits,G,N,K,rows", [
+    (4, 64, 16384, 3584, ()), (4, 64, 16400, 3584, (2, 3, 4)), (4, 128, 24576, 2048, (2, 3, 4)), (4, 64, 24592, 2048, ()), (4, 32, 18944, 3584, ()),
+    (8, 64, 16384, 3584, ()), (8, 64, 16400, 3584, (3, 4)), (8, 128, 24576, 2048, (3, 4)), (4, 64, 18944, 1920, ()), (4, 64, 18304, 4096, (2, 3, 4)), (4, 64, 18320, 4096, ()),
+    (4, 64, 4096, 4096, ()), (4, 64, 5120, 5120, ()), (8, 64, 5120, 5120, ()), (4, 64, 13824, 5120, ()),
+])
+def test_k_run_lines_of_few_rows(bits, G, N, K, rows):
+    """2, 3 and 4 rows on tall matrices: one rule of sizes, on both sides of each line."""
+    on = tuple(M for M in (2, 3, 4) if "qmv_runs_kernel" in ops.plan("qmm", DType.BF16, bits, G, M, N, K)[1][0][0])
+    assert on == rows
+
+
 @pytest.mark.parametrize("dt,bits,G,M,N,K,first", [
     (DType.BF16, 4, 64, 4, 1024, 18688, "qmv_mfma_kernel"),          # K slices; two passes of two rows
     (DType.BF16, 8, 64, 3, 3584, 18944, "qmv_mfma_kernel"),
