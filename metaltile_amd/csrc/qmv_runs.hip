@@ -3,7 +3,7 @@
 
 namespace mtq {
 
-// Steps of a wave's run, rounded up: K / 16 codes in steps of 128 (64 of 8-bit codes).
+// Steps of a sixteenth of a row, rounded up: K / 16 codes in steps of 128 (64 of 8-bit codes). (Where eight waves share a row, a run is two sixteenths.)
 static uint32_t runs_steps(int bits, uint32_t K) {
     const uint32_t per = 16u * (bits == 4 ? 128u : 64u);
     return (K + per - 1u) / per;
@@ -21,10 +21,10 @@ static bool runs_aligned(const void* w, const void* s, const void* b, const void
 }
 
 // (instances: qmv_runs_pick.h, one translation unit per element type)
-const void* qmv_runs_pick_f16(int bits, uint32_t G, bool sliced, uint32_t xs);
-const void* qmv_runs_pick_bf16(int bits, uint32_t G, bool sliced, uint32_t xs);
-static const void* runs_pick(int dtype, int bits, uint32_t G, bool sliced, uint32_t xs) {
-    return dtype == DT_BF16 ? qmv_runs_pick_bf16(bits, G, sliced, xs) : qmv_runs_pick_f16(bits, G, sliced, xs);
+RunsInstance qmv_runs_pick_f16(int bits, uint32_t G, bool sliced, uint32_t xs, bool few);
+RunsInstance qmv_runs_pick_bf16(int bits, uint32_t G, bool sliced, uint32_t xs, bool few);
+static RunsInstance runs_pick(int dtype, int bits, uint32_t G, bool sliced, uint32_t xs, uint32_t M) {
+    return dtype == DT_BF16 ? qmv_runs_pick_bf16(bits, G, sliced, xs, M <= 8) : qmv_runs_pick_f16(bits, G, sliced, xs, M <= 8);
 }
 
 bool qmv_runs_takes(const QmvParams& p, const QmvBatch& b) {
@@ -38,40 +38,45 @@ bool qmv_runs_takes(const QmvParams& p, const QmvBatch& b) {
 // the same bits), so a call of one matrix pays for what the projections of a layer gain in one call. The lines lie where two
 // matrices of a size together gain more than one alone loses. us, bf16, groups of 64, weights from memory, others -> this, one
 // matrix | two in a batch, 5, 9 and 16 rows:
-//   2048 x 2048     5.6  8.1  8.1 ->  5.3  5.5  6.1 | 11.4 16.0 16.1 ->  5.6  5.6  6.2
-//   4096 x 4096     7.9 10.0 10.0 ->  7.0  7.6  8.8 | 15.4 19.6 20.1 ->  9.9 10.4 11.7     8 bits 17.1 21.9 22.7 -> 12.7 13.2 14.5
-//   5120 x 5120    11.4 11.1 11.5 -> 11.3 12.1 13.8 | 22.7 22.1 22.8 -> 14.2 15.0 16.7     8 bits 33.1 28.1 29.1 -> 20.7 21.4 23.3
-//   16384 x 2048    8.8  9.2  9.3 -> 10.0 10.4 11.1 | 17.7 18.4 18.5 -> 14.3 14.7 15.4     8 bits 23.3 22.3 22.8 -> 19.2 19.3 20.0
-//   14336 x 4096   12.3 13.5 13.6 -> 13.8 14.4 15.8 | 24.8 26.9 27.1 -> 19.7 20.1 21.5     8 bits 37.8 36.9 37.5 -> 31.6 32.0 33.9
-//   13824 x 5120   16.3 16.0 16.6 -> 17.0 17.8 19.5 | 32.6 32.1 32.9 -> 25.6 26.3 28.3     (70.8 M codes; 16384 x 5120, 84 M, 16 rows 17.0 -> 19.9 | 34.1 -> 31.5;
-//   28672 x 4096, 117 M, 5 rows 19.3 -> 19.9 | 35.9 -> 34.4; 8 bits 16384 x 5120, 16 rows 24.3 -> 28.6 | 48.7 -> 48.9)
-//   7168 x 7168    13.9 14.8 15.0 -> 15.6 16.6 18.9 | 27.9 29.6 29.9 -> 23.6 24.5 27.0
-//   1024 x 8192     9.9  9.8 10.2 -> 10.2 11.4 13.8 | 19.6 19.7 20.7 -> 10.8 12.0 14.5
-//   2048 x 8192     9.4  9.4  9.5 -> 10.8 11.8 14.4 | 18.7 18.7 18.9 -> 11.7 12.7 15.3
-//   16384 x 512     7.9  5.8  5.8 ->  8.4  8.2  8.3 | 15.7 11.6 11.6 -> 12.2 12.3 12.4
+//   2048 x 2048     5.5  7.7  7.7 ->  4.9  5.0  5.2 | 11.0  8.2  8.2 ->  5.2  5.2  5.6     8 bits 14.8 10.4 10.6 ->  6.0  6.0  6.4
+//   4096 x 4096     7.8 10.1 10.0 ->  6.8  7.2  7.4 | 15.6 19.7 20.8 ->  9.0  9.5  9.4     8 bits 17.2 22.3 23.6 -> 13.2 13.2 13.4
+//   5120 x 5120    11.4 11.2 11.8 ->  9.8  9.7  9.7 | 22.9 22.3 23.6 -> 13.2 13.1 13.2     8 bits 33.3 28.6 30.2 -> 19.3 19.5 19.4
+//   16384 x 2048    8.9  9.7  9.9 ->  8.7  8.6  8.8 | 18.6 19.4 19.7 -> 13.0 13.0 13.4     8 bits 24.2 23.5 24.2 -> 17.8 17.9 18.3
+//   14336 x 4096   12.9 14.0 14.2 -> 13.6 13.6 14.1 | 25.1 27.8 28.0 -> 19.5 19.5 20.2     8 bits 39.1 37.7 38.5 -> 34.1 33.9 31.9
+//   13824 x 5120   16.5 16.5 17.0 -> 15.1 15.7 15.3 | 33.0 32.7 33.9 -> 23.5 24.1 24.1     (70.8 M codes)
+//   7168 x 7168    14.2 15.1 15.4 -> 13.7 13.5 14.1 | 28.0 30.3 30.8 -> 21.5 21.6 22.1
+//   8192 x 8192    15.0 16.8 17.1 -> 16.3 16.3 16.3 | 30.0 33.1 35.2 -> 25.4 25.3 25.6
+//   1024 x 8192     9.8  9.7 10.3 -> 10.3 10.3 10.3 | 11.1 11.0 11.8 -> 10.7 10.7 10.8
+//   2048 x 8192     9.4  9.4  9.5 -> 10.4 10.4 10.5 | 18.5 18.6 18.8 -> 12.3 12.3 12.4
+//   8192 x 1024     5.6  6.6  6.7 ->  6.0  6.0  6.0 | 11.3  7.3  7.4 ->  7.7  7.7  7.8     8 bits 12.6  8.5  8.8 ->  7.9  7.9  7.9
+//   16384 x 512     7.8  6.0  6.0 ->  7.4  7.5  7.5 | 15.7 11.9 12.0 -> 11.7 11.7 11.7     8 bits 15.6 12.5 12.7 -> 10.2 10.3 10.4
+//   16384 x 5120   17.8 18.0 18.3 -> 15.9 15.5 15.6 | 34.4 35.3 36.7 -> 26.4 26.1 26.8     8 bits 76.9 48.2 50.5 -> 42.1 42.5 43.0     (83.9 M)
+//   28672 x 4096   19.3 19.6 21.0 -> 19.7 20.4 20.7 | 37.3 38.4 41.9 -> 32.2 33.5 34.0     8 bits 63.2 66.5 69.7 -> 58.8 59.0 59.7     (117 M)
 // and 2, 3 and 4 rows:
-//   512 x 3584      5.9  7.1  7.6 ->  5.9  6.0  6.1 | 11.7 14.2 15.2 ->  6.1  6.1  6.3
-//   1024 x 4096     5.9  7.2  8.2 ->  6.2  6.3  6.5 | 12.2 14.7 16.8 ->  6.4  6.6  6.9     8 bits 12.7 14.9 16.8 -> 7.8 8.2 8.4
-//   768 x 3072      5.3  6.5  7.1 ->  5.9  6.0  6.1 | 10.7 13.2 14.2 ->  6.1  6.2  6.3     8 bits 4.4 5.1 5.6 -> 6.7 6.9 7.0 | 8.7 10.1 11.1 -> 6.9 7.1 7.3
-//   1280 x 5120     5.1  5.5  5.7 ->  7.5  7.7  8.0 | 10.0 10.9 11.1 ->  7.7  7.9  8.0
-//   512 x 8192      6.3  7.6  8.8 ->  9.5  9.9 10.3 | 13.0 15.5 17.9 ->  9.8 10.2 10.6
-//   4096 x 1024     3.6  3.8  3.8 ->  5.3  5.3  5.4 |  7.1  7.4  7.4 ->  6.4  6.4  6.5
-// 2 to 4 rows on more than 16384 weight rows: the GEMV's 256 workgroups of sixteen waves hold four rows a wave at once, past that
-// every one walks a second block of them (bf16, 2 | 3 | 4 rows alone, then a pair at 4 rows; groups of 64):
-//   16384 x 3584    9.7 | 10.0 | 10.0 -> 13.3 | 13.4 | 13.4, 20.0 -> 19.4        8 bits 14.8 | 15.5 | 15.9 -> 16.7 | 16.7 | 16.7, 32.0 -> 28.7
-//   16512 x 3584   13.5 | 13.9 | 13.9 -> 14.0 | 14.1 | 14.0, 27.9 -> 20.3        8 bits 17.9 | 18.8 | 19.1 -> 19.2 | 19.1 | 19.2, 38.0 -> 31.1
-//   18944 x 3584   13.7 | 14.1 | 14.0 -> 14.5 | 14.6 | 14.4, 28.2 -> 23.0        8 bits 18.4 | 19.2 | 19.6 -> 19.9 | 20.0 | 20.0, 39.2 -> 34.1
-//   16512 x 2048    9.6 | 10.2 | 10.3 -> 10.3 | 10.3 | 10.5, 20.5 -> 15.0        8 bits 13.5 | 14.2 | 14.2 -> 12.7 | 12.7 | 12.6, 28.5 -> 18.7
-//   24576 x 3072   13.9 | 14.4 | 14.4 -> 14.7 | 14.8 | 14.8, 28.8 -> 24.0        8 bits 17.7 | 19.8 | 19.9 -> 20.7 | 21.0 | 20.8, 39.9 -> 37.3
-//   28672 x 2560   13.8 | 14.3 | 14.3 -> 16.3 | 16.4 | 16.4, 28.4 -> 26.3 (seven blocks of 4096 rows each on a workgroup: past six, no)
-//   16512 x 4096   15.0 | 15.2 | 15.0 -> 14.5 | 14.7 | 14.6, 30.4 -> 21.3        8 bits 20.2 | 21.0 | 21.2 -> 23.4 | 22.7 | 23.2, 42.5 -> 38.4
-// Not in groups of 32, whose scales weigh more here (18944 x 3584, 4 rows 13.7 -> 16.9 | 27.5 -> 27.9), and not with 8 bits at 2 rows
-// (24576 x 3072 17.7 -> 20.7 | a pair 35.3 -> 37.4). Fewer weight rows lose more alone than they are sure to gain: 4096 x 4096, 4 rows
-// 6.0 -> 7.3 | 12.0 -> 9.3, 8192 x 4096 7.4 -> 9.2 | 14.9 -> 14.2; 5120 x 5120, 3 rows 8.5 -> 9.7 | 17.1 -> 13.1.
-// So: below 5 rows the gate and up projections of more than 16384 (to 24576) rows of 2048 to 4096 codes, and short matrices against such rows (the
-// K and V projections of grouped-query attention), both with 8-bit codes from 3 rows; from 5 rows up to 75 M codes (60 M of 8 bits), and from 9 rows, where the others take tiles, no more than
-// 1024 weight rows of more than 6144 codes (four steps a run, whose registers leave one block in flight) and no more than 8192 of
-// fewer than 2048 (some of the sixteen waves have no step, and a workgroup has more than two blocks to walk).
+//   512 x 2048      3.9  4.6  5.2 ->  4.7  4.7  4.8 |  7.9  9.3 10.3 ->  4.9  4.9  5.0     8 bits 10.9 12.8 14.5 ->  5.5  5.5  5.6
+//   512 x 3584      5.7  7.0  7.5 ->  6.1  6.2  6.2 | 11.6 14.0 15.0 ->  6.4  6.4  6.5     8 bits 12.1 14.2 15.3 ->  6.7  6.7  6.7
+//   1024 x 4096     5.9  7.1  8.1 ->  6.3  6.3  6.4 | 11.8 14.1 16.3 ->  6.6  6.6  6.6     8 bits 12.6 14.7 16.6 ->  7.2  7.1  7.1
+//   768 x 3072      5.2  6.5  7.0 ->  6.2  6.2  6.3 | 10.4 13.0 13.9 ->  6.4  6.5  6.5     8 bits  4.3  5.0  5.5 ->  6.5  6.5  6.5 | 8.7 10.0 11.0 -> 6.8 6.8 6.8
+//   1280 x 5120     5.0  5.4  5.5 ->  7.3  7.4  7.4 |  9.9 10.8 11.1 ->  7.7  7.8  7.8
+//   512 x 8192      6.2  7.5  8.6 ->  9.8  9.9  9.9 | 12.5 15.0 17.2 -> 10.1 10.1 10.2
+//   4096 x 1024     3.5  3.6  3.7 ->  4.9  4.9  4.9 |  7.0  7.3  7.3 ->  5.7  5.8  5.8
+//   4096 x 4096     5.2  5.9  6.0 ->  6.7  6.8  6.9 | 10.3 11.7 12.0 ->  8.9  9.0  9.0     8 bits 14.0 14.9 15.5 -> 13.2 13.2 13.3
+//   8192 x 4096     6.8  7.3  7.4 ->  8.9  8.9  8.9 | 13.6 14.5 14.8 -> 14.2 14.2 14.3     8 bits 19.6 20.5 21.2 -> 21.7 21.8 22.2
+//   5120 x 5120     8.2  8.5  8.9 ->  9.7  9.8  9.8 | 16.4 17.0 17.9 -> 13.1 13.4 14.5     8 bits 20.4 21.9 22.9 -> 19.4 19.4 19.5
+// and on more than 16384 weight rows, where the GEMV's 256 workgroups of sixteen waves, four rows a wave at once, come to a second block:
+//   16384 x 3584   10.0 10.5 11.0 -> 13.3 13.3 13.4 | 19.9 20.5 20.5 -> 19.3 19.3 19.4     8 bits 34.5 32.8 33.3 -> 29.2 29.3 29.1
+//   16512 x 3584   13.5 14.0 14.0 -> 13.8 13.9 13.8 | 27.3 28.0 28.1 -> 20.0 20.3 20.1     8 bits 36.1 37.0 38.2 -> 31.4 31.0 31.2
+//   18944 x 3584   13.8 14.2 14.1 -> 14.2 14.3 14.4 | 27.7 28.4 28.5 -> 22.7 22.8 23.0     8 bits 36.9 38.5 39.9 -> 34.0 34.0 34.1
+//   16512 x 2048    9.6 10.2 10.2 -> 10.0 10.1 10.3 | 19.3 20.4 20.4 -> 14.2 14.5 14.7     8 bits 27.0 28.5 28.5 -> 18.2 18.4 18.2
+//   16512 x 4096   15.0 15.2 15.2 -> 14.6 14.4 14.6 | 30.3 30.4 30.6 -> 21.2 21.1 21.3     8 bits 20.1 21.1 21.5 -> 22.9 23.5 23.1 | 40.2 41.9 42.9 -> 37.8 38.5 37.2
+//   24576 x 3072   14.2 14.5 14.5 -> 14.6 14.7 14.9 | 28.1 28.9 29.1 -> 24.1 24.1 24.0     8 bits 35.3 39.5 39.9 -> 37.1 37.6 37.7     (75.5 M)
+//   28672 x 2560   13.9 14.7 14.4 -> 16.1 16.3 16.2 | 27.8 28.6 29.7 -> 26.1 26.4 26.7     (seven blocks of 4096 rows each on a workgroup)
+//   18944 x 3584 in groups of 32, whose scales weigh more here 13.3 13.8 13.7 -> 16.8 16.9 17.0 | 26.6 27.7 27.4 -> 27.7 27.9 27.8
+// So: below 5 rows the gate and up projections of 16385 to 24576 rows of 2048 to 4096 codes in groups of 64 and 128, and short matrices
+// against such rows (the K and V projections of grouped-query attention), both with 8-bit codes from 3 rows; from 5 rows up to 75 M codes
+// (60 M of 8 bits), and from 9 rows, where the others take tiles, no more than 8192 rows of fewer than 2048 codes, and no more than 1024
+// of more than 6144. The last two lines and the 75 M are those of an earlier form of the kernel, with sixteen waves on every row length: past
+// them this one has become the faster (7168 x 7168, 16384 x 5120, 8 bits 16384 x 512), but those calls would no longer have the tiles' bits.
 bool qmv_runs_preferred(int bits, uint32_t G, uint32_t M, uint32_t N, uint32_t K) {
     if (M < 2 || M > 16) return false;
     const uint64_t codes = (uint64_t)N * K;
@@ -130,9 +135,9 @@ int launch_qmv_runs(const QmvParams& p, const QmvBatch& b, const LaunchCtx& lc) 
     a.K = p.K;
     a.slices = 1;
     const uint32_t cus = runs_cus(), wgs = a.blocks < cus ? a.blocks : cus, xs = runs_steps(p.bits, p.K);
-    const void* fn = runs_pick(p.dtype, p.bits, p.group_size, false, xs);
+    const RunsInstance k = runs_pick(p.dtype, p.bits, p.group_size, false, xs, p.M);
     void* args[] = {&a};
-    hipError_t e = launch_kernel(fn, dim3(wgs), dim3(p.bits == 4 && (xs <= 1 || xs == 4) ? 512 : 1024), args, 0, lc);
+    hipError_t e = launch_kernel(k.fn, dim3(wgs), dim3(k.threads), args, 0, lc);
     if (e != hipSuccess) return hip_fail(e, "K-run qmv kernel launch");
     return ERR_OK;
 }
@@ -171,7 +176,8 @@ int launch_qmv_slices(const QmmParams& p, const LaunchCtx& lc, void* scratch) {
     LaunchCtx l1 = lc, l2 = lc;
     l1.stop = nullptr;
     l2.start = nullptr;
-    hipError_t e = launch_kernel(runs_pick(p.dtype, p.bits, p.group_size, true, 0), dim3(wgs), dim3(512), args, 0, l1);
+    const RunsInstance k = runs_pick(p.dtype, p.bits, p.group_size, true, 0, p.M);
+    hipError_t e = launch_kernel(k.fn, dim3(wgs), dim3(k.threads), args, 0, l1);
     if (e != hipSuccess) return hip_fail(e, "K-sliced qmv kernel launch");
     return add_slices(p.dtype, (const float*)scratch, p.out, p.M * p.N, a.slices, l2);
 }

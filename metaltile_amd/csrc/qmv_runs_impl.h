@@ -49,6 +49,12 @@ struct QmvRunsArgs {
     float* part[4];          // and its f32 sums [slice][M][N]
 };
 
+// An instance and the threads of its workgroups (qmv_runs_pick.h).
+struct RunsInstance {
+    const void* fn;
+    uint32_t threads;
+};
+
 typedef uint32_t kr_u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t kr_u32x2 __attribute__((ext_vector_type(2)));
 typedef float kr_f32x4 __attribute__((ext_vector_type(4)));
@@ -137,7 +143,7 @@ template <int DT, int BITS> __device__ __forceinline__ kr_u32x4 kr_weights(const
 
 // DT, BITS (4 or 8), G (32, 64, 128), XS: steps of a wave's run at most, PF: blocks whose
 // weights are in flight ahead of the one that is worked on.
-template <int KP, bool SLICED, int DT, int BITS, int G, int XS, int PF> __device__ __forceinline__ void qmv_runs_body(const QmvRunsArgs& a) {
+template <int KP, bool SLICED, bool ORDERED, int DT, int BITS, int G, int XS, int PF> __device__ __forceinline__ void qmv_runs_body(const QmvRunsArgs& a) {
     using C = KrCodes<DT, BITS>;
     constexpr int EG = G < C::STEP ? G : C::STEP;   // codes per scale within a step
     constexpr int GPS = C::STEP / EG;               // scales per step: 1, 2 or 4
@@ -246,7 +252,10 @@ template <int KP, bool SLICED, int DT, int BITS, int G, int XS, int PF> __device
 #pragma unroll
             for (int k = 0; k < C::UNITS; k++) xop[n][k] = __builtin_amdgcn_raw_buffer_load_b128(xr, (int)((xo + (uint32_t)(n * C::STEP * 2 + k * 64)) | step_dead[n]), 0, 0);
         __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_barrier();   // no wave's weights ahead of another's activations
+        // No wave's weights ahead of another's activations. Not where a run is short, as the wait for the last of the waves to start
+        // costs more there (us, with -> without): 8 bits, 5 rows 4096 x 2048 6.5 -> 5.9; 4 bits 11008 x 2048 7.8 -> 7.4, groups of 32
+        // 1024 x 2048 5.9 -> 5.4; two steps, 3584 x 3584, 5 rows 7.1 -> 6.8, but 11008 x 4096, 16 rows 11.4 -> 11.9.
+        if constexpr (ORDERED) __builtin_amdgcn_s_barrier();
         kr_for<0, PF>([&](auto p) { load_block(ring[decltype(p)::value], wg + wgs * (uint32_t)decltype(p)::value); });
         __builtin_amdgcn_sched_barrier(0);
         uint32_t from[C::UNITS];
@@ -418,12 +427,12 @@ template <int KP, bool SLICED, int DT, int BITS, int G, int XS, int PF> __device
 }
 
 // XS: steps of a sixteenth of K at most.
-template <int KP, int DT, int BITS, int G, int XS, int PF> __global__ __launch_bounds__(KP * 64) void qmv_runs_kernel(QmvRunsArgs a) {
-    qmv_runs_body<KP, false, DT, BITS, G, XS * 16 / KP, PF>(a);
+template <bool ORDERED, int KP, int DT, int BITS, int G, int XS, int PF> __global__ __launch_bounds__(KP * 64) void qmv_runs_kernel(QmvRunsArgs a) {
+    qmv_runs_body<KP, false, ORDERED, DT, BITS, G, XS * 16 / KP, PF>(a);
 }
 // On one of a.slices slices of K, whose sums a second launch adds; XS: steps of an eighth of a slice at most.
 template <int DT, int BITS, int G, int XS, int PF> __global__ __launch_bounds__(512) void qmv_slices_kernel(QmvRunsArgs a) {
-    qmv_runs_body<8, true, DT, BITS, G, XS, PF>(a);
+    qmv_runs_body<8, true, true, DT, BITS, G, XS, PF>(a);
 }
 
 }  // namespace mtq

@@ -55,6 +55,8 @@ def test_edges(oracle, dt, bits, G, M, K, Ns):
     (DType.F16, 4, 128, 9, 2176, (9001, 7600), "2, 2"), (DType.BF16, 8, 64, 16, 1152, (9001, 8000), "2, 2"),
     (DType.BF16, 4, 64, 5, 5120, (7001, 6000), "3, 1"), (DType.F16, 4, 32, 16, 6272, (7001, 5400), "4, 1"),
     (DType.BF16, 8, 128, 7, 3072, (7001, 6000), "4, 1"), (DType.F16, 8, 32, 3, 4224, (12401,), "5, 1"),
+    (DType.BF16, 8, 64, 16, 1024, (14000, 9001), "1, 3"), (DType.F16, 8, 32, 2, 384, (24601,), "1, 3"), (DType.BF16, 8, 128, 5, 640, (24601,), "1, 3"),
+    (DType.BF16, 4, 64, 8, 4096, (9001, 7600), "2, 2"), (DType.F16, 4, 32, 3, 2176, (16601,), "2, 2"),   # up to 8 rows: no order between the waves' loads
 ])
 def test_many_blocks_per_workgroup(oracle, dt, bits, G, M, K, Ns, instance):
     """The walk: with PF blocks in flight ahead, every workgroup of the 256 has PF + 2 blocks of 16 weight rows or more, so
