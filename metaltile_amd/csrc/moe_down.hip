@@ -181,13 +181,14 @@ int launch_moe_down_swiglu(int dtype, uint32_t group_size, uint32_t n_slots, con
     a.log2g = lg;
     a.n_experts = n_experts;
     a.n_slots = n_slots;
-    // about one workgroup per CU: the SwiGLU staging is repeated by every workgroup
+    // One workgroup per CU, an even share of the rows each: the SwiGLU staging is repeated by every workgroup. us, bf16, shares rounded up
+    // to eight rows -> these: 8 slots of 768 codes, 1024 / 2176 / 3072 rows 7.8 / 11.4 / 11.5 -> 7.4 / 10.2 / 10.8, 1 of 768, 2176 rows 6.4 -> 6.1
     int dev = 0, n_cu = 0;
     if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n_cu <= 0)
         n_cu = 256;
     const uint32_t cus = (uint32_t)n_cu;
     uint32_t rpw = (out_dim + cus - 1) / cus;
-    rpw = (rpw + DOWN_WAVES - 1) / DOWN_WAVES * DOWN_WAVES;
+    if (options().moe_down_rows) rpw = (uint32_t)options().moe_down_rows;
     a.rows_per_wg = rpw;
     const size_t shmem = (size_t)n_slots * in_dim * sizeof(float);
     const void* fn;

@@ -10,7 +10,7 @@ slot weights) with its metric and bounds: max |a-e| / max(|e|, 1e-3) <= 1e-3 (f3
 import numpy as np
 import pytest
 
-from metaltile_amd import DType, GpuBuffer, MtqError, ops, pack_f32, unpack_f32
+from metaltile_amd import DType, GpuBuffer, MtqError, _lib, ops, pack_f32, unpack_f32
 from tests.parity import rel_err
 from tests.test_gpu_batched import _quantize_int4, _ref_err, _source
 
@@ -105,6 +105,30 @@ def test_more_items_than_one_set_and_more_rows_than_waves(oracle, slots, K, N, G
     assert np.isfinite(got).all()
     assert rel_err(got, exp) <= 1e-2
     for buf in gb + ub + bufs + [out]:
+        buf.free()
+
+
+def test_rows_per_workgroup():
+    """"moe_down.rows" asks for a number of rows per workgroup; a row's sums do not depend on it."""
+    print("[case] moe_down_swiglu rows per workgroup", flush=True)
+    lib = _lib.load()
+    dt, slots, K, N, G, E = DType.BF16, 3, 288, 1100, 32, 4
+    rng = np.random.default_rng(17)
+    acts = [GpuBuffer.from_bytes(pack_f32(rng.standard_normal(K).astype(np.float32), dt)) for _ in range(2 * slots)]
+    w, s, b = _quantize_int4(((rng.random(E * N * K, dtype=np.float32) - 0.5) * 0.5).astype(np.float32), E * N, K, G)
+    bufs = [GpuBuffer.from_bytes(v) for v in (np.array([2, 0, 3], dtype="<u4").tobytes(), pack_f32(np.array([0.5, 0.3, 0.2], np.float32), dt), w.tobytes(), pack_f32(s, dt), pack_f32(b, dt))]
+    got = []
+    try:
+        for rows in (0, 1, 9, 4096):
+            assert lib.mtq_set_option(b"moe_down.rows", rows) == 0
+            out = GpuBuffer.from_bytes(b"\xff" * (N * 2 + 64))
+            ops.moe_down_swiglu_accum(dt, G, acts[:slots], acts[slots:], *bufs, out, K, N, E)
+            got.append(out.read_bytes())
+            out.free()
+    finally:
+        lib.mtq_set_option(b"moe_down.rows", 0)
+    assert all(g == got[0] for g in got) and got[0][N * 2:] == b"\xff" * 64 and np.any(unpack_f32(got[0][:N * 2], dt) != 0.0)
+    for buf in acts + bufs:
         buf.free()
 
 
