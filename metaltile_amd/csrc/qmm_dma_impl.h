@@ -546,20 +546,24 @@ __global__ __launch_bounds__(64 * NW) void qmm_dma_kernel(QmmDArgs args) {
 // pieces, so that 128 rows or a few more are one tile and each weight is converted once for them (64-row tiles: two or three
 // times, the last one nearly empty). 160 rows are what three buffers and the scales leave room for in LDS. us, the whole gather with
 // its table, bf16, 64-row tiles -> these: 128 experts of 768 x 2048, 128 rows each 108 -> 95 (8-bit codes 173 -> 120), of 2048 x 768
-// 133 -> 117; 8 experts of 14336 x 4096, 512 rows each 666 -> 603, of 4096 x 14336, 64 / 128 rows each 172 / 261 -> 118 / 165.
+// 133 -> 117; 8 experts of 14336 x 4096, 512 rows each 666 -> 603, of 4096 x 14336, 64 / 128 rows each 172 / 261 -> 118 / 165 (with
+// skewed routing: qmm_direct.hip, grouped_tile_rows).
 // What is left is the start and end of each tile (about 7 us of 22 at 2048 codes): one workgroup fills a compute unit's registers.
-// (Named by the parameters of the 64-row tiles that it takes the place of.)
-namespace tall {
-template <int DT, int MB, int KG, int NW, int NB, bool GR, bool SP, bool WIN, int BITS> __global__ __launch_bounds__(64 * NW) void qmm_dma_kernel(QmmDArgs args) {
-    static_assert(MB == 2 && GR && !SP, "expert-routed rows, 64 rows and more");
+template <int DT, bool WIN, int BITS> __global__ __launch_bounds__(512) void qmm_dma_routed_kernel(QmmDArgs args) {
     uint4 t;
     uint32_t nt;
     if (!qd_routed_tile(args.tiles, args.m_tiles, args.n_tiles, t, nt)) return;
-    if (t.z <= 64) qmm_dma_tile<DT, 2, KG, NW, 0, true, false, WIN, BITS>(args, t, nt);
-    else if (t.z <= 96) qmm_dma_tile<DT, 3, KG, NW, 0, true, false, WIN, BITS>(args, t, nt);
-    else if (t.z <= 128) qmm_dma_tile<DT, 4, KG, NW, 0, true, false, WIN, BITS>(args, t, nt);
-    else qmm_dma_tile<DT, 5, KG, NW, 0, true, false, WIN, BITS>(args, t, nt);
+    if (t.z <= 64) qmm_dma_tile<DT, 2, 2, 8, 0, true, false, WIN, BITS>(args, t, nt);
+    else if (t.z <= 96) qmm_dma_tile<DT, 3, 2, 8, 0, true, false, WIN, BITS>(args, t, nt);
+    else if (t.z <= 128) qmm_dma_tile<DT, 4, 2, 8, 0, true, false, WIN, BITS>(args, t, nt);
+    else qmm_dma_tile<DT, 5, 2, 8, 0, true, false, WIN, BITS>(args, t, nt);
 }
-}  // namespace tall
+
+// Its instances for one code width (a translation unit each, so that they compile beside each other).
+template <int BITS> static const void* qmm_dma_routed_instance(int dtype, bool windowed) {
+    if (dtype == DT_BF16) return windowed ? (const void*)qmm_dma_routed_kernel<DT_BF16, true, BITS> : (const void*)qmm_dma_routed_kernel<DT_BF16, false, BITS>;
+    if (dtype == DT_F16) return windowed ? (const void*)qmm_dma_routed_kernel<DT_F16, true, BITS> : (const void*)qmm_dma_routed_kernel<DT_F16, false, BITS>;
+    return nullptr;
+}
 
 }  // namespace mtq

@@ -5,12 +5,6 @@
 
 namespace mtq {
 
-template <int BITS> static const void* routed_t(int dtype, bool windowed) {
-    if (dtype == DT_BF16) return windowed ? (const void*)tall::qmm_dma_kernel<DT_BF16, 2, 2, 8, 2, true, false, true, BITS> : (const void*)tall::qmm_dma_kernel<DT_BF16, 2, 2, 8, 2, true, false, false, BITS>;
-    if (dtype == DT_F16) return windowed ? (const void*)tall::qmm_dma_kernel<DT_F16, 2, 2, 8, 2, true, false, true, BITS> : (const void*)tall::qmm_dma_kernel<DT_F16, 2, 2, 8, 2, true, false, false, BITS>;
-    return nullptr;
-}
-
 size_t qmm_dma_routed_lds_bytes(uint32_t gpr, bool windowed) {
     const size_t sb = windowed ? 32768 : (size_t)2 * 128 * (((gpr + 3) & ~3u) + 2) * 2;
     return (size_t)3 * QD_ROUTED_ROWS * 2 * 128 + sb;   // (the epilogue's 120 KB fit the ring of three)
@@ -19,7 +13,7 @@ size_t qmm_dma_routed_lds_bytes(uint32_t gpr, bool windowed) {
 const void* qmm_dma_routed_pick_b8(int dtype, bool windowed);
 const void* qmm_dma_routed_pick(int bits, int dtype, bool windowed) {
     if (bits == 8) return qmm_dma_routed_pick_b8(dtype, windowed);
-    return routed_t<4>(dtype, windowed);
+    return qmm_dma_routed_instance<4>(dtype, windowed);
 }
 
 }  // namespace mtq

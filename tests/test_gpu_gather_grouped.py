@@ -302,7 +302,7 @@ def test_grouped_gather_on_tall_row_tiles(oracle, dt, bits, N, K, G, counts):
                 print(f"[case] tall row tiles {view} {dt.name} b{bits} N={N} K={K} {counts} rows={rows}", flush=True)
                 assert lib.mtq_set_option(b"qmm.tile_rows", rows) == 0
                 kernel = ops.plan(f"gather_{view}", dt, bits, G, 1, N, K, E, T)[1][-1][0]
-                assert ("tall::" in kernel) == (rows == 160), kernel
+                assert ("qmm_dma_routed_kernel" in kernel) == (rows == 160), kernel
                 out = GpuBuffer.from_bytes(np.full(T * N + 1024, 0x7B7B, np.uint16).tobytes())
                 fn(dt, bits, G, x, w, s, b, r, out, T, N, K, E)
                 got.append(np.frombuffer(out.read_bytes(), np.uint16))

@@ -212,7 +212,7 @@ def test_benchmark_configurations_are_routed_as_documented():
         ks, ls = kernels(view, DType.BF16, 4, 64, 1, 2048, 768, 128, 33)   # (more than 32 rows: a grid row per expert)
         assert ls[0][1][1] == 128
     ks, _ = kernels("gather_indices", DType.BF16, 4, 64, 1, 4096, 4096, 8, 2048)
-    assert "moe_count_sort_kernel" in ks[0] and "gather_tiles_kernel" in ks[1] and "qmm_dma_kernel<2, 2, 2, 8, 2, true" in ks[2]
+    assert "moe_count_sort_kernel" in ks[0] and "gather_tiles_kernel<true>" in ks[1] and "qmm_dma_routed_kernel<2, false, 4>" in ks[2]
     for bits, M in itertools.product((2, 4, 8), (1, 4)):   # the sweep configuration's cells
         for G in (32, 64, 128):
             ks, _ = kernels("qmv", DType.F16, bits, G, M, 8192, 8192)
@@ -293,7 +293,7 @@ def test_products_without_scratch_memory(dt, bits, G, M, N, K, first):
 def test_tall_routed_lines(bits, E, N, K, per, tall):
     """Where expert-routed rows run on tiles of up to 160 rows, on both sides of each line; the scratch holds their four tables."""
     rc, launches, scratch, _ = ops.plan("gather_csr", DType.BF16, bits, 32 if K % 64 else 64, 1, N, K, E, per * E)
-    assert rc == OK and ("tall::" in launches[-1][0]) == tall, launches
+    assert rc == OK and ("qmm_dma_routed_kernel" in launches[-1][0]) == tall, launches
     rows = 160 if tall else 64
     if bits != 6:
         assert scratch == 16 + (-(-per * E // rows) + E + 1) * 16 * (4 if tall else 1)

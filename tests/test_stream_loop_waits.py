@@ -217,7 +217,7 @@ def test_tall_routed_kernels_wait_only_where_written():
         outs = [_assembly(s, os.path.join(tmp, s + ".s")) for s in ("qmm_dma_routed.hip", "qmm_dma_routed_b8.hip")]
     n = 0
     for lines in outs:
-        starts = [(i, l.split(":")[0]) for i, l in enumerate(lines) if "14qmm_dma_kernel" in l and l.startswith("_ZN3mtq4tall") and "; @" in l]
+        starts = [(i, l.split(":")[0]) for i, l in enumerate(lines) if l.startswith("_ZN3mtq21qmm_dma_routed_kernel") and "; @" in l]
         starts.append((len(lines), ""))
         for (s0, name), (s1, _) in zip(starts, starts[1:]):
             body = lines[s0:s1]
