@@ -295,9 +295,14 @@ static bool runs_barred() {
 }
 
 // A batch on long rows, on the K-run kernel in slices of K.
+static bool tiles_serve(int bits, uint32_t M, uint32_t N, uint32_t K);
 static bool slices_serve(const QmmParams& q) {
     if (runs_barred() || options().qmv_runs == 2 || !qmv_slices_takes(q)) return false;
-    return options().qmv_runs == 3 || qmv_slices_preferred(q.bits, q.group_size, q.M, q.N, q.K);
+    if (options().qmv_runs == 3) return true;
+    if (!qmv_slices_preferred(q.bits, q.group_size, q.M, q.N, q.K)) return false;
+    // 8-bit rows of which the tiles split K, on load-to-LDS instructions, are as well off there (the figures stand at the rule)
+    QmmDLaunch l;
+    return q.bits != 8 || q.K % 256 || !tiles_serve(q.bits, q.M, q.N, q.K) || plan_qmm_direct(q, l) != ERR_OK || !l.dma;
 }
 static int try_slices(int dtype, int bits, uint32_t G, const void* w, const void* s, const void* b, const void* x, void* out,
                       uint32_t M, uint32_t N, uint32_t K, const LaunchCtx& lc) {

@@ -200,6 +200,7 @@ template <int DT> static int choose_dt(int bits, uint32_t kgroups, QmmDLaunch& l
     l.grid = grouped ? (a.m_tiles * a.n_tiles + 7) & ~7u : a.m_tiles * a.n_tiles;   // (expert-routed rows: eight even shares)
     l.block = kgroups == 1 ? 256 : 512;
     l.split = a.ksplit > 1 && !grouped;
+    l.dma = true;
     const void* fn = nullptr;
     // 8-bit codes on short rows gain nothing where the launch leaves compute units idle (14336 x 4096, 128 rows:
     // 36.3 against 34.3 us) or on the 4-K-group tiles (4096 x 4096, 16 / 64 rows 11.6 / 15.3 against 10.9 / 14.6;
@@ -234,6 +235,7 @@ template <int DT> static int choose_dt(int bits, uint32_t kgroups, QmmDLaunch& l
         l.shmem = qmm_dma4_lds_bytes(a.m_tile_rows, a.gpr);
         return ERR_OK;
     }
+    l.dma = false;
     if (a.m_tile_rows == 256) return fail(ERR_UNSUPPORTED, "direct qmm: 256-row tiles need 4- or 8-bit codes, K % 128 == 0 and rows whose scales fit LDS (or, 4-bit codes, groups of 64 or 128 codes)");
     const bool tall = a.m_tile_rows == 128;
     const uint32_t dbn = kgroups == 1 ? 128 : 32 * (8 / kgroups);

@@ -55,6 +55,7 @@ struct QmmDLaunch {
     uint32_t cus = 256;             // compute units of the device
     size_t shmem = 0;
     bool split = false;
+    bool dma = false;               // activations by load-to-LDS instructions
     size_t scratch = 0;             // bytes of f32 partial tiles (0 when K is not split), a multiple of 256
     QmmDArgs a;
 };

@@ -100,7 +100,9 @@ bool qmv_runs_preferred(int bits, uint32_t G, uint32_t M, uint32_t N, uint32_t K
 //     24.4 / 24.8 -> 17.8 / 18.0; 4096 x 11008, 5 / 16 rows 18.1 / 19.0 -> 17.8 / 17.9; but 2048 x 8960 in groups of 128 10.9 -> 11.4, and
 //     up to 8 rows, where the 16-row kernel takes it, 5120 x 13824 15.6 -> 17.9
 //   8 bits, 5..8 rows on less than twice as many codes as weight rows (two passes of the GEMV): 8192 x 10240 36.2 -> 24.9; and from
-//     230 M codes: 8192 x 28672, 16 rows 96.8 -> 64.5 (16384 x 12288, 201 M: 51.9 -> 55.0)
+//     230 M codes where the tiles are register-staged (their scales do not fit LDS): 8192 x 28672, 5 / 16 rows 97.1 / 99.0 -> 66.4 /
+//     69.6, groups of 32 6144 x 40960 138 / 140 -> 73 / 75; load-to-LDS tiles: groups of 128 8192 x 28672, 16 rows 56.5 -> 68.0, 16384 x
+//     14336 54.9 -> 66.9, 14336 x 16384 59.6 -> 65.3 (but 10240 x 24576 84.6 -> 70.4: not there either). 16384 x 12288, 201 M: 51.9 -> 55.0
 bool qmv_slices_preferred(int bits, uint32_t G, uint32_t M, uint32_t N, uint32_t K) {
     if (M < 3 || M > 16 || K <= 8192) return false;
     if (M <= 4) return K > 18432;

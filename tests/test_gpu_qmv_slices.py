@@ -50,6 +50,8 @@ def test_slices(oracle, dt, bits, G, M, K, N):
     (8, 64, 4, 3584, 18944, True), (4, 64, 3, 1024, 18688, True), (4, 64, 4, 4096, 18432, False), (4, 64, 2, 3584, 18944, False),
     (4, 128, 16, 5120, 13824, True), (4, 128, 8, 5120, 13824, False), (4, 64, 16, 5120, 13824, False), (4, 128, 16, 2048, 8960, False),
     (4, 128, 5, 2048, 9344, True), (4, 64, 17, 4096, 9344, False), (8, 64, 8, 8192, 10240, True), (8, 64, 9, 8192, 10240, False), (8, 64, 16, 8192, 28672, True),
+    (8, 128, 16, 8192, 28672, False), (8, 64, 9, 16384, 14336, False), (8, 64, 8, 16384, 14336, True), (8, 32, 5, 28672, 8448, False), (8, 32, 16, 6144, 40960, True),
+    (8, 128, 16, 4096, 9344, True),
 ])
 def test_lines(bits, G, M, N, K, slices):
     """Which matrices the K-sliced form is for, on both sides of each line."""
