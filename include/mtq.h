@@ -120,20 +120,28 @@ MTQ_API int mtq_qmv(int dtype, int bits, uint32_t group_size, const void *w, con
                     uint32_t K);
 
 /* qmm: same product for any M; routes by M like mt_qmm_for
- * (crates/metaltile-std/src/mlx/quantized.rs:5040-5065). 5 to 16 rows on a 4- or 8-bit f16 /
- * bf16 matrix of up to 75 M codes (60 M of 8 bits), K % 128 == 0, K <= 8192 (5120 of 8 bits;
- * from 9 rows with K > 6144 only N <= 1024, with K < 2048 only N <= 8192), and 2 to 4 rows on
- * short ones (2048 <= K <= 4096, 2 N <= K, 4.5 M codes; 8 bits from 3 rows) run on the K-run
- * kernel: exact w_hat; an activation that takes its sums past the f32 range is multiplied with
- * w_hat rounded to the element type. 5 to 8 rows on a 4-bit matrix of 50 M codes or more, 9 to
- * 16 on one of 100 M, run on the 16-row kernel (exact w_hat). Else from 9 rows (from 5 where
- * the rows are long) the MFMA tile kernel (replaces mt_qmm_mma / _m16 / _int8 / _int2 / _b3 /
- * _b5 / _b6, quantized.rs:2106, 2408, 2731, 3330, 3560-3900; w_hat rounded to the element
- * type before the multiply, as there), below that the qmv family (exact w_hat). A matrix takes
- * the same kernel here and in mtq_qmm_batched, whose launch the K-run kernel shares: a single
- * call is up to 4 us slower for it than it could be (8192 x 8192, 8 rows 15.5 -> 17.9 us, a
- * pair 30.7 -> 26.3). MTQ_F32 batches run on the f32 matrix cores from 5 rows. Short, wide
- * matrices split K over workgroups through a library-owned buffer (allocated on first use). */
+ * (crates/metaltile-std/src/mlx/quantized.rs:5040-5065). On 4- and 8-bit f16 / bf16 matrices
+ * the K-run kernel takes, with exact w_hat (an activation that takes its sums past the f32 range
+ * is multiplied with w_hat rounded to the element type):
+ *   5 to 16 rows on up to 75 M codes (60 M of 8 bits), K % 128 == 0, K <= 8192 (5120 of 8 bits;
+ *     from 9 rows with K > 6144 only N <= 1024, with K < 2048 only N <= 8192);
+ *   2 to 4 rows (8 bits: 3 and 4), 2048 <= K <= 4096, on short matrices (2 N <= K, 4.5 M codes)
+ *     and, in groups of 64 or 128, on tall ones (16384 < N <= 24576, 75 M codes);
+ *   in slices of K, whose f32 sums go through a library-owned buffer: 3 and 4 rows of more than
+ *     18432 codes; 5 to 16 rows of more than 8192 whose K is no multiple of 256, or, with 4 bits
+ *     and N >= 4096, whose scales are not whole 16-byte vectors (K / group_size % 8; up to 8 rows
+ *     of K % 512 == 0 from 50 M codes the 16-row kernel); with 8 bits those of 230 M codes, and
+ *     5 to 8 rows with K < 2 N, unless the tile kernel has them on load-to-LDS instructions.
+ * 5 to 8 rows on a 4-bit matrix of 50 M codes or more, 9 to 16 on one of 100 M, run on the
+ * 16-row kernel (exact w_hat). Else from 9 rows (from 5 where the rows are long) the MFMA tile
+ * kernel (replaces mt_qmm_mma / _m16 / _int8 / _int2 / _b3 / _b5 / _b6, quantized.rs:2106, 2408,
+ * 2731, 3330, 3560-3900; w_hat rounded to the element type before the multiply, as there), below
+ * that the qmv family (exact w_hat). A matrix takes the same kernel here and in
+ * mtq_qmm_batched, whose launch the K-run kernel shares: a single call is up to 3 us slower for
+ * it than it could be (8 bits, 16512 x 4096, 3 rows 21.1 -> 23.5 us, a pair 41.9 -> 38.5).
+ * MTQ_F32 batches run on the f32 matrix cores from 5 rows. Short, wide matrices split K over
+ * workgroups through that buffer (allocated on first use); where it cannot be allocated the call
+ * runs on a kernel that needs none. */
 MTQ_API int mtq_qmm(int dtype, int bits, uint32_t group_size, const void *w, const void *scales,
                     const void *biases, const void *x, void *out, uint32_t M, uint32_t N,
                     uint32_t K);
@@ -145,8 +153,8 @@ MTQ_API int mtq_qmm(int dtype, int bits, uint32_t group_size, const void *w, con
  * x [T][K], expert_offsets u32[E+1], out [T][N].
  * Both row views: while experts average at most 8 rows, each expert's rows run on the
  * GEMV kernels (exact w_hat = s*q + b in f32); above that the rows are grouped by expert
- * into 64-row tiles on the MFMA tile kernel, where w_hat is rounded to the element type
- * first, as in the reference's MMA gathers (moe.rs:2256); MTQ_F32 rows always run grouped, in
+ * into tiles of 32, 64 or up to 160 rows on the MFMA tile kernel, where w_hat is rounded to the
+ * element type first, as in the reference's MMA gathers (moe.rs:2256); MTQ_F32 rows always run grouped, in
  * 32-row tiles on the f32 matrix-core kernel (f32 rounding only). The grouping tables live in a
  * library-owned buffer (allocated on first use). Option "gather.grouped": 0 this rule,
  * 1 never grouped, 2 always grouped. Through mtq_dispatch the reference's kernel name decides instead:
