@@ -125,8 +125,12 @@ MTQ_API int mtq_qmv(int dtype, int bits, uint32_t group_size, const void *w, con
  * is multiplied with w_hat rounded to the element type):
  *   5 to 16 rows on up to 75 M codes (60 M of 8 bits), K % 128 == 0, K <= 8192 (5120 of 8 bits;
  *     from 9 rows with K > 6144 only N <= 1024, with K < 2048 only N <= 8192);
- *   2 to 4 rows (8 bits: 3 and 4), 2048 <= K <= 4096, on short matrices (2 N <= K, 4.5 M codes)
- *     and, in groups of 64 or 128, on tall ones (16384 < N <= 24576, 75 M codes);
+ *   3 and 4 rows, 1024 <= K <= 6144 (5120 of 8 bits), on up to 75 M codes: N <= 6144 (with 4 bits
+ *     and K <= 2048 only N <= 2048); N <= 16384 (8192 in groups of 32) on rows of more than 2048
+ *     bytes, but not of 4096; 8192 < N <= 12288 (in groups of 32 with K <= 4096); and, in groups
+ *     of 64 or 128 and 2048 <= K <= 4096, 16384 < N <= 24576;
+ *   2 rows, 4 bits, 2048 <= K <= 4096, on short matrices (2 N <= K, 4.5 M codes) and on the last
+ *     of these;
  *   in slices of K, whose f32 sums go through a library-owned buffer: 3 and 4 rows of more than
  *     18432 codes; 5 to 16 rows of more than 8192 whose K is no multiple of 256, or, with 4 bits
  *     and N >= 4096, whose scales are not whole 16-byte vectors (K / group_size % 8; up to 8 rows
@@ -137,8 +141,8 @@ MTQ_API int mtq_qmv(int dtype, int bits, uint32_t group_size, const void *w, con
  * kernel (replaces mt_qmm_mma / _m16 / _int8 / _int2 / _b3 / _b5 / _b6, quantized.rs:2106, 2408,
  * 2731, 3330, 3560-3900; w_hat rounded to the element type before the multiply, as there), below
  * that the qmv family (exact w_hat). A matrix takes the same kernel here and in
- * mtq_qmm_batched, whose launch the K-run kernel shares: a single call is up to 3 us slower for
- * it than it could be (8 bits, 16512 x 4096, 3 rows 21.1 -> 23.5 us, a pair 41.9 -> 38.5).
+ * mtq_qmm_batched, whose launch the K-run kernel shares: a single call is up to 3.5 us slower for
+ * it than it could be (8 bits, 9216 x 5120, 3 rows 15.5 -> 19.0 us, a pair 31.0 -> 28.7).
  * MTQ_F32 batches run on the f32 matrix cores from 5 rows. Short, wide matrices split K over
  * workgroups through that buffer (allocated on first use); where it cannot be allocated the call
  * runs on a kernel that needs none. */

@@ -52,38 +52,53 @@ bool qmv_runs_takes(const QmvParams& p, const QmvBatch& b) {
 //   16384 x 512     7.8  6.0  6.0 ->  7.4  7.5  7.5 | 15.7 11.9 12.0 -> 11.7 11.7 11.7     8 bits 15.6 12.5 12.7 -> 10.2 10.3 10.4
 //   16384 x 5120   17.8 18.0 18.3 -> 15.9 15.5 15.6 | 34.4 35.3 36.7 -> 26.4 26.1 26.8     8 bits 76.9 48.2 50.5 -> 42.1 42.5 43.0     (83.9 M)
 //   28672 x 4096   19.3 19.6 21.0 -> 19.7 20.4 20.7 | 37.3 38.4 41.9 -> 32.2 33.5 34.0     8 bits 63.2 66.5 69.7 -> 58.8 59.0 59.7     (117 M)
-// and 2, 3 and 4 rows:
-//   512 x 2048      3.9  4.6  5.2 ->  4.7  4.7  4.8 |  7.9  9.3 10.3 ->  4.9  4.9  5.0     8 bits 10.9 12.8 14.5 ->  5.5  5.5  5.6
-//   512 x 3584      5.7  7.0  7.5 ->  6.1  6.2  6.2 | 11.6 14.0 15.0 ->  6.4  6.4  6.5     8 bits 12.1 14.2 15.3 ->  6.7  6.7  6.7
-//   1024 x 4096     5.9  7.1  8.1 ->  6.3  6.3  6.4 | 11.8 14.1 16.3 ->  6.6  6.6  6.6     8 bits 12.6 14.7 16.6 ->  7.2  7.1  7.1
-//   768 x 3072      5.2  6.5  7.0 ->  6.2  6.2  6.3 | 10.4 13.0 13.9 ->  6.4  6.5  6.5     8 bits  4.3  5.0  5.5 ->  6.5  6.5  6.5 | 8.7 10.0 11.0 -> 6.8 6.8 6.8
-//   1280 x 5120     5.0  5.4  5.5 ->  7.3  7.4  7.4 |  9.9 10.8 11.1 ->  7.7  7.8  7.8
-//   512 x 8192      6.2  7.5  8.6 ->  9.8  9.9  9.9 | 12.5 15.0 17.2 -> 10.1 10.1 10.2
-//   4096 x 1024     3.5  3.6  3.7 ->  4.9  4.9  4.9 |  7.0  7.3  7.3 ->  5.7  5.8  5.8
-//   4096 x 4096     5.2  5.9  6.0 ->  6.7  6.8  6.9 | 10.3 11.7 12.0 ->  8.9  9.0  9.0     8 bits 14.0 14.9 15.5 -> 13.2 13.2 13.3
-//   8192 x 4096     6.8  7.3  7.4 ->  8.9  8.9  8.9 | 13.6 14.5 14.8 -> 14.2 14.2 14.3     8 bits 19.6 20.5 21.2 -> 21.7 21.8 22.2
-//   5120 x 5120     8.2  8.5  8.9 ->  9.7  9.8  9.8 | 16.4 17.0 17.9 -> 13.1 13.4 14.5     8 bits 20.4 21.9 22.9 -> 19.4 19.4 19.5
-// and on more than 16384 weight rows, where the GEMV's 256 workgroups of sixteen waves, four rows a wave at once, come to a second block:
-//   16384 x 3584   10.0 10.5 11.0 -> 13.3 13.3 13.4 | 19.9 20.5 20.5 -> 19.3 19.3 19.4     8 bits 34.5 32.8 33.3 -> 29.2 29.3 29.1
-//   16512 x 3584   13.5 14.0 14.0 -> 13.8 13.9 13.8 | 27.3 28.0 28.1 -> 20.0 20.3 20.1     8 bits 36.1 37.0 38.2 -> 31.4 31.0 31.2
-//   18944 x 3584   13.8 14.2 14.1 -> 14.2 14.3 14.4 | 27.7 28.4 28.5 -> 22.7 22.8 23.0     8 bits 36.9 38.5 39.9 -> 34.0 34.0 34.1
-//   16512 x 2048    9.6 10.2 10.2 -> 10.0 10.1 10.3 | 19.3 20.4 20.4 -> 14.2 14.5 14.7     8 bits 27.0 28.5 28.5 -> 18.2 18.4 18.2
-//   16512 x 4096   15.0 15.2 15.2 -> 14.6 14.4 14.6 | 30.3 30.4 30.6 -> 21.2 21.1 21.3     8 bits 20.1 21.1 21.5 -> 22.9 23.5 23.1 | 40.2 41.9 42.9 -> 37.8 38.5 37.2
-//   24576 x 3072   14.2 14.5 14.5 -> 14.6 14.7 14.9 | 28.1 28.9 29.1 -> 24.1 24.1 24.0     8 bits 35.3 39.5 39.9 -> 37.1 37.6 37.7     (75.5 M)
-//   28672 x 2560   13.9 14.7 14.4 -> 16.1 16.3 16.2 | 27.8 28.6 29.7 -> 26.1 26.4 26.7     (seven blocks of 4096 rows each on a workgroup)
-//   18944 x 3584 in groups of 32, whose scales weigh more here 13.3 13.8 13.7 -> 16.8 16.9 17.0 | 26.6 27.7 27.4 -> 27.7 27.9 27.8
-// So: below 5 rows the gate and up projections of 16385 to 24576 rows of 2048 to 4096 codes in groups of 64 and 128, and short matrices
-// against such rows (the K and V projections of grouped-query attention), both with 8-bit codes from 3 rows; from 5 rows up to 75 M codes
-// (60 M of 8 bits), and from 9 rows, where the others take tiles, no more than 8192 rows of fewer than 2048 codes, and no more than 1024
-// of more than 6144. The last two lines and the 75 M are those of an earlier form of the kernel, with sixteen waves on every row length: past
-// them this one has become the faster (7168 x 7168, 16384 x 5120, 8 bits 16384 x 512), but those calls would no longer have the tiles' bits.
+// and 3 and 4 rows (2 rows in the last lines):
+//   512 x 1024       4.1  4.1 ->  4.7  4.8 |  8.3  8.1 ->  5.0  5.0     8 bits  4.3  4.7 ->  4.3  4.3 |  8.6  9.5 ->  4.5  4.6
+//   2048 x 2048      4.3  4.3 ->  4.9  4.9 |  8.5  8.7 ->  5.1  5.2     8 bits  5.9  6.4 ->  5.5  5.5 | 11.7 12.7 ->  5.9  5.9
+//   4096 x 2048      4.2  4.3 ->  5.3  5.3 |  8.4  8.6 ->  6.5  6.6     8 bits  5.8  5.9 ->  5.9  5.9 | 11.6 11.8 ->  7.7  7.6
+//   1536 x 1536      4.3  4.3 ->  4.8  4.8 |  8.6  8.6 ->  5.1  5.1     8 bits  5.7  5.8 ->  5.4  5.4 | 11.4 11.5 ->  5.7  5.7
+//   512 x 3584       7.0  7.5 ->  6.2  6.2 | 14.1 15.0 ->  6.4  6.5     8 bits  7.1  7.7 ->  6.5  6.5 | 14.2 15.3 ->  6.8  6.7
+//   4096 x 4096      5.9  6.0 ->  6.8  6.8 | 11.8 12.0 ->  9.0  9.0     8 bits  7.5  7.8 ->  8.9  8.9 | 14.9 15.4 -> 13.2 13.3
+//   5120 x 5120      8.5  8.9 ->  9.8  9.8 | 17.1 18.0 -> 13.2 13.1     8 bits 11.1 11.7 -> 13.5 13.4 | 22.0 23.2 -> 19.5 19.5
+//   1024 x 5120      5.3  6.0 ->  7.3  7.3 | 10.7 11.8 ->  7.6  7.7     8 bits  6.5  7.1 ->  8.6  8.7 | 13.1 14.1 ->  9.2  9.2
+//   6144 x 6144      9.3  9.5 -> 10.7 10.7 | 18.7 19.2 -> 15.4 14.7
+//   4096 x 7168      7.4  7.8 -> 10.9 11.0 | 14.9 15.6 -> 13.8 13.8     (four steps a run, on eight waves)
+//   6144 x 4096      6.8  7.0 ->  8.7  8.7 | 13.7 13.9 -> 11.4 11.4     8 bits  9.7 10.1 -> 11.6 11.7 | 19.4 20.2 -> 18.0 18.0
+//   8192 x 4096      7.3  7.4 ->  8.9  8.9 | 14.6 14.8 -> 14.3 14.3     8 bits 10.3 10.8 -> 14.0 14.0 | 20.5 21.7 -> 21.8 22.0
+//   10240 x 4096     9.6  9.7 -> 11.0 11.1 | 19.4 19.3 -> 15.3 15.4     8 bits 15.5 16.0 -> 16.3 16.2 | 30.9 31.8 -> 26.2 26.6
+//   13824 x 4096    10.0 10.0 -> 13.6 13.7 | 20.2 20.2 -> 19.3 19.2     8 bits 16.3 16.6 -> 19.3 19.4 | 32.7 33.8 -> 32.0 32.3
+//   8192 x 5120     10.0  9.6 -> 10.5 10.5 | 18.9 19.2 -> 15.7 15.7     8 bits 13.7 14.2 -> 14.7 14.7 | 27.8 28.6 -> 23.9 23.9
+//   13824 x 5120    13.0 13.4 -> 15.2 15.2 | 25.9 26.7 -> 23.7 24.0     8 bits 20.1 20.6 -> 23.0 22.9 | 40.6 41.1 -> 38.5 38.3
+//   18944 x 3584    14.2 14.1 -> 14.3 14.4 | 28.4 28.5 -> 22.8 23.0     8 bits 38.5 39.9 -> 34.0 34.1
+//   28672 x 2560    14.7 14.4 -> 16.3 16.2 | 28.6 29.7 -> 26.4 26.7     (seven blocks of 4096 rows each on a workgroup)
+//   in groups of 32: 4096 x 2048 4.2 4.3 -> 5.9 5.9 | 8.5 8.6 -> 7.7 7.8, 4608 x 1536 5.0 4.9 -> 6.8 6.9 | 9.9 10.0 -> 8.4 8.4,
+//     13824 x 5120 13.9 14.2 -> 16.8 16.9 | 27.7 28.3 -> 26.9 26.8
+//   2 rows: 512 x 2048 3.9 -> 4.7 | 7.9 -> 4.9; 1024 x 4096 5.9 -> 6.2 | 11.7 -> 6.5; 18944 x 3584 13.8 -> 14.2 | 27.7 -> 22.7;
+//     4096 x 4096 5.2 -> 6.8 | 10.3 -> 9.0, 5120 x 5120 8.2 -> 9.7 | 16.4 -> 13.1 (pairs gain less, a lone output projection loses more)
+// The others' time steps up behind 4096, 8192 and 16384 weight rows (the GEMV's 256 workgroups of sixteen waves hold 16384 rows, four
+// a wave), this kernel's with each 4096, 256 blocks of 16: so at 3 and 4 rows up to 6144 weight rows (2048 of 4-bit rows of up to 2048
+// codes), from 8193 to 12288 and from 16385 to 24576 (of 2048 to 4096 codes), and up to 16384 where rows of more than 2048 bytes make the
+// others slower, except rows of 4096 bytes, which are slower here (8192 x 4096 of 8 bits 14.0, 8192 x 3584 11.0); up to 75 M codes and
+// three steps a run (8 bits: five). The four products of a dense layer, 22 families of sizes in groups of 32, 64 and 128, 4 and 8 bits:
+// 1.16 and 1.18 times as fast at 3 and 4 rows, none slower (5120, 17408 wide, 8 bits in groups of 32 124 -> 118, 129 -> 121; 1536, 4608
+// wide, whose down projection alone loses 2 us, 8 bits 42 -> 27, 4 bits 33 -> 27).
+// 2 rows, 4 bits: the short matrices of grouped-query attention and 16385 to 24576 weight rows.
+// From 5 rows up to 75 M codes (60 M of 8 bits), and from 9 rows, where the others take tiles, no more than 8192 weight rows of fewer than
+// 2048 codes, and no more than 1024 of more than 6144. The last two lines and the 75 M are those of an earlier form of the kernel, with
+// sixteen waves on every row length: past them this one has become the faster (7168 x 7168, 16384 x 5120, 8 bits 16384 x 512), but
+// those calls would no longer have the tiles' bits.
 bool qmv_runs_preferred(int bits, uint32_t G, uint32_t M, uint32_t N, uint32_t K) {
     if (M < 2 || M > 16) return false;
     const uint64_t codes = (uint64_t)N * K;
+    if (M < 5 && codes > 75000000ull) return false;
+    const bool tall = N > 16384 && N <= 24576 && K >= 2048 && K <= 4096 && G >= 64;
+    if (M == 2) return bits == 4 && (tall || ((uint64_t)N * 2 <= K && codes <= 4500000ull && K >= 2048 && K <= 4096));
     if (M < 5) {
-        if (K < 2048 || K > 4096 || (bits == 8 && M == 2)) return false;
-        const bool tall = N > 16384 && N <= 24576 && codes <= 75000000ull && G >= 64;
-        return tall || ((uint64_t)N * 2 <= K && codes <= 4500000ull);
+        if (K < 1024 || K > (bits == 4 ? 6144u : 5120u)) return false;
+        const uint32_t row = K * (uint32_t)bits / 8u;   // bytes from weight row to weight row
+        if (N <= 6144) return bits == 8 || K > 2048 || N <= 2048;
+        if (N <= 16384 && row > 2048 && row != 4096 && (G >= 64 || N <= 8192)) return true;
+        return tall || (N > 8192 && N <= 12288 && (G >= 64 || K <= 4096));
     }
     if (M > 8 && ((K > 6144 && N > 1024) || (K < 2048 && N > 8192))) return false;
     return codes <= (bits == 4 ? 75000000ull : 60000000ull);

@@ -85,6 +85,33 @@ def test_many_blocks_per_workgroup(oracle, dt, bits, G, M, K, Ns, instance):
             b.free()
 
 
+@pytest.mark.parametrize("dt,bits,G,M,K,Ns", [
+    (DType.BF16, 4, 64, 3, 4096, (4096, 1024, 1024)), (DType.F16, 4, 128, 4, 5120, (5120, 5120, 5120)), (DType.BF16, 4, 32, 3, 6144, (6144, 50)),
+    (DType.F16, 4, 64, 4, 1024, (1000, 12288)), (DType.BF16, 8, 64, 4, 3584, (3584, 512, 512)), (DType.F16, 8, 32, 3, 5120, (6144, 8192)), (DType.BF16, 4, 64, 4, 4480, (16384, 9001)),
+])
+def test_layers_of_three_and_four_rows(oracle, dt, bits, G, M, K, Ns):
+    """The projections of dense layers by the rule of sizes, no option set: one launch, exact results, the bits of single calls."""
+    print(f"[case] K-run qmv layer {dt.name} b{bits} g{G} M{M} K{K} N={Ns}", flush=True)
+    cases = [make_case(970 + j + M, dt, bits, G, M, N, K, bias_rule="midpoint") for j, N in enumerate(Ns)]
+    x = GpuBuffer.from_bytes(cases[0].x_bytes)
+    ws, ss, bs = ([GpuBuffer.from_bytes(v) for v in part] for part in zip(*((c.w.tobytes(), c.scales_bytes, c.biases_bytes) for c in cases)))
+    guard = b"\xcd" * 64
+    outs = [GpuBuffer.from_bytes(b"\xff" * (M * N * 2) + guard) for N in Ns]
+    assert all("qmv_runs_kernel" in ops.plan("qmm", dt, bits, G, M, N, K)[1][0][0] for N in Ns)
+    ops.qmm_batched(dt, bits, G, ws, ss, bs, x, outs, list(Ns), M, K)
+    for j, (c, N) in enumerate(zip(cases, Ns)):
+        raw = outs[j].read_bytes(M * N * 2 + 64)
+        assert raw[-64:] == guard
+        exp = oracle.qmm_f64(c.w, c.scales_f, c.biases_f, cases[0].x_f, M, N, K, bits, G, threads=8).reshape(-1)
+        assert rel_err(unpack_f32(raw[:-64], dt), exp) <= TOL[dt], j
+        single = GpuBuffer(M * N * 2)
+        ops.qmm(dt, bits, G, ws[j], ss[j], bs[j], x, single, M, N, K)
+        assert single.read_bytes(M * N * 2) == raw[:-64], j
+        single.free()
+    for b in [x] + ws + ss + bs + outs:
+        b.free()
+
+
 def test_mixed_batch_keeps_bits():
     """Three rows: the short matrices share a launch, the long one goes its own way; the bits are those of single calls."""
     dt, M, K, Ns = DType.BF16, 3, 2048, (4096, 256, 256)

@@ -236,7 +236,7 @@ def test_bit_stream_tiles_at_65_to_128_rows(bits, M, N, K, G, tile, ksplit):
 
 
 @pytest.mark.parametrize("bits,M,N,K,runs", [
-    (4, 2, 1024, 4096, True), (8, 2, 1024, 4096, False), (8, 3, 1024, 4096, True), (4, 4, 1024, 1024, False), (4, 4, 512, 2048, True), (4, 4, 2048, 2048, False),
+    (4, 2, 1024, 4096, True), (8, 2, 1024, 4096, False), (8, 3, 1024, 4096, True), (4, 4, 512, 2048, True), (4, 2, 2048, 2048, False),
     (4, 3, 512, 8192, False), (4, 2, 4096, 1024, False), (4, 5, 8192, 8192, True), (4, 9, 8192, 8192, False), (4, 16, 1024, 8192, True), (4, 9, 1025, 8192, False),
     (4, 9, 1040, 6144, True), (4, 16, 8192, 512, True), (4, 16, 8208, 512, False), (4, 8, 16384, 512, True), (8, 16, 16384, 2048, True), (4, 16, 13824, 5120, True),
     (4, 16, 16384, 5120, False), (8, 16, 14336, 4096, True), (8, 16, 16384, 4096, False), (4, 1, 1024, 4096, False), (4, 17, 1024, 4096, False),
@@ -249,11 +249,18 @@ def test_k_run_lines(bits, M, N, K, runs):
 
 @pytest.mark.parametrize("bits,G,N,K,rows", [
     (4, 64, 16384, 3584, ()), (4, 64, 16400, 3584, (2, 3, 4)), (4, 128, 24576, 2048, (2, 3, 4)), (4, 64, 24592, 2048, ()), (4, 32, 18944, 3584, ()),
-    (8, 64, 16384, 3584, ()), (8, 64, 16400, 3584, (3, 4)), (8, 128, 24576, 2048, (3, 4)), (4, 64, 18944, 1920, ()), (4, 64, 18304, 4096, (2, 3, 4)), (4, 64, 18320, 4096, ()),
-    (4, 64, 4096, 4096, ()), (4, 64, 5120, 5120, ()), (8, 64, 5120, 5120, ()), (4, 64, 13824, 5120, ()),
+    (8, 64, 16400, 3584, (3, 4)), (8, 128, 24576, 2048, (3, 4)), (4, 64, 18944, 1920, ()), (4, 64, 18304, 4096, (2, 3, 4)), (4, 64, 18320, 4096, ()),
+    # up to 6144 weight rows of three steps a run (8 bits: five)
+    (4, 64, 4096, 4096, (3, 4)), (8, 32, 3584, 3584, (3, 4)), (4, 128, 6144, 6144, (3, 4)), (4, 64, 6144, 6272, ()), (8, 64, 6144, 5120, (3, 4)), (8, 64, 4096, 5248, ()),
+    (4, 64, 6160, 4096, ()), (4, 64, 512, 1024, (3, 4)), (4, 64, 512, 896, ()), (4, 64, 2048, 2048, (3, 4)), (4, 64, 2064, 2048, ()), (4, 32, 2064, 2176, (3, 4)), (8, 64, 2064, 2048, (3, 4)),
+    # rows of more than 2048 bytes, but 4096
+    (4, 64, 8192, 4096, ()), (4, 64, 8192, 4224, (3, 4)), (4, 64, 13824, 5120, (3, 4)), (4, 64, 16384, 4480, (3, 4)), (4, 64, 16400, 4480, ()), (4, 32, 8192, 5120, (3, 4)),
+    (4, 32, 8208, 5120, ()), (8, 64, 16384, 3584, (3, 4)), (8, 64, 13824, 4096, ()), (8, 64, 8192, 2048, ()), (8, 64, 8192, 2176, (3, 4)), (8, 32, 8192, 2560, (3, 4)),
+    # 8193 to 12288 rows
+    (4, 64, 8208, 4096, (3, 4)), (4, 64, 12288, 1024, (3, 4)), (4, 64, 12304, 4096, ()), (8, 128, 12288, 4096, (3, 4)), (8, 32, 10240, 4096, (3, 4)), (4, 32, 12288, 2048, (3, 4)),
 ])
 def test_k_run_lines_of_few_rows(bits, G, N, K, rows):
-    """2, 3 and 4 rows on tall matrices: one rule of sizes, on both sides of each line."""
+    """2, 3 and 4 rows: one rule of sizes, the same at 3 and 4, on both sides of each line."""
     on = tuple(M for M in (2, 3, 4) if "qmv_runs_kernel" in ops.plan("qmm", DType.BF16, bits, G, M, N, K)[1][0][0])
     assert on == rows
 
