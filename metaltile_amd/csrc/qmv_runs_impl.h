@@ -13,7 +13,7 @@
 // 16x16x32 MFMA and keeps in registers: from then on the only loads are weights, scales and biases, PF blocks ahead.
 // (Vector loads complete in order: activations read along the way, even from the L2, make a wave wait for all weights
 // asked for before them. The same kernel with activations read per block streamed at half the rate.) The KP sums of
-// a result meet in LDS. The split of K depends on K alone: a matrix gives the same bits in whatever batch of matrices.
+// a result meet in LDS. The split of K depends on K and the code width: a matrix gives the same bits in whatever batch of matrices.
 //
 // A step is 128 codes of a row (64 of 8-bit codes), 64 bytes, of which lane (j, q) = (lane % 16, lane / 16) multiplies the 16 bytes
 // of row j at 16 q: 32 codes (16). What bounded the kernel was finding the lines: with neighbouring lanes in sixteen different rows
