@@ -545,9 +545,9 @@ __global__ __launch_bounds__(64 * NW) void qmm_dma_kernel(QmmDArgs args) {
 // Many rows per expert: row tiles of up to 160 rows, each on as many 32-row blocks as it has. An expert's rows are cut into even
 // pieces, so that 128 rows or a few more are one tile and each weight is converted once for them (64-row tiles: two or three
 // times, the last one nearly empty). 160 rows are what three buffers and the scales leave room for in LDS. us, the whole gather with
-// its table, bf16, 64-row tiles -> these: 128 experts of 768 x 2048, 128 rows each 108 -> 95 (8-bit codes 173 -> 120), of 2048 x 768
-// 133 -> 117; 8 experts of 14336 x 4096, 512 rows each 666 -> 603, of 4096 x 14336, 64 / 128 rows each 172 / 261 -> 118 / 165 (with
-// skewed routing: qmm_direct.hip, grouped_tile_rows).
+// its table, bf16, rows by even / random routing, 64-row tiles -> these: 128 experts of 768 x 2048, 128 rows each 78 / 97 -> 71 / 76 (8-bit
+// codes, random, 172 -> 102), of 2048 x 768 95 / 113 -> 92 / 98; 8 experts of 14336 x 4096, 512 rows each 620 / 648 -> 526 / 562, of 4096 x
+// 14336, 128 rows each 170 / 240 -> 141 / 158 (skewed routing and fewer rows: qmm_direct.hip, grouped_tile_rows).
 // What is left is the start and end of each tile (about 7 us of 22 at 2048 codes): one workgroup fills a compute unit's registers.
 template <int DT, bool WIN, int BITS> __global__ __launch_bounds__(512) void qmm_dma_routed_kernel(QmmDArgs args) {
     uint4 t;
