@@ -21,10 +21,11 @@ static bool runs_aligned(const void* w, const void* s, const void* b, const void
 }
 
 // (instances: qmv_runs_pick.h, one translation unit per element type)
-RunsInstance qmv_runs_pick_f16(int bits, uint32_t G, bool sliced, uint32_t xs, bool few);
-RunsInstance qmv_runs_pick_bf16(int bits, uint32_t G, bool sliced, uint32_t xs, bool few);
-static RunsInstance runs_pick(int dtype, int bits, uint32_t G, bool sliced, uint32_t xs, uint32_t M) {
-    return dtype == DT_BF16 ? qmv_runs_pick_bf16(bits, G, sliced, xs, M <= 8) : qmv_runs_pick_f16(bits, G, sliced, xs, M <= 8);
+RunsInstance qmv_runs_pick_f16(bool paired, int bits, uint32_t G, bool sliced, uint32_t xs, bool few);
+RunsInstance qmv_runs_pick_bf16(bool paired, int bits, uint32_t G, bool sliced, uint32_t xs, bool few);
+static RunsInstance runs_pick(int dtype, int bits, uint32_t G, uint32_t K, bool sliced, uint32_t xs, uint32_t M) {
+    const bool paired = (uint64_t)K * bits / 8 % 128 == 0;   // rows of whole 128-byte lines
+    return dtype == DT_BF16 ? qmv_runs_pick_bf16(paired, bits, G, sliced, xs, M <= 8) : qmv_runs_pick_f16(paired, bits, G, sliced, xs, M <= 8);
 }
 
 bool qmv_runs_takes(const QmvParams& p, const QmvBatch& b) {
@@ -152,7 +153,7 @@ int launch_qmv_runs(const QmvParams& p, const QmvBatch& b, const LaunchCtx& lc) 
     a.K = p.K;
     a.slices = 1;
     const uint32_t cus = runs_cus(), wgs = a.blocks < cus ? a.blocks : cus, xs = runs_steps(p.bits, p.K);
-    const RunsInstance k = runs_pick(p.dtype, p.bits, p.group_size, false, xs, p.M);
+    const RunsInstance k = runs_pick(p.dtype, p.bits, p.group_size, p.K, false, xs, p.M);
     void* args[] = {&a};
     hipError_t e = launch_kernel(k.fn, dim3(wgs), dim3(k.threads), args, 0, lc);
     if (e != hipSuccess) return hip_fail(e, "K-run qmv kernel launch");
@@ -193,7 +194,7 @@ int launch_qmv_slices(const QmmParams& p, const LaunchCtx& lc, void* scratch) {
     LaunchCtx l1 = lc, l2 = lc;
     l1.stop = nullptr;
     l2.start = nullptr;
-    const RunsInstance k = runs_pick(p.dtype, p.bits, p.group_size, true, 0, p.M);
+    const RunsInstance k = runs_pick(p.dtype, p.bits, p.group_size, p.K, true, 0, p.M);
     hipError_t e = launch_kernel(k.fn, dim3(wgs), dim3(k.threads), args, 0, l1);
     if (e != hipSuccess) return hip_fail(e, "K-sliced qmv kernel launch");
     return add_slices(p.dtype, (const float*)scratch, p.out, p.M * p.N, a.slices, l2);

@@ -3,6 +3,6 @@
 
 namespace mtq {
 
-RunsInstance qmv_runs_pick_f16(int bits, uint32_t G, bool sliced, uint32_t xs, bool few) { return runs_pick_type<DT_F16>(bits, G, sliced, xs, few); }
+RunsInstance qmv_runs_pick_f16(bool paired, int bits, uint32_t G, bool sliced, uint32_t xs, bool few) { return runs_pick_type<DT_F16>(paired, bits, G, sliced, xs, few); }
 
 }  // namespace mtq

@@ -15,8 +15,8 @@
 // asked for before them. The same kernel with activations read per block streamed at half the rate.) The KP sums of
 // a result meet in LDS. The split of K depends on K and the code width: a matrix gives the same bits in whatever batch of matrices.
 //
-// A step is 128 codes of a row (64 of 8-bit codes), 64 bytes, of which lane (j, q) = (lane % 16, lane / 16) multiplies the 16 bytes
-// of row j at 16 q: 32 codes (16). What bounded the kernel was finding the lines: with neighbouring lanes in sixteen different rows
+// A step is 128 codes of a row (64 of 8-bit codes), 64 bytes, two neighbouring ones of which are loaded together; of a step lane (j, q) = (lane % 16, lane / 16) multiplies the
+// 16 bytes of row j at 16 q: 32 codes (16). What bounded the kernel was finding the lines: with neighbouring lanes in sixteen different rows
 // a load of 1 KB occupies the compute unit's address path four times as long as with four neighbours in one row, about 64 clk
 // against 16, and that was all of a block's 5000 clk at 16 rows (64 weight and scale loads of it). So four neighbours load a row's
 // step, and the pieces are turned in LDS (one write and one read of 16 bytes, conflict-free). 16 rows, us, groups of 128, before ->
@@ -28,10 +28,8 @@
 // Every load is a buffer load whose out-of-range offsets read zeros without a memory access: rows past the matrix or
 // the batch, steps past a wave's run and blocks past the last one are given such offsets, so that every wave issues the
 // same loads in the same order.
-#include "mtq_device.h"
+#include "mfma16.h"
 #include "mtq_internal.h"
-
-#include <type_traits>
 
 namespace mtq {
 
@@ -54,48 +52,6 @@ struct RunsInstance {
     const void* fn;
     uint32_t threads;
 };
-
-typedef uint32_t kr_u32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t kr_u32x2 __attribute__((ext_vector_type(2)));
-typedef float kr_f32x4 __attribute__((ext_vector_type(4)));
-
-template <int DT> __device__ __forceinline__ kr_f32x4 kr_mfma(kr_u32x4 a, kr_u32x4 b, kr_f32x4 c) {
-    if constexpr (DT == DT_BF16) {
-        typedef __attribute__((ext_vector_type(8))) __bf16 v8;
-        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8, a), __builtin_bit_cast(v8, b), c, 0, 0, 0);
-    } else {
-        typedef __attribute__((ext_vector_type(8))) _Float16 v8;
-        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8, a), __builtin_bit_cast(v8, b), c, 0, 0, 0);
-    }
-}
-
-template <int B, int E, class F> __device__ __forceinline__ void kr_for(F&& f) {
-    if constexpr (B < E) {
-        f(std::integral_constant<int, B>{});
-        kr_for<B + 1, E>(f);
-    }
-}
-
-// Between a wave's writes to its own LDS and its reads of what other lanes wrote (LDS operations of a wave complete in order: no wait).
-__device__ __forceinline__ void kr_turned() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
-}
-
-constexpr uint32_t KR_OOB = 0x80000000u;   // every buffer is shorter than 2 GiB (host): base + KR_OOB is out of range for any base below 2 GiB
-constexpr int KR_NT = 2;                   // cache policy of the weights: read once
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t kr_rsrc(uint64_t a, uint32_t bytes) {
-    // (the base is the same in every lane: the descriptor is kept in scalar registers)
-    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a), hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
-    return __builtin_amdgcn_make_buffer_rsrc((void*)(((uint64_t)hi << 32) | lo), 0, __builtin_amdgcn_readfirstlane(bytes), 0x00020000);
-}
-
-template <int DT> __device__ __forceinline__ float kr_elem(uint32_t dw, int odd) {
-    if constexpr (DT == DT_BF16) return __uint_as_float(odd ? (dw & 0xFFFF0000u) : (dw << 16));
-    else return f16_bits_to_f32(odd ? (dw >> 16) : (dw & 0xFFFFu));
-}
 
 // What a code width fixes: the codes a lane loads per step, the MFMAs of a step, the dwords an MFMA's 8 codes per lane
 // come in, and the offset its conversion adds to every code.
@@ -141,9 +97,9 @@ template <int DT, int BITS> __device__ __forceinline__ kr_u32x4 kr_weights(const
     return o;
 }
 
-// DT, BITS (4 or 8), G (32, 64, 128), XS: steps of a wave's run at most, PF: blocks whose
+// PAIRED: a row is a whole number of 128 bytes. DT, BITS (4 or 8), G (32, 64, 128), XS: steps of a wave at most, PF: blocks whose
 // weights are in flight ahead of the one that is worked on.
-template <int KP, bool SLICED, bool ORDERED, int DT, int BITS, int G, int XS, int PF> __device__ __forceinline__ void qmv_runs_body(const QmvRunsArgs& a) {
+template <bool PAIRED, int KP, bool SLICED, bool ORDERED, int DT, int BITS, int G, int XS, int PF> __device__ __forceinline__ void qmv_runs_body(const QmvRunsArgs& a) {
     using C = KrCodes<DT, BITS>;
     constexpr int EG = G < C::STEP ? G : C::STEP;   // codes per scale within a step
     constexpr int GPS = C::STEP / EG;               // scales per step: 1, 2 or 4
@@ -153,7 +109,9 @@ template <int KP, bool SLICED, bool ORDERED, int DT, int BITS, int G, int XS, in
     constexpr int SR = (XS + 3) / 4;                // scale registers: lanes (j, q) hold steps q, q + 4 of row j
     constexpr bool HOLD = XS * GPS <= (KP == 16 ? 4 : 5);   // the activations' sums stay in registers
     constexpr bool SUMS = !HOLD && KP != 16;                // or in LDS
-    constexpr int SLOTS = C::UNITS;                         // KB of LDS in which a wave turns a step's weights, or its activations
+    constexpr int PAIRS = PAIRED ? XS / 2 : 0;              // pairs of steps of a wave; of an odd number the last step stands alone
+    constexpr int SLOTS = C::UNITS;                         // KB of LDS in which a wave turns two steps' weights, or a step's activations
+    static_assert(SLOTS >= 2, "a pair of steps is 2 KB");
     __shared__ float red[2][KP * 256];
     __shared__ kr_u32x4 turned[KP * SLOTS * 64];
     __shared__ __attribute__((aligned(16))) float sums[SUMS ? KP * XS * GPS * 16 : 4];
@@ -171,10 +129,19 @@ template <int KP, bool SLICED, bool ORDERED, int DT, int BITS, int G, int XS, in
         wg = blockIdx.x / a.slices;
         slice = blockIdx.x - wg * a.slices;
         wgs = gridDim.x / a.slices;
-        first_step = all_steps * slice / a.slices;
-        steps = all_steps * (slice + 1u) / a.slices - first_step;
+        const uint32_t unit = PAIRED ? 2u : 1u;   // (of paired rows a whole number of pairs)
+        first_step = all_steps / unit * slice / a.slices * unit;
+        steps = all_steps / unit * (slice + 1u) / a.slices * unit - first_step;
     }
-    const uint32_t t_in = steps * kp / KP, t0 = first_step + t_in, cnt = steps * (kp + 1u) / KP - t_in;   // cnt <= XS (host)
+    // Of the slice's steps, wave kp has the pairs kp, kp + KP, ... and, of what lies behind PAIRS * KP pairs, the kp-th step: two
+    // neighbouring steps are the 128 bytes of a line, and the same loads streamed 58 MB at 4.4 TB/s in pieces of 64 bytes of
+    // a row, at 5.8 in pieces of 128. 16 rows, us, a run of steps a wave -> pairs: 2 x 13824 x 5120 in groups of 128 22.0 -> 20.6,
+    // 2 x 14336 x 4096 20.0 -> 18.7, 8 rows of 8192 x 8192 16.1 -> 13.7; 8 bits, 4 rows, 2 x 18944 x 3584 31.5 -> 26.9. Where rows are
+    // an odd number of steps a pair of every second row lies in two lines, and a run of steps a wave is the faster (4736 x 4736 9.6
+    // against 10.1). steps <= XS * KP (host).
+    const uint32_t run0 = steps * kp / KP, run = steps * (kp + 1u) / KP - run0;
+    auto step_of = [&](uint32_t n) { return !PAIRED ? run0 + n : n < 2u * PAIRS ? 2u * (kp + KP * (n >> 1)) + (n & 1u) : 2u * (uint32_t)(KP * PAIRS) + kp; };
+    auto has_step = [&](uint32_t n) { return PAIRED ? n < (uint32_t)XS && step_of(n) < steps : n < run; };
 
     // What a lane loads: slot ls of row lr, of the four 16-byte pieces that a step has of a row; the pieces of a row are dealt to
     // its slots so that the sixteen rows' reads from LDS do not meet in a bank.
@@ -182,16 +149,23 @@ template <int KP, bool SLICED, bool ORDERED, int DT, int BITS, int G, int XS, in
     const uint32_t my_row = j * 4u, my_turn = (j >> 1) & 3u;   // (row j, piece p) lies in slot my_row + (p ^ my_turn)
     kr_u32x4* const swap_lds = turned + kp * (uint32_t)(SLOTS * 64);
 
-    const uint32_t wlane = lr * wrow_bytes + t0 * 64u + lpiece * 16u;
+    // Weights of a pair: load 0 has rows 0 .. 7, load 1 rows 8 .. 15, slot lane % 8 of row lane / 8 of the eight pieces; these too
+    // are dealt to the slots so that the reads do not meet in a bank. Of a step alone: as the activations.
+    const uint32_t pr = lane >> 3, ppiece = (lane ^ pr) & 7u;
+    const uint32_t plane = pr * wrow_bytes + first_step * 64u + ppiece * 16u, wlane = lr * wrow_bytes + first_step * 64u + lpiece * 16u;
+    uint32_t pair_dead[PAIRS ? PAIRS : 1];   // this lane's piece lies past the slice
+#pragma unroll
+    for (int n = 0; n < PAIRS; n++) pair_dead[n] = (steps - 1u - step_of(2 * n) - (ppiece >> 2)) & KR_OOB;
+    const uint32_t pair_row = (j >> 3) * 64u + (j & 7u) * 8u, pair_turn = j & 7u;   // (row j, piece p) lies in slot pair_row + (p ^ pair_turn)
     uint32_t slane[SR];
 #pragma unroll
     for (int i = 0; i < SR; i++) {
-        const uint32_t n = ls + 4u * i, at = t0 + n;
-        slane[i] = n < cnt ? lr * gpr * 2u + (G > C::STEP ? at / (uint32_t)(G / EG) : at * GPS) * 2u : KR_OOB;
+        const uint32_t n = ls + 4u * i, at = first_step + step_of(n);
+        slane[i] = has_step(n) ? lr * gpr * 2u + (G > C::STEP ? at / (uint32_t)(G / EG) : at * GPS) * 2u : KR_OOB;
     }
-    uint32_t step_dead[XS];   // steps past the run
+    uint32_t step_dead[XS];   // steps past the slice
 #pragma unroll
-    for (int n = 0; n < XS; n++) step_dead[n] = (cnt - (uint32_t)(n + 1)) & KR_OOB;
+    for (int n = 0; n < XS; n++) step_dead[n] = (PAIRED ? steps - 1u - step_of(n) : run - 1u - (uint32_t)n) & KR_OOB;
 
     // The matrix of a block, by sums of masked differences on the scalar unit. (Selections among the arguments become an
     // indexed read of a copy of them in scratch memory, with a wait for every load in flight.)
@@ -218,7 +192,7 @@ template <int KP, bool SLICED, bool ORDERED, int DT, int BITS, int G, int XS, in
         const __amdgpu_buffer_rsrc_t wr = kr_rsrc(pick(a.w, at_blk), N * wrow_bytes), sr = kr_rsrc(pick(a.scales, at_blk), N * gpr * 2u),
                                      br = kr_rsrc(pick(a.biases, at_blk), N * gpr * 2u);
         const uint32_t dead = (rows - 1u - lr) & KR_OOB;
-        const uint32_t wo = (wlane + row0 * wrow_bytes) | dead, s0 = row0 * gpr * 2u;
+        const uint32_t w0 = row0 * wrow_bytes, s0 = row0 * gpr * 2u;
 #pragma unroll
         for (int i = 0; i < SR; i++) {
             const uint32_t o = (slane[i] + s0) | dead;
@@ -234,7 +208,12 @@ template <int KP, bool SLICED, bool ORDERED, int DT, int BITS, int G, int XS, in
             }
         }
 #pragma unroll
-        for (int n = 0; n < XS; n++) d.w[n] = __builtin_amdgcn_raw_buffer_load_b128(wr, (int)((wo + 64u * n) | step_dead[n]), 0, KR_NT);
+        for (int n = 0; n < PAIRS; n++)
+#pragma unroll
+            for (uint32_t h = 0; h < 2; h++)
+                d.w[2 * n + h] = __builtin_amdgcn_raw_buffer_load_b128(wr, (int)((plane + w0 + 8u * h * wrow_bytes + 64u * step_of(2 * n)) | pair_dead[n] | ((rows - 1u - pr - 8u * h) & KR_OOB)), 0, KR_NT);
+#pragma unroll
+        for (int n = 2 * PAIRS; n < XS; n++) d.w[n] = __builtin_amdgcn_raw_buffer_load_b128(wr, (int)((wlane + w0 + 64u * step_of(n)) | step_dead[n] | dead), 0, KR_NT);
     };
 
     Block ring[PF + 1];
@@ -246,11 +225,11 @@ template <int KP, bool SLICED, bool ORDERED, int DT, int BITS, int G, int XS, in
     kr_u32x4 xop[XS][C::UNITS];
     {
         const __amdgpu_buffer_rsrc_t xr = kr_rsrc((uint64_t)a.x, a.M * K * 2u);
-        const uint32_t xo = ((lr * K + t0 * (uint32_t)C::STEP + lpiece * 8u) * 2u) | ((a.M - 1u - lr) & KR_OOB);
+        const uint32_t xo = ((lr * K + first_step * (uint32_t)C::STEP + lpiece * 8u) * 2u) | ((a.M - 1u - lr) & KR_OOB);
 #pragma unroll
         for (int n = 0; n < XS; n++)
 #pragma unroll
-            for (int k = 0; k < C::UNITS; k++) xop[n][k] = __builtin_amdgcn_raw_buffer_load_b128(xr, (int)((xo + (uint32_t)(n * C::STEP * 2 + k * 64)) | step_dead[n]), 0, 0);
+            for (int k = 0; k < C::UNITS; k++) xop[n][k] = __builtin_amdgcn_raw_buffer_load_b128(xr, (int)((xo + step_of(n) * (uint32_t)(C::STEP * 2) + (uint32_t)(k * 64)) | step_dead[n]), 0, 0);
         __builtin_amdgcn_sched_barrier(0);
         // No wave's weights ahead of another's activations. Not where a run is short, as the wait for the last of the waves to start
         // costs more there (us, with -> without): 8 bits, 5 rows 4096 x 2048 6.5 -> 5.9; 4 bits 11008 x 2048 7.8 -> 7.4, groups of 32
@@ -345,9 +324,19 @@ template <int KP, bool SLICED, bool ORDERED, int DT, int BITS, int G, int XS, in
         kr_for<0, XS>([&](auto n_c) {
             constexpr int n = decltype(n_c)::value;
             uint32_t v[4];
-            swap_lds[n % SLOTS * 64 + lane] = d.w[n];
-            kr_turned();
-            codes_of(swap_lds[n % SLOTS * 64 + my_row + (q ^ my_turn)], v);
+            if constexpr (n < 2 * PAIRS) {
+                constexpr int at = n / 2 * 2 % SLOTS * 64;
+                if constexpr (n % 2 == 0) {
+                    swap_lds[at + lane] = d.w[n];
+                    swap_lds[at + 64 + lane] = d.w[n + 1];
+                    kr_turned();
+                }
+                codes_of(swap_lds[at + pair_row + ((q + 4u * (n % 2)) ^ pair_turn)], v);
+            } else {
+                swap_lds[n % SLOTS * 64 + lane] = d.w[n];
+                kr_turned();
+                codes_of(swap_lds[n % SLOTS * 64 + my_row + (q ^ my_turn)], v);
+            }
             const int src = (int)((my_row + (n % 4)) * 4u);   // the lane that holds this step's scales of row j
             kr_for<0, GPS>([&](auto g_c) {
                 constexpr int g = decltype(g_c)::value;
@@ -378,8 +367,10 @@ template <int KP, bool SLICED, bool ORDERED, int DT, int BITS, int G, int XS, in
             const __amdgpu_buffer_rsrc_t wr = kr_rsrc(pick(a.w, at_blk), N * wrow_bytes), sr = kr_rsrc(pick(a.scales, at_blk), N * gpr * 2u),
                                          br = kr_rsrc(pick(a.biases, at_blk), N * gpr * 2u), xr = kr_rsrc((uint64_t)a.x, a.M * K * 2u);
 #pragma unroll 1
-            for (uint32_t k0 = t0 * (uint32_t)C::STEP, end = k0 + cnt * (uint32_t)C::STEP; k0 < end; k0 += 32u) {
-                const uint32_t k = k0 + 8u * q, wo = (row0 + j) * wrow_bytes + k / 8u * BITS, so = ((row0 + j) * gpr + k / (uint32_t)G) * 2u;   // rows past the last: zeros
+            for (uint32_t i = 0; i < (uint32_t)(XS * C::UNITS); i++) {
+                const uint32_t n = i / C::UNITS;
+                if (!has_step(n)) continue;   // (the same in every lane)
+                const uint32_t k = (first_step + step_of(n)) * (uint32_t)C::STEP + i % C::UNITS * 32u + 8u * q, wo = (row0 + j) * wrow_bytes + k / 8u * BITS, so = ((row0 + j) * gpr + k / (uint32_t)G) * 2u;   // rows past the last: zeros
                 uint32_t d[2] = {};
                 d[0] = __builtin_amdgcn_raw_buffer_load_b32(wr, (int)wo, 0, 0);
                 if constexpr (BITS == 8) d[1] = __builtin_amdgcn_raw_buffer_load_b32(wr, (int)wo + 4, 0, 0);
@@ -427,12 +418,12 @@ template <int KP, bool SLICED, bool ORDERED, int DT, int BITS, int G, int XS, in
 }
 
 // XS: steps of a sixteenth of K at most.
-template <bool ORDERED, int KP, int DT, int BITS, int G, int XS, int PF> __global__ __launch_bounds__(KP * 64) void qmv_runs_kernel(QmvRunsArgs a) {
-    qmv_runs_body<KP, false, ORDERED, DT, BITS, G, XS * 16 / KP, PF>(a);
+template <bool PAIRED, bool ORDERED, int KP, int DT, int BITS, int G, int XS, int PF> __global__ __launch_bounds__(KP * 64) void qmv_runs_kernel(QmvRunsArgs a) {
+    qmv_runs_body<PAIRED, KP, false, ORDERED, DT, BITS, G, XS * 16 / KP, PF>(a);
 }
 // On one of a.slices slices of K, whose sums a second launch adds; XS: steps of an eighth of a slice at most.
-template <int DT, int BITS, int G, int XS, int PF> __global__ __launch_bounds__(512) void qmv_slices_kernel(QmvRunsArgs a) {
-    qmv_runs_body<8, true, true, DT, BITS, G, XS, PF>(a);
+template <bool PAIRED, int DT, int BITS, int G, int XS, int PF> __global__ __launch_bounds__(512) void qmv_slices_kernel(QmvRunsArgs a) {
+    qmv_runs_body<PAIRED, 8, true, true, DT, BITS, G, XS, PF>(a);
 }
 
 }  // namespace mtq

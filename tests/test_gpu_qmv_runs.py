@@ -201,3 +201,33 @@ def test_operands_off_16_bytes(oracle, which):
         assert rel_err(unpack_f32(raw[off["out"]:-64], dt), exp) <= 1e-2, batch
     for b in bufs.values():
         b.free()
+
+
+@pytest.mark.parametrize("dt", [DType.F16, DType.BF16], ids=lambda d: d.name)
+@pytest.mark.parametrize("option,bits,G,M,N,K", [
+    (2, 4, 64, 16, 40, 256), (2, 4, 128, 9, 24, 768), (2, 4, 64, 5, 33, 4352), (2, 4, 32, 16, 20, 4864), (2, 4, 64, 3, 17, 6400),
+    (2, 8, 64, 16, 40, 128), (2, 8, 32, 7, 24, 2176), (2, 8, 128, 16, 33, 4224), (2, 8, 64, 4, 17, 4992),
+    (3, 4, 64, 16, 40, 8448), (3, 4, 128, 5, 33, 13824), (3, 8, 64, 9, 24, 5248), (3, 8, 128, 3, 40, 15232),
+])
+def test_pairs_of_steps(oracle, dt, option, bits, G, M, N, K):
+    """Rows of whole 128-byte lines, whose steps are dealt to the waves in pairs: fewer pairs than waves, pairs that leave some waves
+    one round less, single steps behind the pairs, slices of an odd number of pairs."""
+    print(f"[case] K-run qmv, pairs {dt.name} b{bits} g{G} M{M} N{N} K{K}", flush=True)
+    lib = _ensure_init()
+    c = make_case(970 + M, dt, bits, G, M, N, K, bias_rule="midpoint")
+    bufs = [GpuBuffer.from_bytes(v) for v in (c.w.tobytes(), c.scales_bytes, c.biases_bytes, c.x_bytes)]
+    guard = b"\xcd" * 64
+    out = GpuBuffer.from_bytes(b"\xff" * (M * N * 2) + guard)
+    try:
+        assert lib.mtq_set_option(b"qmv.runs", option) == 0
+        name = ops.plan("qmm", dt, bits, G, M, N, K)[1][0][0]
+        assert ("qmv_runs_kernel<true" if option == 2 else "qmv_slices_kernel<true") in name
+        ops.qmm(dt, bits, G, *bufs, out, M, N, K)
+        raw = out.read_bytes(M * N * 2 + 64)
+        assert raw[-64:] == guard
+        exp = oracle.qmm_f64(c.w, c.scales_f, c.biases_f, c.x_f, M, N, K, bits, G).reshape(-1)
+        assert rel_err(unpack_f32(raw[:-64], dt), exp) <= TOL[dt]
+    finally:
+        lib.mtq_set_option(b"qmv.runs", 0)
+        for b in bufs + [out]:
+            b.free()
