@@ -450,6 +450,11 @@ MTQ_API int mtq_flush_cache(void);
  *   "qmv.gated_fused"      mtq_gated_rms_norm_qmv as one launch of the streaming kernel (hv * dv a multiple of 2048 up to
  *                          16384, dv = 32 .. 2048 in powers of two): 0 = for f16 / bf16, 1 = never (the activation is staged
  *                          in the library's buffer), 2 = wherever the shape allows
+ *   "qmv.held"             GEMV that holds its activations in LDS (f16 / bf16, codes of 2..6 and 8 bits, groups of 32, 64, 128,
+ *                          K % 128 == 0; one row, normalised first or not, or up to 16 that fit): 0 = where it is the fastest,
+ *                          1 = never, 2 = wherever the shape allows
+ *   "qmv.held_kp"          and its waves that share 16 weight rows: 0 = choose, or 1, 2, 4, 8, 16
+ *   "qmv.held_nb"          and such rows side by side in a workgroup: 0 = choose, or 1..16
  *   "qmv.norm_mfma"        mtq_rms_norm_qmv with the norm applied inside the matrix-core GEMV (4-bit codes, f16 / bf16):
  *                          0 = where it is faster than the streaming kernel's fused form, 1 = never, 2 = wherever the
  *                          shape allows

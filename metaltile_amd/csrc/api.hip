@@ -342,12 +342,60 @@ static int run_runs(int dtype, int bits, uint32_t G, int n, const void* const* w
     return launch_qmv_runs(p, all, l2);
 }
 
+// Whether a route that the caller has asked for stands against the GEMV that holds its activations in LDS.
+static bool held_barred() { return options().qmv_held == 1 || (options().qmv_held == 0 && (runs_barred() || options().qmv_runs || options().qmv_mfma || options().qmv_norm_mfma || options().qmv_gated_fused)); }
+
+// One activation row, normalised first or not, on that kernel; `preferred`: where the choice is its own.
+static int try_held(int dtype, int bits, uint32_t G, int n, const void* const* w, const void* const* s, const void* const* b, const void* x,
+                    void* const* outs, const uint32_t* N, uint32_t K, const HeldNorm& norm, bool preferred, const LaunchCtx& lc) {
+    if (held_barred() || (options().qmv_held == 0 && !preferred)) return ERR_UNSUPPORTED;
+    QmvParams p;
+    p.dtype = dtype; p.bits = bits; p.group_size = G; p.x = x; p.M = 1; p.K = K;
+    QmvBatch all;
+    all.n = n;
+    for (int j = 0; j < n; j++) { all.w[j] = w[j]; all.scales[j] = s[j]; all.biases[j] = b[j]; all.out[j] = outs[j]; all.N[j] = N[j]; }
+    if (!qmv_held_takes(p, all, norm)) return ERR_UNSUPPORTED;
+    return launch_qmv_held(p, all, norm, lc);
+}
+
+// The matrices of a batch that it is for, in one launch; taken[j] as in run_runs, where matrices marked already are left out.
+static int run_held(int dtype, int bits, uint32_t G, int n, const void* const* w, const void* const* s, const void* const* b, const void* x,
+                    void* const* outs, uint32_t M, const uint32_t* N, uint32_t K, bool* taken, const LaunchCtx& lc) {
+    if (held_barred()) return ERR_OK;
+    QmvParams p;
+    p.dtype = dtype; p.bits = bits; p.group_size = G; p.x = x; p.M = M; p.K = K;
+    QmvBatch all;
+    all.n = 0;
+    int left = 0;
+    bool mine[4] = {}, started = false;
+    for (int j = 0; j < n; j++) {
+        if (taken[j]) { started = true; continue; }
+        QmvBatch one;
+        one.n = 1;
+        one.w[0] = w[j]; one.scales[0] = s[j]; one.biases[0] = b[j]; one.out[0] = outs[j]; one.N[0] = N[j];
+        mine[j] = (options().qmv_held == 2 || qmv_held_preferred(bits, M, N[j], K)) && qmv_held_takes(p, one, HeldNorm());
+        if (!mine[j]) { left++; continue; }
+        const int i = all.n++;
+        all.w[i] = w[j]; all.scales[i] = s[j]; all.biases[i] = b[j]; all.out[i] = outs[j]; all.N[i] = N[j];
+    }
+    if (all.n == 0) return ERR_OK;
+    LaunchCtx l2 = lc;
+    if (started) l2.start = nullptr;
+    if (left) l2.stop = nullptr;
+    for (int j = 0; j < n; j++) taken[j] = taken[j] || mine[j];
+    return launch_qmv_held(p, all, HeldNorm(), l2);
+}
+
 static int op_qmv(int dtype, int bits, uint32_t G, const void* w, const void* s, const void* b,
                   const void* x, void* out, uint32_t M, uint32_t N, uint32_t K, const LaunchCtx& lc) {
     int rc = check_common(dtype, bits, G, N, K);
     if (rc) return rc;
     if (M == 0) return ERR_OK;
     if (!w || !s || !b || !x || !out) return fail(ERR_BAD_ARG, "null buffer");
+    if (M == 1) {
+        rc = try_held(dtype, bits, G, 1, &w, &s, &b, x, &out, &N, K, HeldNorm(), false, lc);
+        if (rc != ERR_UNSUPPORTED) return rc;
+    }
     rc = try_wide(dtype, bits, G, w, s, b, x, out, M, N, K, true, lc);
     if (rc != ERR_UNSUPPORTED) return rc;
     if (dtype == DT_F32) {
@@ -390,8 +438,10 @@ static int op_qmm(int dtype, int bits, uint32_t G, const void* w, const void* s,
     if (!w || !s || !b || !x || !out) return fail(ERR_BAD_ARG, "null buffer");
     if (dtype == DT_F32 && options().qmm_f32_tiles != 1) return op_qmv(dtype, bits, G, w, s, b, x, out, M, N, K, lc);
     if (!force_mma) {
-        bool taken;
-        rc = run_runs(dtype, bits, G, 1, &w, &s, &b, x, &out, M, &N, K, &taken, lc);
+        bool taken = false;
+        rc = options().qmv_held == 2 ? ERR_OK : run_runs(dtype, bits, G, 1, &w, &s, &b, x, &out, M, &N, K, &taken, lc);
+        if (rc || taken) return rc;
+        rc = run_held(dtype, bits, G, 1, &w, &s, &b, x, &out, M, &N, K, &taken, lc);
         if (rc || taken) return rc;
         rc = try_slices(dtype, bits, G, w, s, b, x, out, M, N, K, lc);
         if (rc != ERR_UNSUPPORTED) return rc;
@@ -528,6 +578,13 @@ static int op_rms_norm_qmv(int dtype, int bits, uint32_t G, const void* x, const
     QmvParams p;
     p.dtype = dtype; p.bits = bits; p.group_size = G; p.w = w; p.scales = s; p.biases = b; p.x = x; p.out = out;
     p.N = N; p.K = K;
+    HeldNorm hn;
+    hn.mode = 1; hn.weight = norm_w; hn.eps = eps;
+    const bool held = qmv_held_norm_preferred(bits, G, N, K);
+    if (options().qmv_held == 2) {
+        rc = try_held(dtype, bits, G, 1, &w, &s, &b, x, &out, &N, K, hn, true, lc);
+        if (rc != ERR_UNSUPPORTED) return rc;
+    }
     // 4-bit f16 / bf16: the norm applied as the matrix-core GEMV stages its row (two staged rows share one set of 4;
     // no per-workgroup renormalisation beyond the sum of squares). us, streaming kernel -> this: 14336 x 4096 12.6 ->
     // 10.6, 6144 x 4096 8.1 -> 7.3; it loses on short matrices and long rows (4096 x 4096 6.2 -> 6.4, 4096 x 14336 13.7 -> 14.1).
@@ -551,6 +608,10 @@ static int op_rms_norm_qmv(int dtype, int bits, uint32_t G, const void* x, const
         rc = launch_qmv_rows_norm(p, norm_w, eps, lc);
         if (rc != ERR_UNSUPPORTED) return rc;
     }
+    if (bits == 4) {
+        rc = try_held(dtype, bits, G, 1, &w, &s, &b, x, &out, &N, K, hn, held, lc);
+        if (rc != ERR_UNSUPPORTED) return rc;
+    }
     const bool norm_on_mfma = options().qmv_norm_mfma == 2 ||
                               (options().qmv_norm_mfma == 0 && K <= 8192 && (uint64_t)N * K >= 24000000ull);
     if (bits == 4 && dtype != DT_F32 && norm_on_mfma) {
@@ -561,7 +622,13 @@ static int op_rms_norm_qmv(int dtype, int bits, uint32_t G, const void* x, const
         rc = launch_qmv_mfma(pm, lc);
         if (rc != ERR_UNSUPPORTED) return rc;
     }
+    if (bits == 2) {   // (2 bits: the rows that the streaming kernel takes too)
+        rc = try_held(dtype, bits, G, 1, &w, &s, &b, x, &out, &N, K, hn, held, lc);
+        if (rc != ERR_UNSUPPORTED) return rc;
+    }
     rc = launch_qmv_norm(p, norm_w, eps, lc);
+    if (rc != ERR_UNSUPPORTED) return rc;
+    rc = try_held(dtype, bits, G, 1, &w, &s, &b, x, &out, &N, K, hn, held, lc);
     if (rc != ERR_UNSUPPORTED) return rc;
     return qmv_of_staged_row(dtype, bits, G, w, s, b, out, N, K, lc, [&](void* dst, const LaunchCtx& ctx) {
         return launch_rms_norm(dtype, x, norm_w, eps, dst, K, ctx);
@@ -581,6 +648,12 @@ static int op_gated_rms_norm_qmv(int dtype, uint32_t G, const float* y, const vo
     int rc = check_common(dtype, 4, G, N, K);
     if (rc) return rc;
     if (!y || !z || !norm_w || !eps || !w || !s || !b || !out) return fail(ERR_BAD_ARG, "null buffer");
+    HeldNorm hn;
+    hn.mode = 2; hn.weight = norm_w; hn.gate = z; hn.eps = eps; hn.dv = dv;
+    if (options().qmv_held == 2) {
+        rc = try_held(dtype, 4, G, 1, &w, &s, &b, y, &out, &N, K, hn, true, lc);
+        if (rc != ERR_UNSUPPORTED) return rc;
+    }
     // One launch: the streaming kernel gates and normalises the slice each thread holds. us per call, staged (three
     // launches; two for f32) -> one launch, dv 128: bf16 hv 16, 2048 rows 7.7 -> 5.1 (the plain qmv of that matrix: 3.3);
     // hv 32, 1024 rows 10.3 -> 5.7; hv 32, 4096 rows 9.3 -> 8.0; hv 64, 8192 rows 14.8 -> 14.5. f32 stays staged (6.3 -> 6.9,
@@ -592,6 +665,10 @@ static int op_gated_rms_norm_qmv(int dtype, uint32_t G, const float* y, const vo
         rc = launch_qmv_gated_norm(p, z, norm_w, eps, dv, lc);
         if (rc != ERR_UNSUPPORTED) return rc;
     }
+    // row lengths that it does not take: the GEMV that holds the row in LDS (2560 rows, hv 8 / 24 / 40 of dv 128, us, norm, GEMV and sum
+    // -> this: 11.1 -> 6.3, 12.2 -> 7.7, 12.6 -> 9.5)
+    rc = try_held(dtype, 4, G, 1, &w, &s, &b, y, &out, &N, K, hn, true, lc);
+    if (rc != ERR_UNSUPPORTED) return rc;
     return qmv_of_staged_row(dtype, 4, G, w, s, b, out, N, K, lc, [&](void* dst, const LaunchCtx& ctx) {
         return launch_gated_rms_norm(dtype, y, z, norm_w, eps, dst, hv, dv, ctx);
     });
@@ -613,7 +690,11 @@ static int op_qmv_batched(int dtype, int bits, uint32_t G, int n, const void* co
         QmvBatch qb;
         qb.n = n;
         for (int j = 0; j < n; j++) { qb.w[j] = w[j]; qb.scales[j] = s[j]; qb.biases[j] = b[j]; qb.out[j] = outs[j]; qb.N[j] = N[j]; }
-        int rc = launch_qmv_batched(p, qb, lc);
+        int rc = options().qmv_held == 2 ? ERR_UNSUPPORTED : launch_qmv_batched(p, qb, lc);
+        if (rc != ERR_UNSUPPORTED) return rc;
+        // row lengths that the batched kernels do not take, or widths (4096, 2048, 16, 16 rows, us, a launch each -> this: 1024 codes
+        // 17.0 -> 8.4, 2304 19.6 -> 8.1, 4736 21.1 -> 10.5)
+        rc = try_held(dtype, bits, G, n, w, s, b, x, outs, N, K, HeldNorm(), true, lc);
         if (rc != ERR_UNSUPPORTED) return rc;
     }
     for (int j = 0; j < n; j++) {
@@ -644,7 +725,9 @@ static int op_qmm_batched(int dtype, int bits, uint32_t G, int n, const void* co
         if (!w[j] || !s[j] || !b[j] || !outs[j]) return fail(ERR_BAD_ARG, "null buffer");
     bool taken[4] = {};
     if (!exact) {
-        int rc = run_runs(dtype, bits, G, n, w, s, b, x, outs, M, N, K, taken, lc);
+        int rc = options().qmv_held == 2 ? ERR_OK : run_runs(dtype, bits, G, n, w, s, b, x, outs, M, N, K, taken, lc);
+        if (rc) return rc;
+        rc = run_held(dtype, bits, G, n, w, s, b, x, outs, M, N, K, taken, lc);
         if (rc) return rc;
     }
     // what is left of the batch on the tile kernels goes there together
@@ -1877,6 +1960,21 @@ int mtq_set_option(const char* name, int value) {
     if (!strcmp(name, "moe_down.rows")) {
         if (value < 0 || value > 4096) return fail(ERR_BAD_ARG, "moe_down.rows must be in 0..4096");
         options().moe_down_rows = value;
+        return MTQ_OK;
+    }
+    if (!strcmp(name, "qmv.held")) {
+        if (value < 0 || value > 2) return fail(ERR_BAD_ARG, "qmv.held must be 0 (auto), 1 (off) or 2 (wherever the shape allows)");
+        options().qmv_held = value;
+        return MTQ_OK;
+    }
+    if (!strcmp(name, "qmv.held_kp")) {
+        if (value != 0 && value != 1 && value != 2 && value != 4 && value != 8 && value != 16) return fail(ERR_BAD_ARG, "qmv.held_kp must be 0, 1, 2, 4, 8 or 16");
+        options().qmv_held_kp = value;
+        return MTQ_OK;
+    }
+    if (!strcmp(name, "qmv.held_nb")) {
+        if (value < 0 || value > 16) return fail(ERR_BAD_ARG, "qmv.held_nb must be in 0..16");
+        options().qmv_held_nb = value;
         return MTQ_OK;
     }
     if (!strcmp(name, "qmv.kernel")) {

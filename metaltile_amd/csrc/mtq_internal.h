@@ -119,6 +119,9 @@ struct Options {
     int qmv_wide_nb = 0;          // 16-row matrix-core GEMV: row blocks per wave (0 = choose; 1, 2)
     int gather_wide = 0;          // expert-routed rows on the 16-row matrix-core GEMV: 0 = choose, 1 = never, 2 = wherever the shape allows
     int qmv_runs = 0;             // K-run matrix-core GEMV for batches of up to 16 rows: 0 = choose per shape, 1 = never, 2 = wherever the shape allows, 3 = the K-sliced form wherever the shape allows
+    int qmv_held = 0;             // GEMV with its activations in LDS: 0 = choose per shape, 1 = never, 2 = wherever the shape allows
+    int qmv_held_kp = 0;          // and its waves that share 16 weight rows (0 = choose; 1, 2, 4, 8, 16),
+    int qmv_held_nb = 0;          // its blocks side by side in a workgroup (0 = choose)
     int scratch_most_kb = 0;      // largest library-owned scratch buffer (0 = no limit): a call that needs more finds no memory
     int qmv_wide = 0;             // 16-row matrix-core GEMV for batches of 5..16 rows: 0 = choose per shape, 1 = never, 2 = wherever the shape allows
 };
@@ -196,6 +199,20 @@ bool qmv_slices_takes(const QmmParams& p);
 bool qmv_slices_preferred(int bits, uint32_t G, uint32_t M, uint32_t N, uint32_t K);
 size_t qmv_slices_scratch_bytes(const QmmParams& p);
 int launch_qmv_slices(const QmmParams& p, const LaunchCtx& lc, void* scratch);
+// GEMV with its activations in LDS (qmv_held.hip): 1..16 activation rows (as many as fit) against 1..4 matrices of one row length, f16 /
+// bf16, codes of 2..6 and 8 bits, K % 128 == 0, groups of 32, 64, 128 (p: dtype, bits, group size, x, M, K). The one row may be
+// RMS-normalised or gated and normalised per head first. A matrix gives the same bits alone and in a batch.
+struct HeldNorm {
+    int mode = 0;                    // 0 none, 1 RMS norm, 2 gated norm (x: f32 [K], heads of dv)
+    const void* weight = nullptr;
+    const void* gate = nullptr;
+    const float* eps = nullptr;
+    uint32_t dv = 0;
+};
+bool qmv_held_takes(const QmvParams& p, const QmvBatch& b, const HeldNorm& n);
+bool qmv_held_norm_preferred(int bits, uint32_t G, uint32_t N, uint32_t K);
+bool qmv_held_preferred(int bits, uint32_t M, uint32_t N, uint32_t K);   // one matrix's sizes
+int launch_qmv_held(const QmvParams& p, const QmvBatch& b, const HeldNorm& n, const LaunchCtx& lc);
 // Adds f32 partial results [slices][total] in slice order and rounds to the element type (qmv_wide.hip).
 int add_slices(int dtype, const float* part, void* out, uint32_t total, uint32_t slices, const LaunchCtx& lc);
 // f32 operands on the f32 matrix cores, any code width (qmm_f32.hip).

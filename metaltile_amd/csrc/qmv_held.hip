@@ -1,0 +1,147 @@
+// Host side of the GEMV with its activations in LDS (kernel in qmv_held_impl.h): which calls it takes and its geometry.
+#include "qmv_held_pick.h"
+
+namespace mtq {
+
+// (instances: one translation unit per element type and kind of group)
+HeldInstance qmv_held_pick_f16(int bits, int mode, uint32_t rows);
+HeldInstance qmv_held_pick_f16_g32(int bits, int mode, uint32_t rows);
+HeldInstance qmv_held_pick_bf16(int bits, int mode, uint32_t rows);
+HeldInstance qmv_held_pick_bf16_g32(int bits, int mode, uint32_t rows);
+
+static HeldInstance held_pick(int dtype, int bits, uint32_t G, int mode, uint32_t rows) {
+    if (dtype == DT_BF16) return G == 32 ? qmv_held_pick_bf16_g32(bits, mode, rows) : qmv_held_pick_bf16(bits, mode, rows);
+    return G == 32 ? qmv_held_pick_f16_g32(bits, mode, rows) : qmv_held_pick_f16(bits, mode, rows);
+}
+
+static uint32_t held_log2rp(uint32_t rows) {
+    uint32_t l = 0;
+    while ((1u << l) < rows) l++;
+    return l;
+}
+static uint32_t held_cus() {
+    int dev = 0, cus = 256;
+    if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    return (uint32_t)cus;
+}
+
+// The waves of a workgroup: KP share 16 weight rows, NB such rows side by side.
+struct HeldGeometry {
+    HeldInstance k;
+    uint32_t kpl, nb, per_cu;   // per_cu: workgroups on a compute unit
+    uint32_t lds;
+};
+static bool held_geometry(int dtype, int bits, uint32_t G, int mode, uint32_t rows, uint32_t K, uint32_t blocks, HeldGeometry& g) {
+    const Options& o = options();
+    const uint32_t cus = held_cus(), rpl = held_log2rp(rows), pairs = (K / 128u + 1u) / 2u;
+    g.k = held_pick(dtype, bits, G, mode, rows);
+    if (!g.k.fn) return false;
+    // KP: what brings a thousand waves to the matrix, each with two and a half steps of 128 codes or more; at least four on long
+    // rows. bf16, groups of 64, RMS norm included, KP 1 / 2 / 4 / 8, us: 1536 x 1280 7.0 5.8 5.6 5.5, 2816 x 2304 9.4 7.6 6.6 7.0, 14080 x 2304 11.7
+    // 9.4 10.5 11.8, 88612 x 2816 27.7 29.0 29.7 39.3, 5 bits 20480 x 2560 14.3 14.9 15.1 15.1, 57344 x 7808 77.2 80.5 70.7 72.0, 6 bits 86686 x 1408
+    // 24.6 26.5 26.0; without a norm 3 bits 5120 x 5120 15.3 11.8 9.0 9.9, 5 bits 2560 x 10240 29.3 17.8 11.4 10.1. For several rows by the row length alone, so that a matrix gives the same bits alone and in a batch (5 rows, 5
+    // bits, 3 x 3456 x 3456 13.0 12.0 14.6, 2 x 14720 x 3456 22.5 22.8 24.1).
+    uint32_t kpl = K > 4608 ? 2 : 0;
+    const bool fixed = mode == HELD_PLAIN && rows > 1;
+    while (kpl < (fixed ? 2u : 4u) && (fixed || (blocks << kpl) < 1024u) && (K / 128u) * 2u >= 5u << (kpl + 1)) kpl++;
+    if (o.qmv_held_kp) for (kpl = 0; (2u << kpl) <= (uint32_t)o.qmv_held_kp; kpl++) {}
+    while (kpl && (1u << kpl) > pairs) kpl--;
+    // a normalised row: at most two pieces of 16 elements a thread
+    const uint32_t least = mode == HELD_PLAIN ? 1u : (K / 16u + 127u) / 128u;
+    for (uint32_t most = 8; most <= 16; most += 8) {   // waves
+        if ((1u << kpl) > most) continue;
+        uint32_t nb = most >> kpl;
+        while (nb > 1 && g.k.lds(K, rpl, nb << kpl) > 160u * 1024u) nb--;
+        g.lds = g.k.lds(K, rpl, nb << kpl);
+        if (g.lds > 160u * 1024u) return false;
+        g.per_cu = most == 8 && g.lds <= 80u * 1024u ? 2u : 1u;
+        const uint32_t want = (blocks + cus * g.per_cu - 1u) / (cus * g.per_cu);
+        if (nb > want) nb = want ? want : 1u;
+        if (o.qmv_held_nb && (uint32_t)o.qmv_held_nb <= most >> kpl) nb = (uint32_t)o.qmv_held_nb;
+        while ((nb << kpl) < least && ((nb + 1u) << kpl) <= most) nb++;
+        g.kpl = kpl;
+        g.nb = nb;
+        g.lds = g.k.lds(K, rpl, nb << kpl);
+        if ((nb << kpl) >= least && g.lds <= 160u * 1024u && (most == 16 || g.per_cu == 2)) return true;
+    }
+    return false;
+}
+
+// p: dtype, bits, group size, x, M, K
+bool qmv_held_takes(const QmvParams& p, const QmvBatch& b, const HeldNorm& n) {
+    const uint32_t G = p.group_size, K = p.K, rows = n.mode == HELD_PLAIN ? p.M : 2u;
+    if ((p.dtype != DT_F16 && p.dtype != DT_BF16) || (p.bits != 2 && p.bits != 3 && p.bits != 4 && p.bits != 5 && p.bits != 6 && p.bits != 8)) return false;
+    if ((G != 32 && G != 64 && G != 128) || K == 0 || K % 128 || K % G || rows == 0 || rows > 16 || b.n < 1 || b.n > 4 || K > (1u << 17)) return false;
+    if ((uintptr_t)p.x % 16) return false;
+    if (n.mode != HELD_PLAIN && ((uintptr_t)n.weight % 16 || (uintptr_t)n.eps % 4)) return false;
+    if (n.mode == HELD_GATED && ((uintptr_t)n.gate % 16 || n.dv < 16 || n.dv > 1024 || (n.dv & (n.dv - 1)))) return false;   // a head's pieces in neighbouring lanes of a wave
+    uint64_t blocks = 0;
+    for (int j = 0; j < b.n; j++) {
+        if (b.N[j] == 0 || (uintptr_t)b.w[j] % 16 || (uintptr_t)b.scales[j] % 4 || (uintptr_t)b.biases[j] % 4) return false;
+        blocks += (b.N[j] + 15u) / 16u;
+    }
+    HeldGeometry g;
+    return blocks < (1u << 26) && held_geometry(p.dtype, p.bits, G, n.mode, rows, K, (uint32_t)blocks, g);
+}
+
+// Where the kernel stands against the others: they have a launch per matrix, or three where a row is normalised first and their
+// row lengths are not the ones it is fused for. us, bf16, groups of 64, others -> this.
+// RMS norm, 4 bits: 1280 x 1024 9.5 -> 5.0, 2816 x 2304 11.1 -> 6.8, 5248 x 4224 14.0 -> 10.0 (norm, GEMV, sum); against the norm inside the
+// matrix-core GEMV, from 24 M codes: 14080 x 2304 10.4 -> 9.4, 19200 x 3200 15.9 -> 14.7, 67882 x 2304 26.0 -> 21.3, 25344 x 4224 24.7 -> 19.2,
+// but 23040 x 3840 15.1 -> 15.6, 32256 x 5376 21.4 -> 22.2, 46080 x 7680 36.7 -> 39.8. 2 bits 4096 x 1024 11.1 -> 5.6, 16384 x 4096 15.2 -> 10.6, 32768 x
+// 8192 31.3 -> 25.9; 3 bits 14720 x 3456 16.3 -> 11.4, 5 bits 20480 x 2560 23.8 -> 14.8, 57344 x 7808 83.2 -> 80.7, 6 bits 131838 x 1408 54.6 -> 35.0;
+// 8 bits 14336 x 1664 14.2 -> 9.5, 30000 x 3712 31.6 -> 24.0, but 20480 x 5120 23.1 -> 24.3. 4 bits in groups of 32: 14080 x 2304 11.2 -> 10.1,
+// 86686 x 1280 20.2 -> 18.5, but 86686 x 1664 21.5 -> 24.7.
+bool qmv_held_norm_preferred(int bits, uint32_t G, uint32_t N, uint32_t K) {
+    if (bits == 8) return K < 5120;
+    if (bits == 4 && G == 32 && K > 1600 && (uint64_t)N * K >= 60000000ull) return false;
+    return bits != 4 || (uint64_t)N * K < 24000000ull || K <= 3200 || (K > 4096 && K < 5120);
+}
+// Batches of 2..16 rows, of the widths that the K-run kernel has not (alone | three, or two tall ones, in a call):
+// 3 bits, 4 rows 4096 x 4096 6.6 -> 7.3 | 19.8 -> 9.2; 5 bits, 5 rows 3456 x 3456 8.4 -> 8.6 | 25.1 -> 13.0; 14720 x 3456 15.2 -> 13.9 | 30.5 -> 22.4;
+// 6 bits, 8 rows 1024 x 4096 10.2 -> 8.0, 14336 x 4096 17.6 -> 15.3; 3 bits, 9 rows 1152 x 1152 9.3 -> 6.4; 5 bits, 16 rows 2048 x 2048 9.8 -> 7.6, 4096 x
+// 4096 12.0 -> 11.7, but 14336 x 4096 18.6 -> 21.3 (tiles); 2 bits, 4 rows 2304 x 2304 6.7 -> 7.1, 20000 x 2048 13.2 -> 9.5, 16 rows 3328 x 3328
+// 13.5 -> 8.6, 13312 x 3328 15.7 -> 12.6. Rows of more than 8192 codes leave a compute unit one workgroup: 3 bits, 4 rows 4096 x 11008
+// 11.1 -> 13.4.
+bool qmv_held_preferred(int bits, uint32_t M, uint32_t N, uint32_t K) {
+    if (M < 2 || M > 16 || bits == 4 || bits == 8) return false;
+    return M <= 8 ? K <= 8192 : K <= 4096 && (N <= 8192 || bits == 2);
+}
+
+int launch_qmv_held(const QmvParams& p, const QmvBatch& b, const HeldNorm& n, const LaunchCtx& lc) {
+    if (!qmv_held_takes(p, b, n)) return fail(ERR_UNSUPPORTED, "GEMV with its activations in LDS: shape not taken");
+    const uint32_t rows = n.mode == HELD_PLAIN ? p.M : 2u;
+    QmvHeldArgs a{};
+    for (int j = 0; j < 4; j++) {
+        a.first[j] = 0x7FFFFFFFu;
+        if (j >= b.n) continue;
+        a.w[j] = (const unsigned char*)b.w[j];
+        a.scales[j] = (const unsigned char*)b.scales[j];
+        a.biases[j] = (const unsigned char*)b.biases[j];
+        a.out[j] = (uint16_t*)b.out[j];
+        a.N[j] = b.N[j];
+        a.first[j] = a.blocks;
+        a.blocks += (b.N[j] + 15u) / 16u;
+    }
+    a.x = (const unsigned char*)p.x;
+    a.norm_w = (const unsigned char*)n.weight;
+    a.gate = (const unsigned char*)n.gate;
+    a.eps = n.eps;
+    a.dv = n.dv;
+    a.M = n.mode == HELD_PLAIN ? p.M : 1u;
+    a.K = p.K;
+    while ((1u << a.log2g) < p.group_size) a.log2g++;
+    HeldGeometry g;
+    if (!held_geometry(p.dtype, p.bits, p.group_size, n.mode, rows, p.K, a.blocks, g)) return fail(ERR_UNSUPPORTED, "GEMV with its activations in LDS: geometry");
+    a.log2kp = g.kpl;
+    a.log2rp = held_log2rp(rows);
+    a.waves = g.nb << g.kpl;
+    const uint32_t tasks = (a.blocks + g.nb - 1u) / g.nb, most = held_cus() * g.per_cu, wgs = tasks < most ? tasks : most;
+    hipError_t e = set_max_dynamic_lds(g.k.fn, g.lds);
+    if (e != hipSuccess) return hip_fail(e, "GEMV with its activations in LDS: LDS");
+    void* args[] = {&a};
+    e = launch_kernel(g.k.fn, dim3(wgs), dim3(a.waves * 64u), args, g.lds, lc);
+    return e == hipSuccess ? ERR_OK : hip_fail(e, "GEMV with its activations in LDS: kernel launch");
+}
+
+}  // namespace mtq

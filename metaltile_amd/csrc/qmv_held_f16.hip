@@ -1,0 +1,7 @@
+#include "qmv_held_pick.h"
+
+namespace mtq {
+
+HeldInstance qmv_held_pick_f16(int bits, int mode, uint32_t rows) { return held_pick_bits<DT_F16, false>(bits, mode, rows); }
+
+}  // namespace mtq
