@@ -24,7 +24,9 @@ static bool runs_aligned(const void* w, const void* s, const void* b, const void
 RunsInstance qmv_runs_pick_f16(bool paired, int bits, uint32_t G, bool sliced, uint32_t xs, bool few);
 RunsInstance qmv_runs_pick_bf16(bool paired, int bits, uint32_t G, bool sliced, uint32_t xs, bool few);
 static RunsInstance runs_pick(int dtype, int bits, uint32_t G, uint32_t K, bool sliced, uint32_t xs, uint32_t M) {
-    const bool paired = (uint64_t)K * bits / 8 % 128 == 0;   // rows of whole 128-byte lines
+    // Rows of whole 128-byte lines; not where sixteen waves have a pair each and a few of them a step more, which the others wait for
+    // (bf16, groups of 64, 5 rows, 2 x 10240, us, runs -> pairs: K = 4352 17.5 -> 18.0, 4608 17.5 -> 18.5, but 5120 and 5376 alike or faster).
+    const bool paired = (uint64_t)K * bits / 8 % 128 == 0 && !(bits == 4 && !sliced && K > 4096 && K < 5120);
     return dtype == DT_BF16 ? qmv_runs_pick_bf16(paired, bits, G, sliced, xs, M <= 8) : qmv_runs_pick_f16(paired, bits, G, sliced, xs, M <= 8);
 }
 

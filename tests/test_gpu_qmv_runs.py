@@ -205,7 +205,7 @@ def test_operands_off_16_bytes(oracle, which):
 
 @pytest.mark.parametrize("dt", [DType.F16, DType.BF16], ids=lambda d: d.name)
 @pytest.mark.parametrize("option,bits,G,M,N,K", [
-    (2, 4, 64, 16, 40, 256), (2, 4, 128, 9, 24, 768), (2, 4, 64, 5, 33, 4352), (2, 4, 32, 16, 20, 4864), (2, 4, 64, 3, 17, 6400),
+    (2, 4, 64, 16, 40, 256), (2, 4, 128, 9, 24, 768), (2, 4, 64, 5, 33, 5376), (2, 4, 32, 16, 20, 5888), (2, 4, 64, 3, 17, 6400),
     (2, 8, 64, 16, 40, 128), (2, 8, 32, 7, 24, 2176), (2, 8, 128, 16, 33, 4224), (2, 8, 64, 4, 17, 4992),
     (3, 4, 64, 16, 40, 8448), (3, 4, 128, 5, 33, 13824), (3, 8, 64, 9, 24, 5248), (3, 8, 128, 3, 40, 15232),
 ])
