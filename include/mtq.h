@@ -455,6 +455,11 @@ MTQ_API int mtq_flush_cache(void);
  *                          1 = never, 2 = wherever the shape allows
  *   "qmv.held_kp"          and its waves that share 16 weight rows: 0 = choose, or 1, 2, 4, 8, 16
  *   "qmv.held_nb"          and such rows side by side in a workgroup: 0 = choose, or 1..16
+ *   "qmv.codes"            GEMV on codes, activations streamed through LDS (f16 / bf16, codes of 2..6 and 8 bits, groups of 32, 64, 128,
+ *                          K % 128 == 0, up to 1024 rows): 0 = where it is the fastest, 1 = never, 2 = wherever the shape allows
+ *   "qmv.codes_kw" / "qmv.codes_nw" / "qmv.codes_stage" / "qmv.codes_slices"
+ *                          and its waves that share weight rows (1, 2, 4, 8), waves along N (up to 16), steps of activations between
+ *                          barriers (1, 2, 4) and slices of K (up to 64); 0 = choose
  *   "qmv.norm_mfma"        mtq_rms_norm_qmv with the norm applied inside the matrix-core GEMV (4-bit codes, f16 / bf16):
  *                          0 = where it is faster than the streaming kernel's fused form, 1 = never, 2 = wherever the
  *                          shape allows

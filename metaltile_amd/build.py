@@ -27,8 +27,8 @@ HIPFLAGS = [
 ]
 # per-source additions: the wave-per-four-rows GEMV keeps its matrix-core results in ordinary vector registers (no accumulator-register copies)
 EXTRA_FLAGS = {"qmv_rows.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"], "qmv_rows_few.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"], "qmv_rows_walk.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
-EXTRA_FLAGS.update({f"qmv_held_{d}{g}.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"] for d in ("f16", "bf16") for g in ("", "_g32")})
-SOURCES = ["api.hip", "qmv.hip", "qmv_f32.hip", "qmv_f16.hip", "qmv_bf16.hip", "qmv_mfma.hip", "qmv_mfma_f16.hip", "qmv_mfma_bf16.hip", "qmv_mfma_f16_odd.hip", "qmv_mfma_bf16_odd.hip", "qmv_wide.hip", "qmv_wide_gather.hip", "qmv_runs.hip", "qmv_runs_f16.hip", "qmv_runs_bf16.hip", "qmv_held.hip", "qmv_held_f16.hip", "qmv_held_f16_g32.hip", "qmv_held_bf16.hip", "qmv_held_bf16_g32.hip", "generic.hip", "qmm.hip", "qmm_direct.hip", "qmm_direct_odd.hip", "qmm_dma.hip", "qmm_dma_b8.hip", "qmm_dma_routed.hip", "qmm_dma_routed_b8.hip", "qmm_f32.hip", "affine.hip", "norm.hip", "moe.hip", "moe_down.hip", "qvm.hip", "qmv_rows.hip", "qmv_rows_few.hip", "qmv_rows_walk.hip"]
+EXTRA_FLAGS.update({f"qmv_{k}_{d}{g}.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"] for k in ("codes", "held") for d in ("f16", "bf16") for g in ("", "_g32")})
+SOURCES = ["api.hip", "qmv.hip", "qmv_f32.hip", "qmv_f16.hip", "qmv_bf16.hip", "qmv_mfma.hip", "qmv_mfma_f16.hip", "qmv_mfma_bf16.hip", "qmv_mfma_f16_odd.hip", "qmv_mfma_bf16_odd.hip", "qmv_wide.hip", "qmv_wide_gather.hip", "qmv_runs.hip", "qmv_runs_f16.hip", "qmv_runs_bf16.hip", "qmv_codes.hip", "qmv_codes_f16.hip", "qmv_codes_f16_g32.hip", "qmv_codes_bf16.hip", "qmv_codes_bf16_g32.hip", "qmv_held.hip", "qmv_held_f16.hip", "qmv_held_f16_g32.hip", "qmv_held_bf16.hip", "qmv_held_bf16_g32.hip", "generic.hip", "qmm.hip", "qmm_direct.hip", "qmm_direct_odd.hip", "qmm_dma.hip", "qmm_dma_b8.hip", "qmm_dma_routed.hip", "qmm_dma_routed_b8.hip", "qmm_f32.hip", "affine.hip", "norm.hip", "moe.hip", "moe_down.hip", "qvm.hip", "qmv_rows.hip", "qmv_rows_few.hip", "qmv_rows_walk.hip"]
 
 
 def _headers():

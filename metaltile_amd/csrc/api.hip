@@ -386,6 +386,76 @@ static int run_held(int dtype, int bits, uint32_t G, int n, const void* const* w
     return launch_qmv_held(p, all, HeldNorm(), l2);
 }
 
+// Whether a matrix is for the GEMV on codes. Of more than 96 rows only what the tiles cannot split (at K >= 8192 they mostly can, in tiles of 128
+// rows: 3584 x 12928, 5 bits, 126 rows 40.6 us in K splits, 55.2 here, 96 rows 38.5 and 36.2; 2304 x 8320, unsplit, 126 rows 100.8 -> 30.4).
+static bool codes_serve(const QmmParams& q) {
+    if (!qmv_codes_takes(q)) return false;
+    if (options().qmv_codes == 2) return true;
+    if (!qmv_codes_preferred(q.bits, q.M, q.N, q.K) || !tiles_serve(q.bits, q.M, q.N, q.K) || slices_serve(q) || wide_serves(q, false)) return false;
+    QmmDLaunch l;
+    return q.M <= 96 || plan_qmm_direct(q, l) != ERR_OK || !l.split;
+}
+
+// The matrices of a batch (or the one of a single call) that the GEMV on codes is for, in one launch; taken[j] as above, where
+// matrices marked already are left out.
+static int run_codes(int dtype, int bits, uint32_t G, int n, const void* const* w, const void* const* s, const void* const* b,
+                     const void* x, void* const* outs, uint32_t M, const uint32_t* N, uint32_t K, bool* taken, const LaunchCtx& lc) {
+    const Options& o = options();
+    if (o.qmv_codes == 1 || (o.qmv_codes == 0 && (runs_barred() || o.qmv_runs || o.qmv_held))) return ERR_OK;
+    QmmParams q;
+    q.dtype = dtype; q.bits = bits; q.group_size = G; q.x = x; q.M = M; q.K = K;
+    QmvBatch all;
+    all.n = 0;
+    CodesSplit split[4];
+    size_t needs[4], total = 0;
+    bool started = false, tried = false;
+    int at[4], left = 0;
+    auto gather = [&](bool fits) {   // fits: only what there is memory for by itself
+        all.n = left = 0;
+        total = 0;
+        started = false;
+        for (int j = 0; j < n; j++) {
+            if (taken[j]) { started = true; continue; }
+            q.w = w[j]; q.scales = s[j]; q.biases = b[j]; q.out = outs[j]; q.N = N[j];
+            if (!codes_serve(q)) { left++; continue; }
+            const CodesSplit sp = qmv_codes_split(q);
+            const size_t need = qmv_codes_scratch_bytes(q, sp);
+            if (fits && need && ensure_scratch(g.scratch_held + need)) { left++; continue; }
+            const int i = all.n++;
+            at[i] = j;
+            split[i] = sp;
+            needs[i] = need;
+            total += need;
+            all.w[i] = w[j]; all.scales[i] = s[j]; all.biases[i] = b[j]; all.out[i] = outs[j]; all.N[i] = N[j];
+        }
+    };
+    gather(false);
+    // without memory for all sums at once one matrix follows the other; without any for a matrix it is left to the other kernels
+    if (total && ensure_scratch(g.scratch_held + total)) {
+        tried = true;
+        gather(true);
+    }
+    if (all.n == 0) return ERR_OK;
+    const int per = tried ? 1 : all.n;
+    for (int i = 0; i < all.n; i += per) {
+        QmvBatch now;
+        now.n = per;
+        size_t need = 0;
+        for (int k = 0; k < per; k++) {
+            now.w[k] = all.w[i + k]; now.scales[k] = all.scales[i + k]; now.biases[k] = all.biases[i + k]; now.out[k] = all.out[i + k]; now.N[k] = all.N[i + k];
+            need += needs[i + k];
+            taken[at[i + k]] = true;
+        }
+        LaunchCtx l2 = lc;
+        if (started) l2.start = nullptr;
+        if (left || i + per < all.n) l2.stop = nullptr;
+        started = true;
+        int rc = launch_qmv_codes(q, now, split + i, need ? (char*)g.scratch_buf + g.scratch_held : nullptr, l2);
+        if (rc) return rc;
+    }
+    return ERR_OK;
+}
+
 static int op_qmv(int dtype, int bits, uint32_t G, const void* w, const void* s, const void* b,
                   const void* x, void* out, uint32_t M, uint32_t N, uint32_t K, const LaunchCtx& lc) {
     int rc = check_common(dtype, bits, G, N, K);
@@ -439,9 +509,13 @@ static int op_qmm(int dtype, int bits, uint32_t G, const void* w, const void* s,
     if (dtype == DT_F32 && options().qmm_f32_tiles != 1) return op_qmv(dtype, bits, G, w, s, b, x, out, M, N, K, lc);
     if (!force_mma) {
         bool taken = false;
-        rc = options().qmv_held == 2 ? ERR_OK : run_runs(dtype, bits, G, 1, &w, &s, &b, x, &out, M, &N, K, &taken, lc);
-        if (rc || taken) return rc;
-        rc = run_held(dtype, bits, G, 1, &w, &s, &b, x, &out, M, &N, K, &taken, lc);
+        if (options().qmv_codes != 2) {
+            rc = options().qmv_held == 2 ? ERR_OK : run_runs(dtype, bits, G, 1, &w, &s, &b, x, &out, M, &N, K, &taken, lc);
+            if (rc || taken) return rc;
+            rc = run_held(dtype, bits, G, 1, &w, &s, &b, x, &out, M, &N, K, &taken, lc);
+            if (rc || taken) return rc;
+        }
+        rc = run_codes(dtype, bits, G, 1, &w, &s, &b, x, &out, M, &N, K, &taken, lc);
         if (rc || taken) return rc;
         rc = try_slices(dtype, bits, G, w, s, b, x, out, M, N, K, lc);
         if (rc != ERR_UNSUPPORTED) return rc;
@@ -725,9 +799,14 @@ static int op_qmm_batched(int dtype, int bits, uint32_t G, int n, const void* co
         if (!w[j] || !s[j] || !b[j] || !outs[j]) return fail(ERR_BAD_ARG, "null buffer");
     bool taken[4] = {};
     if (!exact) {
-        int rc = options().qmv_held == 2 ? ERR_OK : run_runs(dtype, bits, G, n, w, s, b, x, outs, M, N, K, taken, lc);
-        if (rc) return rc;
-        rc = run_held(dtype, bits, G, n, w, s, b, x, outs, M, N, K, taken, lc);
+        int rc = ERR_OK;
+        if (options().qmv_codes != 2) {
+            rc = options().qmv_held == 2 ? ERR_OK : run_runs(dtype, bits, G, n, w, s, b, x, outs, M, N, K, taken, lc);
+            if (rc) return rc;
+            rc = run_held(dtype, bits, G, n, w, s, b, x, outs, M, N, K, taken, lc);
+            if (rc) return rc;
+        }
+        rc = run_codes(dtype, bits, G, n, w, s, b, x, outs, M, N, K, taken, lc);
         if (rc) return rc;
     }
     // what is left of the batch on the tile kernels goes there together
@@ -1975,6 +2054,31 @@ int mtq_set_option(const char* name, int value) {
     if (!strcmp(name, "qmv.held_nb")) {
         if (value < 0 || value > 16) return fail(ERR_BAD_ARG, "qmv.held_nb must be in 0..16");
         options().qmv_held_nb = value;
+        return MTQ_OK;
+    }
+    if (!strcmp(name, "qmv.codes")) {
+        if (value < 0 || value > 2) return fail(ERR_BAD_ARG, "qmv.codes must be 0 (auto), 1 (off) or 2 (wherever the shape allows)");
+        options().qmv_codes = value;
+        return MTQ_OK;
+    }
+    if (!strcmp(name, "qmv.codes_kw")) {
+        if (value != 0 && value != 1 && value != 2 && value != 4 && value != 8) return fail(ERR_BAD_ARG, "qmv.codes_kw must be 0, 1, 2, 4 or 8");
+        options().qmv_codes_kw = value;
+        return MTQ_OK;
+    }
+    if (!strcmp(name, "qmv.codes_nw")) {
+        if (value < 0 || value > 16) return fail(ERR_BAD_ARG, "qmv.codes_nw must be in 0..16");
+        options().qmv_codes_nw = value;
+        return MTQ_OK;
+    }
+    if (!strcmp(name, "qmv.codes_stage")) {
+        if (value != 0 && value != 1 && value != 2 && value != 4) return fail(ERR_BAD_ARG, "qmv.codes_stage must be 0, 1, 2 or 4");
+        options().qmv_codes_stage = value;
+        return MTQ_OK;
+    }
+    if (!strcmp(name, "qmv.codes_slices")) {
+        if (value < 0 || value > 64) return fail(ERR_BAD_ARG, "qmv.codes_slices must be in 0..64");
+        options().qmv_codes_slices = value;
         return MTQ_OK;
     }
     if (!strcmp(name, "qmv.kernel")) {

@@ -122,6 +122,11 @@ struct Options {
     int qmv_held = 0;             // GEMV with its activations in LDS: 0 = choose per shape, 1 = never, 2 = wherever the shape allows
     int qmv_held_kp = 0;          // and its waves that share 16 weight rows (0 = choose; 1, 2, 4, 8, 16),
     int qmv_held_nb = 0;          // its blocks side by side in a workgroup (0 = choose)
+    int qmv_codes = 0;            // matrix-core GEMV on codes (1..1024 rows): 0 = choose per shape, 1 = never, 2 = wherever the shape allows
+    int qmv_codes_kw = 0;         // and its waves that share weight rows (0 = choose; 1, 2, 4, 8),
+    int qmv_codes_nw = 0;         // its waves along N (0 = choose),
+    int qmv_codes_stage = 0;      // its steps of activations between barriers (0 = choose; 1, 2, 4),
+    int qmv_codes_slices = 0;     // its slices of K (0 = choose)
     int scratch_most_kb = 0;      // largest library-owned scratch buffer (0 = no limit): a call that needs more finds no memory
     int qmv_wide = 0;             // 16-row matrix-core GEMV for batches of 5..16 rows: 0 = choose per shape, 1 = never, 2 = wherever the shape allows
 };
@@ -213,6 +218,17 @@ bool qmv_held_takes(const QmvParams& p, const QmvBatch& b, const HeldNorm& n);
 bool qmv_held_norm_preferred(int bits, uint32_t G, uint32_t N, uint32_t K);
 bool qmv_held_preferred(int bits, uint32_t M, uint32_t N, uint32_t K);   // one matrix's sizes
 int launch_qmv_held(const QmvParams& p, const QmvBatch& b, const HeldNorm& n, const LaunchCtx& lc);
+// Matrix-core GEMV on codes (qmv_codes.hip): 1..1024 activation rows, f16 / bf16, codes of 2..6 and 8 bits, K % 128 == 0, the matrices of
+// `b` (1..4, same row length) in one launch (p: dtype, bits, group size, x, M, K). A matrix gives the same bits alone and in a batch.
+// split: qmv_codes_split of each matrix; scratch: the sum of qmv_codes_scratch_bytes over the matrices (0: may be null).
+struct CodesSplit {
+    uint32_t kwl = 0, slices = 0;   // log2 of the waves that share weight rows; slices of K (0: no geometry fits)
+};
+bool qmv_codes_takes(const QmmParams& p);
+bool qmv_codes_preferred(int bits, uint32_t M, uint32_t N, uint32_t K);
+CodesSplit qmv_codes_split(const QmmParams& p);
+size_t qmv_codes_scratch_bytes(const QmmParams& p, const CodesSplit& s);
+int launch_qmv_codes(const QmmParams& p, const QmvBatch& b, const CodesSplit* split, void* scratch, const LaunchCtx& lc);
 // Adds f32 partial results [slices][total] in slice order and rounds to the element type (qmv_wide.hip).
 int add_slices(int dtype, const float* part, void* out, uint32_t total, uint32_t slices, const LaunchCtx& lc);
 // f32 operands on the f32 matrix cores, any code width (qmm_f32.hip).

@@ -1,0 +1,248 @@
+// Host side of the matrix-core GEMV on codes (kernel in qmv_codes_impl.h): which calls it takes and its geometry.
+#include "qmv_codes_pick.h"
+
+namespace mtq {
+
+// (instances: one translation unit per element type, kind of group and row count)
+CodesInstance qmv_codes_pick_f16(int bits, uint32_t mt);
+CodesInstance qmv_codes_pick_f16_g32(int bits, uint32_t mt);
+CodesInstance qmv_codes_pick_bf16(int bits, uint32_t mt);
+CodesInstance qmv_codes_pick_bf16_g32(int bits, uint32_t mt);
+
+static CodesInstance codes_pick(int dtype, int bits, uint32_t G, uint32_t mt) {
+    if (dtype == DT_BF16) return G == 32 ? qmv_codes_pick_bf16_g32(bits, mt) : qmv_codes_pick_bf16(bits, mt);
+    return G == 32 ? qmv_codes_pick_f16_g32(bits, mt) : qmv_codes_pick_f16(bits, mt);
+}
+
+constexpr uint32_t QC_LDS = 160u * 1024u;   // of a compute unit
+
+// Tiles of up to 48 activation rows, all of one height but the last.
+struct CodesRows {
+    uint32_t tiles, rows, mt;   // mt: 16-row operand tiles of one
+};
+static CodesRows codes_rows(uint32_t M) {
+    CodesRows r;
+    r.tiles = (M + 47u) / 48u;
+    r.rows = (M + r.tiles - 1u) / r.tiles;
+    r.mt = (r.rows + 15u) / 16u;
+    r.tiles = (M + r.rows - 1u) / r.rows;
+    return r;
+}
+
+bool qmv_codes_takes(const QmmParams& p) {
+    const uint32_t G = p.group_size, M = p.M, N = p.N, K = p.K;
+    if ((p.dtype != DT_F16 && p.dtype != DT_BF16) || (p.bits != 2 && p.bits != 3 && p.bits != 4 && p.bits != 5 && p.bits != 6 && p.bits != 8)) return false;
+    if ((G != 32 && G != 64 && G != 128) || M == 0 || M > 1024 || N == 0 || K == 0 || K % 128 || K % G) return false;
+    if ((uintptr_t)p.w % 16 || (uintptr_t)p.x % 16 || (uintptr_t)p.scales % 4 || (uintptr_t)p.biases % 4) return false;
+    // offsets of 32 bits: into 32 weight rows, into x; workgroups and partial results
+    return (uint64_t)K * p.bits / 8 * 32 < (1ull << 31) && (uint64_t)M * K * 2 < (1ull << 31) && N < (1u << 24) && (uint64_t)M * N < (1ull << 31);
+}
+
+// How a matrix is split, by what its own launch would take (us, about): workgroups fill the chip in rounds, one to a compute unit; a
+// step of 128 codes takes a workgroup 1.45 us, of eight waves as of five; slices of K cost a second launch. Tall matrices come in pairs, whose
+// waves cannot share rows in another way than those of one alone (2 x 8704 x 3712, 5 bits, 20 rows 37.9 -> 34.6).
+CodesSplit qmv_codes_split(const QmmParams& p) {
+    const CodesRows r = codes_rows(p.M);
+    const CodesInstance k = codes_pick(p.dtype, p.bits, p.group_size, r.mt);
+    const uint32_t N = p.N, steps = p.K / 128u, pair = N >= 2 * (uint64_t)p.K ? 2u : 1u;
+    const Options& o = options();
+    CodesSplit best;
+    float least = 1e30f;
+    for (uint32_t kwl = 0; kwl <= 3; kwl++) {
+        if (o.qmv_codes_kw && (1u << kwl) != (uint32_t)o.qmv_codes_kw) continue;
+        for (uint32_t nw = qc_min_nw(r.mt); nw << kwl <= QC_WAVES; nw++) {
+            if ((o.qmv_codes_nw && nw != (uint32_t)o.qmv_codes_nw) || k.lds(1u << kwl, 1, nw << kwl) > QC_LDS) continue;
+            const uint32_t tiles = (N + 32u * nw - 1u) / (32u * nw);
+            const float step_us = (r.mt == 1 ? 1.2f : r.mt == 2 ? 1.45f : 1.8f) * ((nw << kwl) <= 4 ? 0.8f : 1.0f);
+            for (uint32_t s = 1; s <= 16 && s <= steps; s++) {
+                if (o.qmv_codes_slices && s != (uint32_t)o.qmv_codes_slices) continue;
+                if (s > 1 && !o.qmv_codes_slices && (steps >> kwl) < 3u * s) break;
+                const uint32_t wgs = (tiles * s + 7u) / 8u * 8u * r.tiles * pair, per = (((steps + s - 1u) / s + 1u) / 2u + (1u << kwl) - 1u) >> kwl;
+                float us = 4.f + (float)((wgs + 255u) / 256u) * ((float)(2u * per) * step_us + 1.5f);
+                if (s > 1) us += 4.f + (float)(pair * s) * (float)p.M * (float)N * 8.0f / 4e6f;
+                if (us < least) { least = us; best = CodesSplit{kwl, s}; }
+            }
+        }
+    }
+    return best;
+}
+size_t qmv_codes_scratch_bytes(const QmmParams& p, const CodesSplit& s) { return s.slices > 1 ? ((size_t)s.slices * p.M * p.N * sizeof(float) + 255) & ~(size_t)255 : 0; }
+
+// Where the kernel stands against the tile kernels, which split K over workgroups only where it is a multiple of 256: short of
+// that a workgroup walks the whole row. us, bf16, groups of 64, tiles -> this:
+//                          16 rows            24                32                48                64                96                128
+//   4736 x 4736, 5 bits    54.6 -> 14.2       55.1 -> 17.2      56.1 -> 17.8      57.4 -> 20.6      58.5 -> 24.7      53.9 -> 27.6      54.4 -> 31.2
+//                4 bits                       32.4 -> 15.4      32.6 -> 15.9      33.2 -> 18.9      33.3 -> 21.4      32.5 -> 24.6      33.1 -> 27.3
+//   4736 x 20096, 5 bits   255 -> 31          259 -> 39         263 -> 39         270 -> 43         278 -> 65         95 -> 64          101 -> 84
+//                4 bits                       111 -> 33         112 -> 34         115 -> 38         120 -> 56         112 -> 55         45 -> 71
+//   2 x 20096 x 4736, 5 b. 121 -> 55          123 -> 64         124 -> 66         126 -> 77         130 -> 113        132 -> 130        141 -> 144
+//                4 bits    66 -> 46           67 -> 54          68 -> 57          69 -> 67          70 -> 97          94 -> 116
+//   3 matrices of 3200 x 1664, 5 bits         18.8 -> 12.3      19.0 -> 12.5      19.3 -> 15.0      19.6 -> 12.7      18.9 -> 16.9      19.0 -> 19.0
+//                4 bits                       13.9 -> 11.1      14.0 -> 11.4      14.0 -> 13.9      14.2 -> 11.6      14.1 -> 15.8
+// (4 bits, up to 16 rows: the K-run kernel, but for more than 75 M codes.) A matrix's route cannot depend on whether it comes in a batch,
+// and the tile kernels take the matrices of a batch in the time of one as long as they fill the chip together no more than once: so
+// not the tall matrices that come in pairs (2 x 9472 x 2176, 4 bits, 24 rows 22.6 -> 26.9; 2 x 8704 x 3968, 51 rows 30.9 -> 44.6; 2 x 5888 x 1664, 3 bits, 24 / 43 rows
+// 17.5 -> 12.1, 18.4 -> 20.0), and 4-bit
+// projections up to 48 rows only (5760 x 5760, 52 rows 39.2 -> 24.1, but three of them 40.6 -> 64.6).
+// Where the tiles split K they are the faster (4096 x 4096, 5 bits, 32 rows 13.1 -> 14.8; 2 x 14336 x 4096 40.0 -> 42.6), except for the
+// bit-stream widths on long rows (4096 x 14336, 5 bits, 16 / 32 / 48 rows 28.1 -> 20.5, 29.1 -> 25.4, 32.9 -> 29.3) and up to 16 rows of
+// many (14336 x 4096 18.8 -> 16.0).
+// A matrix of a fifth of its row length and less is a key or value projection, which comes beside a square one of its row length and goes
+// where that one goes (768 x 6528 next to 6528 x 6528, 4 bits, 55 rows: apart from it the layer 228 -> 242).
+bool qmv_codes_preferred(int bits, uint32_t M, uint32_t N, uint32_t K) {
+    const bool stream = bits == 3 || bits == 5 || bits == 6, tall = N >= 2 * (uint64_t)K, narrow = K >= 5 * (uint64_t)N, wide = K >= 2 * (uint64_t)N && !narrow;
+    const uint64_t codes = narrow ? (uint64_t)K * K : (uint64_t)N * K;
+    if (M < 5 || M > 128 || K < 1024) return false;
+    if (K % 256 == 0) return stream && M <= 48 && ((K > 8192 && K >= 2 * (uint64_t)N) || (M >= 9 && M <= 16 && N > 8192));
+    if (M <= 16) return stream || (uint64_t)N * K > 75000000ull;
+    if (wide) return stream || M <= 96;
+    if (tall) return M <= (bits == 3 ? 32u : 48u) && (stream || (M <= 32 && (codes > 90000000ull || K < 1536)));
+    if (M <= 48) return true;
+    return (stream || bits == 8) && (M <= 64 || (K >= 2048 && codes <= 40000000ull));
+}
+
+struct CodesReduceArgs {
+    const float* part[4];
+    uint16_t* out[4];
+    uint32_t total[4];    // results
+    uint32_t slices[4];
+    uint32_t first[4];    // first workgroup, of 1024 results each; 0x7FFFFFFF past the last matrix
+};
+
+// Adds the slices' f32 sums in slice order. One thread has four results in a row.
+template <int DT> __global__ __launch_bounds__(256) void qmv_codes_reduce_kernel(CodesReduceArgs a) {
+    uint32_t i = 0;
+#pragma unroll
+    for (uint32_t k = 1; k < 4; k++) i += blockIdx.x >= a.first[k] ? 1u : 0u;
+    const float* part = a.part[0];
+    uint16_t* out = a.out[0];
+    uint32_t total = a.total[0], slices = a.slices[0], first = a.first[0];
+#pragma unroll
+    for (uint32_t k = 1; k < 4; k++)
+        if (i == k) { part = a.part[k]; out = a.out[k]; total = a.total[k]; slices = a.slices[k]; first = a.first[k]; }
+    const uint32_t at = ((blockIdx.x - first) * 256u + threadIdx.x) * 4u;
+    if (at >= total) return;
+    if (total % 4u == 0 && (uintptr_t)out % 8u == 0) {
+        kr_f32x4 s = *(const kr_f32x4*)(part + at);
+        for (uint32_t k = 1; k < slices; k++) s += *(const kr_f32x4*)(part + (size_t)k * total + at);
+        *(kr_u32x2*)(out + at) = kr_u32x2{f32_to_elem_bits<DT>(s[0]) | ((uint32_t)f32_to_elem_bits<DT>(s[1]) << 16),
+                                          f32_to_elem_bits<DT>(s[2]) | ((uint32_t)f32_to_elem_bits<DT>(s[3]) << 16)};
+        return;
+    }
+    for (uint32_t e = at; e < at + 4u && e < total; e++) {
+        float s = part[e];
+        for (uint32_t k = 1; k < slices; k++) s += part[(size_t)k * total + e];
+        out[e] = f32_to_elem_bits<DT>(s);
+    }
+}
+
+// The matrices of `b` whose waves share rows alike, in one launch (p: dtype, bits, group size, x, M, K); the sums of sliced ones go to
+// `scratch` from `at` on.
+static int launch_codes_alike(const QmmParams& p, const QmvBatch& b, const CodesSplit* split, const bool* in, void* scratch, size_t& at, CodesReduceArgs& r, uint32_t& n_sliced,
+                              uint32_t& rblocks, const LaunchCtx& lc) {
+    const CodesRows rows = codes_rows(p.M);
+    const CodesInstance k = codes_pick(p.dtype, p.bits, p.group_size, rows.mt);
+    QmvCodesArgs a{};
+    uint32_t n = 0, kwl = 0, nw = QC_WAVES;
+    uint32_t tile_slices[4] = {};
+    for (int j = 0; j < b.n; j++) {
+        if (!in[j]) continue;
+        kwl = split[j].kwl;
+        a.w[n] = (const unsigned char*)b.w[j];
+        a.scales[n] = (const unsigned char*)b.scales[j];
+        a.biases[n] = (const unsigned char*)b.biases[j];
+        a.out[n] = (uint16_t*)b.out[j];
+        a.N[n] = b.N[j];
+        a.slices[n] = split[j].slices;
+        if (a.slices[n] > 1) {
+            if (!scratch) return fail(ERR_UNSUPPORTED, "GEMV on codes: no scratch");
+            a.part[n] = (float*)((char*)scratch + at);
+            at += ((size_t)a.slices[n] * p.M * b.N[j] * sizeof(float) + 255) & ~(size_t)255;
+            r.part[n_sliced] = a.part[n];
+            r.out[n_sliced] = a.out[n];
+            r.total[n_sliced] = p.M * b.N[j];
+            r.slices[n_sliced] = a.slices[n];
+            r.first[n_sliced++] = rblocks;
+            rblocks += (p.M * b.N[j] + 1023u) / 1024u;
+        }
+        n++;
+    }
+    // waves along N: the fewest rounds of workgroups over the chip, and of those the most waves
+    uint32_t least = ~0u;
+    for (uint32_t t = qc_min_nw(rows.mt); t << kwl <= QC_WAVES; t++) {
+        if (k.lds(1u << kwl, 1, t << kwl) > QC_LDS) break;
+        uint32_t wgs = 0;
+        for (uint32_t j = 0; j < n; j++) wgs += ((a.N[j] + 32u * t - 1u) / (32u * t) * a.slices[j] + 7u) / 8u * 8u * rows.tiles;
+        if ((wgs + 255u) / 256u < least) { least = (wgs + 255u) / 256u; nw = t; }
+    }
+    if (options().qmv_codes_nw) nw = (uint32_t)options().qmv_codes_nw;
+    uint32_t stage = k.stage;
+    if (options().qmv_codes_stage && (uint32_t)options().qmv_codes_stage < stage) stage = (uint32_t)options().qmv_codes_stage;
+    while (stage > 1 && k.lds(1u << kwl, stage, nw << kwl) > QC_LDS) stage /= 2;
+    const uint32_t shmem = k.lds(1u << kwl, stage, nw << kwl);
+    if (nw < qc_min_nw(rows.mt) || (nw << kwl) > QC_WAVES || shmem > QC_LDS) return fail(ERR_BAD_ARG, "GEMV on codes: geometry");
+    uint32_t wgs = 0;
+    for (uint32_t j = 0; j < 4; j++) {
+        a.first[j] = 0x7FFFFFFFu;
+        if (j >= n) { a.slices[j] = 1; continue; }
+        a.first[j] = wgs;
+        tile_slices[j] = (a.N[j] + 32u * nw - 1u) / (32u * nw) * a.slices[j];
+        wgs += (tile_slices[j] + 7u) / 8u * 8u * rows.tiles;
+    }
+    a.x = (const unsigned char*)p.x;
+    a.M = p.M;
+    a.K = p.K;
+    a.m_tiles = rows.tiles;
+    a.m_rows = rows.rows;
+    while ((1u << a.log2g) < p.group_size) a.log2g++;
+    a.log2kw = kwl;
+    a.waves = nw << kwl;
+    a.log2stage = stage == 4 ? 2u : stage == 2 ? 1u : 0u;
+    hipError_t e = set_max_dynamic_lds(k.fn, shmem);
+    if (e != hipSuccess) return hip_fail(e, "GEMV on codes: LDS");
+    void* args[] = {&a};
+    e = launch_kernel(k.fn, dim3(wgs), dim3(a.waves * 64u), args, shmem, lc);
+    return e == hipSuccess ? ERR_OK : hip_fail(e, "GEMV on codes: kernel launch");
+}
+
+int launch_qmv_codes(const QmmParams& p, const QmvBatch& b, const CodesSplit* split, void* scratch, const LaunchCtx& lc) {
+    bool done[4] = {}, any_sliced = false;
+    for (int j = 0; j < b.n; j++) {
+        QmmParams q = p;
+        q.w = b.w[j]; q.scales = b.scales[j]; q.biases = b.biases[j]; q.out = b.out[j]; q.N = b.N[j];
+        if (!qmv_codes_takes(q)) return fail(ERR_UNSUPPORTED, "GEMV on codes: shape not taken");
+        if (split[j].slices == 0) return fail(ERR_BAD_ARG, "GEMV on codes: geometry");
+        any_sliced = any_sliced || split[j].slices > 1;
+    }
+    CodesReduceArgs r{};
+    uint32_t n_sliced = 0, rblocks = 0;
+    size_t at = 0;
+    int left = b.n;
+    bool started = false;
+    while (left) {
+        bool in[4] = {};
+        int kwl = -1;
+        for (int j = 0; j < b.n; j++) {
+            if (done[j] || (kwl >= 0 && split[j].kwl != (uint32_t)kwl)) continue;
+            kwl = (int)split[j].kwl;
+            in[j] = done[j] = true;
+            left--;
+        }
+        LaunchCtx l = lc;
+        if (started) l.start = nullptr;
+        if (left || any_sliced) l.stop = nullptr;
+        started = true;
+        int rc = launch_codes_alike(p, b, split, in, scratch, at, r, n_sliced, rblocks, l);
+        if (rc) return rc;
+    }
+    if (!n_sliced) return ERR_OK;
+    for (uint32_t j = n_sliced; j < 4; j++) r.first[j] = 0x7FFFFFFFu;
+    LaunchCtx l2 = lc;
+    l2.start = nullptr;
+    void* rargs[] = {&r};
+    const void* fn = p.dtype == DT_BF16 ? (const void*)qmv_codes_reduce_kernel<DT_BF16> : (const void*)qmv_codes_reduce_kernel<DT_F16>;
+    hipError_t e = launch_kernel(fn, dim3(rblocks), dim3(256), rargs, 0, l2);
+    return e == hipSuccess ? ERR_OK : hip_fail(e, "GEMV on codes: reduce kernel launch");
+}
+
+}  // namespace mtq

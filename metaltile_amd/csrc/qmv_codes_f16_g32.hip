@@ -1,0 +1,7 @@
+#include "qmv_codes_pick.h"
+
+namespace mtq {
+
+CodesInstance qmv_codes_pick_f16_g32(int bits, uint32_t mt) { return codes_pick<DT_F16, true>(bits, mt); }
+
+}  // namespace mtq
