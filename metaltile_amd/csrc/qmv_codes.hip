@@ -70,23 +70,28 @@ size_t qmv_codes_scratch_bytes(const QmmParams& p, const CodesSplit& s) { return
 
 // Where the kernel stands against the tile kernels, which split K over workgroups only where it is a multiple of 256: short of
 // that a workgroup walks the whole row. us, bf16, groups of 64, tiles -> this:
-//                          16 rows            24                32                48                64                96                128
-//   4736 x 4736, 5 bits    54.6 -> 14.2       55.1 -> 17.2      56.1 -> 17.8      57.4 -> 20.6      58.5 -> 24.7      53.9 -> 27.6      54.4 -> 31.2
-//                4 bits                       32.4 -> 15.4      32.6 -> 15.9      33.2 -> 18.9      33.3 -> 21.4      32.5 -> 24.6      33.1 -> 27.3
-//   4736 x 20096, 5 bits   255 -> 31          259 -> 39         263 -> 39         270 -> 43         278 -> 65         95 -> 64          101 -> 84
-//                4 bits                       111 -> 33         112 -> 34         115 -> 38         120 -> 56         112 -> 55         45 -> 71
-//   2 x 20096 x 4736, 5 b. 121 -> 55          123 -> 64         124 -> 66         126 -> 77         130 -> 113        132 -> 130        141 -> 144
-//                4 bits    66 -> 46           67 -> 54          68 -> 57          69 -> 67          70 -> 97          94 -> 116
-//   3 matrices of 3200 x 1664, 5 bits         18.8 -> 12.3      19.0 -> 12.5      19.3 -> 15.0      19.6 -> 12.7      18.9 -> 16.9      19.0 -> 19.0
-//                4 bits                       13.9 -> 11.1      14.0 -> 11.4      14.0 -> 13.9      14.2 -> 11.6      14.1 -> 15.8
-// (4 bits, up to 16 rows: the K-run kernel, but for more than 75 M codes.) A matrix's route cannot depend on whether it comes in a batch,
-// and the tile kernels take the matrices of a batch in the time of one as long as they fill the chip together no more than once: so
-// not the tall matrices that come in pairs (2 x 9472 x 2176, 4 bits, 24 rows 22.6 -> 26.9; 2 x 8704 x 3968, 51 rows 30.9 -> 44.6; 2 x 5888 x 1664, 3 bits, 24 / 43 rows
-// 17.5 -> 12.1, 18.4 -> 20.0), and 4-bit
-// projections up to 48 rows only (5760 x 5760, 52 rows 39.2 -> 24.1, but three of them 40.6 -> 64.6).
+//                                   20 rows            32                40                48                60                96               128
+//   4736 x 4736, 5 bits             55.1 -> 17.2       56.1 -> 17.8                        57.4 -> 20.6      58.5 -> 24.7      53.9 -> 27.6     54.4 -> 31.2
+//                4 bits             32.4 -> 15.4       32.6 -> 15.9                        33.2 -> 18.9      33.3 -> 21.4      32.5 -> 24.6     33.1 -> 27.3
+//   4736 x 20096, 5 bits            259 -> 39          263 -> 39                           270 -> 43         278 -> 65         95 -> 64         101 -> 84
+//                4 bits             111 -> 33          112 -> 34                           115 -> 38         120 -> 56         112 -> 55        45 -> 71
+//   2 x 20096 x 4736, 5 bits        120.9 -> 70.7      124.3 -> 72.5     124.6 -> 74.3     125.9 -> 76.1     128.0 -> 112.5    132 -> 130
+//                4 bits             66.3 -> 58.8       67.4 -> 60.6      68.2 -> 64.6      68.6 -> 66.8      69.4 -> 96.3
+//                8 bits             107.3 -> 71.9      108.1 -> 73.6     108.3 -> 75.9     108.7 -> 77.8     109.9 -> 115.1
+//   2 x 9472 x 2176, 5 bits         28.2 -> 19.6       28.7 -> 20.3      28.8 -> 23.4      29.1 -> 23.9      29.3 -> 27.7
+//                4 bits             21.2 -> 17.3       21.1 -> 18.1      21.3 -> 21.0      21.4 -> 21.4      21.8 -> 24.0
+//                8 bits             25.5 -> 21.2       26.0 -> 21.9      26.2 -> 24.7      26.3 -> 25.0      26.7 -> 29.2
+//   2 x 8704 x 3968, 5 bits         49.8 -> 27.9       51.0 -> 28.6      51.3 -> 32.6      51.8 -> 33.0      52.8 -> 55.4
+//   1664, 1664, 1664 x 1664, 5 bits 21.7 -> 12.5       22.3 -> 13.0      22.4 -> 15.2      22.5 -> 16.0      22.9 -> 13.3
+//                4 bits             16.6 -> 11.2       16.6 -> 11.6      16.7 -> 13.9      16.7 -> 14.8      16.8 -> 12.0
+//   3968, 992, 992 x 3968, 4 bits   28.6 -> 15.4       28.9 -> 16.8      29.1 -> 21.1      29.5 -> 29.8      29.6 -> 26.6
+// (2 bits as 4, 3 and 6 bits as 5; up to 16 rows 4- and 8-bit codes have the K-run kernel, but for more than 75 M codes: 4736 x 4736, 5 bits, 54.6 -> 14.2.) A
+// matrix's route cannot depend on whether it comes in a batch, and the tile kernels take the matrices of a batch in the time of one
+// as long as they fill the chip together no more than once: three of 5760 x 5760, 4 bits, 20 / 48 rows 39.2 -> 45.2, 40.5 -> 51.1, one of
+// them 39.2 -> 24.1, which a layer has beside the three; at 60 rows 40.9 -> 64.9, so up to 48 rows there.
 // Where the tiles split K they are the faster (4096 x 4096, 5 bits, 32 rows 13.1 -> 14.8; 2 x 14336 x 4096 40.0 -> 42.6), except for the
 // bit-stream widths on long rows (4096 x 14336, 5 bits, 16 / 32 / 48 rows 28.1 -> 20.5, 29.1 -> 25.4, 32.9 -> 29.3) and up to 16 rows of
-// many (14336 x 4096 18.8 -> 16.0).
+// many (2 x 14336 x 4096, 5 bits, 12 rows 35.9 -> 27.3).
 // A matrix of a fifth of its row length and less is a key or value projection, which comes beside a square one of its row length and goes
 // where that one goes (768 x 6528 next to 6528 x 6528, 4 bits, 55 rows: apart from it the layer 228 -> 242).
 bool qmv_codes_preferred(int bits, uint32_t M, uint32_t N, uint32_t K) {
@@ -96,8 +101,8 @@ bool qmv_codes_preferred(int bits, uint32_t M, uint32_t N, uint32_t K) {
     if (K % 256 == 0) return stream && M <= 48 && ((K > 8192 && K >= 2 * (uint64_t)N) || (M >= 9 && M <= 16 && N > 8192));
     if (M <= 16) return stream || (uint64_t)N * K > 75000000ull;
     if (wide) return stream || M <= 96;
-    if (tall) return M <= (bits == 3 ? 32u : 48u) && (stream || (M <= 32 && (codes > 90000000ull || K < 1536)));
-    if (M <= 48) return true;
+    if (tall) return M <= (stream ? (K < 2304 || codes > 90000000ull ? 64u : 48u) : bits == 8 || codes > 90000000ull ? 48u : 32u);
+    if (M <= 48 || (M <= 64 && K <= 5632)) return true;
     return (stream || bits == 8) && (M <= 64 || (K >= 2048 && codes <= 40000000ull));
 }
 
