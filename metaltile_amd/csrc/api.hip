@@ -391,7 +391,7 @@ static int run_held(int dtype, int bits, uint32_t G, int n, const void* const* w
 static bool codes_serve(const QmmParams& q) {
     if (!qmv_codes_takes(q)) return false;
     if (options().qmv_codes == 2) return true;
-    if (!qmv_codes_preferred(q.bits, q.M, q.N, q.K) || !tiles_serve(q.bits, q.M, q.N, q.K) || slices_serve(q) || wide_serves(q, false)) return false;
+    if (!qmv_codes_preferred(q.bits, q.group_size, q.M, q.N, q.K) || !tiles_serve(q.bits, q.M, q.N, q.K) || slices_serve(q) || wide_serves(q, false)) return false;
     QmmDLaunch l;
     return q.M <= 96 || plan_qmm_direct(q, l) != ERR_OK || !l.split;
 }

@@ -225,7 +225,7 @@ struct CodesSplit {
     uint32_t kwl = 0, slices = 0;   // log2 of the waves that share weight rows; slices of K (0: no geometry fits)
 };
 bool qmv_codes_takes(const QmmParams& p);
-bool qmv_codes_preferred(int bits, uint32_t M, uint32_t N, uint32_t K);
+bool qmv_codes_preferred(int bits, uint32_t G, uint32_t M, uint32_t N, uint32_t K);
 CodesSplit qmv_codes_split(const QmmParams& p);
 size_t qmv_codes_scratch_bytes(const QmmParams& p, const CodesSplit& s);
 int launch_qmv_codes(const QmmParams& p, const QmvBatch& b, const CodesSplit* split, void* scratch, const LaunchCtx& lc);
