@@ -77,6 +77,7 @@ size_t qmv_codes_scratch_bytes(const QmmParams& p, const CodesSplit& s) { return
 //                4 bits             111 -> 33          112 -> 34                           115 -> 38         120 -> 56         112 -> 55        45 -> 71
 //   2 x 20096 x 4736, 5 bits        120.9 -> 70.7      124.3 -> 72.5     124.6 -> 74.3     125.9 -> 76.1     128.0 -> 112.5    132 -> 130
 //                4 bits             66.3 -> 58.8       67.4 -> 60.6      68.2 -> 64.6      68.6 -> 66.8      69.4 -> 96.3
+// (one of them alone, 4 bits, 20 / 48 rows 34.9 -> 35.9, 36.9 -> 42.1: 4 bits up to 32 rows)
 //                8 bits             107.3 -> 71.9      108.1 -> 73.6     108.3 -> 75.9     108.7 -> 77.8     109.9 -> 115.1
 //   2 x 9472 x 2176, 5 bits         28.2 -> 19.6       28.7 -> 20.3      28.8 -> 23.4      29.1 -> 23.9      29.3 -> 27.7
 //                4 bits             21.2 -> 17.3       21.1 -> 18.1      21.3 -> 21.0      21.4 -> 21.4      21.8 -> 24.0
@@ -90,24 +91,21 @@ size_t qmv_codes_scratch_bytes(const QmmParams& p, const CodesSplit& s) { return
 // as long as they fill the chip together no more than once: three of 5760 x 5760, 4 bits, 20 / 48 rows 39.2 -> 45.2, 40.5 -> 51.1, one of
 // them 39.2 -> 24.1, which a layer has beside the three; at 60 rows 40.9 -> 64.9, so up to 48 rows there.
 // Where the tiles split K (rows of a multiple of 256 codes; a matrix of at most half as many tiles of 128 columns as there are compute units) they
-// are the faster: 4096 x 4096, 5 bits, 32 rows 13.1 -> 14.8; 2 x 8192 x 2048, 4 bits, 20 rows 9.7 -> 11.8. They are not on the tall matrices
-// that are just past that, as long as the workgroups of a pair come to one round, or to full ones, over the chip (2 x N x K; us, tiles -> this):
-//                          20 rows         48              77                         20 rows         48              77
-//   9216 x 2304, 6 bits    31.1 -> 19.6    38.8 -> 23.4    54.4 -> 32.3    4 bits     24.3 -> 17.0    30.9 -> 20.9    37.0 -> 29.0
-//   10240 x 2560           26.3 -> 20.1    35.8 -> 24.0    46.8 -> 34.8               21.1 -> 17.1    27.9 -> 21.2    34.7 -> 31.3
-//   11008 x 4096           36.6 -> 27.8    51.0 -> 33.0    68.6 -> 54.3               26.6 -> 23.8    34.6 -> 28.9    45.6 -> 46.9
-//   14336 x 4096           37.7 -> 33.3    51.7 -> 39.4    70.3 -> 59.0               27.4 -> 26.2    36.1 -> 31.2    50.0 -> 49.7
-//   18944 x 3584           43.6 -> 39.5    62.7 -> 46.9    74.8 -> 94.0               31.1 -> 33.5    46.2 -> 42.1    57.9 -> 75.4
-//   22016 x 4096           47.0 -> 46.9    72.0 -> 56.9    86.3 -> 101.8              33.4 -> 38.0    49.0 -> 47.9    64.8 -> 81.3
-//   28672 x 8192           124.7 -> 98.1   176.9 -> 121.0  252.5 -> 217.7             67.8 -> 79.8    106.4 -> 97.3   127.5 -> 181.1
-//   8192 x 2048            11.9 -> 15.1    15.7 -> 21.2    27.5 -> 21.2               9.7 -> 11.8     12.1 -> 18.7    21.9 -> 18.6
-// (8 bits: as 4 at 10240 and 77 rows, 45.2 -> 37.5, and as 6 at 28672 and up to 48, 157.8 -> 125.3; alone, 28672 x 4096 at 77 rows, 6 bits 56.0 -> 58.8,
-// 128256 x 4096 194.6 -> 241.8.) And not on long rows: bit-stream widths past 8192 codes (4096 x 14336, 5 bits, 16 / 32 / 48 rows 28.1 -> 20.5,
+// are the faster: 4096 x 4096, 5 bits, 32 rows 13.1 -> 14.8; 2 x 8192 x 2048, 4 bits, 20 rows 9.7 -> 11.8. Past that pairs of matrices are faster here up to
+// 48 rows, but one of them alone is not, on half the workgroups (us, 6 bits, tiles -> this, 20 and 48 rows):
+//   2 x 14336 x 4096   37.7 -> 33.3   51.7 -> 39.4    one   18.8 -> 21.2   25.9 -> 31.8
+//   2 x 18944 x 3584   43.6 -> 39.5   62.7 -> 46.9    one   29.0 -> 29.7   42.6 -> 34.9
+//   28672 x 4096                                      one   34.1 -> 33.7   49.1 -> 41.2
+//   2 x 28672 x 8192   124.7 -> 98.1  176.9 -> 121.0  57344 x 8192 120.2 -> 98.4  202.1 -> 120.0
+//   128256 x 4096                                     one   130.5 -> 111.1 147.5 -> 135.0
+// So from 16385 rows of weights on, where a pair's workgroups come to one round over the chip or to full ones. 8 bits: the last two only (57344 x 8192 124.1 -> 112.3,
+// 151.1 -> 128.9; 128256 x 4096 131.2 -> 130.1, 167.8 -> 145.7; 28672 x 4096 33.1 -> 38.6); 3 bits from 33 rows on (28672 x 4096, 20 / 48 rows 25.5 -> 30.9, 38.6
+// -> 37.7); 4 bits are not (2 x 28672 x 8192 67.8 -> 79.8). Past 48 rows neither are
+// the others (128256 x 4096, 6 bits, 77 rows 194.6 -> 241.8). On long rows: bit-stream widths past 8192 codes (4096 x 14336, 5 bits, 16 / 32 / 48 rows 28.1 -> 20.5,
 // 29.1 -> 25.4, 32.9 -> 29.3; 5120 x 20480, 6 bits, 77 rows 85.0 -> 67.4, but 3584 x 18944 45.0 -> 47.9), 8 bits past 16384 (5120 x 20480, 48 / 77 rows 60.5 -> 44.0,
 // 138 -> 66.7; 20 rows 30.9 -> 38.3), 4 bits there at few rows of weights (3584 x 18944, 77 rows 51.1 -> 42.0, 8192 x 28672 88.2 -> 95.0).
-// Groups of 32 cost the tiles nothing and a second product per operand here: 2- and 4-bit codes are left there on rows of 1152 (1152 x 1152, 20 rows 10.8
-// -> 12.3), on 2 x 14336 x 4096 (28.3 -> 31.6) and from 49 rows on (2 x 10496 x 2560, 77 rows 34.8 -> 38.5), bit-stream widths on the smaller
-// long rows (2560 x 10496, 3 bits, 30 rows 17.1 -> 18.8).
+// Groups of 32 cost the tiles nothing and a second scaling per group here: 2- and 4-bit codes are left there on rows of 1152 (1152 x 1152, 20 rows 10.8
+// -> 12.3), bit-stream widths on the smaller long rows (2560 x 10496, 3 bits, 30 rows 17.1 -> 18.8).
 // A matrix of a fifth of its row length and less is a key or value projection, which comes beside a square one of its row length and goes
 // where that one goes (768 x 6528 next to 6528 x 6528, 4 bits, 55 rows: apart from it the layer 228 -> 242); so is a wider one on rows shorter
 // than any that MLP activations have, or a quarter of rows that are long for them.
@@ -119,23 +117,18 @@ bool qmv_codes_preferred(int bits, uint32_t G, uint32_t M, uint32_t N, uint32_t 
     if (M < 5 || M > 128 || K < 1024 || (g32 && K < 1280 && M > 16)) return false;
     if (K % 256 == 0) {
         if (K >= 2 * (uint64_t)N) {
-            if (stream) return K > 8192 && (M <= 48 || (M <= 96 && N >= 5120)) && (G != 32 || (uint64_t)N * K > 33000000ull);
+            if (stream) return K > 8192 && (M <= 48 || (M <= 96 && N >= 5120 && K > 16384)) && (G != 32 || (uint64_t)N * K > 33000000ull);
             return K > 16384 && M <= 96 && (bits == 8 ? M > 32 : M > 48 && N <= 5120);
         }
-        if (!tall || M < 9) return false;
-        if (M <= 16) return stream && N > 8192;
-        if (M <= 48 && N > 8192) {
-            if (N <= 16384) return !g32 || N <= 12288;
-            const uint32_t tiles = 2 * ((N + 255) / 256), rounds = (tiles + 255) / 256;
-            if (!stream && bits != 8) return M > 32 && N < 24576 && !g32;
-            return tiles * 5 >= rounds * 256 * 4 ? stream || K >= 8192 || M > 32 : (stream || M > 32) && rounds == 1;
-        }
-        if (M <= 48 || M > 96 || N < 6144 || g32) return false;
-        return stream ? N <= 16384 && (M > 64 || N >= 12800) : M > 64 && codes <= 28000000ull;
+        if (!tall || M < 9 || M > 48) return false;
+        if (M <= 16) return stream && N > 8192 && (bits != 3 || N <= 16384);
+        if (N <= 16384 || (!stream && bits != 8) || (M <= 32 && (bits == 3 || K < 2048))) return false;
+        const uint32_t tiles = 2 * ((N + 255) / 256), rounds = (tiles + 255) / 256;
+        return tiles * 5 >= rounds * 256 * 4 ? stream || K >= 8192 || N > 65536 : stream && rounds == 1;
     }
     if (M <= 16) return stream || (uint64_t)N * K > 75000000ull;
     if (wide) return stream || M <= 96;
-    if (tall) return M <= (stream ? (K < 2304 || codes > 90000000ull ? 64u : 48u) : bits == 8 || codes > 90000000ull ? 48u : 32u);
+    if (tall) return M <= (stream ? (K < 2304 || codes > 90000000ull ? 64u : 48u) : bits == 8 ? 48u : 32u);
     if (M <= 48 || (M <= 64 && K <= 5632)) return true;
     return (stream || bits == 8) && (M <= 64 || (K >= 2048 && codes <= 40000000ull));
 }

@@ -1,6 +1,6 @@
 // The matrix-core GEMV on codes (see qmv_codes.hip for the routing and the geometry): kernel and argument block.
 #pragma once
-// Batches of 5 to 128 activation rows against one or several weight matrices of the same row length, f16 / bf16, codes of
+// Batches of activation rows (5 to 128 where it is chosen) against one or several weight matrices of the same row length, f16 / bf16, codes of
 // 2, 3, 4, 5, 6 and 8 bits, rows of any whole number of 128 codes, with exact-dequant arithmetic:
 // out[m][n] = sum_g (s[n][g] * sum_k q[n][k] x[m][k] + b[n][g] * sum_k x[m][k]), the rows of mt_qmm
 // (crates/metaltile-std/src/mlx/quantized.rs:1330-1500).
@@ -22,6 +22,9 @@
 // neighbouring lanes on neighbouring 16 bytes of a row (in operand order, 16 rows next to each other, a load occupies the
 // compute unit's address path four times as long), two steps ahead, and turned in an LDS area of the wave's own; rows
 // there are 16 bytes apart from a multiple of 128 so that the operand reads spread over the banks.
+// A step of eight waves (256 x 128 codes) takes 1.2 / 1.45 / 1.8 us at 16 / 32 / 48 activation rows: 5.2 TB/s of 6-bit codes at 16 rows, less than half of that of
+// 4-bit codes at 48, where the LDS traffic of operands (98 KB of activations and 48 KB of codes in and out) and the conversion stand beside the MFMAs. us, tiles -> this:
+// 4736 x 20096, 5 bits, 32 rows 263 -> 39; 2 x 8704 x 3968, 8 bits, 40 rows 45.1 -> 34.7 (the table is at qmv_codes_preferred).
 // Every load is a buffer load whose out-of-range offsets read zeros without a memory access: rows past the matrix or the
 // batch and steps past the slice are given such offsets.
 #include "codes16.h"

@@ -74,7 +74,7 @@ def test_without_memory_for_the_sums(oracle, codes, kb):
     run(oracle, DType.BF16, 5, 64, 20, 1152, (58, 83), more=0.045 if kb == 1 else 0.0)
 
 
-@pytest.mark.parametrize("bits,G,M,N,K", [(5, 64, 24, 1664, 1664), (3, 32, 32, 2944, 1408), (4, 64, 33, 1152, 1152), (6, 128, 24, 4096, 8448), (8, 64, 60, 1920, 1920), (4, 128, 45, 9216, 1024), (8, 64, 40, 72, 16640)])
+@pytest.mark.parametrize("bits,G,M,N,K", [(5, 64, 24, 1664, 1664), (3, 32, 32, 2944, 1408), (4, 64, 33, 1152, 1152), (6, 128, 24, 4096, 8448), (8, 64, 60, 1920, 1920), (6, 128, 45, 18944, 1024), (8, 64, 40, 72, 16640)])
 def test_chosen(oracle, bits, G, M, N, K):
     print(f"[case] chosen codes qmm b{bits} g{G} M{M} N{N} K{K}", flush=True)
     assert "qmv_codes_kernel" in ops.plan("qmm", DType.BF16, bits, G, M, N, K)[1][0][0]

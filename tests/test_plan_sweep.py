@@ -265,6 +265,26 @@ def test_k_run_lines_of_few_rows(bits, G, N, K, rows):
     assert on == rows
 
 
+@pytest.mark.parametrize("bits,G,M,N,K,codes", [
+    # rows that the tiles cannot split
+    (5, 64, 16, 4736, 4736, True), (4, 64, 16, 4736, 4736, False), (4, 64, 17, 4736, 4736, True), (4, 64, 64, 5504, 5504, True), (4, 64, 64, 5760, 5760, False),
+    (4, 64, 48, 5760, 5760, True), (8, 64, 96, 4736, 4736, True), (5, 64, 128, 4736, 4736, True), (4, 64, 65, 4736, 4736, False), (5, 64, 129, 4736, 4736, False),
+    (4, 64, 96, 2304, 8320, True), (4, 64, 97, 2304, 8320, False), (5, 64, 126, 2304, 8320, True), (5, 64, 126, 3584, 12928, False), (5, 64, 96, 3584, 12928, True),   # (split)
+    (4, 64, 32, 9472, 2176, True), (4, 64, 33, 9472, 2176, False), (8, 64, 48, 9472, 2176, True), (5, 64, 64, 9472, 2176, True), (5, 64, 65, 9472, 2176, False),
+    (4, 64, 60, 768, 6528, False), (4, 64, 60, 768, 4736, True), (2, 128, 72, 512, 1152, False), (4, 32, 20, 1152, 1152, False), (4, 64, 20, 1152, 1152, True),
+    # rows that they can
+    (5, 64, 32, 4096, 4096, False), (6, 64, 20, 8192, 2048, False), (6, 64, 20, 16384, 4096, False), (6, 64, 17, 18944, 3584, True), (6, 64, 48, 18944, 3584, True),
+    (4, 64, 20, 28672, 8192, False), (8, 64, 20, 28672, 8192, True), (8, 64, 48, 28672, 4096, False), (8, 64, 48, 18944, 3584, False), (8, 64, 17, 128256, 4096, True),
+    (6, 64, 49, 28672, 8192, False), (6, 64, 48, 128256, 4096, True), (6, 64, 20, 40960, 4096, False),
+    (5, 64, 48, 4096, 14336, True), (5, 64, 49, 4096, 14336, False), (6, 64, 77, 5120, 20480, True), (6, 64, 77, 3584, 18944, False), (8, 64, 33, 5120, 20480, True), (8, 64, 32, 5120, 20480, False),
+    (4, 64, 49, 3584, 18944, True), (4, 64, 77, 8192, 28672, False), (3, 32, 30, 2560, 10496, False), (7, 64, 24, 4736, 4736, False), (4, 64, 24, 4736, 4672, False),
+])
+def test_gemv_on_codes_lines(bits, G, M, N, K, codes):
+    """Which matrices the GEMV on codes is for, on both sides of each line."""
+    rc, launches, _, _ = ops.plan("qmm", DType.BF16, bits, G, M, N, K)
+    assert rc == 0 and ("qmv_codes_kernel" in launches[0][0]) == codes, launches[0][0]
+
+
 @pytest.mark.parametrize("dt,bits,G,M,N,K,first", [
     (DType.BF16, 4, 64, 4, 1024, 18688, "qmv_mfma_kernel"),          # K slices; two passes of two rows
     (DType.BF16, 8, 64, 3, 3584, 18944, "qmv_mfma_kernel"),
