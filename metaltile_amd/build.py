@@ -102,8 +102,8 @@ SAN_FLAGS = ["-Xarch_host", "-fsanitize=address", "-Xarch_host", "-fsanitize=und
 
 def build_sanitized(verbose: bool = True) -> dict:
     """The library's HOST code (routing, geometry, argument checks, the C-ABI) compiled with the address and
-    undefined-behaviour sanitizers and linked into two programs under _build/san/: plan_sweep (walks mtq_plan over
-    a grid of shapes, no GPU needed) and tile_bench. Only the host side of every source is compiled
+    undefined-behaviour sanitizers and linked into three programs under _build/san/: plan_sweep (walks mtq_plan over
+    a grid of shapes, no GPU needed), scratch_failures (batches while allocations fail; it answers the HIP calls itself) and tile_bench. Only the host side of every source is compiled
     (--cuda-host-only: no device code, so nothing here can be launched); the GPU library is not touched."""
     os.makedirs(SAN_DIR, exist_ok=True)
     inc = os.path.join(HERE, "..", "include")
@@ -111,13 +111,13 @@ def build_sanitized(verbose: bool = True) -> dict:
 
     def one(src):
         obj = os.path.join(SAN_DIR, os.path.splitext(src)[0] + ".o")
-        r = subprocess.run([HIPCC] + flags + ["-c", os.path.join(CSRC, src), "-o", obj], capture_output=True, text=True)
+        r = subprocess.run([HIPCC] + flags + (["-x", "hip"] if src.endswith(".cpp") else []) + ["-c", os.path.join(CSRC, src), "-o", obj], capture_output=True, text=True)
         if r.returncode != 0:
             raise RuntimeError(f"sanitized compile of {src} failed:\n{r.stderr}")
         return obj
 
     with concurrent.futures.ThreadPoolExecutor(max_workers=8) as ex:
-        objs = list(ex.map(one, SOURCES))
+        *objs, failures = ex.map(one, SOURCES + ["scratch_failures.cpp"])
     out = {}
     # A host-only object still refers to the device code bundle its registration hands to the runtime at load
     # time. Give each an empty bundle (the bundle magic and an entry count of zero): nothing is ever launched here.
@@ -138,9 +138,10 @@ def build_sanitized(verbose: bool = True) -> dict:
     if not os.path.exists(clangxx):
         clangxx = "/opt/rocm/lib/llvm/bin/clang++"
     rocm_lib = os.path.join(os.path.dirname(os.path.realpath(HIPCC)), "..", "lib")
-    for prog in ("plan_sweep", "tile_bench"):
+    for prog in ("plan_sweep", "scratch_failures", "tile_bench"):
         exe = os.path.join(SAN_DIR, prog)
-        cmd = [clangxx, os.path.join(CSRC, prog + ".cpp")] + objs + \
+        own = failures if prog == "scratch_failures" else os.path.join(CSRC, prog + ".cpp")
+        cmd = [clangxx, own] + objs + (["-rdynamic"] if own == failures else []) + \
               ["-O1", "-g", "-std=c++17", "-I", inc, "-fsanitize=address", "-fsanitize=undefined", "-fno-sanitize-recover=all",
                "-L", rocm_lib, "-lamdhip64", "-ldl", f"-Wl,-rpath,{rocm_lib}", "-o", exe]
         r = subprocess.run(cmd, capture_output=True, text=True)

@@ -408,49 +408,36 @@ static int run_codes(int dtype, int bits, uint32_t G, int n, const void* const* 
     all.n = 0;
     CodesSplit split[4];
     size_t needs[4], total = 0;
-    bool started = false, tried = false;
+    bool started = false;
     int at[4], left = 0;
-    auto gather = [&](bool fits) {   // fits: only what there is memory for by itself
-        all.n = left = 0;
-        total = 0;
-        started = false;
-        for (int j = 0; j < n; j++) {
-            if (taken[j]) { started = true; continue; }
-            q.w = w[j]; q.scales = s[j]; q.biases = b[j]; q.out = outs[j]; q.N = N[j];
-            if (!codes_serve(q)) { left++; continue; }
-            const CodesSplit sp = qmv_codes_split(q);
-            const size_t need = qmv_codes_scratch_bytes(q, sp);
-            if (fits && need && ensure_scratch(g.scratch_held + need)) { left++; continue; }
-            const int i = all.n++;
-            at[i] = j;
-            split[i] = sp;
-            needs[i] = need;
-            total += need;
-            all.w[i] = w[j]; all.scales[i] = s[j]; all.biases[i] = b[j]; all.out[i] = outs[j]; all.N[i] = N[j];
-        }
-    };
-    gather(false);
-    // without memory for all sums at once one matrix follows the other; without any for a matrix it is left to the other kernels
-    if (total && ensure_scratch(g.scratch_held + total)) {
-        tried = true;
-        gather(true);
+    for (int j = 0; j < n; j++) {
+        if (taken[j]) { started = true; continue; }
+        q.w = w[j]; q.scales = s[j]; q.biases = b[j]; q.out = outs[j]; q.N = N[j];
+        if (!codes_serve(q)) { left++; continue; }
+        const int i = all.n++;
+        at[i] = j;
+        split[i] = qmv_codes_split(q);
+        total += needs[i] = qmv_codes_scratch_bytes(q, split[i]);
+        all.w[i] = w[j]; all.scales[i] = s[j]; all.biases[i] = b[j]; all.out[i] = outs[j]; all.N[i] = N[j];
     }
     if (all.n == 0) return ERR_OK;
-    const int per = tried ? 1 : all.n;
+    // Without memory for all sums at once one matrix follows the other, and one without any for its own is left to the other kernels. (The
+    // memory is asked for at each launch: a growth that fails takes the buffer that was there with it.)
+    const bool together = !total || ensure_scratch(g.scratch_held + total) == ERR_OK;
+    const int per = together ? all.n : 1;
     for (int i = 0; i < all.n; i += per) {
+        if (!together && needs[i] && ensure_scratch(g.scratch_held + needs[i])) { left++; continue; }
         QmvBatch now;
         now.n = per;
-        size_t need = 0;
         for (int k = 0; k < per; k++) {
             now.w[k] = all.w[i + k]; now.scales[k] = all.scales[i + k]; now.biases[k] = all.biases[i + k]; now.out[k] = all.out[i + k]; now.N[k] = all.N[i + k];
-            need += needs[i + k];
             taken[at[i + k]] = true;
         }
         LaunchCtx l2 = lc;
         if (started) l2.start = nullptr;
         if (left || i + per < all.n) l2.stop = nullptr;
         started = true;
-        int rc = launch_qmv_codes(q, now, split + i, need ? (char*)g.scratch_buf + g.scratch_held : nullptr, l2);
+        int rc = launch_qmv_codes(q, now, split + i, g.scratch_buf ? (char*)g.scratch_buf + g.scratch_held : nullptr, l2);
         if (rc) return rc;
     }
     return ERR_OK;

@@ -1,5 +1,6 @@
 """Host code under the address and undefined-behaviour sanitizers (no GPU): the library's routing, geometry and
-argument checks walked by csrc/plan_sweep.cpp through mtq_plan (about 600 000 plans), the bench driver's start-up,
+argument checks walked by csrc/plan_sweep.cpp through mtq_plan (about 600 000 plans), batches while allocations of the library's
+scratch fail (csrc/scratch_failures.cpp), the bench driver's start-up,
 and the oracle's restatement over small ragged shapes (oracle/san_check.c). A sanitizer report ends a program with
 a non-zero exit code (-fno-sanitize-recover), so the exit codes are the test."""
 import os
@@ -26,6 +27,12 @@ def _run(cmd, **kw):
 
 def test_plan_sweep_under_sanitizers(programs):
     r, text = _run([programs["plan_sweep"]])
+    assert r.returncode == 0, text[-4000:]
+    assert " 0 violations" in text
+
+
+def test_batches_when_scratch_cannot_be_had(programs):
+    r, text = _run([programs["scratch_failures"]])
     assert r.returncode == 0, text[-4000:]
     assert " 0 violations" in text
 
