@@ -51,7 +51,9 @@ template <int BITS, bool G32> struct QhLds {
     static constexpr uint32_t TB = 16 * TS;
     static constexpr uint32_t SG = G32 ? 16 : 8;      // scales of four steps: [group or 64 codes][weight row], then biases less MAGIC scales
     static constexpr uint32_t WB = TB + 2 * SG * 64;  // a wave's own part
-    static constexpr uint32_t xbytes(uint32_t K, uint32_t rpl) { return (K * 2u + K / (G32 ? 32u : 64u) * 4u) << rpl; }
+    static_assert(WB % 16 == 0, "16-byte LDS accesses");
+    // rows and their sums; the waves' parts behind them begin on 16 bytes (one row in groups of 64: 264 bytes per 128 codes)
+    static constexpr uint32_t xbytes(uint32_t K, uint32_t rpl) { return (((K * 2u + K / (G32 ? 32u : 64u) * 4u) << rpl) + 15u) & ~15u; }
     static constexpr uint32_t bytes(uint32_t K, uint32_t rpl, uint32_t waves) { return xbytes(K, rpl) + waves * WB + ((2u * waves * 64u) << rpl) + 64u; }
 };
 

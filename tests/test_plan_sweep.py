@@ -285,6 +285,20 @@ def test_gemv_on_codes_lines(bits, G, M, N, K, codes):
     assert rc == 0 and ("qmv_codes_kernel" in launches[0][0]) == codes, launches[0][0]
 
 
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("K", [128, 256, 1152, 1664, 4736])
+def test_activations_in_lds_end_on_16_bytes(bits, K):
+    """The GEMV that holds its activations in LDS has 16-byte accesses behind the rows and their sums (264 bytes per 128 codes of one
+    row); all else in its LDS is a multiple of 16."""
+    lib = _lib.load()
+    assert lib.mtq_set_option(b"qmv.held", 2) == OK
+    try:
+        _, launches, _, _ = ops.plan("qmv", DType.BF16, bits, 64, 1, 1000, K)
+    finally:
+        lib.mtq_set_option(b"qmv.held", 0)
+    assert "qmv_held_kernel" in launches[0][0] and launches[0][3] % 16 == 0
+
+
 @pytest.mark.parametrize("dt,bits,G,M,N,K,first", [
     (DType.BF16, 4, 64, 4, 1024, 18688, "qmv_mfma_kernel"),          # K slices; two passes of two rows
     (DType.BF16, 8, 64, 3, 3584, 18944, "qmv_mfma_kernel"),
