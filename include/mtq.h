@@ -458,8 +458,9 @@ MTQ_API int mtq_flush_cache(void);
  *   "qmv.codes"            GEMV on codes, activations streamed through LDS (f16 / bf16, codes of 2..6 and 8 bits, groups of 32, 64, 128,
  *                          K % 128 == 0, up to 1024 rows): 0 = where it is the fastest, 1 = never, 2 = wherever the shape allows
  *   "qmv.codes_kw" / "qmv.codes_nw" / "qmv.codes_stage" / "qmv.codes_slices"
- *                          and its waves that share weight rows (1, 2, 4, 8), waves along N (up to 16), steps of activations between
- *                          barriers (1, 2, 4) and slices of K (up to 64); 0 = choose
+ *                          and its waves that share weight rows (1, 2, 4), waves along N (2..8), steps of activations between
+ *                          barriers (1, 2, 4) and slices of K (up to 16 and K / 128); 0 = choose. Calls that the values do not fit
+ *                          (more than 8 waves in all, too few for the rows) go to the other kernels
  *   "qmv.norm_mfma"        mtq_rms_norm_qmv with the norm applied inside the matrix-core GEMV (4-bit codes, f16 / bf16):
  *                          0 = where it is faster than the streaming kernel's fused form, 1 = never, 2 = wherever the
  *                          shape allows

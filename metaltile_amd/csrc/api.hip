@@ -388,12 +388,15 @@ static int run_held(int dtype, int bits, uint32_t G, int n, const void* const* w
 
 // Whether a matrix is for the GEMV on codes. Of more than 96 rows only what the tiles cannot split (at K >= 8192 they mostly can, in tiles of 128
 // rows: 3584 x 12928, 5 bits, 126 rows 40.6 us in K splits, 55.2 here, 96 rows 38.5 and 36.2; 2304 x 8320, unsplit, 126 rows 100.8 -> 30.4).
-static bool codes_serve(const QmmParams& q) {
+static bool codes_serve(const QmmParams& q, CodesSplit& split) {
     if (!qmv_codes_takes(q)) return false;
-    if (options().qmv_codes == 2) return true;
-    if (!qmv_codes_preferred(q.bits, q.group_size, q.M, q.N, q.K) || !tiles_serve(q.bits, q.M, q.N, q.K) || slices_serve(q) || wide_serves(q, false)) return false;
-    QmmDLaunch l;
-    return q.M <= 96 || plan_qmm_direct(q, l) != ERR_OK || !l.split;
+    if (options().qmv_codes != 2) {
+        if (!qmv_codes_preferred(q.bits, q.group_size, q.M, q.N, q.K) || !tiles_serve(q.bits, q.M, q.N, q.K) || slices_serve(q) || wide_serves(q, false)) return false;
+        QmmDLaunch l;
+        if (q.M > 96 && plan_qmm_direct(q, l) == ERR_OK && l.split) return false;
+    }
+    split = qmv_codes_split(q);
+    return split.slices != 0;   // (a geometry that the caller has asked for does not fit every call)
 }
 
 // The matrices of a batch (or the one of a single call) that the GEMV on codes is for, in one launch; taken[j] as above, where
@@ -413,10 +416,9 @@ static int run_codes(int dtype, int bits, uint32_t G, int n, const void* const* 
     for (int j = 0; j < n; j++) {
         if (taken[j]) { started = true; continue; }
         q.w = w[j]; q.scales = s[j]; q.biases = b[j]; q.out = outs[j]; q.N = N[j];
-        if (!codes_serve(q)) { left++; continue; }
+        if (!codes_serve(q, split[all.n])) { left++; continue; }
         const int i = all.n++;
         at[i] = j;
-        split[i] = qmv_codes_split(q);
         total += needs[i] = qmv_codes_scratch_bytes(q, split[i]);
         all.w[i] = w[j]; all.scales[i] = s[j]; all.biases[i] = b[j]; all.out[i] = outs[j]; all.N[i] = N[j];
     }
@@ -2049,12 +2051,12 @@ int mtq_set_option(const char* name, int value) {
         return MTQ_OK;
     }
     if (!strcmp(name, "qmv.codes_kw")) {
-        if (value != 0 && value != 1 && value != 2 && value != 4 && value != 8) return fail(ERR_BAD_ARG, "qmv.codes_kw must be 0, 1, 2, 4 or 8");
+        if (value != 0 && value != 1 && value != 2 && value != 4) return fail(ERR_BAD_ARG, "qmv.codes_kw must be 0, 1, 2 or 4");
         options().qmv_codes_kw = value;
         return MTQ_OK;
     }
     if (!strcmp(name, "qmv.codes_nw")) {
-        if (value < 0 || value > 16) return fail(ERR_BAD_ARG, "qmv.codes_nw must be in 0..16");
+        if (value != 0 && (value < 2 || value > 8)) return fail(ERR_BAD_ARG, "qmv.codes_nw must be 0 or in 2..8");
         options().qmv_codes_nw = value;
         return MTQ_OK;
     }
@@ -2064,7 +2066,7 @@ int mtq_set_option(const char* name, int value) {
         return MTQ_OK;
     }
     if (!strcmp(name, "qmv.codes_slices")) {
-        if (value < 0 || value > 64) return fail(ERR_BAD_ARG, "qmv.codes_slices must be in 0..64");
+        if (value < 0 || value > 16) return fail(ERR_BAD_ARG, "qmv.codes_slices must be in 0..16");
         options().qmv_codes_slices = value;
         return MTQ_OK;
     }

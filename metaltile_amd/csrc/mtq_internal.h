@@ -123,10 +123,10 @@ struct Options {
     int qmv_held_kp = 0;          // and its waves that share 16 weight rows (0 = choose; 1, 2, 4, 8, 16),
     int qmv_held_nb = 0;          // its blocks side by side in a workgroup (0 = choose)
     int qmv_codes = 0;            // matrix-core GEMV on codes (1..1024 rows): 0 = choose per shape, 1 = never, 2 = wherever the shape allows
-    int qmv_codes_kw = 0;         // and its waves that share weight rows (0 = choose; 1, 2, 4, 8),
-    int qmv_codes_nw = 0;         // its waves along N (0 = choose),
+    int qmv_codes_kw = 0;         // and its waves that share weight rows (0 = choose; 1, 2, 4),
+    int qmv_codes_nw = 0;         // its waves along N (0 = choose; 2..8),
     int qmv_codes_stage = 0;      // its steps of activations between barriers (0 = choose; 1, 2, 4),
-    int qmv_codes_slices = 0;     // its slices of K (0 = choose)
+    int qmv_codes_slices = 0;     // its slices of K (0 = choose; 1..16)
     int scratch_most_kb = 0;      // largest library-owned scratch buffer (0 = no limit): a call that needs more finds no memory
     int qmv_wide = 0;             // 16-row matrix-core GEMV for batches of 5..16 rows: 0 = choose per shape, 1 = never, 2 = wherever the shape allows
 };

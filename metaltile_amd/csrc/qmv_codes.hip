@@ -48,9 +48,9 @@ CodesSplit qmv_codes_split(const QmmParams& p) {
     const Options& o = options();
     CodesSplit best;
     float least = 1e30f;
-    for (uint32_t kwl = 0; kwl <= 3; kwl++) {
+    for (uint32_t kwl = 0; kwl <= 2; kwl++) {
         if (o.qmv_codes_kw && (1u << kwl) != (uint32_t)o.qmv_codes_kw) continue;
-        for (uint32_t nw = qc_min_nw(r.mt); nw << kwl <= QC_WAVES; nw++) {
+        for (uint32_t nw = qc_min_nw(r.mt); nw << kwl <= QC_WAVES; nw++) {   // (two waves along N at least: four share rows at most)
             if ((o.qmv_codes_nw && nw != (uint32_t)o.qmv_codes_nw) || k.lds(1u << kwl, 1, nw << kwl) > QC_LDS) continue;
             const uint32_t tiles = (N + 32u * nw - 1u) / (32u * nw);
             const float step_us = (r.mt == 1 ? 1.2f : r.mt == 2 ? 1.45f : 1.8f) * ((nw << kwl) <= 4 ? 0.8f : 1.0f);

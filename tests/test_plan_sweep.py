@@ -285,6 +285,28 @@ def test_gemv_on_codes_lines(bits, G, M, N, K, codes):
     assert rc == 0 and ("qmv_codes_kernel" in launches[0][0]) == codes, launches[0][0]
 
 
+@pytest.mark.parametrize("mode", [0, 2])
+@pytest.mark.parametrize("kw,nw,slices", [(4, 0, 0), (4, 3, 0), (0, 2, 0), (1, 8, 16), (2, 8, 0), (0, 0, 11)])
+def test_geometries_that_do_not_fit(mode, kw, nw, slices):
+    """A geometry of the GEMV on codes that is asked for and fits a call is used; calls that it does not fit are served all the same."""
+    lib = _lib.load()
+    names = (b"qmv.codes", b"qmv.codes_kw", b"qmv.codes_nw", b"qmv.codes_slices")
+    assert all(lib.mtq_set_option(n, v) == OK for n, v in zip(names, (mode, kw, nw, slices)))
+    try:
+        for M, K in ((9, 8320), (20, 1152), (33, 1152), (48, 1664), (60, 4736), (128, 1152)):
+            rc, launches, _, n = ops.plan("qmm", DType.BF16, 5, 64, M, 1664, K)
+            assert rc == OK and n >= 1
+            mt = -(-(-(-M // -(-M // 48))) // 16)   # operand tiles of 16 rows
+            waves = [w for w in range(max(2, mt), 9) for k in (1, 2, 4) if (not nw or w == nw) and (not kw or k == kw) and w * k <= 8]
+            fits = bool(waves) and slices <= K // 128
+            assert ("qmv_codes_kernel" in launches[0][0]) == fits, (M, K, launches[0][0])
+    finally:
+        for n in names:
+            lib.mtq_set_option(n, 0)
+    for n, v in ((b"qmv.codes_kw", 8), (b"qmv.codes_nw", 1), (b"qmv.codes_nw", 9), (b"qmv.codes_slices", 17)):
+        assert lib.mtq_set_option(n, v) == BAD_ARG
+
+
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("K", [128, 256, 1152, 1664, 4736])
 def test_activations_in_lds_end_on_16_bytes(bits, K):
