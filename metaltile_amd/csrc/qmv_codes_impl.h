@@ -78,7 +78,8 @@ template <int DT, int BITS, bool G32, int MT> __global__ __launch_bounds__(QC_WA
     constexpr int R = 2, NL = BITS, XU = QcShape<MT>::XU;
     constexpr int U = G32 ? 1 : 2;                      // steps per f32 MFMA of the bias term (four sums)
     constexpr uint32_t ROWS = L::ROWS, QS = L::QS, XB = L::XB, XSB = L::XSB;
-    constexpr float MAGIC = QcCodes<DT, BITS>::MAGIC;
+    using C = QcCodes<DT, BITS, false>;
+    constexpr float MAGIC = C::MAGIC;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
 
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -222,7 +223,7 @@ template <int DT, int BITS, bool G32, int MT> __global__ __launch_bounds__(QC_WA
 #pragma unroll
         for (int t = 0; t < MT; t++) tot[r][t] = zero;
 
-    uint32_t kor = DT == DT_BF16 ? 0x43004300u : 0x64006400u;
+    uint32_t kor = C::KOR;
     asm volatile("" : "+v"(kor));
 
     load_s(0);
@@ -274,7 +275,7 @@ template <int DT, int BITS, bool G32, int MT> __global__ __launch_bounds__(QC_WA
             kr_u32x4 wo[R][2];
 #pragma unroll
             for (int r = 0; r < R; r++) {
-                qc_convert<DT, BITS>(d[hb][r], kor, wo[r]);
+                qc_convert<DT, BITS, false>(d[hb][r], kor, wo[r]);
                 if constexpr (G32) {
                     // operand u of lanes 0..3: the pairs of pieces 2 u, 2 u + 1 (first halves), then their second halves
 #pragma unroll

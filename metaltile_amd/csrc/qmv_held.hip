@@ -4,14 +4,16 @@
 namespace mtq {
 
 // (instances: one translation unit per element type and kind of group)
-HeldInstance qmv_held_pick_f16(int bits, int mode, uint32_t rows);
-HeldInstance qmv_held_pick_f16_g32(int bits, int mode, uint32_t rows);
-HeldInstance qmv_held_pick_bf16(int bits, int mode, uint32_t rows);
-HeldInstance qmv_held_pick_bf16_g32(int bits, int mode, uint32_t rows);
+HeldInstance qmv_held_pick_f16(int bits, int mode, uint32_t rows, bool least);
+HeldInstance qmv_held_pick_f16_g32(int bits, int mode, uint32_t rows, bool least);
+HeldInstance qmv_held_pick_bf16(int bits, int mode, uint32_t rows, bool least);
+HeldInstance qmv_held_pick_bf16_g32(int bits, int mode, uint32_t rows, bool least);
 
-static HeldInstance held_pick(int dtype, int bits, uint32_t G, int mode, uint32_t rows) {
-    if (dtype == DT_BF16) return G == 32 ? qmv_held_pick_bf16_g32(bits, mode, rows) : qmv_held_pick_bf16(bits, mode, rows);
-    return G == 32 ? qmv_held_pick_f16_g32(bits, mode, rows) : qmv_held_pick_f16(bits, mode, rows);
+static HeldInstance held_pick(int dtype, int bits, uint32_t G, int mode, uint32_t rows, uint32_t K) {
+    // (the streaming kernel's norm takes rows of whole 2048 codes; plain ones are its and the one-shot kernel's at every length)
+    const bool least = mode == HELD_NORM ? K % 2048 == 0 : rows == 1;
+    if (dtype == DT_BF16) return G == 32 ? qmv_held_pick_bf16_g32(bits, mode, rows, least) : qmv_held_pick_bf16(bits, mode, rows, least);
+    return G == 32 ? qmv_held_pick_f16_g32(bits, mode, rows, least) : qmv_held_pick_f16(bits, mode, rows, least);
 }
 
 static uint32_t held_log2rp(uint32_t rows) {
@@ -34,7 +36,7 @@ struct HeldGeometry {
 static bool held_geometry(int dtype, int bits, uint32_t G, int mode, uint32_t rows, uint32_t K, uint32_t blocks, HeldGeometry& g) {
     const Options& o = options();
     const uint32_t cus = held_cus(), rpl = held_log2rp(rows), pairs = (K / 128u + 1u) / 2u;
-    g.k = held_pick(dtype, bits, G, mode, rows);
+    g.k = held_pick(dtype, bits, G, mode, rows, K);
     if (!g.k.fn) return false;
     // KP: what brings a thousand waves to the matrix, each with two and a half steps of 128 codes or more; at least four on long
     // rows. bf16, groups of 64, RMS norm included, KP 1 / 2 / 4 / 8, us: 1536 x 1280 7.0 5.8 5.6 5.5, 2816 x 2304 9.4 7.6 6.6 7.0, 14080 x 2304 11.7

@@ -57,11 +57,12 @@ template <int BITS, bool G32> struct QhLds {
     static constexpr uint32_t bytes(uint32_t K, uint32_t rpl, uint32_t waves) { return xbytes(K, rpl) + waves * WB + ((2u * waves * 64u) << rpl) + 64u; }
 };
 
-// DT, BITS, groups of 32 (else 64 or 128), NR: result registers that hold rows (1: one row, 2: value and remainder, 4), MODE
-template <int DT, int BITS, bool G32, int NR, int MODE> __global__ __launch_bounds__(1024) void qmv_held_kernel(QmvHeldArgs a) {
+// DT, BITS, groups of 32 (else 64 or 128), NR: result registers that hold rows (1: one row, 2: value and remainder, 4), MODE, LEAST: of QcCodes
+template <int DT, int BITS, bool G32, int NR, int MODE, bool LEAST> __global__ __launch_bounds__(1024) void qmv_held_kernel(QmvHeldArgs a) {
     using L = QhLds<BITS, G32>;
     constexpr int NL = (BITS + 1) / 2;                  // 16-byte loads of two steps: 32 * BITS pieces
-    constexpr float MAGIC = QcCodes<DT, BITS>::MAGIC;
+    using C = QcCodes<DT, BITS, LEAST>;
+    constexpr float MAGIC = C::MAGIC;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
 
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -274,7 +275,7 @@ template <int DT, int BITS, bool G32, int NR, int MODE> __global__ __launch_boun
     }
     barrier();
 
-    uint32_t kor = DT == DT_BF16 ? 0x43004300u : 0x64006400u;
+    uint32_t kor = C::KOR;
     asm volatile("" : "+v"(kor));
     const uint32_t odd = (BITS == 3 || BITS == 5) ? (q & 1u) * 2u : 0u;
     const uint32_t tread = j * L::TS + ((q * (2u * BITS)) & ~3u);
@@ -287,7 +288,7 @@ template <int DT, int BITS, bool G32, int NR, int MODE> __global__ __launch_boun
     auto operands = [&](int hb, kr_u32x4 (&wo)[2]) {   // hb: half of 64 codes of the two steps
         uint32_t d[4];
         qc_read<BITS>(own + tread + hb * 8 * BITS, odd, d);
-        qc_convert<DT, BITS>(d, kor, wo);
+        qc_convert<DT, BITS, LEAST>(d, kor, wo);
         if constexpr (G32) {
             // operand u of lanes 0..3: the pairs of pieces 2 u, 2 u + 1 (first halves), then their second halves
 #pragma unroll

@@ -9,8 +9,9 @@ import numpy as np
 import pytest
 
 from metaltile_amd import DType, GpuBuffer, ops, pack_f32, unpack_f32
+from metaltile_amd.dtypes import round_through
 from metaltile_amd.runtime import _ensure_init
-from metaltile_amd.synth import make_case
+from metaltile_amd.synth import make_case, pack_codes
 from tests.parity import rel_err
 
 pytestmark = pytest.mark.gpu
@@ -137,4 +138,52 @@ def test_infinite_activations(oracle, held, dt, bits, G, M, N, K):
     rest = [m for m in range(M) if m != 1]
     np.testing.assert_array_equal(got[0][rest], got[1][rest])
     for v in bufs:
+        v.free()
+
+
+@pytest.mark.parametrize("op,dt,bits,N,K", [
+    ("norm", DType.F16, 4, 512, 4096), ("norm", DType.F16, 4, 256, 2048), ("norm", DType.F16, 4, 1024, 8192), ("norm", DType.F16, 2, 512, 4096), ("norm", DType.BF16, 4, 512, 4096),
+    ("batch", DType.F16, 4, 512, 1024), ("batch", DType.F16, 8, 512, 512), ("batch", DType.BF16, 8, 512, 512), ("batch", DType.F16, 3, 512, 1152), ("norm", DType.F16, 5, 512, 2304),
+])
+def test_no_more_of_the_codes_offset_than_before(op, dt, bits, N, K):
+    """The error of the f32 sums, bare of the result's rounding: the biases of a row's last two groups are set so that its exact
+    result is all but 0. The root of its mean square over N rows is no larger than that of the kernels that take these calls without this
+    one (half as much again: both are estimates, and the orders of their sums differ), or 2^-20 of what a row's result is without
+    those biases: a hundredth of an f16 rounding, and what sums of some hundred f32 terms leave in any order."""
+    G, n = 64, K // 64
+    rng = np.random.default_rng(K + bits)
+    codes = rng.integers(0, 1 << bits, size=(N, n, G), dtype=np.uint8)
+    scale = round_through((0.02 * np.abs(rng.standard_normal((N, n))) + 1e-3).astype(np.float32).reshape(-1), dt).reshape(N, n)
+    bias = round_through((-(1 << (bits - 1)) * scale + 1e-3 * rng.standard_normal((N, n))).astype(np.float32).reshape(-1), dt).reshape(N, n)
+    x = rng.standard_normal((n, G)).astype(np.float32)
+    x[-2:] = np.abs(x[-2:])
+    x = round_through(x.reshape(-1), dt).reshape(n, G)
+    v = x.astype(np.float64) / (np.sqrt(np.mean(x.astype(np.float64) ** 2) + float(np.float32(1e-5))) if op == "norm" else 1.0)
+    plain = np.sqrt(np.mean((scale[:, :, None] * codes + bias[:, :, None]) ** 2) * (v * v).sum())
+    part = scale * np.einsum("rgk,gk->rg", codes.astype(np.float64), v)
+    for g in (-2, -1):
+        rest = part.sum(1) + (np.delete(bias, n + g, 1).astype(np.float64) * np.delete(v, n + g, 0).sum(1)).sum(1)
+        bias[:, g] = round_through((-rest / v[g].sum()).astype(np.float32), dt)
+    exact = part.sum(1) + (bias.astype(np.float64) * v.sum(1)).sum(1)
+    bufs = [GpuBuffer.from_bytes(t) for t in (pack_codes(codes.reshape(N, K), bits).tobytes(), pack_f32(scale.reshape(-1), dt), pack_f32(bias.reshape(-1), dt),
+                                              pack_f32(x.reshape(-1), dt), pack_f32(np.ones(K, np.float32), dt), np.float32(1e-5).tobytes())]
+    w, s, b, xb, nw, eps = bufs
+    out = GpuBuffer(2 * N * 2)
+    lib = _ensure_init()
+    rms = []
+    for held in (1, 0):
+        assert lib.mtq_set_option(b"qmv.held", held) == 0
+        try:
+            if op == "norm":
+                assert ("qmv_held_kernel" in ops.plan("rms_norm_qmv", dt, bits, G, 1, N, K)[1][0][0]) == (held == 0)
+                ops.rms_norm_qmv(dt, bits, G, xb, nw, w, s, b, out, eps, N, K)
+            else:
+                ops.qmv_batched(dt, bits, G, [w, w], [s, s], [b, b], xb, [out.ptr, out.ptr + N * 2], [N, N], K)
+            got = unpack_f32(out.read_bytes(N * 2), dt).astype(np.float64)
+        finally:
+            lib.mtq_set_option(b"qmv.held", 0)
+        rms.append(np.sqrt(np.mean((got - exact) ** 2)))
+    print(f"[case] {op} {dt.name} b{bits} {N} x {K}: {rms[0]:.2e} without, {rms[1]:.2e} with, of {plain:.2f}", flush=True)
+    assert rms[1] <= max(1.5 * rms[0], 2.0 ** -20 * plain)
+    for v in bufs + [out]:
         v.free()
