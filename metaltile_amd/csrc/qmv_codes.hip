@@ -15,6 +15,11 @@ static CodesInstance codes_pick(int dtype, int bits, uint32_t G, uint32_t mt) {
 }
 
 constexpr uint32_t QC_LDS = 160u * 1024u;   // of a compute unit
+static uint32_t codes_cus() {
+    int dev = 0, cus = 256;
+    if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    return (uint32_t)cus;
+}
 
 // Tiles of up to 48 activation rows, all of one height but the last.
 struct CodesRows {
@@ -44,7 +49,7 @@ bool qmv_codes_takes(const QmmParams& p) {
 CodesSplit qmv_codes_split(const QmmParams& p) {
     const CodesRows r = codes_rows(p.M);
     const CodesInstance k = codes_pick(p.dtype, p.bits, p.group_size, r.mt);
-    const uint32_t N = p.N, steps = p.K / 128u, pair = N >= 2 * (uint64_t)p.K ? 2u : 1u;
+    const uint32_t N = p.N, steps = p.K / 128u, pair = N >= 2 * (uint64_t)p.K ? 2u : 1u, cus = codes_cus();
     const Options& o = options();
     CodesSplit best;
     float least = 1e30f;
@@ -58,7 +63,7 @@ CodesSplit qmv_codes_split(const QmmParams& p) {
                 if (o.qmv_codes_slices && s != (uint32_t)o.qmv_codes_slices) continue;
                 if (s > 1 && !o.qmv_codes_slices && (steps >> kwl) < 3u * s) break;
                 const uint32_t wgs = (tiles * s + 7u) / 8u * 8u * r.tiles * pair, per = (((steps + s - 1u) / s + 1u) / 2u + (1u << kwl) - 1u) >> kwl;
-                float us = 4.f + (float)((wgs + 255u) / 256u) * ((float)(2u * per) * step_us + 6.5f);
+                float us = 4.f + (float)((wgs + cus - 1u) / cus) * ((float)(2u * per) * step_us + 6.5f);
                 if (s > 1) us += 4.f + (float)(pair * s) * (float)p.M * (float)N * 8.0f / 4e6f;
                 if (us < least) { least = us; best = CodesSplit{kwl, s}; }
             }
@@ -123,8 +128,8 @@ bool qmv_codes_preferred(int bits, uint32_t G, uint32_t M, uint32_t N, uint32_t 
         if (!tall || M < 9 || M > 48) return false;
         if (M <= 16) return stream && N > 8192 && (bits != 3 || N <= 16384);
         if (N <= 16384 || (!stream && bits != 8) || (M <= 32 && (bits == 3 || K < 2048))) return false;
-        const uint32_t tiles = 2 * ((N + 255) / 256), rounds = (tiles + 255) / 256;
-        return tiles * 5 >= rounds * 256 * 4 ? stream || K >= 8192 || N > 65536 : stream && rounds == 1;
+        const uint32_t cus = codes_cus(), tiles = 2 * ((N + 255) / 256), rounds = (tiles + cus - 1) / cus;
+        return tiles * 5 >= rounds * cus * 4 ? stream || K >= 8192 || N > 65536 : stream && rounds == 1;
     }
     if (M <= 16) return stream || (uint64_t)N * K > 75000000ull;
     if (wide) return stream || M <= 96;
@@ -200,12 +205,13 @@ static int launch_codes_alike(const QmmParams& p, const QmvBatch& b, const Codes
         n++;
     }
     // waves along N: the fewest rounds of workgroups over the chip, and of those the most waves
+    const uint32_t cus = codes_cus();
     uint32_t least = ~0u;
     for (uint32_t t = qc_min_nw(rows.mt); t << kwl <= QC_WAVES; t++) {
         if (k.lds(1u << kwl, 1, t << kwl) > QC_LDS) break;
         uint32_t wgs = 0;
         for (uint32_t j = 0; j < n; j++) wgs += ((a.N[j] + 32u * t - 1u) / (32u * t) * a.slices[j] + 7u) / 8u * 8u * rows.tiles;
-        if ((wgs + 255u) / 256u < least) { least = (wgs + 255u) / 256u; nw = t; }
+        if ((wgs + cus - 1u) / cus < least) { least = (wgs + cus - 1u) / cus; nw = t; }
     }
     if (options().qmv_codes_nw) nw = (uint32_t)options().qmv_codes_nw;
     uint32_t stage = k.stage;

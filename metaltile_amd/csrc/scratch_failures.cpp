@@ -2,7 +2,7 @@
 // host code makes are answered here: an allocation is host memory or, by a schedule, fails as it does on a full card (the
 // buffer it was to replace is gone by then), and a launch is looked at instead of made. Whatever the schedule, each matrix of
 // a batch is worked out once, every kernel's partial results lie inside memory that is allocated at its launch, and the
-// call's two timestamps are each taken once. Built with the sanitizers from the library's own host code (metaltile_amd/build.py,
+// call's two timestamps are each taken once. And the slices of the GEMV on codes follow the device's compute units. Built with the sanitizers from the library's own host code (metaltile_amd/build.py,
 // build_sanitized). Exit code 0 = all of that holds.
 #include "qmm_direct_plan.h"
 #include "qmv_codes_impl.h"
@@ -23,6 +23,8 @@ std::map<char*, size_t> g_live;   // allocated memory
 unsigned g_fail = 0;              // bit i: the i-th allocation from here on fails
 int g_allocs = 0, g_starts = 0, g_stops = 0, g_bad = 0;
 bool g_after_stop = false;
+int g_cus = 256;                    // compute units of the device
+uint32_t g_slices = 0;              // most slices of K of a matrix on the GEMV on codes
 std::multiset<const void*> g_out;   // results that the launches so far work out
 const char* g_case = "";
 
@@ -43,6 +45,7 @@ hipError_t launch(const void* fn, void** args) {
         const mtq::QmvCodesArgs& a = *(const mtq::QmvCodesArgs*)args[0];
         for (int j = 0; j < 4 && a.first[j] != 0x7FFFFFFFu; j++) {
             g_out.insert(a.out[j]);
+            if (a.slices[j] > g_slices) g_slices = a.slices[j];
             if (a.slices[j] > 1) inside(a.part[j], (size_t)a.slices[j] * a.M * a.N[j] * 4);
         }
     } else if (strstr(name, "qmm_direct_kernel") || strstr(name, "qmm_dma_kernel")) {
@@ -66,7 +69,7 @@ hipError_t hipGetDeviceCount(int* n) { *n = 1; return hipSuccess; }
 hipError_t hipSetDevice(int) { return hipSuccess; }
 hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
 hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600* p, int) { memset(p, 0, sizeof *p); strcpy(p->gcnArchName, "gfx950"); return hipSuccess; }
-hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) { *v = 256; return hipSuccess; }
+hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) { *v = g_cus; return hipSuccess; }
 hipError_t hipGetSymbolAddress(void** p, const void* s) { *p = (void*)s; return hipSuccess; }
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { *s = (hipStream_t)8; return hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
@@ -112,6 +115,7 @@ static void batch(int dtype, int bits, uint32_t G, uint32_t M, uint32_t K, const
     g_fail = fail;
     g_allocs = g_starts = g_stops = 0;
     g_after_stop = false;
+    g_slices = 0;
     g_out.clear();
     mtq_timed_begin();
     if (mtq_qmm_batched(dtype, bits, G, 3, w, s, b, at(12), outs, N, M, K) != MTQ_OK) complain("the batch");
@@ -139,6 +143,17 @@ int main() {
                     batch(MTQ_BF16, 4, 64, 130, 4096, N, before, fail);
                     n += 2;
                 }
+    // a device of fewer compute units is filled with fewer slices
+    g_case = "GEMV on codes, slices";
+    const uint32_t N[3] = {1100, 1100, 1100};
+    uint32_t slices[2];
+    for (int i = 0; i < 2; i++) {
+        g_cus = i ? 32 : 256;
+        batch(MTQ_BF16, 5, 64, 20, 4736, N, false, 0);
+        slices[i] = g_slices;
+        n++;
+    }
+    if (slices[1] == 0 || slices[1] >= slices[0]) complain("as many slices for 32 compute units as for 256");
     printf("scratch_failures: %ld batches, %d violations\n", n, g_bad);
     return g_bad ? 1 : 0;
 }
