@@ -271,7 +271,11 @@ def test_k_run_lines_of_few_rows(bits, G, N, K, rows):
     (4, 64, 48, 5760, 5760, True), (8, 64, 96, 4736, 4736, True), (5, 64, 128, 4736, 4736, True), (4, 64, 65, 4736, 4736, False), (5, 64, 129, 4736, 4736, False),
     (4, 64, 96, 2304, 8320, True), (4, 64, 97, 2304, 8320, False), (5, 64, 126, 2304, 8320, True), (5, 64, 126, 3584, 12928, False), (5, 64, 96, 3584, 12928, True),   # (split)
     (4, 64, 32, 9472, 2176, True), (4, 64, 33, 9472, 2176, False), (8, 64, 48, 9472, 2176, True), (5, 64, 64, 9472, 2176, True), (5, 64, 65, 9472, 2176, False),
-    (4, 64, 60, 768, 6528, False), (4, 64, 60, 768, 4736, True), (2, 128, 72, 512, 1152, False), (4, 32, 20, 1152, 1152, False), (4, 64, 20, 1152, 1152, True),
+    (4, 64, 60, 768, 6528, True), (4, 64, 60, 768, 4736, True), (2, 128, 72, 512, 1152, False), (4, 32, 20, 1152, 1152, False), (4, 64, 20, 1152, 1152, True),
+    # few weight rows, past 64 activation rows
+    (4, 64, 60, 1792, 7040, True), (4, 64, 96, 1792, 7040, True), (8, 64, 96, 1792, 7040, True), (4, 64, 64, 512, 1664, True), (4, 64, 65, 512, 1664, False),
+    (4, 64, 65, 1120, 4480, False), (4, 64, 65, 1184, 4736, True), (8, 64, 65, 512, 1920, False), (8, 64, 65, 512, 2176, True), (5, 64, 128, 1792, 7040, True), (5, 64, 65, 256, 1664, False),
+    (8, 64, 128, 1024, 6528, True), (4, 64, 97, 1792, 7040, False),
     # rows that they can
     (5, 64, 32, 4096, 4096, False), (6, 64, 20, 8192, 2048, False), (6, 64, 20, 16384, 4096, False), (6, 64, 17, 18944, 3584, True), (6, 64, 48, 18944, 3584, True),
     (4, 64, 20, 28672, 8192, False), (8, 64, 20, 28672, 8192, True), (8, 64, 48, 28672, 4096, False), (8, 64, 48, 18944, 3584, False), (8, 64, 17, 128256, 4096, True),
