@@ -471,7 +471,8 @@ MTQ_API int mtq_flush_cache(void);
  *   "qmv.runs"             K-run matrix-core GEMV for batches of up to 16 rows (4- and 8-bit codes, f16 / bf16, K % 128 == 0,
  *                          K <= 8192, 5120 for 8-bit codes; the matrices of mtq_qmm_batched in one launch): 0 = where it is
  *                          the fastest kernel, 1 = never, 2 = wherever the shape allows, 3 = in slices of K (one matrix of rows
- *                          of more than 5120 codes, f32 sums in the library's buffer) wherever the shape allows
+ *                          of more than 5120 codes, f32 sums in the library's buffer) wherever the shape allows;
+ *                          2 and 3 deal the steps of rows of whole 128-byte lines to the waves in pairs, 0 where that is faster
  *   "qmv.wide"             16-row matrix-core GEMV for batches of 5..16 rows (4-bit codes, f16 / bf16, K % 512 == 0):
  *                          0 = where it is the fastest kernel, 1 = never, 2 = wherever the shape allows
  *   "qmv.wide_kp"          that kernel: waves that share a row block, 0 = choose, or 1 / 2 / 4 / 8 / 16

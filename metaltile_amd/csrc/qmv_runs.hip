@@ -23,10 +23,23 @@ static bool runs_aligned(const void* w, const void* s, const void* b, const void
 // (instances: qmv_runs_pick.h, one translation unit per element type)
 RunsInstance qmv_runs_pick_f16(bool paired, int bits, uint32_t G, bool sliced, uint32_t xs, bool few);
 RunsInstance qmv_runs_pick_bf16(bool paired, int bits, uint32_t G, bool sliced, uint32_t xs, bool few);
+// Whether the steps of a row are dealt to the waves in pairs: of rows of whole 128-byte lines, 8-bit and sliced ones always (2 x 3072 x 1024,
+// 8 bits, 4 rows 5.6 -> 5.4, 2 x 12288 x 4096 29.1 -> 21.1), 4-bit ones where that is the faster at every batch. bf16, groups of 64, us, runs -> pairs, three square
+// matrices and two of twice or three times as many rows, 5 | 16 rows:
+//   K = 512   5.0 5.0 -> 5.1 5.1 | 5.0 5.0 -> 5.1 5.2     1536  6.1 7.2 -> 6.1 7.0 | 6.1 7.2 -> 6.1 7.1      1792  6.3 7.3 -> 6.2 7.2 | 6.3 7.4 -> 6.2 7.3
+//       2304  7.8 11.2 -> 7.9 11.2 | 8.3 11.6 -> 8.4 11.6   2560  8.0 11.8 -> 7.9 11.4 | 8.4 12.0 -> 8.5 11.9   3584  10.4 15.1 -> 9.4 13.9 | 10.9 15.3 -> 10.2 14.7
+//       4096  11.3 -> 10.4, 2 x 14336 18.4 -> 16.6 | 11.7 -> 10.7, 18.7 -> 17.2      8192 (one)  14.7 -> 12.5 | 16.2 -> 16.1
+// A wave of rows of 4097 to 6144 codes has a pair and some have a step of their own beside it, half of a line whose other half is another wave's. Which
+// form is the faster there depends on the device and on how much of the weights its last-level cache still holds: three layers of 5120, 13824 wide, in groups
+// of 128 at 16 rows, runs -> pairs on eight devices 185 -> 178, 185.5 -> 178, 187 -> 186, 188 -> 188, 187 -> 188, 188 -> 194, 189 -> 195, 195 -> 205. So
+// runs there. (qmv.runs = 2 and 3: pairs wherever rows are whole lines.)
+static bool runs_paired(int bits, uint32_t K, bool sliced) {
+    if ((uint64_t)K * bits / 8 % 128) return false;
+    if (bits == 8 || sliced || options().qmv_runs >= 2) return true;
+    return K > 4096 ? K > 6144 : K > 2048 ? K >= 2560 : K >= 1792;
+}
 static RunsInstance runs_pick(int dtype, int bits, uint32_t G, uint32_t K, bool sliced, uint32_t xs, uint32_t M) {
-    // Rows of whole 128-byte lines; not where sixteen waves have a pair each and a few of them a step more, which the others wait for
-    // (bf16, groups of 64, 5 rows, 2 x 10240, us, runs -> pairs: K = 4352 17.5 -> 18.0, 4608 17.5 -> 18.5, but 5120 and 5376 alike or faster).
-    const bool paired = (uint64_t)K * bits / 8 % 128 == 0 && !(bits == 4 && !sliced && K > 4096 && K < 5120);
+    const bool paired = runs_paired(bits, K, sliced);
     return dtype == DT_BF16 ? qmv_runs_pick_bf16(paired, bits, G, sliced, xs, M <= 8) : qmv_runs_pick_f16(paired, bits, G, sliced, xs, M <= 8);
 }
 

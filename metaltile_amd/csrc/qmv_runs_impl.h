@@ -15,7 +15,7 @@
 // asked for before them. The same kernel with activations read per block streamed at half the rate.) The KP sums of
 // a result meet in LDS. The split of K depends on K and the code width: a matrix gives the same bits in whatever batch of matrices.
 //
-// A step is 128 codes of a row (64 of 8-bit codes), 64 bytes, two neighbouring ones of which are loaded together; of a step lane (j, q) = (lane % 16, lane / 16) multiplies the
+// A step is 128 codes of a row (64 of 8-bit codes), 64 bytes, two neighbouring ones of which are loaded together where rows are dealt in pairs; of a step lane (j, q) = (lane % 16, lane / 16) multiplies the
 // 16 bytes of row j at 16 q: 32 codes (16). What bounded the kernel was finding the lines: with neighbouring lanes in sixteen different rows
 // a load of 1 KB occupies the compute unit's address path four times as long as with four neighbours in one row, about 64 clk
 // against 16, and that was all of a block's 5000 clk at 16 rows (64 weight and scale loads of it). So four neighbours load a row's
@@ -135,10 +135,8 @@ template <bool PAIRED, int KP, bool SLICED, bool ORDERED, int DT, int BITS, int 
     }
     // Of the slice's steps, wave kp has the pairs kp, kp + KP, ... and, of what lies behind PAIRS * KP pairs, the kp-th step: two
     // neighbouring steps are the 128 bytes of a line, and the same loads streamed 58 MB at 4.4 TB/s in pieces of 64 bytes of
-    // a row, at 5.8 in pieces of 128. 16 rows, us, a run of steps a wave -> pairs: 2 x 13824 x 5120 in groups of 128 22.0 -> 20.6,
-    // 2 x 14336 x 4096 20.0 -> 18.7, 8 rows of 8192 x 8192 16.1 -> 13.7; 8 bits, 4 rows, 2 x 18944 x 3584 31.5 -> 26.9. Where rows are
-    // an odd number of steps a pair of every second row lies in two lines, and a run of steps a wave is the faster (4736 x 4736 9.6
-    // against 10.1). steps <= XS * KP (host).
+    // a row, at 5.8 in pieces of 128 (figures and lines: runs_paired). Where rows are an odd number of steps a pair of every second row
+    // lies in two lines, and a run of steps a wave is the faster (4736 x 4736 9.6 against 10.1). steps <= XS * KP (host).
     const uint32_t run0 = steps * kp / KP, run = steps * (kp + 1u) / KP - run0;
     auto step_of = [&](uint32_t n) { return !PAIRED ? run0 + n : n < 2u * PAIRS ? 2u * (kp + KP * (n >> 1)) + (n & 1u) : 2u * (uint32_t)(KP * PAIRS) + kp; };
     auto has_step = [&](uint32_t n) { return PAIRED ? n < (uint32_t)XS && step_of(n) < steps : n < run; };
@@ -152,7 +150,7 @@ template <bool PAIRED, int KP, bool SLICED, bool ORDERED, int DT, int BITS, int 
     // Weights of a pair: load 0 has rows 0 .. 7, load 1 rows 8 .. 15, slot lane % 8 of row lane / 8 of the eight pieces; these too
     // are dealt to the slots so that the reads do not meet in a bank. Of a step alone: as the activations.
     const uint32_t pr = lane >> 3, ppiece = (lane ^ pr) & 7u;
-    const uint32_t plane = pr * wrow_bytes + first_step * 64u + ppiece * 16u, wlane = lr * wrow_bytes + first_step * 64u + lpiece * 16u;
+    const uint32_t plane = pr * wrow_bytes + (first_step + 2u * kp) * 64u + ppiece * 16u, wlane = lr * wrow_bytes + (first_step + (PAIRED ? kp : run0)) * 64u + lpiece * 16u;
     uint32_t pair_dead[PAIRS ? PAIRS : 1];   // this lane's piece lies past the slice
 #pragma unroll
     for (int n = 0; n < PAIRS; n++) pair_dead[n] = (steps - 1u - step_of(2 * n) - (ppiece >> 2)) & KR_OOB;
@@ -192,7 +190,7 @@ template <bool PAIRED, int KP, bool SLICED, bool ORDERED, int DT, int BITS, int 
         const __amdgpu_buffer_rsrc_t wr = kr_rsrc(pick(a.w, at_blk), N * wrow_bytes), sr = kr_rsrc(pick(a.scales, at_blk), N * gpr * 2u),
                                      br = kr_rsrc(pick(a.biases, at_blk), N * gpr * 2u);
         const uint32_t dead = (rows - 1u - lr) & KR_OOB;
-        const uint32_t w0 = row0 * wrow_bytes, s0 = row0 * gpr * 2u;
+        const uint32_t w0 = row0 * wrow_bytes, s0 = row0 * gpr * 2u, wo = (wlane + w0) | dead;
 #pragma unroll
         for (int i = 0; i < SR; i++) {
             const uint32_t o = (slane[i] + s0) | dead;
@@ -211,9 +209,9 @@ template <bool PAIRED, int KP, bool SLICED, bool ORDERED, int DT, int BITS, int 
         for (int n = 0; n < PAIRS; n++)
 #pragma unroll
             for (uint32_t h = 0; h < 2; h++)
-                d.w[2 * n + h] = __builtin_amdgcn_raw_buffer_load_b128(wr, (int)((plane + w0 + 8u * h * wrow_bytes + 64u * step_of(2 * n)) | pair_dead[n] | ((rows - 1u - pr - 8u * h) & KR_OOB)), 0, KR_NT);
+                d.w[2 * n + h] = __builtin_amdgcn_raw_buffer_load_b128(wr, (int)((plane + w0 + 8u * h * wrow_bytes + 128u * KP * n) | pair_dead[n] | ((rows - 1u - pr - 8u * h) & KR_OOB)), 0, KR_NT);
 #pragma unroll
-        for (int n = 2 * PAIRS; n < XS; n++) d.w[n] = __builtin_amdgcn_raw_buffer_load_b128(wr, (int)((wlane + w0 + 64u * step_of(n)) | step_dead[n] | dead), 0, KR_NT);
+        for (int n = 2 * PAIRS; n < XS; n++) d.w[n] = __builtin_amdgcn_raw_buffer_load_b128(wr, (int)((wo + 64u * (PAIRED ? 2 * KP * PAIRS : n)) | step_dead[n]), 0, KR_NT);
     };
 
     Block ring[PF + 1];
@@ -225,11 +223,11 @@ template <bool PAIRED, int KP, bool SLICED, bool ORDERED, int DT, int BITS, int 
     kr_u32x4 xop[XS][C::UNITS];
     {
         const __amdgpu_buffer_rsrc_t xr = kr_rsrc((uint64_t)a.x, a.M * K * 2u);
-        const uint32_t xo = ((lr * K + first_step * (uint32_t)C::STEP + lpiece * 8u) * 2u) | ((a.M - 1u - lr) & KR_OOB);
+        const uint32_t xo = ((lr * K + (first_step + (PAIRED ? 0u : run0)) * (uint32_t)C::STEP + lpiece * 8u) * 2u) | ((a.M - 1u - lr) & KR_OOB);
 #pragma unroll
         for (int n = 0; n < XS; n++)
 #pragma unroll
-            for (int k = 0; k < C::UNITS; k++) xop[n][k] = __builtin_amdgcn_raw_buffer_load_b128(xr, (int)((xo + step_of(n) * (uint32_t)(C::STEP * 2) + (uint32_t)(k * 64)) | step_dead[n]), 0, 0);
+            for (int k = 0; k < C::UNITS; k++) xop[n][k] = __builtin_amdgcn_raw_buffer_load_b128(xr, (int)((xo + (PAIRED ? step_of(n) : (uint32_t)n) * (uint32_t)(C::STEP * 2) + (uint32_t)(k * 64)) | step_dead[n]), 0, 0);
         __builtin_amdgcn_sched_barrier(0);
         // No wave's weights ahead of another's activations. Not where a run is short, as the wait for the last of the waves to start
         // costs more there (us, with -> without): 8 bits, 5 rows 4096 x 2048 6.5 -> 5.9; 4 bits 11008 x 2048 7.8 -> 7.4, groups of 32

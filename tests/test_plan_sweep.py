@@ -265,6 +265,15 @@ def test_k_run_lines_of_few_rows(bits, G, N, K, rows):
     assert on == rows
 
 
+@pytest.mark.parametrize("bits,K,paired", [(4, 1536, False), (4, 1792, True), (4, 1920, False), (4, 2048, True), (4, 2304, False), (4, 2560, True), (4, 4096, True), (4, 4352, False),
+                                           (4, 5120, False), (4, 6144, False), (4, 6400, True), (4, 8192, True), (8, 1152, True), (8, 5120, True)])
+def test_k_run_steps_in_pairs(bits, K, paired):
+    """Which row lengths have their steps dealt to the waves in pairs, on both sides of each line."""
+    for M in (5, 8) + ((9, 16) if K <= 6144 else ()):
+        name = ops.plan("qmm", DType.BF16, bits, 64, M, 2048, K)[1][0][0]
+        assert ("qmv_runs_kernel<true" if paired else "qmv_runs_kernel<false") in name
+
+
 @pytest.mark.parametrize("bits,G,M,N,K,codes", [
     # rows that the tiles cannot split
     (5, 64, 16, 4736, 4736, True), (4, 64, 16, 4736, 4736, False), (4, 64, 17, 4736, 4736, True), (4, 64, 64, 5504, 5504, True), (4, 64, 64, 5760, 5760, False),
