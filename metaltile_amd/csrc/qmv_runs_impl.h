@@ -100,6 +100,7 @@ template <int DT, int BITS> __device__ __forceinline__ kr_u32x4 kr_weights(const
 // PAIRED: a row is a whole number of 128 bytes. DT, BITS (4 or 8), G (32, 64, 128), XS: steps of a wave at most, PF: blocks whose
 // weights are in flight ahead of the one that is worked on.
 template <bool PAIRED, int KP, bool SLICED, bool ORDERED, int DT, int BITS, int G, int XS, int PF> __device__ __forceinline__ void qmv_runs_body(const QmvRunsArgs& a) {
+    static_assert(PAIRED || BITS == 4, "rows of 8-bit codes are whole lines");
     using C = KrCodes<DT, BITS>;
     constexpr int EG = G < C::STEP ? G : C::STEP;   // codes per scale within a step
     constexpr int GPS = C::STEP / EG;               // scales per step: 1, 2 or 4

@@ -21,10 +21,11 @@ template <bool PAIRED, int DT, int BITS, int G> static RunsInstance runs_pick_st
         return {xs <= 4 ? (const void*)qmv_runs_kernel<PAIRED, true, 16, DT, 8, G, 4, 1> : (const void*)qmv_runs_kernel<PAIRED, true, 16, DT, 8, G, 5, 1>, 1024};
     }
 }
-// paired: rows are whole numbers of 128 bytes
+// paired: rows are whole numbers of 128 bytes (of 8-bit codes every row is)
 template <bool PAIRED, int DT> static RunsInstance runs_pick_type(int bits, uint32_t G, bool sliced, uint32_t xs, bool few) {
-    if (bits == 4) return G == 32 ? runs_pick_steps<PAIRED, DT, 4, 32>(sliced, xs, few) : G == 64 ? runs_pick_steps<PAIRED, DT, 4, 64>(sliced, xs, few) : runs_pick_steps<PAIRED, DT, 4, 128>(sliced, xs, few);
-    return G == 32 ? runs_pick_steps<PAIRED, DT, 8, 32>(sliced, xs, few) : G == 64 ? runs_pick_steps<PAIRED, DT, 8, 64>(sliced, xs, few) : runs_pick_steps<PAIRED, DT, 8, 128>(sliced, xs, few);
+    if constexpr (PAIRED)
+        if (bits == 8) return G == 32 ? runs_pick_steps<true, DT, 8, 32>(sliced, xs, few) : G == 64 ? runs_pick_steps<true, DT, 8, 64>(sliced, xs, few) : runs_pick_steps<true, DT, 8, 128>(sliced, xs, few);
+    return G == 32 ? runs_pick_steps<PAIRED, DT, 4, 32>(sliced, xs, few) : G == 64 ? runs_pick_steps<PAIRED, DT, 4, 64>(sliced, xs, few) : runs_pick_steps<PAIRED, DT, 4, 128>(sliced, xs, few);
 }
 template <int DT> static RunsInstance runs_pick_type(bool paired, int bits, uint32_t G, bool sliced, uint32_t xs, bool few) {
     return paired ? runs_pick_type<true, DT>(bits, G, sliced, xs, few) : runs_pick_type<false, DT>(bits, G, sliced, xs, few);
