@@ -99,15 +99,42 @@ bool qmv_held_norm_preferred(int bits, uint32_t G, uint32_t N, uint32_t K) {
     if (bits == 4 && G == 32 && K > 1600 && (uint64_t)N * K >= 60000000ull) return false;
     return bits != 4 || (uint64_t)N * K < 24000000ull || K <= 3200 || (K > 4096 && K < 5120);
 }
-// Batches of 2..16 rows, of the widths that the K-run kernel has not (alone | three, or two tall ones, in a call):
-// 3 bits, 4 rows 4096 x 4096 6.6 -> 7.3 | 19.8 -> 9.2; 5 bits, 5 rows 3456 x 3456 8.4 -> 8.6 | 25.1 -> 13.0; 14720 x 3456 15.2 -> 13.9 | 30.5 -> 22.4;
-// 6 bits, 8 rows 1024 x 4096 10.2 -> 8.0, 14336 x 4096 17.6 -> 15.3; 3 bits, 9 rows 1152 x 1152 9.3 -> 6.4; 5 bits, 16 rows 2048 x 2048 9.8 -> 7.6, 4096 x
-// 4096 12.0 -> 11.7, but 14336 x 4096 18.6 -> 21.3 (tiles); 2 bits, 4 rows 2304 x 2304 6.7 -> 7.1, 20000 x 2048 13.2 -> 9.5, 16 rows 3328 x 3328
-// 13.5 -> 8.6, 13312 x 3328 15.7 -> 12.6. Rows of more than 8192 codes leave a compute unit one workgroup: 3 bits, 4 rows 4096 x 11008
-// 11.1 -> 13.4.
+// Batches of 2..16 rows, of the widths that the K-run kernel has not. As there, a matrix's route cannot depend on whether it comes in a batch, so the
+// lines lie where two matrices of a size, or a square one with the two of a quarter of its rows that come with it, together gain more than one alone
+// loses. us on the device (bf16, groups of 64, weights from memory), others -> this, alone | together (q: 1, 1/4, 1/4; 2: two):
+//                  2 rows                     4 rows                     8 rows                      16 rows
+//   2 bits  2048 x 2048   4.2 -> 4.6 | q 12.1 -> 4.8    4.7 -> 4.7 | 14.7 -> 4.8    6.4 -> 5.3 | 15.8 -> 5.6     9.1 -> 6.4 | 9.5 -> 6.7
+//           4096 x 4096   5.3 -> 6.1 | q 15.4 -> 7.4    5.8 -> 6.7 | 19.6 -> 8.2    8.0 -> 7.9 | 17.6 -> 8.6    10.7 -> 10.1 | 21.2 -> 13.1
+//           14336 x 4096  9.4 -> 9.5 | 2 18.6 -> 15.1  10.1 -> 9.9 | 19.9 -> 15.6  12.9 -> 11.0 | 25.4 -> 18.2  15.6 -> 19.1 | 31.0 -> 28.3 (not taken)
+//           8192 x 8192   7.9 -> 11.5 | q 18.7 -> 14.9 (not taken)  9.8 -> 11.7 | 22.9 -> 14.2  20.6 -> 13.4 | 38.0 -> 19.4
+//           28672 x 8192 24.4 -> 25.4 | 2 49.0 -> 41.7 29.4 -> 26.6 | 58.8 -> 48.1 41.3 -> 31.4 | 81.9 -> 50.8
+//   3 bits  1024 x 1024   3.7 -> 4.4 | q 10.5 -> 4.4    4.4 -> 4.4 | 12.5 -> 4.5    6.0 -> 4.9 | 12.0 -> 5.0     6.4 -> 6.1 | 6.8 -> 6.0
+//           4096 x 4096   5.5 -> 6.8 | q 18.1 -> 8.2    6.3 -> 7.3 | 23.0 -> 9.4    8.2 -> 8.5 | 17.9 -> 9.7    11.0 -> 10.7 | 21.6 -> 13.9
+//           14336 x 4096 11.2 -> 12.0 | 2 22.3 -> 19.1 11.4 -> 12.3 | 22.5 -> 19.5 14.6 -> 12.9 | 28.8 -> 21.4
+//           28672 x 8192 29.9 -> 33.1 | 2 59.3 -> 54.4 31.5 -> 34.3 | 62.9 -> 62.6 (not taken)  44.0 -> 45.5 | 88.9 -> 83.6
+//           8192 x 1024                                                                         7.0 -> 7.8 | 7.8 -> 7.9 (not taken)
+//   5 bits  3072 x 3072   5.3 -> 7.0 | q 16.8 -> 8.6    6.5 -> 7.4 | 21.1 -> 9.4    8.0 -> 8.2 | 20.5 -> 9.5    14.0 -> 9.9 | 14.1 -> 10.9
+//           4096 x 4096   5.8 -> 7.6 | q 18.4 -> 9.4    7.0 -> 8.2 | 23.9 -> 10.4   8.7 -> 9.3 | 18.8 -> 10.8   12.2 -> 11.4 | 23.7 -> 15.3
+//           8192 x 4096   7.9 -> 9.7 | 2 15.6 -> 14.7   8.6 -> 10.7 | 16.8 -> 15.2 (neither taken)  10.8 -> 11.3 | 21.7 -> 17.0  14.8 -> 15.2 | 29.4 -> 22.7
+//           14336 x 4096 12.8 -> 14.2 | 2 25.1 -> 23.9 13.0 -> 14.6 | 25.8 -> 24.5 (neither)        16.2 -> 15.4 | 32.1 -> 26.7
+//           10240 x 5120 14.5 -> 16.2 | 2 28.7 -> 22.3 15.4 -> 17.0 | 30.5 -> 23.0 18.8 -> 15.4 | 37.5 -> 29.1
+//           21504 x 6144 25.2 -> 25.4 | 2 50.2 -> 46.0 26.5 -> 31.5 | 52.4 -> 47.6 (not taken)      34.6 -> 28.5 | 68.1 -> 50.5
+//   6 bits  2048 x 2048   3.9 -> 5.4 | q 12.5 -> 5.8    4.9 -> 5.4 | 15.5 -> 5.7    6.5 -> 6.2 | 16.5 -> 6.4     9.6 -> 7.2 | 10.9 -> 7.6
+//           7168 x 2048   6.0 -> 7.1 | 2 11.8 -> 9.5    6.2 -> 7.1 | 12.2 -> 9.7    7.5 -> 8.6 | 14.8 -> 10.3   11.0 -> 8.8 | 11.6 -> 13.4
+//           14336 x 4096 13.3 -> 13.6 | 2 26.4 -> 23.8 13.8 -> 14.1 | 27.1 -> 24.1 17.7 -> 15.2 | 34.6 -> 25.9
+//           8192 x 8192  14.2 -> 15.4 | q 27.6 -> 21.9 15.2 -> 15.8 | 31.5 -> 21.0 23.8 -> 20.6 | 43.2 -> 26.9
+// (3 rows as 4, 12 as 16. At 5 bits up to 4 rows the others lose little on rows of whole 2048 codes, whose steps of 512 the waves of the GEMV of up to 8 rows
+// share evenly: tall matrices of those are left there.)
+// From 9 rows past 8192 weight rows the tiles are ahead (14336 x 4096, 16 rows, 5 bits 18.6 -> 21.3), but at 2 bits; rows of more than 8192 codes leave a
+// compute unit one workgroup: 3 bits, 4 rows 4096 x 11008 11.1 -> 13.4.
 bool qmv_held_preferred(int bits, uint32_t M, uint32_t N, uint32_t K) {
     if (M < 2 || M > 16 || bits == 4 || bits == 8) return false;
-    return M <= 8 ? K <= 8192 : K <= 4096 && (N <= 8192 || bits == 2);
+    const bool tall = N >= 2 * (uint64_t)K;
+    if (M > 8) return K <= 4096 && (N <= 8192 || (bits == 2 && (M <= 12 || K <= 3328))) && !(bits != 6 && K <= 1024 && N > 4096);
+    if (K > 8192) return false;
+    if (bits == 5 && M <= 4 && tall && K % 2048 == 0) return false;
+    if (bits == 3 && M >= 3 && M <= 4 && K > 6144 && N >= 3 * (uint64_t)K) return false;
+    return !(bits == 2 && M == 2 && K > 6144 && N <= 2 * (uint64_t)K);
 }
 
 int launch_qmv_held(const QmvParams& p, const QmvBatch& b, const HeldNorm& n, const LaunchCtx& lc) {

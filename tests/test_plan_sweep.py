@@ -274,6 +274,20 @@ def test_k_run_steps_in_pairs(bits, K, paired):
         assert ("qmv_runs_kernel<true" if paired else "qmv_runs_kernel<false") in name
 
 
+@pytest.mark.parametrize("bits,M,N,K,held", [
+    (3, 1, 2048, 2048, False), (3, 2, 2048, 2048, True), (4, 8, 2304, 2304, False), (8, 4, 2304, 2304, False), (6, 8, 8192, 8192, True), (6, 8, 8192, 8320, False), (6, 9, 4096, 4096, True), (6, 9, 4096, 4352, False),
+    (5, 4, 8192, 4096, False), (5, 5, 8192, 4096, True), (5, 4, 8064, 4096, True), (5, 4, 10240, 5120, True), (5, 2, 21504, 6144, False), (6, 2, 21504, 6144, True), (5, 4, 4096, 4096, True),
+    (3, 4, 28672, 8192, False), (3, 2, 28672, 8192, True), (3, 5, 28672, 8192, True), (3, 4, 16384, 8192, True), (2, 2, 8192, 8192, False), (2, 3, 8192, 8192, True), (2, 2, 28672, 8192, True), (2, 2, 6144, 6144, True),
+    (2, 16, 14336, 4096, False), (2, 12, 14336, 4096, True), (2, 16, 13312, 3328, True), (5, 16, 8192, 2048, True), (5, 16, 8200, 2048, False),
+    (3, 16, 8192, 1024, False), (3, 16, 4096, 1024, True), (6, 16, 8192, 1024, True), (3, 8, 8192, 1024, True),
+])
+def test_held_gemv_lines(bits, M, N, K, held):
+    """Which batches the GEMV with its activations in LDS is for, on both sides of each line."""
+    op = "qmm" if M > 1 else "qmv"
+    rc, launches, _, _ = ops.plan(op, DType.BF16, bits, 64, M, N, K)
+    assert rc == 0 and ("qmv_held_kernel" in launches[0][0]) == held, launches[0][0]
+
+
 @pytest.mark.parametrize("bits,G,M,N,K,codes", [
     # rows that the tiles cannot split
     (5, 64, 16, 4736, 4736, True), (4, 64, 16, 4736, 4736, False), (4, 64, 17, 4736, 4736, True), (4, 64, 64, 5504, 5504, True), (4, 64, 64, 5760, 5760, False),
