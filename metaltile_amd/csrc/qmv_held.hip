@@ -31,12 +31,14 @@ static uint32_t held_cus() {
 struct HeldGeometry {
     HeldInstance k;
     uint32_t kpl, nb, per_cu;   // per_cu: workgroups on a compute unit
+    uint32_t cus;               // of the device
     uint32_t lds;
 };
 static bool held_geometry(int dtype, int bits, uint32_t G, int mode, uint32_t rows, uint32_t K, uint32_t blocks, HeldGeometry& g) {
     const Options& o = options();
     const uint32_t cus = held_cus(), rpl = held_log2rp(rows), pairs = (K / 128u + 1u) / 2u;
     g.k = held_pick(dtype, bits, G, mode, rows, K);
+    g.cus = cus;
     if (!g.k.fn) return false;
     // KP: what brings a thousand waves to the matrix, each with two and a half steps of 128 codes or more; at least four on long
     // rows. bf16, groups of 64, RMS norm included, KP 1 / 2 / 4 / 8, us: 1536 x 1280 7.0 5.8 5.6 5.5, 2816 x 2304 9.4 7.6 6.6 7.0, 14080 x 2304 11.7
@@ -69,8 +71,8 @@ static bool held_geometry(int dtype, int bits, uint32_t G, int mode, uint32_t ro
     return false;
 }
 
-// p: dtype, bits, group size, x, M, K
-bool qmv_held_takes(const QmvParams& p, const QmvBatch& b, const HeldNorm& n) {
+// p: dtype, bits, group size, x, M, K; g: the geometry of a call that is taken
+static bool held_plan(const QmvParams& p, const QmvBatch& b, const HeldNorm& n, HeldGeometry& g) {
     const uint32_t G = p.group_size, K = p.K, rows = n.mode == HELD_PLAIN ? p.M : 2u;
     if ((p.dtype != DT_F16 && p.dtype != DT_BF16) || (p.bits != 2 && p.bits != 3 && p.bits != 4 && p.bits != 5 && p.bits != 6 && p.bits != 8)) return false;
     if ((G != 32 && G != 64 && G != 128) || K == 0 || K % 128 || K % G || rows == 0 || rows > 16 || b.n < 1 || b.n > 4 || K > (1u << 17)) return false;
@@ -82,8 +84,11 @@ bool qmv_held_takes(const QmvParams& p, const QmvBatch& b, const HeldNorm& n) {
         if (b.N[j] == 0 || (uintptr_t)b.w[j] % 16 || (uintptr_t)b.scales[j] % 4 || (uintptr_t)b.biases[j] % 4) return false;
         blocks += (b.N[j] + 15u) / 16u;
     }
-    HeldGeometry g;
     return blocks < (1u << 26) && held_geometry(p.dtype, p.bits, G, n.mode, rows, K, (uint32_t)blocks, g);
+}
+bool qmv_held_takes(const QmvParams& p, const QmvBatch& b, const HeldNorm& n) {
+    HeldGeometry g;
+    return held_plan(p, b, n, g);
 }
 
 // Where the kernel stands against the others: they have a launch per matrix, or three where a row is normalised first and their
@@ -138,7 +143,8 @@ bool qmv_held_preferred(int bits, uint32_t M, uint32_t N, uint32_t K) {
 }
 
 int launch_qmv_held(const QmvParams& p, const QmvBatch& b, const HeldNorm& n, const LaunchCtx& lc) {
-    if (!qmv_held_takes(p, b, n)) return fail(ERR_UNSUPPORTED, "GEMV with its activations in LDS: shape not taken");
+    HeldGeometry g;
+    if (!held_plan(p, b, n, g)) return fail(ERR_UNSUPPORTED, "GEMV with its activations in LDS: shape not taken");
     const uint32_t rows = n.mode == HELD_PLAIN ? p.M : 2u;
     QmvHeldArgs a{};
     for (int j = 0; j < 4; j++) {
@@ -160,13 +166,11 @@ int launch_qmv_held(const QmvParams& p, const QmvBatch& b, const HeldNorm& n, co
     a.M = n.mode == HELD_PLAIN ? p.M : 1u;
     a.K = p.K;
     while ((1u << a.log2g) < p.group_size) a.log2g++;
-    HeldGeometry g;
-    if (!held_geometry(p.dtype, p.bits, p.group_size, n.mode, rows, p.K, a.blocks, g)) return fail(ERR_UNSUPPORTED, "GEMV with its activations in LDS: geometry");
     a.log2kp = g.kpl;
     a.log2rp = held_log2rp(rows);
     a.waves = g.nb << g.kpl;
-    const uint32_t tasks = (a.blocks + g.nb - 1u) / g.nb, most = held_cus() * g.per_cu, wgs = tasks < most ? tasks : most;
-    hipError_t e = set_max_dynamic_lds(g.k.fn, g.lds);
+    const uint32_t tasks = (a.blocks + g.nb - 1u) / g.nb, most = g.cus * g.per_cu, wgs = tasks < most ? tasks : most;
+    hipError_t e = g.lds > 64u * 1024u ? set_max_dynamic_lds(g.k.fn, g.lds) : hipSuccess;   // (what a launch may have unasked: no static LDS here)
     if (e != hipSuccess) return hip_fail(e, "GEMV with its activations in LDS: LDS");
     void* args[] = {&a};
     e = launch_kernel(g.k.fn, dim3(wgs), dim3(a.waves * 64u), args, g.lds, lc);
