@@ -40,14 +40,17 @@ static bool held_geometry(int dtype, int bits, uint32_t G, int mode, uint32_t ro
     g.k = held_pick(dtype, bits, G, mode, rows, K);
     g.cus = cus;
     if (!g.k.fn) return false;
-    // KP: what brings a thousand waves to the matrix, each with two and a half steps of 128 codes or more; at least four on long
+    // KP: what brings more than a thousand waves to the matrix, each with two and a half steps of 128 codes or more; at least four on long
     // rows. bf16, groups of 64, RMS norm included, KP 1 / 2 / 4 / 8, us: 1536 x 1280 7.0 5.8 5.6 5.5, 2816 x 2304 9.4 7.6 6.6 7.0, 14080 x 2304 11.7
     // 9.4 10.5 11.8, 88612 x 2816 27.7 29.0 29.7 39.3, 5 bits 20480 x 2560 14.3 14.9 15.1 15.1, 57344 x 7808 77.2 80.5 70.7 72.0, 6 bits 86686 x 1408
-    // 24.6 26.5 26.0; without a norm 3 bits 5120 x 5120 15.3 11.8 9.0 9.9, 5 bits 2560 x 10240 29.3 17.8 11.4 10.1. For several rows by the row length alone, so that a matrix gives the same bits alone and in a batch (5 rows, 5
-    // bits, 3 x 3456 x 3456 13.0 12.0 14.6, 2 x 14720 x 3456 22.5 22.8 24.1).
+    // 24.6 26.5 26.0; without a norm 3 bits 5120 x 5120 15.3 11.8 9.0 9.9, 5 bits 2560 x 10240 29.3 17.8 11.4 10.1. A thousand and 24 waves, four to a compute unit,
+    // are too few where two waves or one share rows, or a wave has more than 12 steps: 16384 x 4096, 2 bits 15.4 -> 10.8; 8192 x 2304 9.1 -> 7.8, x 3584, gated norm,
+    // 14.3 -> 9.8; 4096 x 9216, 3 bits 13.4 -> 10.9, but x 4736 8.2 -> 9.0. For several rows by the row length alone, so that a matrix gives the
+    // same bits alone and in a batch (5 rows, 5 bits, 3 x 3456 x 3456 13.0 12.0 14.6, 2 x 14720 x 3456 22.5 22.8 24.1).
     uint32_t kpl = K > 4608 ? 2 : 0;
     const bool fixed = mode == HELD_PLAIN && rows > 1;
-    while (kpl < (fixed ? 2u : 4u) && (fixed || (blocks << kpl) < 1024u) && (K / 128u) * 2u >= 5u << (kpl + 1)) kpl++;
+    auto few = [&]() { return (blocks << kpl) < 1024u || ((blocks << kpl) == 1024u && (kpl < 2 || (K / 128u) >> kpl > 12u)); };
+    while (kpl < (fixed ? 2u : 4u) && (fixed || few()) && (K / 128u) * 2u >= 5u << (kpl + 1)) kpl++;
     if (o.qmv_held_kp) for (kpl = 0; (2u << kpl) <= (uint32_t)o.qmv_held_kp; kpl++) {}
     while (kpl && (1u << kpl) > pairs) kpl--;
     // a normalised row: at most two pieces of 16 elements a thread

@@ -274,6 +274,14 @@ def test_k_run_steps_in_pairs(bits, K, paired):
         assert ("qmv_runs_kernel<true" if paired else "qmv_runs_kernel<false") in name
 
 
+@pytest.mark.parametrize("N,K,waves", [(16384, 3584, 2048), (16000, 3584, 2000), (8192, 3584, 2048), (8000, 3584, 2000), (8208, 3584, 1028), (4096, 3584, 1024), (4096, 9216, 2048), (2048, 9216, 1024), (2048, 18944, 2048)])
+def test_held_gemv_waves_of_a_matrix(N, K, waves):
+    """More than 1024 waves, or 1024 where four and more share rows and have a few steps each."""
+    _, launches, _, _ = ops.plan("rms_norm_qmv", DType.BF16, 3, 64, 1, N, K)
+    kernel, grid, block, _ = launches[0]
+    assert "qmv_held_kernel" in kernel and grid[0] * (block[0] // 64) == waves
+
+
 @pytest.mark.parametrize("bits,M,N,K,held", [
     (3, 1, 2048, 2048, False), (3, 2, 2048, 2048, True), (4, 8, 2304, 2304, False), (8, 4, 2304, 2304, False), (6, 8, 8192, 8192, True), (6, 8, 8192, 8320, False), (6, 9, 4096, 4096, True), (6, 9, 4096, 4352, False),
     (5, 4, 8192, 4096, False), (5, 5, 8192, 4096, True), (5, 4, 8064, 4096, True), (5, 4, 10240, 5120, True), (5, 2, 21504, 6144, False), (6, 2, 21504, 6144, True), (5, 4, 4096, 4096, True),
