@@ -7,9 +7,9 @@ namespace mtq {
 // What the conversion adds to every code: the power of two in whose mantissa (10 bits in f16, 7 in bf16) a code that stands AT bits up is the
 // code itself. The f32 sums carry the offset, so it is to be small, and AT large. LEAST: the one that leaves no more room than the
 // code needs, and 8-bit codes with the offset taken out again by a packed subtraction; else the largest that leaves one of the shifts below
-// free, as AT = 0 does. Error of the sums of a row of 4096 f16 4-bit codes, of a result of 6.2, with 1024, 64 and 16: 1.6e-4, 1.1e-5 and 3.4e-6;
-// 3.5e-6 in the streaming kernel, whose calls LEAST is for. It costs a shift in eight or an addition to each pair (67882 x 2304, 4 bits, norm
-// included, 22.3 -> 23.0 us; 14336 x 1664, 8 bits, 9.3 -> 9.8).
+// free, as AT = 0 does. Error of the sums of a row of 1024 f16 4-bit codes, of a result of 2.9, with 1024, 64 and 16: 1.0e-4, 6.4e-6 and 2.2e-6;
+// 2.0e-6 in the kernels whose calls LEAST is for. It costs a shift in eight or an addition to each pair (67882 x 2304, 4 bits, norm included, 22.3 ->
+// 23.0 us; 14336 x 1664, 8 bits, 9.3 -> 9.8).
 template <int DT, int BITS, bool LEAST> struct QcCodes {
     static_assert(!LEAST || DT == DT_F16, "bf16: 128 and less in every kernel");
     static constexpr int ROOM = (DT == DT_F16 ? 10 : 7) - BITS;

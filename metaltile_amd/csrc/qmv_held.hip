@@ -4,16 +4,14 @@
 namespace mtq {
 
 // (instances: one translation unit per element type and kind of group)
-HeldInstance qmv_held_pick_f16(int bits, int mode, uint32_t rows, bool least);
-HeldInstance qmv_held_pick_f16_g32(int bits, int mode, uint32_t rows, bool least);
-HeldInstance qmv_held_pick_bf16(int bits, int mode, uint32_t rows, bool least);
-HeldInstance qmv_held_pick_bf16_g32(int bits, int mode, uint32_t rows, bool least);
+HeldInstance qmv_held_pick_f16(int bits, int mode, uint32_t rows);
+HeldInstance qmv_held_pick_f16_g32(int bits, int mode, uint32_t rows);
+HeldInstance qmv_held_pick_bf16(int bits, int mode, uint32_t rows);
+HeldInstance qmv_held_pick_bf16_g32(int bits, int mode, uint32_t rows);
 
-static HeldInstance held_pick(int dtype, int bits, uint32_t G, int mode, uint32_t rows, uint32_t K) {
-    // (the streaming kernel's norm takes rows of whole 2048 codes; plain ones are its and the one-shot kernel's at every length)
-    const bool least = mode == HELD_NORM ? K % 2048 == 0 : rows == 1;
-    if (dtype == DT_BF16) return G == 32 ? qmv_held_pick_bf16_g32(bits, mode, rows, least) : qmv_held_pick_bf16(bits, mode, rows, least);
-    return G == 32 ? qmv_held_pick_f16_g32(bits, mode, rows, least) : qmv_held_pick_f16(bits, mode, rows, least);
+static HeldInstance held_pick(int dtype, int bits, uint32_t G, int mode, uint32_t rows) {
+    if (dtype == DT_BF16) return G == 32 ? qmv_held_pick_bf16_g32(bits, mode, rows) : qmv_held_pick_bf16(bits, mode, rows);
+    return G == 32 ? qmv_held_pick_f16_g32(bits, mode, rows) : qmv_held_pick_f16(bits, mode, rows);
 }
 
 static uint32_t held_log2rp(uint32_t rows) {
@@ -37,7 +35,7 @@ struct HeldGeometry {
 static bool held_geometry(int dtype, int bits, uint32_t G, int mode, uint32_t rows, uint32_t K, uint32_t blocks, HeldGeometry& g) {
     const Options& o = options();
     const uint32_t cus = held_cus(), rpl = held_log2rp(rows), pairs = (K / 128u + 1u) / 2u;
-    g.k = held_pick(dtype, bits, G, mode, rows, K);
+    g.k = held_pick(dtype, bits, G, mode, rows);
     g.cus = cus;
     if (!g.k.fn) return false;
     // KP: what brings more than a thousand waves to the matrix, each with two and a half steps of 128 codes or more; at least four on long
@@ -96,16 +94,29 @@ bool qmv_held_takes(const QmvParams& p, const QmvBatch& b, const HeldNorm& n) {
 
 // Where the kernel stands against the others: they have a launch per matrix, or three where a row is normalised first and their
 // row lengths are not the ones it is fused for. us, bf16, groups of 64, others -> this.
-// RMS norm, 4 bits: 1280 x 1024 9.5 -> 5.0, 2816 x 2304 11.1 -> 6.8, 5248 x 4224 14.0 -> 10.0 (norm, GEMV, sum); against the norm inside the
-// matrix-core GEMV, from 24 M codes: 14080 x 2304 10.4 -> 9.4, 19200 x 3200 15.9 -> 14.7, 67882 x 2304 26.0 -> 21.3, 25344 x 4224 24.7 -> 19.2,
-// but 23040 x 3840 15.1 -> 15.6, 32256 x 5376 21.4 -> 22.2, 46080 x 7680 36.7 -> 39.8. 2 bits 4096 x 1024 11.1 -> 5.6, 16384 x 4096 15.2 -> 10.6, 32768 x
-// 8192 31.3 -> 25.9; 3 bits 14720 x 3456 16.3 -> 11.4, 5 bits 20480 x 2560 23.8 -> 14.8, 57344 x 7808 83.2 -> 80.7, 6 bits 131838 x 1408 54.6 -> 35.0;
-// 8 bits 14336 x 1664 14.2 -> 9.5, 30000 x 3712 31.6 -> 24.0, but 20480 x 5120 23.1 -> 24.3. 4 bits in groups of 32: 14080 x 2304 11.2 -> 10.1,
-// 86686 x 1280 20.2 -> 18.5, but 86686 x 1664 21.5 -> 24.7.
+// RMS norm, 4 bits: 1280 x 1024 9.5 -> 5.0, 2816 x 2304 11.1 -> 6.8, 512 x 9216 11.8 -> 10.8 (norm, GEMV, sum); against the norm inside the
+// matrix-core GEMV, from 24 M codes: 14080 x 2304 10.4 -> 9.4, 19200 x 3200 15.9 -> 14.7, 67882 x 2304 26.0 -> 21.3, 25600 x 3328 / 3968 / 4224 / 4608 / 4736 / 4864 / 4992 / 5248 / 5632
+// 14.8 17.1 24.4 22.8 22.0 18.7 22.5 22.2 19.1 -> 15.1 17.7 19.4 19.2 22.4 20.8 23.0 24.1 22.7, 46080 x 4224 / 4736 / 4864 / 4992 34.3 32.6 28.0 33.5 -> 29.9 30.7 28.2 32.0. Rows of whole 2048 codes are
+// the streaming kernel's, which takes them in one launch too: 512 x 2048 4.4 -> 5.2, 1000 x 4096 4.7 -> 6.5, 8192 5.1 -> 10.2, 1500 x 12288 11.3 -> 12.2. 4 bits in groups
+// of 32: 14080 x 2304 11.2 -> 10.1, 86686 x 1280 20.2 -> 18.5, but 86686 x 1664 21.5 -> 24.7.
+// 2 bits 4096 x 1024 9.6 -> 5.4, 8192 x 8192 14.2 -> 11.7; 3 bits 14720 x 3456 16.3 -> 11.4, 5 bits 20480 x 2560 23.8 -> 14.4, 57344 x 8192 78.8 -> 73.5, 6 bits
+// 131838 x 1408 54.6 -> 37; 8 bits 14336 x 1664 14.2 -> 9.3, 32768 x 4608 38.9 -> 27.8, but 20480 x 5120 23.1 -> 24.3.
+// Heads of more than 65536 rows, of which the GEMV of the others reads 2- to 5-bit codes faster: 70000 / 100000 / 150000 x 3968, 2 bits 31.5 / 39.8 / 53.1 -> 36.7 / 50.7 / 64.3, 3 bits
+// 43 / 56 / 75 -> 46 / 63 / 81, 100000 x 4096, 5 bits 73 -> 79; 100000 x 3328, 2 bits 35.0 -> 38.5, 3584, 3 bits 50.2 -> 52.5; 7168 and 7936, 2 bits 61 and 64 -> 65 and 69, 7936, 3 bits
+// 150000 130 -> 135. Rows of more than 16384 codes leave a compute unit one workgroup, whose second round costs the most there: 5120 x 18944, 5 bits 32.2 -> 36.5, 8192 38.8 -> 38.9;
+// 8192 x 28672, 2 bits 36.0 -> 42.1, 16384 55.5 -> 47.5.
 bool qmv_held_norm_preferred(int bits, uint32_t G, uint32_t N, uint32_t K) {
     if (bits == 8) return K < 5120;
-    if (bits == 4 && G == 32 && K > 1600 && (uint64_t)N * K >= 60000000ull) return false;
-    return bits != 4 || (uint64_t)N * K < 24000000ull || K <= 3200 || (K > 4096 && K < 5120);
+    if (K > 16384 && N > 4096 && N < (K > 20480 ? 16384u : 8192u)) return false;
+    if (N > 65536 && K > 3200 && bits != 6) {
+        if (bits == 2 && (K <= 4096 || (K >= 7168 && K < 8192))) return false;
+        if (bits == 3 && ((K > 3456 && K <= 4096) || (K > 7680 && K <= 8192))) return false;
+        if (bits == 5 && K > 3968 && K <= 4096) return false;
+    }
+    if (bits != 4) return true;
+    if (K % 2048 == 0) return false;
+    if (G == 32 && K > 1600 && (uint64_t)N * K >= 60000000ull) return false;
+    return (uint64_t)N * K < 24000000ull || K <= 3200 || (K > 4096 && K < 5120 && (K <= 4608 || K % 256));
 }
 // Batches of 2..16 rows, of the widths that the K-run kernel has not. As there, a matrix's route cannot depend on whether it comes in a batch, so the
 // lines lie where two matrices of a size, or a square one with the two of a quarter of its rows that come with it, together gain more than one alone

@@ -2,6 +2,6 @@
 
 namespace mtq {
 
-HeldInstance qmv_held_pick_bf16_g32(int bits, int mode, uint32_t rows, bool least) { return held_pick_bits<DT_BF16, true>(bits, mode, rows, least); }
+HeldInstance qmv_held_pick_bf16_g32(int bits, int mode, uint32_t rows) { return held_pick_bits<DT_BF16, true>(bits, mode, rows); }
 
 }  // namespace mtq

@@ -57,10 +57,12 @@ template <int BITS, bool G32> struct QhLds {
     static constexpr uint32_t bytes(uint32_t K, uint32_t rpl, uint32_t waves) { return xbytes(K, rpl) + waves * WB + ((2u * waves * 64u) << rpl) + 64u; }
 };
 
-// DT, BITS, groups of 32 (else 64 or 128), NR: result registers that hold rows (1: one row, 2: value and remainder, 4), MODE, LEAST: of QcCodes
-template <int DT, int BITS, bool G32, int NR, int MODE, bool LEAST> __global__ __launch_bounds__(1024) void qmv_held_kernel(QmvHeldArgs a) {
+// DT, BITS, groups of 32 (else 64 or 128), NR: result registers that hold rows (1: one row, 2: value and remainder, 4), MODE
+template <int DT, int BITS, bool G32, int NR, int MODE> __global__ __launch_bounds__(1024) void qmv_held_kernel(QmvHeldArgs a) {
     using L = QhLds<BITS, G32>;
     constexpr int NL = (BITS + 1) / 2;                  // 16-byte loads of two steps: 32 * BITS pieces
+    // (one row of f16 4- and 8-bit codes came from the streaming and one-shot kernels)
+    constexpr bool LEAST = NR == 1 && DT == DT_F16 && (BITS == 4 || BITS == 8);
     using C = QcCodes<DT, BITS, LEAST>;
     constexpr float MAGIC = C::MAGIC;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];

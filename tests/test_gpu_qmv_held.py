@@ -142,8 +142,8 @@ def test_infinite_activations(oracle, held, dt, bits, G, M, N, K):
 
 
 @pytest.mark.parametrize("op,dt,bits,N,K", [
-    ("norm", DType.F16, 4, 512, 4096), ("norm", DType.F16, 4, 256, 2048), ("norm", DType.F16, 4, 1024, 8192), ("norm", DType.F16, 2, 512, 4096), ("norm", DType.BF16, 4, 512, 4096),
-    ("batch", DType.F16, 4, 512, 1024), ("batch", DType.F16, 8, 512, 512), ("batch", DType.BF16, 8, 512, 512), ("batch", DType.F16, 3, 512, 1152), ("norm", DType.F16, 5, 512, 2304),
+    ("norm", DType.F16, 4, 512, 2304), ("norm", DType.F16, 2, 512, 4096), ("norm", DType.BF16, 4, 512, 2304), ("norm", DType.F16, 5, 512, 2304), ("norm", DType.F16, 8, 512, 1152),
+    ("batch", DType.F16, 4, 512, 1024), ("batch", DType.F16, 8, 512, 512), ("batch", DType.BF16, 8, 512, 512), ("batch", DType.F16, 3, 512, 1152),
 ])
 def test_no_more_of_the_codes_offset_than_before(op, dt, bits, N, K):
     """The error of the f32 sums, bare of the result's rounding: the biases of a row's last two groups are set so that its exact

@@ -274,6 +274,19 @@ def test_k_run_steps_in_pairs(bits, K, paired):
         assert ("qmv_runs_kernel<true" if paired else "qmv_runs_kernel<false") in name
 
 
+@pytest.mark.parametrize("bits,G,N,K,held", [
+    (4, 64, 256, 2048, False), (4, 64, 1000, 4096, False), (4, 64, 1500, 8192, False), (4, 64, 512, 18432, False), (4, 64, 500, 2304, True), (4, 64, 256, 3072, True), (4, 64, 6000, 3840, True), (4, 64, 6400, 3840, False),
+    (4, 64, 70000, 3200, True), (4, 64, 7000, 4224, True), (4, 64, 7000, 4736, True), (4, 64, 7000, 4864, False), (4, 64, 7000, 5248, False), (4, 32, 70000, 1408, True), (4, 32, 70000, 1664, False),
+    (2, 64, 16384, 4096, True), (2, 64, 65536, 4096, True), (2, 64, 65537, 4096, False), (2, 64, 70000, 3200, True), (2, 64, 70000, 6656, True), (2, 64, 70000, 7168, False), (2, 64, 70000, 8192, True),
+    (3, 64, 100000, 3456, True), (3, 64, 100000, 3584, False), (3, 64, 100000, 4224, True), (3, 64, 100000, 7936, False), (5, 64, 100000, 3968, True), (5, 64, 100000, 4096, False), (6, 64, 100000, 4096, True),
+    (5, 64, 4096, 18944, True), (5, 64, 5120, 18944, False), (6, 64, 8192, 18944, True), (2, 64, 8192, 28672, False), (2, 64, 16384, 28672, True), (8, 64, 4096, 4992, True), (8, 64, 4096, 5248, False),
+])
+def test_held_norm_lines(bits, G, N, K, held):
+    """Which RMS-normalised rows the GEMV with its activations in LDS is for, on both sides of each line."""
+    rc, launches, _, _ = ops.plan("rms_norm_qmv", DType.BF16, bits, G, 1, N, K)
+    assert rc == 0 and ("qmv_held_kernel" in launches[0][0]) == held, launches[0][0]
+
+
 @pytest.mark.parametrize("N,K,waves", [(16384, 3584, 2048), (16000, 3584, 2000), (8192, 3584, 2048), (8000, 3584, 2000), (8208, 3584, 1028), (4096, 3584, 1024), (4096, 9216, 2048), (2048, 9216, 1024), (2048, 18944, 2048)])
 def test_held_gemv_waves_of_a_matrix(N, K, waves):
     """More than 1024 waves, or 1024 where four and more share rows and have a few steps each."""
