@@ -728,9 +728,8 @@ static int op_gated_rms_norm_qmv(int dtype, uint32_t G, const float* y, const vo
         rc = launch_qmv_gated_norm(p, z, norm_w, eps, dv, lc);
         if (rc != ERR_UNSUPPORTED) return rc;
     }
-    // row lengths that it does not take: the GEMV that holds the row in LDS (2560 rows, hv 8 / 24 / 40 of dv 128, us, norm, GEMV and sum
-    // -> this: 11.1 -> 6.3, 12.2 -> 7.7, 12.6 -> 9.5)
-    rc = try_held(dtype, 4, G, 1, &w, &s, &b, y, &out, &N, K, hn, true, lc);
+    // row lengths that it does not take: the GEMV that holds the row in LDS, where it is the faster
+    rc = try_held(dtype, 4, G, 1, &w, &s, &b, y, &out, &N, K, hn, qmv_held_gated_preferred(N, K), lc);
     if (rc != ERR_UNSUPPORTED) return rc;
     return qmv_of_staged_row(dtype, 4, G, w, s, b, out, N, K, lc, [&](void* dst, const LaunchCtx& ctx) {
         return launch_gated_rms_norm(dtype, y, z, norm_w, eps, dst, hv, dv, ctx);

@@ -118,6 +118,17 @@ bool qmv_held_norm_preferred(int bits, uint32_t G, uint32_t N, uint32_t K) {
     if (G == 32 && K > 1600 && (uint64_t)N * K >= 60000000ull) return false;
     return (uint64_t)N * K < 24000000ull || K <= 3200 || (K > 4096 && K < 5120 && (K <= 4608 || K % 256));
 }
+// Gated norm, 4 bits, row lengths that the streaming kernel does not take (norm, GEMV of two rows and sum -> this): 512 / 2560 / 5120 / 16384 rows x 2304 9.3 8.7 10.2 13.2 -> 6.6
+// 6.9 9.2 10.4, x 4608 9.6 10.6 12.8 18.4 -> 9.4 9.8 12.0 14.9. Longer rows take a compute unit's LDS for two workgroups of few waves: 512 / 2048 / 2560 / 4096 / 5120 / 8192 / 12288 rows x
+// 5376 8.7 9.6 10.3 10.5 12.5 13.0 14.9 -> 9.3 9.8 9.6 9.8 13.7 13.8 16.5, x 6016 8.9 9.3 10.6 10.8 13.7 14.4 17.3 -> 9.4 10.0 9.6 9.7 13.9 14.1 16.7, x 7680 10.8 10.4 10.9 11.3 13.2 14.2 18.5 ->
+// 9.8 10.2 10.1 10.2 15.3 15.4 18.7, x 9216 9.2 10.8 12.6 13.2 14.6 16.5 20.1 -> 11.9 12.5 12.1 12.3 14.8 15.0 21.3; 5120 / 8192 x 5120 12.5 12.9 -> 12.0 12.2.
+bool qmv_held_gated_preferred(uint32_t N, uint32_t K) {
+    if (K <= 4608) return true;
+    if (K > 6144 && K <= 8192) return N <= 4096 || N > 8192;
+    if (N <= 2048) return false;
+    if (K > 8192) return N <= 8192;
+    return N <= 4096 || K <= 5120 || K > 5632;
+}
 // Batches of 2..16 rows, of the widths that the K-run kernel has not. As there, a matrix's route cannot depend on whether it comes in a batch, so the
 // lines lie where two matrices of a size, or a square one with the two of a quarter of its rows that come with it, together gain more than one alone
 // loses. us on the device (bf16, groups of 64, weights from memory), others -> this, alone | together (q: 1, 1/4, 1/4; 2: two):

@@ -2,7 +2,8 @@
 // host code makes are answered here: an allocation is host memory or, by a schedule, fails as it does on a full card (the
 // buffer it was to replace is gone by then), and a launch is looked at instead of made. Whatever the schedule, each matrix of
 // a batch is worked out once, every kernel's partial results lie inside memory that is allocated at its launch, and the
-// call's two timestamps are each taken once. And the slices of the GEMV on codes follow the device's compute units. Built with the sanitizers from the library's own host code (metaltile_amd/build.py,
+// call's two timestamps are each taken once. And the slices of the GEMV on codes follow the device's compute units, and the gated
+// norm, of which mtq_plan knows nothing, goes where its lines say. Built with the sanitizers from the library's own host code (metaltile_amd/build.py,
 // build_sanitized). Exit code 0 = all of that holds.
 #include "qmm_direct_plan.h"
 #include "qmv_codes_impl.h"
@@ -25,6 +26,7 @@ int g_allocs = 0, g_starts = 0, g_stops = 0, g_bad = 0;
 bool g_after_stop = false;
 int g_cus = 256;                    // compute units of the device
 uint32_t g_slices = 0;              // most slices of K of a matrix on the GEMV on codes
+int g_held = 0, g_others = 0;       // launches of the GEMV with its activations in LDS, and of kernels not looked into
 std::multiset<const void*> g_out;   // results that the launches so far work out
 const char* g_case = "";
 
@@ -56,8 +58,10 @@ hipError_t launch(const void* fn, void** args) {
             g_out.insert(a.more.out[j]);
             if (a.ksplit > 1) inside(a.more.part[j], (size_t)a.ksplit * a.M * a.more.N[j] * 4);
         }
+    } else if (strstr(name, "qmv_held_kernel")) {
+        g_held++;
     } else if (!strstr(name, "reduce") && !strstr(name, "add")) {
-        complain(name);
+        g_others++;
     }
     return hipSuccess;
 }
@@ -116,11 +120,13 @@ static void batch(int dtype, int bits, uint32_t G, uint32_t M, uint32_t K, const
     g_allocs = g_starts = g_stops = 0;
     g_after_stop = false;
     g_slices = 0;
+    g_held = g_others = 0;
     g_out.clear();
     mtq_timed_begin();
     if (mtq_qmm_batched(dtype, bits, G, 3, w, s, b, at(12), outs, N, M, K) != MTQ_OK) complain("the batch");
     for (void* o : outs)
         if (g_out.count(o) != 1) complain(g_out.count(o) ? "a matrix worked out twice" : "a matrix left out");
+    if (g_held || g_others) complain("kernels of others");
     if (g_starts != 1 || g_stops != 1) complain("timestamps");
     g_after_stop = false;
     g_fail = 0;
@@ -128,8 +134,30 @@ static void batch(int dtype, int bits, uint32_t G, uint32_t M, uint32_t K, const
     if (!g_live.empty()) complain("scratch not given back");
 }
 
+// Whether the gated norm of a row of `hv` heads of 128 goes with its projection to the GEMV that holds it in LDS.
+static void gated(uint32_t N, uint32_t hv, bool held) {
+    static char operands[4096];
+    auto at = [&](int i) { return (void*)(((uintptr_t)operands + 255) / 256 * 256 + 256 * i); };
+    g_fail = 0;
+    if (mtq_init(0) != MTQ_OK) return complain("mtq_init");
+    g_held = g_others = 0;
+    g_after_stop = false;
+    if (mtq_gated_rms_norm_qmv(MTQ_BF16, 64, (const float*)at(0), at(1), at(2), (const float*)at(3), at(4), at(5), at(6), at(7), hv, 128, N) != MTQ_OK) complain("gated norm");
+    if (g_held != held || (g_others == 0) != held) complain("gated norm on another kernel");
+    mtq_shutdown();
+}
+
 int main() {
     long n = 0;
+    const struct { uint32_t N, hv; bool held; } lines[] = {
+        {64, 36, true}, {16384, 36, true}, {2048, 40, false}, {2049, 40, true}, {8192, 40, true}, {4096, 42, true}, {4097, 42, false}, {8192, 47, true}, {2048, 47, false}, {512, 50, true},
+        {4096, 56, true}, {4097, 56, false}, {8192, 56, false}, {8193, 56, true}, {2048, 72, false}, {2049, 72, true}, {8193, 72, false}, {512, 16, false},
+    };
+    for (const auto& l : lines) {
+        g_case = "gated norm";
+        gated(l.N, l.hv, l.held);
+        n++;
+    }
     const uint32_t orders[6][3] = {{600, 1100, 300}, {600, 300, 1100}, {1100, 600, 300}, {1100, 300, 600}, {300, 600, 1100}, {300, 1100, 600}};
     for (const auto& N : orders)
         for (int slices : {3, 0})
