@@ -93,8 +93,16 @@ size_t qmv_codes_scratch_bytes(const QmmParams& p, const CodesSplit& s) { return
 //   3968, 992, 992 x 3968, 4 bits   28.6 -> 15.4       28.9 -> 16.8      29.1 -> 21.1      29.5 -> 29.8      29.6 -> 26.6
 // (2 bits as 4, 3 and 6 bits as 5; up to 16 rows 4- and 8-bit codes have the K-run kernel, but for more than 75 M codes: 4736 x 4736, 5 bits, 54.6 -> 14.2.) A
 // matrix's route cannot depend on whether it comes in a batch, and the tile kernels take the matrices of a batch in the time of one
-// as long as they fill the chip together no more than once: three of 5760 x 5760, 4 bits, 20 / 48 rows 39.2 -> 45.2, 40.5 -> 51.1, one of
-// them 39.2 -> 24.1, which a layer has beside the three; at 60 rows 40.9 -> 64.9, so up to 48 rows there.
+// as long as they fill the chip together no more than once; so the lines of square matrices lie where one of them alone and one with the two of an
+// eighth or a quarter of its rows (q8, q4) gain more together than three of them lose (us, tiles -> this):
+//                         alone          q8             q4             three
+//   4 bits,  20 rows, 5760   38.2 -> 18.5                                39.2 -> 45.2     48 rows  39.0 -> 22.1                                40.3 -> 51.0
+//            64 rows, 4992   35.2 -> 21.3   35.2 -> 34.5   35.6 -> 37.5   36.0 -> 40.8     8064     54.0 -> 30.9   54.8 -> 48.0   55.2 -> 54.5   57.1 -> 85.9
+//            72 rows, 4992   34.0 -> 23.8   34.2 -> 37.5   34.4 -> 40.8   35.6 -> 57.0     8064     52.0 -> 35.8   52.5 -> 54.1   52.7 -> 59.8   106 -> 94.8  (neither)
+//   2 bits,  64 rows, 6784   63.2 -> 26.0   61.5 -> 40.9   63.8 -> 48.7   65.5 -> 71.5
+//   3 bits, 128 rows, 4992   52.9 -> 27.3   54.2 -> 44.6   52.9 -> 54.7   56.8 -> 69.1     8064     88.1 -> 55.2   88.9 -> 70.6   88.2 -> 76.3   179 -> 159
+//   5 bits,  96 rows, 6784   84.5 -> 39.2   85.9 -> 59.0   87.0 -> 64.9   173 -> 103
+//   8 bits, 112 rows, 4992   56.8 -> 31.1   55.0 -> 49.0   54.9 -> 62.2   57.2 -> 81.7     8064     92.3 -> 67.6   93.1 -> 81.2   93.4 -> 91.4   187 -> 197
 // Where the tiles split K (rows of a multiple of 256 codes; a matrix of at most half as many tiles of 128 columns as there are compute units) they
 // are the faster: 4096 x 4096, 5 bits, 32 rows 13.1 -> 14.8; 2 x 8192 x 2048, 4 bits, 20 rows 9.7 -> 11.8. Past that pairs of matrices are faster here up to
 // 48 rows, but one of them alone is not, on half the workgroups (us, 6 bits, tiles -> this, 20 and 48 rows):
@@ -111,11 +119,11 @@ size_t qmv_codes_scratch_bytes(const QmmParams& p, const CodesSplit& s) { return
 // 138 -> 66.7; 20 rows 30.9 -> 38.3), 4 bits there at few rows of weights (3584 x 18944, 77 rows 51.1 -> 42.0, 8192 x 28672 88.2 -> 95.0).
 // Groups of 32 cost the tiles nothing and a second scaling per group here: 2- and 4-bit codes are left there on rows of 1152 (1152 x 1152, 20 rows 10.8
 // -> 12.3), bit-stream widths on the smaller long rows (2560 x 10496, 3 bits, 30 rows 17.1 -> 18.8).
-// A matrix of half its row length and less goes by its own times: past 64 rows, where the square ones of its row length stay on the tiles, it is taken
-// from where the tiles need twice its time on, so that what it gains alone is about what a launch of its own costs behind the tiles' of a batch (bits,
+// A matrix of half its row length and less goes by its own times: past 64 rows, where the square 2- and 4-bit ones of its row length stay on the tiles, it is
+// taken from where the tiles need twice its time on, so that what it gains alone is about what a launch of its own costs behind the tiles' of a batch (bits,
 // rows, us, tiles -> this, alone | two next to the square one):
-//   768 x 6528     4  60   40.4 -> 13.6 | 45.8 -> 60.7     8  96   67.5 -> 17.7      1184 x 4736    4  80   29.9 -> 16.5    8  80   49.3 -> 17.4
-//   1632 x 6528    4  80   43.5 -> 17.6 | 44.5 -> 71.8     1792 x 7040  4  60   48.0 -> 15.4 | 49.1 -> 73.4    5  96   82.6 -> 20.2 | 91.3 -> 121
+//   768 x 6528     4  60   40.4 -> 13.6                    8  96   67.5 -> 17.7      1184 x 4736    4  80   29.9 -> 16.5    8  80   49.3 -> 17.4
+//   1632 x 6528    4  80   43.5 -> 17.6 | 44.5 -> 71.8     1792 x 7040  4  60   48.0 -> 15.4                   5  96   82.6 -> 20.2
 //   544 x 2176     4  80   17.6 -> 12.8 | 18.8 -> 31.0     736 x 2944   4  80   21.0 -> 13.5 | 23.6 -> 37.0    (neither is taken:
 //   1056 x 4224    4  80   27.3 -> 15.1 | 30.1 -> 48.8     512 x 1664   8  80   16.4 -> 13.1                    nor are these)
 //   592 x 4736     8  120  41.7 -> 16.0 | 52.5 -> 48.7     (the square one too)
@@ -137,8 +145,8 @@ bool qmv_codes_preferred(int bits, uint32_t G, uint32_t M, uint32_t N, uint32_t 
     if (M <= 16) return stream || (uint64_t)N * K > 75000000ull;
     if (wide) return M <= 64 || (stream || bits == 8 ? K >= 2048 : M <= 96 && K >= 4608);
     if (tall) return M <= (stream ? (K < 2304 || codes > 90000000ull ? 64u : 48u) : bits == 8 ? 48u : 32u);
-    if (M <= 48 || (M <= 64 && K <= 5632)) return true;
-    return (stream || bits == 8) && (M <= 64 || (K >= 2048 && codes <= 40000000ull));
+    if (M <= 48 || (M <= 64 && codes <= 68000000ull)) return true;
+    return (stream || bits == 8) && (M <= 64 || (K >= 2048 && codes <= 68000000ull));
 }
 
 struct CodesReduceArgs {

@@ -102,14 +102,14 @@ bool qmv_held_takes(const QmvParams& p, const QmvBatch& b, const HeldNorm& n) {
 // 2 bits 4096 x 1024 9.6 -> 5.4, 8192 x 8192 14.2 -> 11.7; 3 bits 14720 x 3456 16.3 -> 11.4, 5 bits 20480 x 2560 23.8 -> 14.4, 57344 x 8192 78.8 -> 73.5, 6 bits
 // 131838 x 1408 54.6 -> 37; 8 bits 14336 x 1664 14.2 -> 9.3, 32768 x 4608 38.9 -> 27.8, but 20480 x 5120 23.1 -> 24.3.
 // Heads of more than 65536 rows, of which the GEMV of the others reads 2- to 5-bit codes faster: 70000 / 100000 / 150000 x 3968, 2 bits 31.5 / 39.8 / 53.1 -> 36.7 / 50.7 / 64.3, 3 bits
-// 43 / 56 / 75 -> 46 / 63 / 81, 100000 x 4096, 5 bits 73 -> 79; 100000 x 3328, 2 bits 35.0 -> 38.5, 3584, 3 bits 50.2 -> 52.5; 7168 and 7936, 2 bits 61 and 64 -> 65 and 69, 7936, 3 bits
+// 43 / 56 / 75 -> 46 / 63 / 81, 100000 x 4096, 5 bits 73 -> 79; 100000 x 3328, 2 bits 35.0 -> 38.5, 3584, 3 bits 50.2 -> 52.5; 6656 and 7936, 2 bits 60 and 64 -> 62 and 69, 7936, 3 bits
 // 150000 130 -> 135. Rows of more than 16384 codes leave a compute unit one workgroup, whose second round costs the most there: 5120 x 18944, 5 bits 32.2 -> 36.5, 8192 38.8 -> 38.9;
 // 8192 x 28672, 2 bits 36.0 -> 42.1, 16384 55.5 -> 47.5.
 bool qmv_held_norm_preferred(int bits, uint32_t G, uint32_t N, uint32_t K) {
     if (bits == 8) return K < 5120;
     if (K > 16384 && N > 4096 && N < (K > 20480 ? 16384u : 8192u)) return false;
     if (N > 65536 && K > 3200 && bits != 6) {
-        if (bits == 2 && (K <= 4096 || (K >= 7168 && K < 8192))) return false;
+        if (bits == 2 && (K <= 4096 || (K >= 6656 && K < 8192))) return false;
         if (bits == 3 && ((K > 3456 && K <= 4096) || (K > 7680 && K <= 8192))) return false;
         if (bits == 5 && K > 3968 && K <= 4096) return false;
     }

@@ -277,7 +277,7 @@ def test_k_run_steps_in_pairs(bits, K, paired):
 @pytest.mark.parametrize("bits,G,N,K,held", [
     (4, 64, 256, 2048, False), (4, 64, 1000, 4096, False), (4, 64, 1500, 8192, False), (4, 64, 512, 18432, False), (4, 64, 500, 2304, True), (4, 64, 256, 3072, True), (4, 64, 6000, 3840, True), (4, 64, 6400, 3840, False),
     (4, 64, 70000, 3200, True), (4, 64, 7000, 4224, True), (4, 64, 7000, 4736, True), (4, 64, 7000, 4864, False), (4, 64, 7000, 5248, False), (4, 32, 70000, 1408, True), (4, 32, 70000, 1664, False),
-    (2, 64, 16384, 4096, True), (2, 64, 65536, 4096, True), (2, 64, 65537, 4096, False), (2, 64, 70000, 3200, True), (2, 64, 70000, 6656, True), (2, 64, 70000, 7168, False), (2, 64, 70000, 8192, True),
+    (2, 64, 16384, 4096, True), (2, 64, 65536, 4096, True), (2, 64, 65537, 4096, False), (2, 64, 70000, 3200, True), (2, 64, 70000, 6400, True), (2, 64, 70000, 6656, False), (2, 64, 70000, 8192, True),
     (3, 64, 100000, 3456, True), (3, 64, 100000, 3584, False), (3, 64, 100000, 4224, True), (3, 64, 100000, 7936, False), (5, 64, 100000, 3968, True), (5, 64, 100000, 4096, False), (6, 64, 100000, 4096, True),
     (5, 64, 4096, 18944, True), (5, 64, 5120, 18944, False), (6, 64, 8192, 18944, True), (2, 64, 8192, 28672, False), (2, 64, 16384, 28672, True), (8, 64, 4096, 4992, True), (8, 64, 4096, 5248, False),
 ])
@@ -311,7 +311,8 @@ def test_held_gemv_lines(bits, M, N, K, held):
 
 @pytest.mark.parametrize("bits,G,M,N,K,codes", [
     # rows that the tiles cannot split
-    (5, 64, 16, 4736, 4736, True), (4, 64, 16, 4736, 4736, False), (4, 64, 17, 4736, 4736, True), (4, 64, 64, 5504, 5504, True), (4, 64, 64, 5760, 5760, False),
+    (5, 64, 16, 4736, 4736, True), (4, 64, 16, 4736, 4736, False), (4, 64, 17, 4736, 4736, True), (4, 64, 64, 5504, 5504, True), (4, 64, 64, 5760, 5760, True), (4, 64, 64, 8064, 8064, True), (4, 64, 65, 8064, 8064, False), (4, 64, 64, 8320, 8320, False),
+    (5, 64, 128, 8064, 8064, True), (5, 64, 65, 8320, 8320, False), (5, 64, 64, 8320, 8320, True), (8, 64, 128, 6784, 6784, True),
     (4, 64, 48, 5760, 5760, True), (8, 64, 96, 4736, 4736, True), (5, 64, 128, 4736, 4736, True), (4, 64, 65, 4736, 4736, False), (5, 64, 129, 4736, 4736, False),
     (4, 64, 96, 2304, 8320, True), (4, 64, 97, 2304, 8320, False), (5, 64, 126, 2304, 8320, True), (5, 64, 126, 3584, 12928, False), (5, 64, 96, 3584, 12928, True),   # (split)
     (4, 64, 32, 9472, 2176, True), (4, 64, 33, 9472, 2176, False), (8, 64, 48, 9472, 2176, True), (5, 64, 64, 9472, 2176, True), (5, 64, 65, 9472, 2176, False),
