@@ -265,6 +265,15 @@ def test_k_run_lines_of_few_rows(bits, G, N, K, rows):
     assert on == rows
 
 
+@pytest.mark.parametrize("bits", [4, 5, 8])
+@pytest.mark.parametrize("M,K", [(17, 2176), (24, 2432), (20, 2944), (64, 2944)])
+def test_gemv_on_codes_of_a_layer_is_one_launch(bits, M, K):
+    """Matrices of an eighth, a quarter and all of the rows that a square one has: as many waves that share rows, and no slices."""
+    for N in (K // 8, K // 4, K):
+        _, launches, _, n = ops.plan("qmm", DType.BF16, bits, 64, M, N, K)
+        assert n == 1 and "qmv_codes_kernel" in launches[0][0] and launches[0][2][0] == 512
+
+
 @pytest.mark.parametrize("bits,K,paired", [(4, 1536, False), (4, 1792, True), (4, 1920, False), (4, 2048, True), (4, 2304, False), (4, 2560, True), (4, 4096, True), (4, 4352, False),
                                            (4, 5120, False), (4, 6144, False), (4, 6400, True), (4, 8192, True), (8, 1152, True), (8, 5120, True)])
 def test_k_run_steps_in_pairs(bits, K, paired):
