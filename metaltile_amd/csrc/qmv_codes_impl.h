@@ -303,17 +303,15 @@ template <int DT, int BITS, bool G32, int MT> __global__ __launch_bounds__(QC_WA
                 }
             }
         }
-        if (p % U == U - 1 || it + 1u == iters) {
-            // (the four sums of groups of 64 codes and more begin with the step before; a last step alone has none behind it)
-            constexpr uint32_t back = U == 2 && p % 2 == 1 ? 1u : 0u;
+        if constexpr (p % U == U - 1) {   // (iters is even)
+            constexpr uint32_t back = U - 1;   // the four sums of groups of 64 codes and more begin with the step before
             const unsigned char* const sums = xs0 + (((((it - back) & 7u) + (G32 ? 0u : (q >> 1))) << kwl) + kw) * XSB + (G32 ? q : (q & 1u)) * (ROWS * 4u) + j * 4u;
             float bp[R];
 #pragma unroll
             for (int r = 0; r < R; r++) bp[r] = sbl[(L::SG + (G32 ? p * 4 : (p - (int)back) * 2) + q) * 32u + 16 * r + j];
 #pragma unroll
             for (int t = 0; t < MT; t++) {
-                float xa = *(const float*)(sums + t * 64);
-                if (U == 2 && p % 2 == 0) xa = q < 2u ? xa : 0.f;
+                const float xa = *(const float*)(sums + t * 64);
 #pragma unroll
                 for (int r = 0; r < R; r++) tot[r][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(xa, bp[r], tot[r][t], 0, 0, 0);
             }
