@@ -206,7 +206,8 @@ size_t qmv_slices_scratch_bytes(const QmmParams& p);
 int launch_qmv_slices(const QmmParams& p, const LaunchCtx& lc, void* scratch);
 // GEMV with its activations in LDS (qmv_held.hip): 1..16 activation rows (as many as fit) against 1..4 matrices of one row length, f16 /
 // bf16, codes of 2..6 and 8 bits, K % 128 == 0, groups of 32, 64, 128 (p: dtype, bits, group size, x, M, K). The one row may be
-// RMS-normalised or gated and normalised per head first. A matrix gives the same bits alone and in a batch.
+// RMS-normalised or gated and normalised per head first. A matrix of 2..16 rows gives the same bits alone and in a batch; for one row the waves
+// that share weight rows follow the blocks of all matrices of the call.
 struct HeldNorm {
     int mode = 0;                    // 0 none, 1 RMS norm, 2 gated norm (x: f32 [K], heads of dv)
     const void* weight = nullptr;

@@ -21,7 +21,7 @@
 // Activations go through LDS a step at a time, turned into operand order, two buffers. Weights are loaded with
 // neighbouring lanes on neighbouring 16 bytes of a row (in operand order, 16 rows next to each other, a load occupies the
 // compute unit's address path four times as long), two steps ahead, and turned in an LDS area of the wave's own; rows
-// there are 16 bytes apart from a multiple of 128 so that the operand reads spread over the banks.
+// there are 16 bytes apart from a multiple of 32 (128 at 4 and 8 bits) so that the operand reads spread over the banks.
 // A step of eight waves (256 x 128 codes) takes 1.2 / 1.45 / 1.8 us at 16 / 32 / 48 activation rows: 5.2 TB/s of 6-bit codes at 16 rows, less than half of that of
 // 4-bit codes at 48, where the LDS traffic of operands (98 KB of activations and 48 KB of codes in and out) and the conversion stand beside the MFMAs. us, tiles -> this:
 // 4736 x 20096, 5 bits, 32 rows 263 -> 39; 2 x 8704 x 3968, 8 bits, 40 rows 45.1 -> 34.7 (the table is at qmv_codes_preferred).

@@ -1,6 +1,6 @@
 // The matrix-core GEMV with its activations held in LDS (see qmv_held.hip for the routing and the geometry).
 #pragma once
-// A few activation rows (as many as fit the LDS: one row of up to 28672 codes, 16 of up to 2560) against one or several
+// A few activation rows (as many as fit the LDS: a normalised one of up to 18944 codes, 28672 at 2 bits; 16 of up to 4096) against one or several
 // weight matrices of the same row length: f16 / bf16, codes of 2, 3, 4, 5, 6 and 8 bits, rows of any whole number of 128
 // codes, groups of 32, 64 and 128, the row optionally RMS-normalised or gated and normalised per head first. Exact-dequant
 // arithmetic: out[m][n] = sum_g (s[n][g] * sum_k q[n][k] x[m][k] + b[n][g] * sum_k x[m][k]), the rows of mt_qmv and mt_qmm
