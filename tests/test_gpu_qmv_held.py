@@ -3,7 +3,7 @@ kernels do not take, batches of 2..16 rows of 2-, 3-, 5- and 6-bit codes): the e
 steps of 128 codes over the waves that share them, of its groups and of its stream over several blocks, against the f64-accumulated oracle.
 
 Bound: exact-dequant arithmetic, so what is left is the rounding of the result (2^-8 of it in bf16, 2^-11 in f16), f32 sums, and the
-offset of up to 1024 that the conversion adds to a code and takes out again (2^-24 * 1024 * sqrt(K) * scale (0.1) * |x| (5) = 4e-4 absolute at
+offset of up to 256 that the conversion adds to a code and takes out again (2^-24 * 256 * sqrt(K) * scale (0.1) * |x| (5) = 5e-4 absolute at
 K = 4736). A normalised row keeps 16 significant bits. max |a-e| / max(|e|, 1) <= 1e-2 (bf16), 3e-3 (f16)."""
 import numpy as np
 import pytest
@@ -113,7 +113,8 @@ def test_gated_norm(oracle, held, dt, G, N, hv, dv):
 
 
 @pytest.mark.parametrize("dt", [DType.F16, DType.BF16], ids=lambda d: d.name)
-@pytest.mark.parametrize("bits,G,M,N,K", [(3, 64, 3, 40, 1152), (6, 32, 8, 300, 768), (8, 128, 2, 33, 1280), (2, 64, 16, 20, 512)])
+@pytest.mark.parametrize("bits,G,M,N,K", [(3, 64, 3, 40, 1152), (6, 32, 8, 300, 768), (8, 128, 2, 33, 1280), (2, 64, 16, 20, 512),
+                                          (5, 64, 2, 30000, 384), (2, 32, 4, 20000, 1280)])   # (several blocks to a wave: the next one's weights are asked for again)
 def test_infinite_activations(oracle, held, dt, bits, G, M, N, K):
     """One infinite activation in a row makes its results infinities of the weight's sign, as a product with the weights does;
     the other rows keep their bits."""
@@ -138,6 +139,32 @@ def test_infinite_activations(oracle, held, dt, bits, G, M, N, K):
     rest = [m for m in range(M) if m != 1]
     np.testing.assert_array_equal(got[0][rest], got[1][rest])
     for v in bufs:
+        v.free()
+
+
+@pytest.mark.parametrize("dt", [DType.F16, DType.BF16], ids=lambda d: d.name)
+@pytest.mark.parametrize("bits,G,N,K,what", [(3, 64, 300, 1152, "row"), (5, 32, 9000, 640, "weight"), (4, 128, 40, 2304, "weight")])
+def test_infinities_in_the_norm(dt, bits, G, N, K, what):
+    """An infinite element of the row leaves no finite result, an infinite norm weight one where the matrix's element is 0 at most: the
+    same elements are finite as without this kernel."""
+    print(f"[case] held rms_norm_qmv, infinite {what} {dt.name} b{bits} g{G} N{N} K{K}", flush=True)
+    c = make_case(790 + bits, dt, bits, G, 1, N, K, bias_rule="midpoint")
+    x, nw = c.x_f.reshape(-1).copy(), np.ones(K, np.float32)
+    (x if what == "row" else nw)[K // 3] = np.inf
+    bufs = upload(c) + [GpuBuffer.from_bytes(v) for v in (pack_f32(x, dt), pack_f32(nw, dt), np.float32(1e-5).tobytes())]
+    w, s, b, xb, nb, eb = bufs
+    out, lib, got = GpuBuffer(N * 2), _ensure_init(), []
+    for option in (2, 1):
+        assert lib.mtq_set_option(b"qmv.held", option) == 0
+        try:
+            assert ("qmv_held_kernel" in ops.plan("rms_norm_qmv", dt, bits, G, 1, N, K)[1][0][0]) == (option == 2)
+            ops.rms_norm_qmv(dt, bits, G, xb, nb, w, s, b, out, eb, N, K)
+            got.append(np.isfinite(unpack_f32(out.read_bytes(N * 2), dt)))
+        finally:
+            lib.mtq_set_option(b"qmv.held", 0)
+    assert not got[0].any()
+    np.testing.assert_array_equal(got[0], got[1])
+    for v in bufs + [out]:
         v.free()
 
 
