@@ -98,15 +98,34 @@ bool qmv_held_takes(const QmvParams& p, const QmvBatch& b, const HeldNorm& n) {
 // matrix-core GEMV, from 24 M codes: 14080 x 2304 10.4 -> 9.4, 19200 x 3200 15.9 -> 14.7, 67882 x 2304 26.0 -> 21.3, 25600 x 3328 / 3968 / 4224 / 4608 / 4736 / 4864 / 4992 / 5248 / 5632
 // 14.8 17.1 24.4 22.8 22.0 18.7 22.5 22.2 19.1 -> 15.1 17.7 19.4 19.2 22.4 20.8 23.0 24.1 22.7, 46080 x 4224 / 4736 / 4864 / 4992 34.3 32.6 28.0 33.5 -> 29.9 30.7 28.2 32.0. Rows of whole 2048 codes are
 // the streaming kernel's, which takes them in one launch too: 512 x 2048 4.4 -> 5.2, 1000 x 4096 4.7 -> 6.5, 8192 5.1 -> 10.2, 1500 x 12288 11.3 -> 12.2. 4 bits in groups
-// of 32: 14080 x 2304 11.2 -> 10.1, 86686 x 1280 20.2 -> 18.5, but 86686 x 1664 21.5 -> 24.7.
+// of 32, where each group is scaled for itself: 14080 x 2304 11.2 -> 10.1, 11936 / 25728 x 2176 10.6 / 15.0 -> 10.1 / 13.7, 86686 x 1280 20.2 -> 18.5, but from 24 M codes 15616 / 33648 x 1664
+// 8.2 / 12.8 -> 9.0 / 14.7, 13536 / 29152 x 1920 8.2 / 11.4 -> 9.1 / 12.6, 20832 x 2688 13.2 -> 15.2, 8112 / 17488 x 3200 8.4 / 13.3 -> 9.3 / 17.4, 6144 / 9456 x 4224 9.9 / 11.6 -> 11.0 / 14.4, 86686 x 1664 21.5 -> 24.7.
 // 2 bits 4096 x 1024 9.6 -> 5.4, 8192 x 8192 14.2 -> 11.7; 3 bits 14720 x 3456 16.3 -> 11.4, 5 bits 20480 x 2560 23.8 -> 14.4, 57344 x 8192 78.8 -> 73.5, 6 bits
 // 131838 x 1408 54.6 -> 37; 8 bits 14336 x 1664 14.2 -> 9.3, 32768 x 4608 38.9 -> 27.8, but 20480 x 5120 23.1 -> 24.3.
 // Heads of more than 65536 rows, of which the GEMV of the others reads 2- to 5-bit codes faster: 70000 / 100000 / 150000 x 3968, 2 bits 31.5 / 39.8 / 53.1 -> 36.7 / 50.7 / 64.3, 3 bits
 // 43 / 56 / 75 -> 46 / 63 / 81, 100000 x 4096, 5 bits 73 -> 79; 100000 x 3328, 2 bits 35.0 -> 38.5, 3584, 3 bits 50.2 -> 52.5; 6656 and 7936, 2 bits 60 and 64 -> 62 and 69, 7936, 3 bits
 // 150000 130 -> 135. Rows of more than 16384 codes leave a compute unit one workgroup, whose second round costs the most there: 5120 x 18944, 5 bits 32.2 -> 36.5, 8192 38.8 -> 38.9;
 // 8192 x 28672, 2 bits 36.0 -> 42.1, 16384 55.5 -> 47.5.
+// A workgroup to a compute unit has eight blocks of 16 rows at a time: a head of a few rows more than full rounds of those (32768 rows on 256 units) takes a round more, while the
+// others' time goes with its rows. Up to two fifths of a round into the third or a later one, us, 68000 | 100651 | (full rounds) 131072 rows: 4 bits x 1792 18.0 -> 19.0 | 22.9 -> 25.6 |
+// 27.3 -> 27.0, 1920 21.7 -> 21.8 | 27.5 -> 30.0 | 31.7 -> 31.6, 2688 29.5 -> 30.0 | 38.9 -> 41.3 | 46.4 -> 43.5, 2944 30.5 -> 32.3 | 40.6 -> 44.5 | 47.7 -> 47.2 (but 2816 27.3 -> 26.4 |
+// 35.9 -> 36.1, 3072 27.8 -> 28.2 | 37.7 -> 39.2 | 46.1 -> 40.7, 2432 29.7 -> 26.8 | 39.6 -> 37.3), in groups of 32 x 1152 17.1 -> 18.1 | 21.5 -> 23.8 | 24.8 -> 24.5; groups of 32 at 70000 |
+// 100651 | 131072 rows: 2 bits x 1920 21.2 -> 22.1 | 25.8 -> 29.8 | 29.8 -> 30.9, 2688 29.4 -> 30.5 | 39.0 -> 41.5 | 46.8 -> 43.6, 3 bits x 3200 39.9 -> 43.1 | 52.7 -> 58.8 | 62.7 -> 62.3, 5 bits x
+// 3712 53.1 -> 60.6 | 72.1 -> 81.6 | 90.7 -> 87.9, 6 bits 58.9 -> 62.3 | 79.4 -> 83.2 | 97.2 -> 89.6, 8 bits 54.3 -> 60.5 | 74.3 -> 82.9 | 93.3 -> 87.8. At any number of rows: x 3200, 4 bits 31.2 -> 36.0 | 40.6 -> 49.4 | 48.5 -> 51.5, 2 bits 38.1 -> 40.7 at 100651, 43.0 -> 43.2 at 131072; 4 bits in
+// groups of 32 x 1408 50257 / 78000 / 115000 rows 14.8 19.1 24.8 -> 15.3 20.4 26.8.
+static bool held_norm_short_round(int bits, uint32_t G, uint32_t N, uint32_t K) {
+    const uint32_t round = 128u * held_cus(), over = N % round;
+    if (N <= 2 * round || over == 0 || over * 5 > 2 * round || K > 4096) return false;
+    const bool odd = K % 256 != 0;
+    if (bits == 4 && G == 32) return K > 1024;
+    if (bits == 4 || (bits == 2 && G == 32)) return (K >= 1792 && K < 2048 && (odd || (bits == 4 && G == 64))) || (K > 2560 && odd);
+    return G == 32 && ((bits == 8 && K > 3328) || (odd && ((bits == 3 && K > 2688) || (bits == 5 && K > 2944) || (bits == 6 && K > 3584))));
+}
 bool qmv_held_norm_preferred(int bits, uint32_t G, uint32_t N, uint32_t K) {
+    if (held_norm_short_round(bits, G, N, K)) return false;
     if (bits == 8) return K < 5120;
+    if (N > 65536 && K == 3200 && (bits == 4 || bits == 2)) return false;
+    if (bits == 4 && G == 32 && N > 32768 && K == 1408) return false;
     if (K > 16384 && N > 4096 && N < (K > 20480 ? 16384u : 8192u)) return false;
     if (N > 65536 && K > 3200 && bits != 6) {
         if (bits == 2 && (K <= 4096 || (K >= 6656 && K < 8192))) return false;
@@ -115,8 +134,9 @@ bool qmv_held_norm_preferred(int bits, uint32_t G, uint32_t N, uint32_t K) {
     }
     if (bits != 4) return true;
     if (K % 2048 == 0) return false;
-    if (G == 32 && K > 1600 && (uint64_t)N * K >= 60000000ull) return false;
-    return (uint64_t)N * K < 24000000ull || K <= 3200 || (K > 4096 && K < 5120 && (K <= 4608 || K % 256));
+    const uint64_t codes = (uint64_t)N * K;
+    if (G == 32 && codes >= 24000000ull) return K <= 1600 || (K > 2048 && K <= 2304 && codes < 60000000ull);
+    return codes < 24000000ull || K <= 3200 || (K > 4096 && K < 5120 && (K <= 4608 || K % 256));
 }
 // Gated norm, 4 bits, row lengths that the streaming kernel does not take (norm, GEMV of two rows and sum -> this): 512 / 2560 / 5120 / 16384 rows x 2304 9.3 8.7 10.2 13.2 -> 6.6
 // 6.9 9.2 10.4, x 4608 9.6 10.6 12.8 18.4 -> 9.4 9.8 12.0 14.9. Longer rows take a compute unit's LDS for two workgroups of few waves: 512 / 2048 / 2560 / 4096 / 5120 / 8192 / 12288 rows x

@@ -285,10 +285,16 @@ def test_k_run_steps_in_pairs(bits, K, paired):
 
 @pytest.mark.parametrize("bits,G,N,K,held", [
     (4, 64, 256, 2048, False), (4, 64, 1000, 4096, False), (4, 64, 1500, 8192, False), (4, 64, 512, 18432, False), (4, 64, 500, 2304, True), (4, 64, 256, 3072, True), (4, 64, 6000, 3840, True), (4, 64, 6400, 3840, False),
-    (4, 64, 70000, 3200, True), (4, 64, 7000, 4224, True), (4, 64, 7000, 4736, True), (4, 64, 7000, 4864, False), (4, 64, 7000, 5248, False), (4, 32, 70000, 1408, True), (4, 32, 70000, 1664, False),
-    (2, 64, 16384, 4096, True), (2, 64, 65536, 4096, True), (2, 64, 65537, 4096, False), (2, 64, 70000, 3200, True), (2, 64, 70000, 6400, True), (2, 64, 70000, 6656, False), (2, 64, 70000, 8192, True),
+    (4, 64, 70000, 3200, False), (4, 64, 7000, 4224, True), (4, 64, 7000, 4736, True), (4, 64, 7000, 4864, False), (4, 64, 7000, 5248, False), (4, 32, 30000, 1408, True), (4, 32, 70000, 1664, False),
+    (2, 64, 16384, 4096, True), (2, 64, 65536, 4096, True), (2, 64, 65537, 4096, False), (2, 64, 70000, 3200, False), (2, 64, 70000, 6400, True), (2, 64, 70000, 6656, False), (2, 64, 70000, 8192, True),
     (3, 64, 100000, 3456, True), (3, 64, 100000, 3584, False), (3, 64, 100000, 4224, True), (3, 64, 100000, 7936, False), (5, 64, 100000, 3968, True), (5, 64, 100000, 4096, False), (6, 64, 100000, 4096, True),
     (5, 64, 4096, 18944, True), (5, 64, 5120, 18944, False), (6, 64, 8192, 18944, True), (2, 64, 8192, 28672, False), (2, 64, 16384, 28672, True), (8, 64, 4096, 4992, True), (8, 64, 4096, 5248, False),
+    (4, 64, 65537, 1792, False), (4, 64, 78643, 1792, False), (4, 64, 78644, 1792, True), (4, 64, 98304, 1792, True), (4, 64, 98305, 1792, False), (4, 64, 68000, 1664, True),
+    (4, 128, 68000, 1792, True), (4, 128, 68000, 1920, False), (4, 64, 68000, 2432, True), (4, 64, 68000, 2688, False), (4, 64, 68000, 2816, True), (4, 64, 34000, 2944, True), (4, 64, 68000, 4224, True),
+    (4, 32, 68000, 1024, True), (4, 32, 68000, 1152, False), (4, 32, 60000, 1152, True), (4, 32, 34000, 1408, False), (2, 64, 100651, 2944, True), (2, 32, 100651, 2944, False), (2, 32, 68000, 1792, True),
+    (3, 32, 100651, 2688, True), (3, 32, 100651, 3200, False), (3, 64, 100651, 3200, True), (5, 32, 100651, 3200, False), (5, 32, 131072, 3200, True), (5, 64, 100651, 3200, True), (6, 32, 100651, 3200, True),
+    (6, 32, 100651, 3712, False), (8, 32, 100651, 3200, True), (8, 32, 100651, 3712, False), (8, 32, 131072, 3712, True), (8, 64, 100651, 3712, True), (4, 32, 14000, 1664, True), (4, 32, 14500, 1664, False),
+    (4, 32, 14080, 2176, True), (4, 32, 14080, 2432, False), (4, 32, 5600, 4224, True), (4, 32, 5700, 4224, False),
 ])
 def test_held_norm_lines(bits, G, N, K, held):
     """Which RMS-normalised rows the GEMV with its activations in LDS is for, on both sides of each line."""
