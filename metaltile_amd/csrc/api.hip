@@ -373,7 +373,7 @@ static int run_held(int dtype, int bits, uint32_t G, int n, const void* const* w
         QmvBatch one;
         one.n = 1;
         one.w[0] = w[j]; one.scales[0] = s[j]; one.biases[0] = b[j]; one.out[0] = outs[j]; one.N[0] = N[j];
-        mine[j] = (options().qmv_held == 2 || qmv_held_preferred(bits, M, N[j], K)) && qmv_held_takes(p, one, HeldNorm());
+        mine[j] = (options().qmv_held == 2 || qmv_held_preferred(bits, G, M, N[j], K)) && qmv_held_takes(p, one, HeldNorm());
         if (!mine[j]) { left++; continue; }
         const int i = all.n++;
         all.w[i] = w[j]; all.scales[i] = s[j]; all.biases[i] = b[j]; all.out[i] = outs[j]; all.N[i] = N[j];

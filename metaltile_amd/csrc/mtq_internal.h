@@ -218,7 +218,7 @@ struct HeldNorm {
 bool qmv_held_takes(const QmvParams& p, const QmvBatch& b, const HeldNorm& n);
 bool qmv_held_norm_preferred(int bits, uint32_t G, uint32_t N, uint32_t K);
 bool qmv_held_gated_preferred(uint32_t N, uint32_t K);
-bool qmv_held_preferred(int bits, uint32_t M, uint32_t N, uint32_t K);   // one matrix's sizes
+bool qmv_held_preferred(int bits, uint32_t G, uint32_t M, uint32_t N, uint32_t K);   // one matrix's sizes
 int launch_qmv_held(const QmvParams& p, const QmvBatch& b, const HeldNorm& n, const LaunchCtx& lc);
 // Matrix-core GEMV on codes (qmv_codes.hip): 1..1024 activation rows, f16 / bf16, codes of 2..6 and 8 bits, K % 128 == 0, the matrices of
 // `b` (1..4, same row length) in one launch (p: dtype, bits, group size, x, M, K). A matrix gives the same bits alone and in a batch.

@@ -177,9 +177,36 @@ bool qmv_held_gated_preferred(uint32_t N, uint32_t K) {
 // share evenly: tall matrices of those are left there.)
 // From 9 rows past 8192 weight rows the tiles are ahead (14336 x 4096, 16 rows, 5 bits 18.6 -> 21.3), but at 2 bits; rows of more than 8192 codes leave a
 // compute unit one workgroup: 3 bits, 4 rows 4096 x 11008 11.1 -> 13.4.
-bool qmv_held_preferred(int bits, uint32_t M, uint32_t N, uint32_t K) {
+// In groups of 32 a group is scaled for itself, which costs a wave of up to four rows most on long rows of tall matrices (alone | two):
+//   2 rows  2 bits 12032 x 6016 10.4 -> 15.2 | 20.5 -> 20.0, 20480 x 5120 14.4 -> 17.0 | 28.1 -> 26.5    3 bits 16384 x 8192 19.8 -> 21.9 | 39.5 -> 39.9    6 bits 28672 x 8192 41.6 -> 47.1 | 83.3 -> 79.5
+//   4 rows  5 bits 18432 x 5120 23.1 -> 30.7 | 45.7 -> 44.6, x 6016 24.0 -> 35.6 | 47.7 -> 52.8    6 bits 18432 x 5120 24.4 -> 30.2 | 48.4 -> 44.2, 16384 x 8192 28.0 -> 35.8 | 55.7 -> 54.1 (none taken)
+//           5 bits 24576 x 5120 27.3 -> 31.6 | 54.1 -> 47.8    6 bits 28672 x 5120 32.3 -> 32.5 | 64.4 -> 58.8    2 bits 16384 x 8192 19.4 -> 20.0 | 39.2 -> 34.2, square and nearly square ones: 5 bits
+//           6016 x 6016 12.7 -> 13.6 | q 26.4 -> 16.8 (taken). Groups of 64, 5 bits: 18432 x 6016 26.2 -> 31.7 | 52.2 -> 47.3 (not)
+// A head has no other beside it and goes by its own times (68000 | 100651 | 131072 rows):
+//   2 rows  2 bits x 3328 23.9 30.5 36.0 -> 26.1 36.2 45.3, x 4096 24.6 32.3 39.7 -> 27.3 38.4 48.6, x 7168 40.1 54.7 70.5 -> 46.7 65.8 83.5, but x 2944 25.6 33.1 -> 23.8 32.6, x 5120 37.1 52.2 66.0 ->
+//           34.6 49.9 61.1    3 bits x 4096 35.0 48.0 55.6 -> 35.0 48.8 60.5, x 6144 47.2 68.7 89.7 -> 50.8 73.6 90.8, x 8192 61.6 87.7 112.1 -> 67.9 97.4 120.2, but x 5120 47.0 67.0 86.6 -> 45.0 63.1 78.7
+//           groups of 32, at 100651: 2 bits x 1536 / 2944 / 4096 / 5120 21.2 34.5 40.8 51.7 -> 26.8 39.2 46.1 59.2, 3 bits x 1536 / 2048 / 4096 27.4 29.2 50.3 -> 29.8 31.8 55.5, but x 2944 47.0 -> 46.0
+//   8 rows  3 bits x 8192 90.3 140.9 173.9 -> 100.7 146.4 185.1    5 bits x 4096 51.1 70.9 89.5 -> 55.0 77.2 89.3, 34000 rows 30.6 -> 34.2, but x 3584 49.8 69.9 88.5 -> 49.4 68.0 78.9
+//           groups of 32 x 2048, 34000 / 68000 rows: 5 bits 19.2 31.1 -> 22.1 34.7, 6 bits 19.9 31.9 -> 21.8 33.6, but x 1664 18.7 29.3 -> 17.6 27.4
+static bool held_head_slower(int bits, uint32_t G, uint32_t M, uint32_t N, uint32_t K) {
+    if (N <= 32768) return false;
+    const bool most = N > 65536, mid = K > 3072 && K <= 4096;
+    if (M > 4) return G == 32 ? bits >= 5 && K == 2048 : (bits == 5 && K > 3840 && K <= 4096) || (bits == 3 && most && K > 7168);
+    if (bits == 2) return G == 32 ? most || K > 2048 : most && (mid || (K > 6144 && K < 8192));
+    if (bits != 3 || !most) return false;
+    return G == 32 ? K <= 2048 || mid : (M == 2 && K > 5120) || (N > 98304 && K > 3584 && K <= 4096);
+}
+bool qmv_held_preferred(int bits, uint32_t G, uint32_t M, uint32_t N, uint32_t K) {
     if (M < 2 || M > 16 || bits == 4 || bits == 8) return false;
     const bool tall = N >= 2 * (uint64_t)K;
+    if (held_head_slower(bits, G, M, N, K)) return false;
+    if (G == 32 && M <= 4) {
+        const bool fewer = bits == 2 ? M == 2 && N > 16384 : bits == 3 ? M == 2 : M > 2 || N > 16384;
+        if (K > 5120 && 2 * (uint64_t)N > 3 * (uint64_t)K && (K % 2048 || fewer)) return false;
+        if (K > 4608 && K <= 5120 && N > 16384 && N <= 20480 && (bits >= 5 ? M > 2 : bits == 2 && M == 2)) return false;
+    } else if (bits == 5 && (M == 3 || M == 4) && K > 5632 && N > 16384 && N <= 20480) {
+        return false;
+    }
     if (M > 8) return K <= 4096 && (N <= 8192 || (bits == 2 && (M <= 12 || K <= 3328))) && !(bits != 6 && K <= 1024 && N > 4096);
     if (K > 8192) return false;
     if (bits == 5 && M <= 4 && tall && K % 2048 == 0) return false;

@@ -324,6 +324,24 @@ def test_held_gemv_lines(bits, M, N, K, held):
     assert rc == 0 and ("qmv_held_kernel" in launches[0][0]) == held, launches[0][0]
 
 
+@pytest.mark.parametrize("bits,G,M,N,K,held", [
+    # groups of 32, long rows of tall matrices
+    (2, 32, 2, 8960, 6016, True), (2, 32, 2, 9040, 6016, False), (2, 32, 4, 12032, 6016, False), (2, 32, 8, 12032, 6016, True), (2, 64, 4, 12032, 6016, True), (2, 32, 2, 16384, 5120, True), (2, 32, 2, 20480, 5120, False),
+    (2, 32, 4, 20480, 5120, True), (2, 32, 4, 16384, 8192, True), (3, 32, 2, 16384, 8192, False), (3, 32, 4, 16384, 8192, True), (6, 32, 2, 16384, 8192, True), (6, 32, 2, 28672, 8192, False),
+    (6, 32, 4, 16384, 8192, False), (5, 32, 4, 20480, 5120, False), (5, 32, 4, 20481, 5120, True), (6, 32, 2, 20480, 5120, True), (5, 64, 4, 18432, 6016, False), (5, 64, 4, 18432, 5632, True), (5, 64, 2, 18432, 6016, True),
+    # heads
+    (2, 64, 2, 65536, 4096, True), (2, 64, 2, 65537, 4096, False), (2, 64, 4, 68000, 3072, True), (2, 64, 4, 68000, 3328, False), (2, 64, 4, 68000, 4224, True), (2, 64, 4, 68000, 7168, False),
+    (2, 64, 8, 68000, 4096, True), (2, 32, 4, 34000, 2048, True), (2, 32, 4, 34000, 2944, False), (2, 32, 4, 68000, 1536, False), (3, 64, 2, 68000, 5120, True), (3, 64, 2, 68000, 5248, False),
+    (3, 64, 3, 68000, 5248, True), (3, 64, 2, 98304, 4096, True), (3, 64, 2, 98305, 4096, False), (3, 32, 2, 68000, 2048, False), (3, 32, 2, 68000, 2944, True), (3, 32, 2, 65536, 2048, True),
+    (3, 64, 8, 68000, 8192, False), (3, 64, 8, 65536, 8192, True), (5, 64, 8, 32768, 4096, True), (5, 64, 8, 32769, 4096, False), (5, 64, 8, 34000, 3840, True), (5, 32, 8, 34000, 2048, False), (5, 32, 8, 34000, 1664, True),
+    (6, 64, 4, 100651, 4096, True),
+])
+def test_held_gemv_lines_of_heads_and_groups_of_32(bits, G, M, N, K, held):
+    """Heads, which come alone, and groups of 32, on both sides of each line."""
+    rc, launches, _, _ = ops.plan("qmm", DType.BF16, bits, G, M, N, K)
+    assert rc == 0 and ("qmv_held_kernel" in launches[0][0]) == held, launches[0][0]
+
+
 @pytest.mark.parametrize("bits,G,M,N,K,codes", [
     # rows that the tiles cannot split
     (5, 64, 16, 4736, 4736, True), (4, 64, 16, 4736, 4736, False), (4, 64, 17, 4736, 4736, True), (4, 64, 64, 5504, 5504, True), (4, 64, 64, 5760, 5760, True), (4, 64, 64, 8064, 8064, True), (4, 64, 65, 8064, 8064, False), (4, 64, 64, 8320, 8320, False),
