@@ -122,14 +122,13 @@ size_t qmv_codes_scratch_bytes(const QmmParams& p, const CodesSplit& s) { return
 // 138 -> 66.7; 20 rows 30.9 -> 38.3), 4 bits there at few rows of weights (3584 x 18944, 77 rows 51.1 -> 42.0, 8192 x 28672 88.2 -> 95.0).
 // Groups of 32 cost the tiles nothing and a second scaling per group here: 2- and 4-bit codes are left there on rows of 1152 (1152 x 1152, 20 rows 10.8
 // -> 12.3), bit-stream widths on the smaller long rows (2560 x 10496, 3 bits, 30 rows 17.1 -> 18.8).
-// A matrix of half its row length and less goes by its own times: past 64 rows, where the square 2- and 4-bit ones of its row length stay on the tiles, it is
-// taken from where the tiles need twice its time on, so that what it gains alone is about what a launch of its own costs behind the tiles' of a batch (bits,
-// rows, us, tiles -> this, alone | two next to the square one):
-//   768 x 6528     4  60   40.4 -> 13.6                    8  96   67.5 -> 17.7      1184 x 4736    4  80   29.9 -> 16.5    8  80   49.3 -> 17.4
-//   1632 x 6528    4  80   43.5 -> 17.6 | 44.5 -> 71.8     1792 x 7040  4  60   48.0 -> 15.4                   5  96   82.6 -> 20.2
-//   544 x 2176     4  80   17.6 -> 12.8 | 18.8 -> 31.0     736 x 2944   4  80   21.0 -> 13.5 | 23.6 -> 37.0    (neither is taken:
-//   1056 x 4224    4  80   27.3 -> 15.1 | 30.1 -> 48.8     512 x 1664   8  80   16.4 -> 13.1                    nor are these)
-//   592 x 4736     8  120  41.7 -> 16.0 | 52.5 -> 48.7     (the square one too)
+// A matrix of half its row length and less goes by its own times. Past 64 rows, where the square 2- and 4-bit ones of its row length stay on the tiles, two of them are worked
+// out beside the square one's tiles for nothing, and here cost what one alone gains: of a quarter of its row length and less they stay on the tiles, which larger
+// ones leave where the tiles need twice the time (bits, rows, us, tiles -> this, alone | two next to the square one):
+//   768 x 6528     4  60   40.4 -> 13.6                    8  96   67.5 -> 17.7      1184 x 4736    8  80   49.3 -> 17.4
+//   592 x 4736     8  120  41.7 -> 16.0 | 52.5 -> 48.7 (the square one too)                1792 x 7040  4  60   48.0 -> 15.4    5  96   82.6 -> 20.2
+// and not taken: 1632 x 6528, 4 bits, 80 rows 43.5 -> 17.6 | 44.5 -> 71.8 (a layer of 7296 with 896 for keys and values, 71 rows, 397 -> 417), 1056 x 4224 27.3 -> 15.1 | 30.1 -> 48.8,
+// 544 x 2176 17.6 -> 12.8 | 18.8 -> 31.0, 736 x 2944 21.0 -> 13.5 | 23.6 -> 37.0, 1184 x 4736 29.9 -> 16.5; 512 x 1664, 8 bits 16.4 -> 13.1.
 bool qmv_codes_preferred(int bits, uint32_t G, uint32_t M, uint32_t N, uint32_t K) {
     const bool stream = bits == 3 || bits == 5 || bits == 6, tall = N >= 2 * (uint64_t)K, wide = K >= 2 * (uint64_t)N, g32 = G == 32 && !stream && bits != 8;
     const uint64_t codes = (uint64_t)N * K;
@@ -146,7 +145,7 @@ bool qmv_codes_preferred(int bits, uint32_t G, uint32_t M, uint32_t N, uint32_t 
         return tiles * 5 >= rounds * cus * 4 ? stream || K >= 8192 || N > 65536 : stream && rounds == 1;
     }
     if (M <= 16) return stream || (uint64_t)N * K > 75000000ull;
-    if (wide) return M <= 64 || (stream || bits == 8 ? K >= 2048 : M <= 96 && K >= 4608);
+    if (wide) return M <= 64 || (stream || bits == 8 ? K >= 2048 : M <= 96 && K >= 4608 && (K > 8192 ? 5 : 4) * (uint64_t)N > K);
     if (tall) return M <= (stream ? (K < 2304 || codes > 90000000ull ? 64u : 48u) : bits == 8 ? 48u : 32u);
     if (M <= 48 || (M <= 64 && codes <= 68000000ull)) return true;
     return (stream || bits == 8) && (M <= 64 || (K >= 2048 && codes <= 68000000ull));

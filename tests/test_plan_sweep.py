@@ -352,7 +352,7 @@ def test_held_gemv_lines_of_heads_and_groups_of_32(bits, G, M, N, K, held):
     (4, 64, 60, 768, 6528, True), (4, 64, 60, 768, 4736, True), (2, 128, 72, 512, 1152, False), (4, 32, 20, 1152, 1152, False), (4, 64, 20, 1152, 1152, True),
     # few weight rows, past 64 activation rows
     (4, 64, 60, 1792, 7040, True), (4, 64, 96, 1792, 7040, True), (8, 64, 96, 1792, 7040, True), (4, 64, 64, 512, 1664, True), (4, 64, 65, 512, 1664, False),
-    (4, 64, 65, 1120, 4480, False), (4, 64, 65, 1184, 4736, True), (8, 64, 65, 512, 1920, False), (8, 64, 65, 512, 2176, True), (5, 64, 128, 1792, 7040, True), (5, 64, 65, 256, 1664, False),
+    (4, 64, 65, 1120, 4480, False), (4, 64, 65, 1184, 4736, False), (4, 64, 65, 1185, 4736, True), (4, 64, 71, 896, 7296, False), (4, 64, 65, 2176, 8320, True), (4, 64, 65, 2048, 8320, True), (4, 64, 65, 1664, 8320, False), (8, 64, 65, 512, 1920, False), (8, 64, 65, 512, 2176, True), (5, 64, 128, 1792, 7040, True), (5, 64, 65, 256, 1664, False),
     (8, 64, 128, 1024, 6528, True), (4, 64, 97, 1792, 7040, False),
     # rows that they can
     (5, 64, 32, 4096, 4096, False), (6, 64, 20, 8192, 2048, False), (6, 64, 20, 16384, 4096, False), (6, 64, 17, 18944, 3584, True), (6, 64, 48, 18944, 3584, True),
