@@ -124,19 +124,18 @@ static bool held_norm_short_round(int bits, uint32_t G, uint32_t N, uint32_t K) 
 bool qmv_held_norm_preferred(int bits, uint32_t G, uint32_t N, uint32_t K) {
     if (held_norm_short_round(bits, G, N, K)) return false;
     if (bits == 8) return K < 5120;
-    if (N > 65536 && K == 3200 && (bits == 4 || bits == 2)) return false;
-    if (bits == 4 && G == 32 && N > 32768 && K == 1408) return false;
     if (K > 16384 && N > 4096 && N < (K > 20480 ? 16384u : 8192u)) return false;
-    if (N > 65536 && K > 3200 && bits != 6) {
-        if (bits == 2 && (K <= 4096 || (K >= 6656 && K < 8192))) return false;
+    if (N > 65536) {
+        if (bits == 2 && ((K > 3072 && K <= 4096) || (K >= 6656 && K < 8192))) return false;
         if (bits == 3 && ((K > 3456 && K <= 4096) || (K > 7680 && K <= 8192))) return false;
         if (bits == 5 && K > 3968 && K <= 4096) return false;
     }
     if (bits != 4) return true;
     if (K % 2048 == 0) return false;
     const uint64_t codes = (uint64_t)N * K;
-    if (G == 32 && codes >= 24000000ull) return K <= 1600 || (K > 2048 && K <= 2304 && codes < 60000000ull);
-    return codes < 24000000ull || K <= 3200 || (K > 4096 && K < 5120 && (K <= 4608 || K % 256));
+    if (codes < 24000000ull) return true;
+    if (G == 32) return K <= (N > 32768 && K % 256 ? 1280 : 1600) || (K > 2048 && K <= 2304 && codes < 60000000ull);
+    return K <= (N > 65536 ? 3072 : 3200) || (K > 4096 && K < 5120 && (K <= 4608 || K % 256));
 }
 // Gated norm, 4 bits, row lengths that the streaming kernel does not take (norm, GEMV of two rows and sum -> this): 512 / 2560 / 5120 / 16384 rows x 2304 9.3 8.7 10.2 13.2 -> 6.6
 // 6.9 9.2 10.4, x 4608 9.6 10.6 12.8 18.4 -> 9.4 9.8 12.0 14.9. Longer rows take a compute unit's LDS for two workgroups of few waves: 512 / 2048 / 2560 / 4096 / 5120 / 8192 / 12288 rows x
