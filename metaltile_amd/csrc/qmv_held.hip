@@ -114,12 +114,13 @@ bool qmv_held_takes(const QmvParams& p, const QmvBatch& b, const HeldNorm& n) {
 // 3712 53.1 -> 60.6 | 72.1 -> 81.6 | 90.7 -> 87.9, 6 bits 58.9 -> 62.3 | 79.4 -> 83.2 | 97.2 -> 89.6, 8 bits 54.3 -> 60.5 | 74.3 -> 82.9 | 93.3 -> 87.8. At any number of rows: x 3200, 4 bits 31.2 -> 36.0 | 40.6 -> 49.4 | 48.5 -> 51.5, 2 bits 38.1 -> 40.7 at 100651, 43.0 -> 43.2 at 131072; 4 bits in
 // groups of 32 x 1408 50257 / 78000 / 115000 rows 14.8 19.1 24.8 -> 15.3 20.4 26.8.
 static bool held_norm_short_round(int bits, uint32_t G, uint32_t N, uint32_t K) {
-    const uint32_t round = 128u * held_cus(), over = N % round;
-    if (N <= 2 * round || over == 0 || over * 5 > 2 * round || K > 4096) return false;
     const bool odd = K % 256 != 0;
-    if (bits == 4 && G == 32) return K > 1024;
-    if (bits == 4 || (bits == 2 && G == 32)) return (K >= 1792 && K < 2048 && (odd || (bits == 4 && G == 64))) || (K > 2560 && odd);
-    return G == 32 && ((bits == 8 && K > 3328) || (odd && ((bits == 3 && K > 2688) || (bits == 5 && K > 2944) || (bits == 6 && K > 3584))));
+    const bool row = bits == 4 && G == 32                  ? K > 1024
+                     : bits == 4 || (bits == 2 && G == 32) ? (K >= 1792 && K < 2048 && (odd || (bits == 4 && G == 64))) || (K > 2560 && odd)
+                                                           : G == 32 && ((bits == 8 && K > 3328) || (odd && ((bits == 3 && K > 2688) || (bits == 5 && K > 2944) || (bits == 6 && K > 3584))));
+    if (!row || K > 4096) return false;   // (first: most calls need not ask the device)
+    const uint32_t round = 128u * held_cus(), over = N % round;
+    return N > 2 * round && over != 0 && over * 5 <= 2 * round;
 }
 bool qmv_held_norm_preferred(int bits, uint32_t G, uint32_t N, uint32_t K) {
     if (held_norm_short_round(bits, G, N, K)) return false;
